@@ -960,130 +960,175 @@ __global__ __launch_bounds__(256) void dequant_native(half_t *__restrict__ out, 
     }
 }
 
-// Writes the 64 codes of one lane (c[8*s + j] = code of its row at column 32*s + 8*q + j of the K block) as the lane's
-// 12 (6-bit formats), 10 (FP5) or 8 (FP4) dwords of a native block.
-template <int FM> __device__ __forceinline__ void store_native_lane(const uint8_t (&c)[64], uint8_t *dst, int lane)
+// Writes one lane's two 192-bit strings of 6-bit fields (MFMA steps 0..3 and 4..7 of a K block, in the order the conversion
+// instruction reads them) into a native block: 12 (6-bit formats), 10 (FP5) or 8 (FP4) dwords at the places of lane `slot`.
+// FP5 and FP4 park the payload bits of the last one or two dwords of a string in the fixed-zero bits of the others.  The stores
+// leave the caches to what the quantizer reads twice (5-12 % off it at 4096x4096 and 8192x28672).
+template <int FM> __device__ __forceinline__ void store_native_strings(v6u s0, v6u s1, uint8_t *dst, int slot)
 {
-    if (Fmt<FM>::bits == 6) {
-        uint32_t d[12];
-        for (int h = 0; h < 2; h++) {
-            uint64_t accb = 0;
-            int      nb = 0, w = 0;
-            for (int i = 0; i < 32; i++) {
-                accb |= (uint64_t)c[32 * h + i] << nb;
-                nb += 6;
-                if (nb >= 32) { d[6 * h + w++] = (uint32_t)accb; accb >>= 32; nb -= 32; }
-            }
-        }
-        for (int i = 0; i < 3; i++) {
-            v4u v = { d[4 * i], d[4 * i + 1], d[4 * i + 2], d[4 * i + 3] };
-            reinterpret_cast<v4u *>(dst)[i * 64 + lane] = v;
-        }
-    } else if (Fmt<FM>::bits == 4) {
-        constexpr uint32_t P = 0xC30C30C3u, Q = 0x30C30C30u, R = 0x0C30C30Cu;
-        for (int h = 0; h < 2; h++) {
-            uint32_t D[6];
-            uint64_t accb = 0;
-            int      nb = 0, w = 0;
-            for (int i = 0; i < 32; i++) {
-                accb |= (uint64_t)((c[32 * h + i] & 15u) << 2) << nb;
-                nb += 6;
-                if (nb >= 32) { D[w++] = (uint32_t)accb; accb >>= 32; nb -= 32; }
-            }
-            v4u v = { D[0] | (D[4] & P), D[1] | (D[5] & Q), D[2] | (D[4] & R), D[3] | (D[5] & P) };
-            reinterpret_cast<v4u *>(dst)[h * 64 + lane] = v;
-        }
-    } else {
+    v4u *d4 = reinterpret_cast<v4u *>(dst) + slot;
+    if constexpr (Fmt<FM>::bits == 6) {
+        __builtin_nontemporal_store((v4u){ s0[0], s0[1], s0[2], s0[3] }, d4);
+        __builtin_nontemporal_store((v4u){ s0[4], s0[5], s1[0], s1[1] }, d4 + 64);
+        __builtin_nontemporal_store((v4u){ s1[2], s1[3], s1[4], s1[5] }, d4 + 128);
+    } else if constexpr (Fmt<FM>::bits == 5) {
         constexpr uint32_t A = 0x10410410u, B = 0x04104104u, C = 0x41041041u;
-        uint32_t           S[2][5];
-        for (int h = 0; h < 2; h++) {
-            uint32_t D[6];
-            uint64_t accb = 0;
-            int      nb = 0, w = 0;
-            for (int i = 0; i < 32; i++) {
-                uint32_t code = c[32 * h + i], field = (code & 15u) | (((code >> 4) & 1u) << 5);
-                accb |= (uint64_t)field << nb;
-                nb += 6;
-                if (nb >= 32) { D[w++] = (uint32_t)accb; accb >>= 32; nb -= 32; }
-            }
-            S[h][0] = D[0] | (D[5] & A);
-            S[h][1] = D[1] | (D[5] & B);
-            S[h][2] = D[2] | ((D[5] >> 1) & C);
-            S[h][3] = D[3] | ((D[5] >> 1) & A);
-            S[h][4] = D[4] | ((D[5] >> 1) & B);
-        }
-        for (int h = 0; h < 2; h++) {
-            v4u v = { S[h][0], S[h][1], S[h][2], S[h][3] };
-            reinterpret_cast<v4u *>(dst)[h * 64 + lane] = v;
-        }
-        v2u sv = { S[0][4], S[1][4] };
-        reinterpret_cast<v2u *>(dst + 2048)[lane] = sv;
+        auto fold = [&](v6u D) { return (v4u){ D[0] | (D[5] & A), D[1] | (D[5] & B), D[2] | ((D[5] >> 1) & C), D[3] | ((D[5] >> 1) & A) }; };
+        __builtin_nontemporal_store(fold(s0), d4);
+        __builtin_nontemporal_store(fold(s1), d4 + 64);
+        __builtin_nontemporal_store((v2u){ s0[4] | ((s0[5] >> 1) & B), s1[4] | ((s1[5] >> 1) & B) }, reinterpret_cast<v2u *>(dst + 2048) + slot);
+    } else {
+        constexpr uint32_t P = 0xC30C30C3u, Q = 0x30C30C30u, R = 0x0C30C30Cu;
+        auto fold = [&](v6u D) { return (v4u){ D[0] | (D[4] & P), D[1] | (D[5] & Q), D[2] | (D[4] & R), D[3] | (D[5] & P) }; };
+        __builtin_nontemporal_store(fold(s0), d4);
+        __builtin_nontemporal_store(fold(s1), d4 + 64);
     }
 }
 
-// Reference layout -> native layout on the device.  One thread per (row tile, K block, lane): it gathers its 64
-// codes bit piece by bit piece from the reference's segment arrays and writes its 8, 10 or 12 native dwords.
-__constant__ uint8_t kInvOrder4[8]  = { 4, 0, 6, 2, 5, 1, 7, 3 };
-__constant__ uint8_t kInvOrder2[16] = { 8, 0, 12, 4, 9, 1, 13, 5, 10, 2, 14, 6, 11, 3, 15, 7 };
-
+// Reference layout -> native layout on the device, HBM-bound (reads and writes the weight bytes once).  One workgroup per 64-row
+// tile of the reference and K block of 256 columns, one wavefront per 16-row block of the tile; lane = (m = l%16, q = l/16) as in
+// the GEMM.  The segment words of a (16 rows x 16 columns) piece are 32 consecutive ones, word 4*(m%8) + t holding columns 2t,
+// 2t+1, 2t+8, 2t+9 of rows m%8 and m%8 + 8.  So the eight columns 8q'..8q'+7 that a lane needs of a piece for one MFMA step are
+// the four words from 4*(m%8) on, one 16-byte load per segment array (a quarter-wavefront reads one 128-byte line), and in each word its two
+// codes sit 16 bits apart at a position that depends on the lane alone: a shift and a mask bring both out at once.  The whole block
+// is in flight before the first use.  11008x4096 FP6: 12.0 us = 5.6 TB/s read + written, where one bit piece per load, a byte array per
+// lane in scratch memory and a loop over its 64 codes took 266 us.
 template <int FM>
 __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restrict__ native, const uint8_t *__restrict__ ref,
                                                              uint32_t M, uint32_t K, uint32_t units)
 {
-    const int      lane = threadIdx.x & 63;
-    const uint32_t blk = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (blk >= (M / 16) * units) return;
-    const uint32_t R = blk / units, U = blk % units;
-    const int      m = lane & 15, q = lane >> 4;
-    const uint32_t row = R * 16 + m, tile = row >> 6, block = (row >> 4) & 3, rin = row & 15, g = rin & 7, rowhalf = rin >> 3;
     // segment arrays: 6 bits = [2-bit | 4-bit], 5 bits = [1-bit | 4-bit], 4 bits = [4-bit]
-    constexpr int   bits = Fmt<FM>::bits;
-    const uint32_t *seg_hi = reinterpret_cast<const uint32_t *>(ref);
-    const uint32_t *seg4   = reinterpret_cast<const uint32_t *>(ref + (size_t)M * K * (bits - 4) / 8);
-    uint8_t         c[64];
-#pragma unroll 1
+    constexpr int  bits = Fmt<FM>::bits, kHiWords = bits == 6 ? 64 : 32; // words of the high segment per 64-row tile and 16 columns
+    const int      lane = threadIdx.x & 63, m = lane & 15, q = lane >> 4;
+    const uint32_t block = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tile = blockIdx.x / units, U = blockIdx.x % units, g = m & 7, rowhalf = m >> 3;
+    const uint32_t slices = K >> 4;
+    const uint32_t *seg_hi = reinterpret_cast<const uint32_t *>(ref) + (size_t)tile * slices * kHiWords + (bits == 6 ? (block >> 1) * 32 : 0) + 4 * g;
+    const uint32_t *seg4   = reinterpret_cast<const uint32_t *>(ref + (size_t)M * K * (bits - 4) / 8) + (size_t)tile * slices * 128 + block * 32 + 4 * g;
+
+    v4u lo[8], hi[8];
+#pragma unroll
     for (int s = 0; s < 8; s++) {
-        uint32_t k0 = U * 256 + 32 * s + 8 * q;
-        for (int j = 0; j < 8; j++) {
-            uint32_t col = k0 + j, code = 0;
-            if (col < K) {
-                uint32_t slice = col >> 4, cc = col & 15, t = (cc & 7) >> 1;
-                uint32_t el = (cc & 1) | (rowhalf << 1) | ((cc >> 3) << 2);
-                uint32_t l32 = 4 * g + t;
-                { // 4-bit piece: q4 = block, pre = el
-                    uint32_t word = seg4[((size_t)(tile * (K / 16) + slice) * 4 + block) * 32 + l32];
-                    code |= (word >> (28 - 4 * kInvOrder4[el])) & 15u;
-                }
-                if (bits == 6) { // 2-bit piece: q2 = block/2, pre = (block%2)*8 + el
-                    uint32_t word = seg_hi[((size_t)(tile * (K / 16) + slice) * 2 + (block >> 1)) * 32 + l32];
-                    code |= ((word >> (30 - 2 * kInvOrder2[(block & 1) * 8 + el])) & 3u) << 4;
-                } else if (bits == 5) { // 1-bit piece: q1 = 0, pre = block*8 + el; order_1 maps p -> pre, inverted arithmetically:
-                    // order_1[p]-1 = 4*(p%8) + {1,3,0,2}[p/8]  =>  p = 8*{2,0,3,1}[pre%4] + pre/4
-                    uint32_t pre = block * 8 + el;
-                    uint32_t p   = 8 * ((0x1302u >> (4 * (pre & 3))) & 3u) + (pre >> 2);
-                    uint32_t word = seg_hi[((size_t)(tile * (K / 16) + slice)) * 32 + l32];
-                    code |= ((word >> (31 - p)) & 1u) << 4;
-                }
+        const uint32_t slice = U * 16 + 2 * s + (q >> 1); // K is a multiple of 64: a 16-column piece lies inside K or beyond it
+        const bool     in = slice < slices;
+        lo[s] = in ? *reinterpret_cast<const v4u *>(seg4 + (size_t)slice * 128) : (v4u){ 0u, 0u, 0u, 0u };
+        if constexpr (bits != 4) hi[s] = in ? *reinterpret_cast<const v4u *>(seg_hi + (size_t)slice * kHiWords) : (v4u){ 0u, 0u, 0u, 0u };
+    }
+    // positions inside a word of the code at the even column (the odd column's is 16 bits above); e = index of the pair among the
+    // four pairs (row half, column half) of a word
+    const uint32_t e = rowhalf + 2 * (q & 1);
+    const uint32_t sh4 = (0x048Cu >> (4 * ((e & 1) * 2 + (e >> 1)))) & 15u; // e = 0, 1, 2, 3: 12, 4, 8, 0
+    uint32_t       sh_hi = 0;
+    if constexpr (bits == 6) { // 2-bit fields from the top of the word: field 8, 12, 9, 13, 10, 14, 11, 15 for pair 4*(block%2) + e
+        const uint32_t pair = (block & 1) * 4 + e;
+        sh_hi = 30 - 2 * (8 + (pair >> 1) + 4 * (pair & 1));
+    }
+    if constexpr (bits == 5) // bits from the top of the word: bit 16 or 24, plus 2*block + column half
+        sh_hi = 31 - (16 + 8 * rowhalf + 2 * block + (q & 1));
+
+    v6u str[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        uint32_t p[16]; // pairs of 6-bit fields
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                uint32_t c = (lo[4 * h + s][t] >> sh4) & 0x000F000Fu; // two codes (their low four bits), 16 bits apart
+                if constexpr (bits == 6) c |= ((hi[4 * h + s][t] >> sh_hi) & 0x00030003u) << 4;
+                if constexpr (bits == 5) c |= ((hi[4 * h + s][t] >> sh_hi) & 0x00010001u) << 5; // the fixed-zero bit goes in above the exponent
+                if constexpr (bits == 4) c <<= 2;                                               // and here two below the mantissa
+                p[4 * s + t] = (c | (c >> 10)) & 0xFFFu;
             }
-            c[8 * s + j] = (uint8_t)code;
+#pragma unroll
+        for (int k = 0; k < 2; k++) { // eight pairs = three dwords
+            const uint32_t *v = p + 8 * k;
+            str[h][3 * k]     = v[0] | v[1] << 12 | v[2] << 24;
+            str[h][3 * k + 1] = v[2] >> 8 | v[3] << 4 | v[4] << 16 | v[5] << 28;
+            str[h][3 * k + 2] = v[5] >> 4 | v[6] << 8 | v[7] << 20;
         }
     }
-    store_native_lane<FM>(c, native + (size_t)blk * Fmt<FM>::block_bytes, lane);
+    store_native_strings<FM>(str[0], str[1], native + ((size_t)(tile * 4 + block) * units + U) * Fmt<FM>::block_bytes, lane);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
 // Quantizer on the device: float weights [M,K] (fp16, bf16 or fp32) -> per-row fp16 scales + native-layout FPx codes.
-// Same arithmetic as the host quantizer of this package, so that both give identical bits:
+// Gives the bits of the host quantizer of this package, which computes in double precision:
 //   scale[row] = fp16_rn(absmax(row) / max_value) (1.0 where that rounds to zero), computed from a double quotient;
-//   code       = nearest representable magnitude to |w / scale| (a double quotient, clamped at max_value), ties to the even
-//                code, with the sign bit of w.  NaN weights become +0, +-Inf saturates, and neither takes part in absmax.
+//   code       = nearest representable magnitude to |w / scale| (clamped at max_value), ties to the even code, with the sign
+//                bit of w.  NaN weights become +0, +-Inf saturates, and neither takes part in absmax.
 // (The reference's only quantizer truncates and is not wired to any API: fp6_llm/csrc/utils/weight_quant.h:9-105.)
+//
+// The codes come from single precision and the packing conversion instruction (v_cvt_scalef32_2xpk16_bf6/fp6_f32: 32 floats to
+// 32 fields, round to nearest even, saturating), and are exact all the same.  A code changes where |w| = t * scale, t a
+// midpoint of at most 5 significant bits; t * scale has at most 16 bits.  A quotient computed as q = |w| * (1/scale)
+// followed by one residual step q += fma(-q, scale, |w|) * (1/scale) is within a hair over half an ulp of the true one, and exact where
+// the quotient is a midpoint.  A 16-bit w that is not on a boundary is at least 2^-16 away from it (relative), so q stays on
+// its side.  A 24-bit w can be as near as 2^-24, where q might round onto the midpoint: for fp32 weights the sign of a second
+// residual turns q into the quotient rounded to odd (truncated, last bit set if inexact), which never sits on a midpoint.
+//
+// HBM-bound.  Two organisations of the same arithmetic.  quant_fused: one workgroup of eight wavefronts per 16-row tile reads
+// its rows, finds the scales, and converts; the last three (fp32: two) blocks of every wavefront are still in its registers then,
+// the others are read again, latest first, out of L2 or the 256 MB last-level cache.  quant_row_scales + quant_blocks: a workgroup takes
+// a row, then a wavefront a block, and all weights are read twice.  bf16, us, fused / two kernels: 8192x8192 47 / 54 (184 MB, 3.9 TB/s), 4096x4096
+// 12.6 / 17.4, 28672x8192 137 / 199, 1024x1024 4.2 / 6.4, but 2048x8192 20 / 17 and 1024x8192 15 / 11: 64 or 128 workgroups do not pull
+// enough from memory to pay for a second pass over a long row.  The lines where the two meet lie near 192 tiles and K = 3072.  (Held
+// blocks and wavefronts at 8192x8192: 1 / 2 / 3 / 4 blocks on eight wavefronts 54 / 50 / 46 / 50, four wavefronts 54-59, sixteen 50-54.)
+// A conversion in double precision, code by code through a byte array in scratch memory, took 532 us for the first of these.
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T> __device__ __forceinline__ float to_float(T v);
-template <> __device__ __forceinline__ float to_float<half_t>(half_t v) { return (float)v; }
-template <> __device__ __forceinline__ float to_float<float>(float v) { return v; }
 struct bf16_t { uint16_t bits; };
-template <> __device__ __forceinline__ float to_float<bf16_t>(bf16_t v) { return __builtin_bit_cast(float, (uint32_t)v.bits << 16); }
+typedef short v2s __attribute__((ext_vector_type(2)));
+
+// Eight consecutive weights as loaded, their widening, and a running maximum of their magnitudes that lets NaN and Inf pass by: magnitude
+// bits order like the values, and adding the distance of the exponent field's top to the sign bit makes Inf and NaN negative.
+template <typename T> struct WeightPiece {
+    v4u x;
+    __device__ __forceinline__ void load(const T *p) { x = *reinterpret_cast<const v4u *>(p); }
+    __device__ __forceinline__ void zero() { x = (v4u){ 0u, 0u, 0u, 0u }; }
+    __device__ __forceinline__ float value(int j) const
+    {
+        const uint32_t w = x[j >> 1];
+        if constexpr (std::is_same<T, bf16_t>::value)
+            return __builtin_bit_cast(float, j & 1 ? w & 0xFFFF0000u : w << 16);
+        else
+            return (float)__builtin_bit_cast(half_t, (uint16_t)(j & 1 ? w >> 16 : w));
+    }
+};
+template <> struct WeightPiece<float> {
+    v4u x, y;
+    __device__ __forceinline__ void load(const float *p) { x = *reinterpret_cast<const v4u *>(p), y = *reinterpret_cast<const v4u *>(p + 4); }
+    __device__ __forceinline__ void zero() { x = y = (v4u){ 0u, 0u, 0u, 0u }; }
+    __device__ __forceinline__ float value(int j) const { return __builtin_bit_cast(float, j < 4 ? x[j] : y[j - 4]); }
+};
+template <typename T> struct MaxMagnitude {
+    static constexpr short kLift = std::is_same<T, bf16_t>::value ? 0x0080 : 0x0400; // 0x8000 - the bits of infinity
+    v2s m = { kLift, kLift };
+    __device__ __forceinline__ void add(const WeightPiece<T> &p)
+    {
+#pragma unroll
+        for (int i = 0; i < 4; i++) m = __builtin_elementwise_max(m, __builtin_bit_cast(v2s, p.x[i] & 0x7FFF7FFFu) + (v2s){ kLift, kLift });
+    }
+    __device__ __forceinline__ float value() const
+    {
+        const uint16_t b = (uint16_t)((m[0] > m[1] ? m[0] : m[1]) - kLift);
+        if constexpr (std::is_same<T, bf16_t>::value)
+            return __builtin_bit_cast(float, (uint32_t)b << 16);
+        else
+            return (float)__builtin_bit_cast(half_t, b);
+    }
+};
+template <> struct MaxMagnitude<float> {
+    int m = 0x00800000;
+    __device__ __forceinline__ void add(const WeightPiece<float> &p)
+    {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            m = max(m, (int)((p.x[i] & 0x7FFFFFFFu) + 0x00800000u));
+            m = max(m, (int)((p.y[i] & 0x7FFFFFFFu) + 0x00800000u));
+        }
+    }
+    __device__ __forceinline__ float value() const { return __builtin_bit_cast(float, m - 0x00800000); }
+};
 
 // round-to-nearest-even of a non-negative double to fp16 without passing through float (no double rounding)
 __device__ __forceinline__ half_t half_rn_from_double(double q)
@@ -1095,99 +1140,182 @@ __device__ __forceinline__ half_t half_rn_from_double(double q)
     double v = scalbn(r, ulp_exp);                   // representable in fp16 unless it overflows
     return v >= 65520.0 ? (half_t)__builtin_inff() : (half_t)(float)v;
 }
-
-// |v| for finite v, 0 for NaN and +-Inf: neither sets a scale
-__device__ __forceinline__ float finite_abs(float v)
+template <int FM> __device__ __forceinline__ half_t row_scale(float amax)
 {
-    const float a = fabsf(v);
-    return a <= 3.4028234663852886e38f ? a : 0.f;
+    const half_t sc = half_rn_from_double((double)amax / Fmt<FM>::max_value);
+    return (float)sc == 0.f ? (half_t)1.0f : sc;
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void quant_row_scales(half_t *__restrict__ scales, const T *__restrict__ Wf, uint32_t M, uint32_t K,
-                                                       double max_value)
+// The 32 weights of one field string (four pieces of eight) against the scale f -> their 6-bit fields.
+template <int FM, typename T> __device__ __forceinline__ v6u quantize_string(const WeightPiece<T> *p, float f)
 {
-    const int      lane = threadIdx.x & 63;
-    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= M) return;
-    const T *p = Wf + (size_t)row * K;
-    float    amax = 0.f;
-    for (uint32_t k = lane * 8; k < K; k += 512)
+    typedef float v16f __attribute__((ext_vector_type(16)));
+    // the fields of FP5 hold a quarter of the value (its grid up to 7 is the e3m2 grid up to 1.75, times 4)
+    constexpr float top = (float)Fmt<FM>::max_value / Fmt<FM>::post_scale, kInf = __builtin_inff();
+    f *= Fmt<FM>::post_scale;
+    const bool  overflown = f == kInf; // a row whose scale left fp16: finite weights become zeros
+    const float rf = overflown ? 0.f : 1.0f / f, fd = overflown ? 0.f : f, limit = overflown ? 3.4028234663852886e38f : kInf;
+    v16f        even, odd;
 #pragma unroll
-        for (int j = 0; j < 8; j++) amax = fmaxf(amax, finite_abs(to_float<T>(p[k + j])));
+    for (int i = 0; i < 32; i++) {
+        const float w = p[i >> 3].value(i & 7), a = __builtin_fabsf(w);
+        float       q = __builtin_fminf(a * rf, 2.f * top);
+        q = __builtin_fminf(__builtin_fmaf(__builtin_fmaf(-q, fd, a), rf, q), top);
+        if constexpr (std::is_same<T, float>::value) {
+            const float r = __builtin_fmaf(-q, fd, a);
+            uint32_t    u = __builtin_bit_cast(uint32_t, q);
+            if (r < 0.f) u -= 1;
+            if (r != 0.f) u |= 1;
+            q = __builtin_bit_cast(float, u);
+        }
+        if constexpr (Fmt<FM>::bits == 4) { // to the coarser grid first (steps of 1/2 below 2, 1 below 4, 2 above): exact in the fields then
+            const float magic = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, __builtin_fmaxf(q, 1.f)) & 0x7F800000u) * 6291456.f; // 1.5 * 2^23 steps
+            q = (q + magic) - magic;
+        }
+        q = a <= limit ? __builtin_copysignf(q, w) : 0.f; // NaN: +0
+        if (i & 1)
+            odd[i >> 1] = q;
+        else
+            even[i >> 1] = q;
+    }
+    if constexpr (Fmt<FM>::hw_e3m2)
+        return __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(even, odd, 1.0f);
+    else
+        return __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(even, odd, 1.0f);
+}
+
+// A lane of the quantizer is (m = l/4, p = l%4): the four lanes of a row read 64 or 128 consecutive bytes, and its codes go to the places
+// of lane (m, q = p) of the native block.  w points at the tile's first row.
+template <typename T> __device__ __forceinline__ void load_quant_block(WeightPiece<T> (&x)[8], const T *w, uint32_t K, uint32_t U, int lane)
+{
+    const T *p = w + (size_t)(lane >> 2) * K + (size_t)U * 256 + 8 * (lane & 3);
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        if (U * 256 + 32 * s < K) // uniform: K is a multiple of 64
+            x[s].load(p + 32 * s);
+        else
+            x[s].zero();
+    }
+}
+// GROUPS: every group of 128 columns of a row also gets the smallest factor 2^k, -15 <= k <= 0, that still holds its largest
+// magnitude, stored as the byte 127 + k, and its codes are chosen against scale * 2^k.  max_value * scale has at most 14 significant bits, so
+// comparing amax with it (by exponent, then by mantissa) decides like the double quotient amax / scale against max_value * 2^k.
+template <int FM, typename T, bool GROUPS>
+__device__ __forceinline__ void quantize_block(const WeightPiece<T> (&x)[8], float sc, uint8_t *native, uint8_t *gexp, size_t blk, uint32_t K, uint32_t U, int lane)
+{
+    v6u str[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        float f = sc;
+        if constexpr (GROUPS) {
+            MaxMagnitude<T> mm;
+#pragma unroll
+            for (int s = 0; s < 4; s++) mm.add(x[4 * h + s]);
+            float amax = mm.value();
+            amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
+            amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
+            const float t = (float)Fmt<FM>::max_value * sc;
+            int         k = __builtin_amdgcn_frexp_expf(amax) - __builtin_amdgcn_frexp_expf(t) + (__builtin_amdgcn_frexp_mantf(amax) > __builtin_amdgcn_frexp_mantf(t) ? 1 : 0);
+            if (amax == 0.f || t == __builtin_inff()) k = -15;
+            k = k < -15 ? -15 : k > 0 ? 0 : k;
+            if (U * 256 + 128 * h >= K) k = 0; // a half block beyond K: factor 1 by convention
+            f = ldexpf(sc, k);
+            if ((lane & 3) == 0) gexp[(blk * 16 + (lane >> 2)) * 2 + h] = (uint8_t)(127 + k);
+        }
+        str[h] = quantize_string<FM, T>(x + 4 * h, f);
+    }
+    store_native_strings<FM>(str[0], str[1], native + blk * Fmt<FM>::block_bytes, (lane >> 2) + 16 * (lane & 3));
+}
+
+template <int FM, typename T, bool GROUPS, int WAVES, int KEEP>
+__global__ __launch_bounds__(WAVES *kWave) void quant_fused(uint8_t *__restrict__ native, half_t *__restrict__ scales, uint8_t *__restrict__ gexp,
+                                                            const T *__restrict__ Wf, uint32_t K, uint32_t units)
+{
+    __shared__ float  wave_max[WAVES][16];
+    __shared__ half_t tile_scale[16];
+    const int         lane = threadIdx.x & 63;
+    const uint32_t    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), R = blockIdx.x;
+    const T          *w = Wf + (size_t)R * 16 * K;
+
+    // blocks wave, wave + WAVES, ...; the last KEEP of them stay in registers (kept[0] is the very last)
+    const uint32_t  mine = wave < units ? (units - wave + WAVES - 1) / WAVES : 0;
+    MaxMagnitude<T> mm;
+    WeightPiece<T>  kept[KEEP][8];
+    for (uint32_t i = 0; i + KEEP < mine; i++) {
+        WeightPiece<T> x[8];
+        load_quant_block<T>(x, w, K, wave + i * WAVES, lane);
+#pragma unroll
+        for (int s = 0; s < 8; s++) mm.add(x[s]);
+    }
+#pragma unroll
+    for (int k = KEEP - 1; k >= 0; k--)
+        if ((uint32_t)k < mine) load_quant_block<T>(kept[k], w, K, wave + (mine - 1 - k) * WAVES, lane);
+#pragma unroll
+    for (int k = KEEP - 1; k >= 0; k--)
+        if ((uint32_t)k < mine) {
+#pragma unroll
+            for (int s = 0; s < 8; s++) mm.add(kept[k][s]);
+        }
+    float amax = mm.value();
+    amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
+    if ((lane & 3) == 0) wave_max[wave][lane >> 2] = amax;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        float a = 0.f;
+#pragma unroll
+        for (int i = 0; i < WAVES; i++) a = fmaxf(a, wave_max[i][threadIdx.x]);
+        const half_t sc = row_scale<FM>(a);
+        tile_scale[threadIdx.x] = sc;
+        scales[R * 16 + threadIdx.x] = sc;
+    }
+    __syncthreads();
+    const float sc = (float)tile_scale[lane >> 2];
+#pragma unroll
+    for (int k = 0; k < KEEP; k++)
+        if ((uint32_t)k < mine) {
+            const uint32_t U = wave + (mine - 1 - k) * WAVES;
+            quantize_block<FM, T, GROUPS>(kept[k], sc, native, gexp, (size_t)R * units + U, K, U, lane);
+        }
+    for (uint32_t i = mine > KEEP ? mine - KEEP : 0; i-- > 0;) {
+        WeightPiece<T> x[8];
+        const uint32_t U = wave + i * WAVES;
+        load_quant_block<T>(x, w, K, U, lane);
+        quantize_block<FM, T, GROUPS>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+    }
+}
+
+template <int FM, typename T>
+__global__ __launch_bounds__(256) void quant_row_scales(half_t *__restrict__ scales, const T *__restrict__ Wf, uint32_t K)
+{
+    __shared__ float wave_max[4];
+    const T         *p = Wf + (size_t)blockIdx.x * K;
+    MaxMagnitude<T>  mm;
+#pragma unroll 4
+    for (uint32_t k = threadIdx.x * 8; k < K; k += 2048) {
+        WeightPiece<T> x;
+        x.load(p + k);
+        mm.add(x);
+    }
+    float amax = mm.value();
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-    if (lane == 0) {
-        half_t sc = half_rn_from_double((double)amax / max_value);
-        scales[row] = (float)sc == 0.f ? (half_t)1.0f : sc;
-    }
+    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = amax;
+    __syncthreads();
+    if (threadIdx.x == 0) scales[blockIdx.x] = row_scale<FM>(fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3])));
 }
 
-// index (= magnitude bits of the code) of the representable magnitude nearest to a, 0 <= a <= max_value
-template <int FM> __device__ __forceinline__ uint32_t nearest_magnitude(double a)
-{
-    constexpr int bias = Fmt<FM>::bias, MB = Fmt<FM>::man;
-    int           e = a > 0.0 ? ilogb(a) : -1000;
-    if (e < 1 - bias) e = 1 - bias;                        // subnormals use the spacing of the first binade
-    double   t = scalbn(a, MB - e);                        // in units of the spacing 2^(e-MB): [0,2^MB) subnormal, [2^MB,2^(MB+1)) normal
-    double   fl = floor(t), frac = t - fl;
-    uint32_t lo = (uint32_t)fl + ((uint32_t)(e + bias - 1) << MB);
-    // (normal: index = (e+bias)*2^MB + (fl-2^MB); subnormal: e = 1-bias, so index = fl)
-    if (frac > 0.5 || (frac == 0.5 && (lo & 1u))) lo += 1;
-    return lo;
-}
-
-// gexp (native order) non-null: besides the row scale every group of 128 columns of a row gets the smallest factor 2^k,
-// -15 <= k <= 0, that still holds its largest magnitude, stored as the byte 127 + k, and its codes are chosen against
-// scale * 2^k.  A wavefront's lanes (m, q = 0..3) hold the group's 128 values between them, 32 each.
-template <int FM, typename T>
-__global__ __launch_bounds__(256) void quant_to_native(uint8_t *__restrict__ native, const half_t *__restrict__ scales, uint8_t *__restrict__ gexp,
-                                                      const T *__restrict__ Wf, uint32_t M, uint32_t K, uint32_t units, double max_value)
+template <int FM, typename T, bool GROUPS>
+__global__ __launch_bounds__(256) void quant_blocks(uint8_t *__restrict__ native, const half_t *__restrict__ scales, uint8_t *__restrict__ gexp,
+                                                   const T *__restrict__ Wf, uint32_t M, uint32_t K, uint32_t units)
 {
     const int      lane = threadIdx.x & 63;
-    const uint32_t blk = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const uint32_t blk = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (blk >= (M / 16) * units) return;
     const uint32_t R = blk / units, U = blk % units;
-    const int      m = lane & 15, q = lane >> 4;
-    const uint32_t row = R * 16 + m;
-    const double   sc = (double)(float)scales[row];
-    const T       *p = Wf + (size_t)row * K;
-    double         factor[2] = { sc, sc };
-    if (gexp) { // uniform
-        for (int h = 0; h < 2; h++) {
-            float amax = 0.f;
-            for (int s = 4 * h; s < 4 * h + 4; s++) {
-                const uint32_t k0 = U * 256 + 32 * s + 8 * q;
-                for (int j = 0; j < 8; j++)
-                    if (k0 + j < K) amax = fmaxf(amax, finite_abs(to_float<T>(p[k0 + j])));
-            }
-            amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-            amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-            const double gmax = (double)amax / sc;
-            int          k = -15;
-            while (k < 0 && !(gmax <= scalbn(max_value, k))) k++;
-            if (U * 256 + 128 * h >= K) k = 0; // a half block beyond K: factor 1 by convention
-            factor[h] = scalbn(sc, k);
-            if (q == 0) gexp[((size_t)blk * 16 + m) * 2 + h] = (uint8_t)(127 + k);
-        }
-    }
-    uint8_t c[64];
-#pragma unroll 1
-    for (int s = 0; s < 8; s++) {
-        const uint32_t k0 = U * 256 + 32 * s + 8 * q;
-        const double   f = factor[s >> 2];
-        for (int j = 0; j < 8; j++) {
-            uint32_t code = 0;
-            if (k0 + j < K) {
-                float  w = to_float<T>(p[k0 + j]);
-                double a = fabs((double)w / f);
-                if (a > max_value) a = max_value; // clamps; +-Inf saturates
-                if (w == w) code = nearest_magnitude<FM>(a) | ((__builtin_bit_cast(uint32_t, w) >> 31) << (Fmt<FM>::bits - 1)); // NaN: +0
-            }
-            c[8 * s + j] = (uint8_t)code;
-        }
-    }
-    store_native_lane<FM>(c, native + (size_t)blk * Fmt<FM>::block_bytes, lane);
+    WeightPiece<T> x[8];
+    load_quant_block<T>(x, Wf + (size_t)R * 16 * K, K, U, lane);
+    quantize_block<FM, T, GROUPS>(x, (float)scales[R * 16 + (lane >> 2)], native, gexp, blk, K, U, lane);
 }
 // ------------------------------------------------------------------------------------------------ launch helpers
 
@@ -1327,8 +1455,7 @@ int op_gemm(const LaunchCfg &c, void *stream, const void *W, const void *sc, con
 template <int FM> int op_relayout(void *stream, void *native, const void *ref, size_t M, size_t K)
 {
     uint32_t units = (uint32_t)((K + 255) / 256);
-    size_t   blocks = (M / 16) * units;
-    hipLaunchKernelGGL(relayout_ref_to_native<FM>, dim3((uint32_t)((blocks + 3) / 4)), dim3(256), 0, static_cast<hipStream_t>(stream),
+    hipLaunchKernelGGL(relayout_ref_to_native<FM>, dim3((uint32_t)((M / 64) * units)), dim3(256), 0, static_cast<hipStream_t>(stream),
                        static_cast<uint8_t *>(native), static_cast<const uint8_t *>(ref), (uint32_t)M, (uint32_t)K, units);
     return (int)hipGetLastError();
 }
@@ -1351,25 +1478,36 @@ template <int FM> int op_dequant(void *stream, void *out, const void *W, const v
 // dtype: 0 = fp16, 1 = bf16, 2 = fp32
 template <int FM> int op_quantize(void *stream, void *native, void *scales, void *gexp, const void *weights, int dtype, size_t M, size_t K)
 {
-    const uint32_t   units = (uint32_t)((K + 255) / 256);
-    const size_t     blocks = (M / 16) * units;
-    const dim3       grid_rows((uint32_t)((M + 3) / 4)), grid_blocks((uint32_t)((blocks + 3) / 4));
-    constexpr double max_value = Fmt<FM>::max_value;
-    hipStream_t      st = static_cast<hipStream_t>(stream);
-    uint8_t         *nat = static_cast<uint8_t *>(native);
-    half_t          *sc = static_cast<half_t *>(scales);
-    auto             run = [&](auto *typed) {
+    const uint32_t units = (uint32_t)((K + 255) / 256);
+    const size_t   blocks = (M / 16) * units;
+    hipStream_t    st = static_cast<hipStream_t>(stream);
+    uint8_t       *nat = static_cast<uint8_t *>(native), *ge = static_cast<uint8_t *>(gexp);
+    half_t        *sc = static_cast<half_t *>(scales);
+    auto           run = [&](auto *typed, auto groups_c) {
         typedef std::remove_cv_t<std::remove_pointer_t<decltype(typed)>> T;
-        hipLaunchKernelGGL(quant_row_scales<T>, grid_rows, dim3(256), 0, st, sc, typed, (uint32_t)M, (uint32_t)K, max_value);
-        hipLaunchKernelGGL((quant_to_native<FM, T>), grid_blocks, dim3(256), 0, st, nat, sc, static_cast<uint8_t *>(gexp), typed, (uint32_t)M,
-                           (uint32_t)K, units, max_value);
+        constexpr bool GROUPS = decltype(groups_c)::value;
+        if (M / 16 >= 192 || K <= 3072) { // (where the two organisations cross: see quant_fused)
+            constexpr int WAVES = 8, KEEP = sizeof(T) == 2 ? 3 : 2;
+            hipLaunchKernelGGL((quant_fused<FM, T, GROUPS, WAVES, KEEP>), dim3((uint32_t)(M / 16)), dim3(WAVES * kWave), 0, st, nat, sc, ge, typed,
+                               (uint32_t)K, units);
+        } else {
+            hipLaunchKernelGGL((quant_row_scales<FM, T>), dim3((uint32_t)M), dim3(256), 0, st, sc, typed, (uint32_t)K);
+            hipLaunchKernelGGL((quant_blocks<FM, T, GROUPS>), dim3((uint32_t)((blocks + 3) / 4)), dim3(256), 0, st, nat, sc, ge, typed, (uint32_t)M,
+                               (uint32_t)K, units);
+        }
     };
-    if (dtype == 0)
-        run(static_cast<const half_t *>(weights));
-    else if (dtype == 1)
-        run(static_cast<const bf16_t *>(weights));
+    auto typed = [&](auto groups_c) {
+        if (dtype == 0)
+            run(static_cast<const half_t *>(weights), groups_c);
+        else if (dtype == 1)
+            run(static_cast<const bf16_t *>(weights), groups_c);
+        else
+            run(static_cast<const float *>(weights), groups_c);
+    };
+    if (gexp)
+        typed(std::true_type{});
     else
-        run(static_cast<const float *>(weights));
+        typed(std::false_type{});
     return (int)hipGetLastError();
 }
 

@@ -795,6 +795,43 @@ def test_device_quantizer_matches_host_bits(E, M, dtype, OC, IC):
     assert np.array_equal(_codes_of_native(native, E, M, OC, IC), c_def)
 
 
+@pytest.mark.parametrize("E,M", FORMATS)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("OC,IC", [(16, 3072), (16, 3136), (3056, 3136), (3072, 6208)])
+def test_device_quantizer_at_the_edges_of_its_kernels(E, M, dtype, OC, IC):
+    """Both organisations on either side of the lines between them (192 row tiles, K = 3072), K blocks cut at 64 columns, more
+    blocks per wavefront than registers hold, and weights on and one step to either side of every rounding boundary.  Rows are
+    independent, so the first and the last row tile stand for the matrix."""
+    print("case quantizer edges", E, M, dtype, OC, IC, flush=True)
+    gen = torch.Generator().manual_seed(OC + IC)
+    w = (torch.randn(OC, IC, generator=gen) * 0.02).to(dtype)
+    top = quant.max_value(E, M)
+    mags = quant.magnitudes(E, M)
+    mids = torch.from_numpy((mags[1:] + mags[:-1]) / 2)
+    for r, sc in ((0, 0.0123), (5, 2.0 ** -6), (OC - 1, 1.7)):
+        sc = float(np.float16(sc))
+        near = (mids * sc).to(dtype)
+        bits = near.view(torch.int32 if dtype == torch.float32 else torch.int16)
+        row = torch.cat([near, (bits + 1).view(dtype), (bits - 1).view(dtype)])
+        row = torch.cat([row, -row, torch.tensor([top * sc, 0.0, -0.0, float("nan"), float("inf")]).to(dtype)])
+        w[r, :] = 0
+        w[r, IC - len(row):] = row
+    native, scales = fp6.weight_quantize_native_cuda(E, M, w.to(DEV))
+    native_g, scales_g, gexp = fp6.weight_quantize_native_cuda(E, M, w.to(DEV), group_scales=True)
+    assert torch.equal(scales, scales_g)
+    per_tile, per_gexp = native.numel() // (OC // 16), gexp.numel() // (OC // 16)
+    for tile in sorted({0, OC // 16 - 1}):
+        rows = w[16 * tile:16 * tile + 16].float().numpy().astype(np.float64)
+        codes, sc_host = quant.quantize_rowwise(rows, E, M)
+        assert np.array_equal(scales[16 * tile:16 * tile + 16].cpu().numpy().view(np.uint16), sc_host.view(np.uint16))
+        want = fp6.weight_prepacking_native_cpu(E, M, torch.from_numpy(quant.pack_raw(codes, E, M)))
+        assert torch.equal(native[per_tile * tile:per_tile * (tile + 1)].cpu(), want)
+        codes, _, ex = quant.quantize_groupwise(rows, E, M)
+        want = fp6.weight_prepacking_native_cpu(E, M, torch.from_numpy(quant.pack_raw(codes, E, M)))
+        assert torch.equal(native_g[per_tile * tile:per_tile * (tile + 1)].cpu(), want)
+        assert torch.equal(gexp[per_gexp * tile:per_gexp * (tile + 1)].cpu(), fp6.pack_group_exps(torch.from_numpy(ex), 16, IC))
+
+
 def test_device_quantizer_rejects_bad_arguments():
     with pytest.raises(ValueError):
         fp6.weight_quantize_native_cuda(3, 2, torch.zeros(256, 100, dtype=torch.float16, device=DEV))
