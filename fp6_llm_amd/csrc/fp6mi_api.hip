@@ -158,7 +158,7 @@ inline bool cfg_fits(const TuneCfg &c, size_t M) { return c.kind != 255 && (c.ki
 // 16384 and 17920 rows differ by 9 % in size but by a whole round of 64-row workgroups; sweeps off the grid showed that
 // this, not the distance, decides which neighbour's shape is right.  Farther neighbours pay 15 % per octave of distance.
 struct TuneGroup { int xb; size_t n, begin, end; }; // entries [begin, end) of kTune share format and batch (the table is sorted by them)
-struct TuneAnswer { bool valid, measured; LaunchCfg cfg[kNumSplits]; float t[kNumSplits]; }; // index i: splitK = kSplits[i]; t in 0.02 us, 0 = no proposal; measured: this very (M, K) at this or the next larger measured batch
+struct TuneAnswer { bool valid, measured, exact; LaunchCfg cfg[kNumSplits]; float t[kNumSplits]; }; // index i: splitK = kSplits[i]; t in 0.02 us, 0 = no proposal; measured: this very (M, K) at this or the next larger measured batch; exact: at this batch
 
 const std::vector<TuneGroup> &tune_groups()
 {
@@ -216,7 +216,7 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
         }
     }
     TuneAnswer a = {};
-    if (count > 0 && dist[0] == 0.f) count = 1, a.measured = true; // measured: nothing to carry over
+    if (count > 0 && dist[0] == 0.f) count = 1, a.measured = true, a.exact = group->n == N; // measured: nothing to carry over
     const size_t units = (K + 255) / 256;
     for (int j = 0; j < count; j++) {
         const TuneEntry &e = *near[j];
@@ -237,6 +237,28 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
     return a.valid ? &slot.a : nullptr;
 }
 
+// Whether gemm_prefill's 128 x 128 tile replaces the shape `c` of another large-batch kernel.  Its workgroups take a CU as long as half a
+// 256 x 128 one does (7 ns per column of K, measured from 64 to 3600 workgroups) and as long as a 256 x 64 one of the same area, so what
+// decides is the number of rounds on the chip.  Over 205 problems (M 1024-57344, K 1024-28672, N 96-4096, three bit widths; time here / time of
+// the shape before):
+//   * 256 x 128: fewer half rounds 0.63-1.00 up to N 2048; as many 0.95-1.00 up to N 1024, 0.99-1.20 above;
+//     beyond N 2048 0.80-0.89 with an eighth fewer and 0.90-1.07 with less gained (3854 columns, 15 half rounds for 16: 1.07);
+//   * 256 x 64: as many rounds or fewer, two at least, 0.83-0.97 up to N 2048 (1.03-1.06 above); a single round 1.02-1.2;
+//   * up to N 144 the second column block is nearly empty (N 128: 1.09, N 135: 1.02, N 166: 0.98);
+//   * beyond N 2048 with rows of a multiple of 8 KB the activation lines crowd the same channels (8192x8192 N 4096: 1.20).
+inline bool prefill_tile_wins(const LaunchCfg &c, size_t M, size_t N, size_t K, int splitK, int cus)
+{
+    if (splitK != 1 || N <= 144 || K > (size_t)1 << 20 || (N > 2048 && K % 4096 == 0)) return false;
+    auto         rounds = [&](size_t rows, size_t cols) { return (M / rows * ((N + cols - 1) / cols) + cus - 1) / cus; };
+    const size_t here = rounds(128, 128);
+    if (c.kind == 1 && c.nt == 8 && c.rt == 2 && c.wr == 8 && c.wk == 1) {
+        const size_t half = 2 * rounds(256, 128);
+        return N <= 1024 ? here <= half : N <= 2048 ? here < half : 8 * here <= 7 * half;
+    }
+    if (c.nt == 4 && c.rt == 2 && c.wr == 8 && (c.kind == 2 || (c.kind == 1 && c.wk == 1))) return rounds(256, 64) >= 2 && here <= rounds(256, 64) && N <= 2048;
+    return false;
+}
+
 // Launch shape for a given splitK.
 //  N <= 16: stream kernel.  Row tiles per wavefront (rt) reuse the activation registers, so rt grows with M; wavefronts
 //           per workgroup follow the K blocks of one split and the register budget (16 wavefronts leave 128 VGPRs each).
@@ -247,7 +269,10 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
     LaunchCfg c;
     if (const int i = split_index(splitK); cus == 256 && i >= 0) {
         if (const TuneAnswer *a = tune_lookup(xbits, M, N, K)) {
-            if (a->t[i] > 0.f) return a->cfg[i];
+            if (a->t[i] > 0.f) { // a problem that was itself measured keeps its shape
+                if (!a->exact && prefill_tile_wins(a->cfg[i], M, N, K, splitK, cus)) return LaunchCfg{ 2, 8, 4, 2, 2 };
+                return a->cfg[i];
+            }
         }
     }
     size_t    tiles = M / 16, units = (K + 255) / 256, per_split = (units + splitK - 1) / splitK;
@@ -294,7 +319,7 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
     tile_estimate_ns(M, N, K, splitK, cus, &t);
     if (!t) t = &kRuleShapes[1]; // 128 x 32, one K wavefront: divides every legal M and needs a single K block
     c.nt = t->nt, c.rt = t->rt, c.wr = t->wr, c.wk = t->wk;
-    return c;
+    return prefill_tile_wins(c, M, N, K, splitK, cus) ? LaunchCfg{ 2, 8, 4, 2, 2 } : c;
 }
 int linear_native(const fp6mi::FormatOps &ops, hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, size_t M, size_t N, size_t K, float *ws,
                   int splitK, const LaunchCfg *forced)

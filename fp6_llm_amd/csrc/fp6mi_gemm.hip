@@ -934,6 +934,217 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// gemm_prefill: the tile GEMM for long prompts, where the matrix cores are the bound.
+//   workgroup = 2 x 2 wavefronts; tile = (2*RT*16) rows x (2*NT*16) columns, (RT*16) x (NT*16) of it per wavefront; grid as gemm_tile
+// What bounds such a GEMM on this chip is that the conversions do not run in the MFMAs' shadow (70-90 cycles against 17 per MFMA) and,
+// in gemm_tile and gemm_ws, the LDS operand reads: there a wavefront owns 32 rows, one read for every two MFMAs.  Here it owns
+// 64 x 64 outputs: a read feeds four MFMAs, a converted fragment sixteen, on a tile half as large as the 256 x 128 one that takes as
+// many cycles per output, so that the last round of workgroups leaves half as much of the chip idle.
+// K is walked in chunks of 128 (half a native block).  The chunk's B operands live in registers, all 4 steps x NT of them;
+// the row tiles pass by one after the other: section r runs 4 * NT MFMAs on row tile r while tile r+1 is converted and the raw
+// codes of tile r+1 of the NEXT chunk are asked for (memory -> registers, a whole chunk ahead).  The activations of the next chunk go
+// memory -> LDS without registers in the first sections, and the last section, behind the only barrier of a chunk, replaces the B
+// operands step by step as its own MFMAs release them.
+// LDS: two stages of [2*NT*16 rows x 256 bytes], piece p of row n (16 bytes) at slot p ^ (n & 15): eight neighbouring columns at one
+// K position then lie in eight different bank groups.
+// 128 x 128 (RT = NT = 4) takes 215-228 registers and 64 KB, two workgroups per CU.  Measured (us, the shape chosen before -> this):
+// FP6 4608x4544 N 777: 59 -> 39, 9984x3328 N 312: 42 -> 29, 28672x8192 N 384: 215 -> 170, N 1024: 446 -> 403; 18944x2432 N 1305: 152 -> 128;
+// FP5 3584x4928 N 3435: 156 -> 125; FP4 6912x4416 N 2563: 194 -> 161.  Where the rounds come out even it is level (8192x8192 N 512: 62.7 both) or
+// behind (N 4096 at K 8192: 484 against 583).  Tiles of 256 x 128 (RT 8, 400+ registers, one wavefront per SIMD: 3-15 % slower than
+// gemm_tile's) and 256 x 256 (RT = NT = 8: spills) were left out.
+// ---------------------------------------------------------------------------------------------------------------
+// f(0), ..., f(RT - 1) with the index as a compile-time constant (a body this long is past what `#pragma unroll` takes)
+template <int RT, int R = 0, typename F> __device__ __forceinline__ void sections(const F &f)
+{
+    f(std::integral_constant<int, R>{});
+    if constexpr (R + 1 < RT) sections<RT, R + 1>(f);
+}
+
+struct RawHalf { v4u p; v2u s; uint32_t g; }; // one lane's codes of half a block of one row tile, as loaded (s, g: where the format has them)
+
+// raw codes of half H of a native block (and its group exponent): what field_string(., H) needs
+template <int FM, bool GS, int H> __device__ __forceinline__ void load_raw_half(RawHalf &f, const uint8_t *block, const uint8_t *gexp32, int lane)
+{
+    constexpr int kPiece = Fmt<FM>::bits == 6 ? 2048 : 1024; // the second half's 16-byte piece (6 bits: pieces a | b | c, b shared)
+    f.p = *reinterpret_cast<const v4u *>(block + H * kPiece + lane * 16);
+    if constexpr (Fmt<FM>::bits == 6) f.s = *reinterpret_cast<const v2u *>(block + 1024 + lane * 16 + 8 * H);
+    if constexpr (Fmt<FM>::bits == 5) f.s[0] = *reinterpret_cast<const uint32_t *>(block + 2048 + lane * 8 + 4 * H);
+    if constexpr (GS) f.g = gexp32[2 * (lane & 15) + H];
+}
+template <int FM, bool GS, int H> __device__ __forceinline__ v32h convert_raw_half(const RawHalf &f)
+{
+    v6u src;
+    if constexpr (Fmt<FM>::bits == 6)
+        src = H == 0 ? (v6u){ f.p[0], f.p[1], f.p[2], f.p[3], f.s[0], f.s[1] } : (v6u){ f.s[0], f.s[1], f.p[0], f.p[1], f.p[2], f.p[3] };
+    else if constexpr (Fmt<FM>::bits == 5)
+        src = fp5_expand(f.p[0], f.p[1], f.p[2], f.p[3], f.s[0]);
+    else
+        src = fp4_expand(f.p);
+    return fields_to_halfs<FM>(src, GS ? __builtin_bit_cast(float, f.g << 23) : 1.0f);
+}
+
+// (no __restrict__ on what the K loop reads: its loads must stay where the waits count them, on their side of the barriers)
+template <int FM, bool GS, int NT, int RT>
+__global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X,
+                                                          half_t *__restrict__ C, float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
+                                                          uint32_t units, uint32_t splitK, uint32_t nblocks)
+{
+    static_assert(RT >= 4 && RT % 2 == 0, "the activation transfers take the first half of the sections");
+    constexpr int TN = 2 * NT * 16, kStage = TN * 256;
+    constexpr int kDma = TN / 16;          // transfers of 1 KB (four rows) per wavefront and chunk
+    constexpr int kDmaSections = RT / 2, kDmaPer = kDma / kDmaSections;
+    static_assert(kDma % kDmaSections == 0, "every section issues the same number of transfers");
+    // loads a wavefront issues for certain after its last transfer of a chunk and before the chunk's barrier
+    constexpr int kRawLoads = (Fmt<FM>::bits == 4 ? 1 : 2) + (GS ? 1 : 0), kAfterDma = (RT - kDmaSections) * kRawLoads;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, q = lane >> 4, wr = wave & 1, wc = wave >> 1;
+
+    uint32_t id = blockIdx.x; // -> (row block, split, column block), every XCD a run of consecutive triples: as in gemm_tile
+    {
+        const uint32_t per = gridDim.x >> 3, r = gridDim.x & 7u, x = id & 7u;
+        id = x * per + (x < r ? x : r) + (id >> 3);
+    }
+    const uint32_t nb = id % nblocks, rest = id / nblocks, split = rest % splitK, mb = rest / splitK;
+    const uint32_t nbase = nb * TN, R0 = (mb * 2 + wr) * RT;
+    uint32_t       u0 = 0, u1 = units;
+    if (splitK > 1) {
+        const uint32_t avg = units / splitK, extra = units % splitK;
+        u0 = split * avg + (split < extra ? split : extra);
+        u1 = u0 + avg + (split < extra ? 1u : 0u);
+    }
+
+    v4f acc[RT][NT];
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[r][t] = (v4f){ 0.f, 0.f, 0.f, 0.f };
+
+    const size_t   tile_stride = (size_t)units * Fmt<FM>::block_bytes;
+    const uint8_t *wgroup = W + (size_t)R0 * tile_stride;
+    const uint8_t *ggroup = GS ? gexp + (size_t)R0 * units * 32 : nullptr;
+    RawHalf        raw[RT];
+    auto           load_raw = [&](auto half_c, int r, uint32_t u) __attribute__((always_inline)) {
+        load_raw_half<FM, GS, decltype(half_c)::value>(raw[r], wgroup + r * tile_stride + (size_t)u * Fmt<FM>::block_bytes,
+                                                       GS ? ggroup + ((size_t)r * units + u) * 32 : nullptr, lane);
+    };
+
+    // transfer j of this wavefront fills rows 4*wave + 16*j .. +3 of a stage: lane l is slot l%16 of row 4*wave + 16*j + l/16, which
+    // holds the piece slot ^ (row & 15), the same piece for every j.  Rows beyond N repeat the last real one (never stored).
+    typedef __attribute__((address_space(3))) void lvoid;
+    // Offsets are formed anew at every use (two instructions): kept, they would take two registers per transfer.
+    const uint32_t xrow0 = 4 * wave + q, xpiece = (lane & 15) ^ xrow0; // xrow0 < 16
+    const uint32_t xoff0 = xrow0 * K * 2, xlast = (N - nbase < (uint32_t)TN ? N - 1 - nbase : TN - 1) * K * 2; // 32 bits: the launcher bounds K
+    auto           row_offset = [&](int j) __attribute__((always_inline)) {
+        uint32_t o = xoff0;
+        asm volatile("" : "+v"(o));
+        o += (uint32_t)j * 32u * K;
+        return o < xlast ? o : xlast;
+    };
+    // Positions beyond K (the last block of a K that is no multiple of 256) are given an offset outside the buffer, which reads as
+    // zero: no branch, and the same number of transfers to wait for in every chunk.  (The buffer form of the instruction also lets the
+    // compiler count the raw codes' loads; behind global_load_lds, which it takes for a flat access, it waits for all of them.)
+    const auto xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(X + (size_t)nbase * K), 0, (int)(xlast + K * 2), 0x00027000);
+    auto       transfer = [&](int j, uint32_t h, uint32_t stage) __attribute__((always_inline)) {
+        const uint32_t beyond = h * 128 + xpiece * 8 < K ? 0u : 0xc0000000u, off = (row_offset(j) + xpiece * 16) | beyond;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, (lvoid *)(lds + stage * kStage + (wave + 4 * j) * 1024), 16, off, h * 256, 0, 0);
+    };
+
+    v8h            b[4][NT];
+    const uint8_t *xread = lds + (wc * NT * 16 + col) * 256;
+    auto           read_b = [&](int s, uint32_t stage) __attribute__((always_inline)) {
+        const uint8_t *p = xread + stage * kStage + (((4 * s + q) ^ col) * 16);
+#pragma unroll
+        for (int t = 0; t < NT; t++) b[s][t] = *reinterpret_cast<const v8h *>(p + t * 16 * 256);
+    };
+
+    typedef std::integral_constant<int, 0> Half0;
+    typedef std::integral_constant<int, 1> Half1;
+
+    // Chunk h: its B operands are in b, its row tile 0 in a, its other raw codes in (or on the way to) raw[1..]; raw[0] is the next
+    // chunk's.  There is no special last chunk: after it a chunk is fetched once more and not used.  One copy of the code per half
+    // keeps the accumulators in place (copies for the ends of K made the compiler move them between the halves of the register file).
+    v32h a;
+    auto chunk = [&](auto half_c, uint32_t h) __attribute__((always_inline)) {
+        constexpr int H = decltype(half_c)::value;
+        typedef std::integral_constant<int, 1 - H> Other;
+        const uint32_t hx = h + 1 < 2 * u1 ? h + 1 : h, u_next = hx >> 1, u_after = h + 2 < 2 * u1 ? (h + 2) >> 1 : h >> 1;
+        sections<RT>([&](auto r_c) __attribute__((always_inline)) {
+            constexpr int r = decltype(r_c)::value;
+            if constexpr (r < kDmaSections) {
+#pragma unroll
+                for (int j = r * kDmaPer; j < (r + 1) * kDmaPer; j++) transfer(j, hx, (h + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (r == RT - 1) { // the next chunk's activations have landed, for every wavefront
+                wait_transfers_and_barrier<kAfterDma>();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            v32h a_next;
+            if constexpr (r + 1 < RT) {
+                a_next = convert_raw_half<FM, GS, H>(raw[r + 1]);
+                load_raw(Other{}, r + 1, u_next);
+            } else {
+                a_next = convert_raw_half<FM, GS, 1 - H>(raw[0]);
+                load_raw(half_c, 0, u_after);
+            }
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(slice8(a, s), b[s][t], acc[r][t], 0, 0, 0);
+                if constexpr (r == RT - 1) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    read_b(s, (h + 1) & 1);
+                }
+            }
+            a = a_next;
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+
+    if (u0 < u1) { // (more splits than K blocks leave some empty: their partial sums are zeros)
+#pragma unroll
+        for (int j = 0; j < kDma; j++) transfer(j, 2 * u0, 0);
+#pragma unroll
+        for (int r = 0; r < RT; r++) load_raw(Half0{}, r, u0);
+        wait_transfers_and_barrier<0>();
+#pragma unroll
+        for (int s = 0; s < 4; s++) read_b(s, 0);
+        a = convert_raw_half<FM, GS, 0>(raw[0]);
+        load_raw(Half1{}, 0, u0);
+        for (uint32_t u = u0; u < u1; u++) {
+            chunk(Half0{}, 2 * u);
+            chunk(Half1{}, 2 * u + 1);
+        }
+    }
+    wait_transfers_and_barrier<0>(); // nothing is on its way to LDS any more, and nobody reads operands
+
+    // output: as in the other tile kernels, through LDS; the row scales are asked for here, one round trip at the end of a long K loop
+    v4h sc4[RT];
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        const half_t *p = scales + (R0 + r) * 16 + 4 * q;
+        sc4[r] = (v4h){ p[0], p[1], p[2], p[3] };
+    }
+    if (splitK == 1) {
+        tile_park<FM, NT, RT, 2, half_t>(acc, sc4, lds + (size_t)wc * NT * 16 * (2 * RT * 16 * 2 + 16), wr, col, q);
+        __syncthreads();
+        tile_flush<2 * NT, RT, 2, 4 * kWave, half_t>(C, lds, M, N, mb, nbase, tid);
+    } else {
+        // fp32 partial sums in two turns, one half of the columns each: both at once would not fit LDS
+        float *out = ws + (size_t)split * N * M;
+#pragma unroll
+        for (int part = 0; part < 2; part++) {
+            if (wc == part) tile_park<FM, NT, RT, 2, float>(acc, sc4, lds, wr, col, q);
+            __syncthreads();
+            tile_flush<NT, RT, 2, 4 * kWave, float>(out, lds, M, N, mb, nbase + part * NT * 16, tid);
+            __syncthreads();
+        }
+    }
+}
+
 // Native layout -> fp16 [M,K], with the GEMM's own conversion code.  One lane per (row tile, K block, lane) triple.
 template <int FM, bool GS>
 __global__ __launch_bounds__(256) void dequant_native(half_t *__restrict__ out, const uint8_t *__restrict__ W, const half_t *__restrict__ scales,
@@ -1404,7 +1615,27 @@ int launch_ws(hipStream_t st, const void *W, const void *sc, const void *gexp, c
         return (int)hipGetLastError();
     }
 }
-// kind 0: gemm_stream (wr == 1, wk = wavefronts per workgroup);  kind 1: gemm_tile (wr x wk wavefronts);  kind 2: gemm_ws (wr arithmetic + wk loading wavefronts)
+template <int FM, bool GS, int NT, int RT>
+int launch_prefill(hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, float *ws, size_t M, size_t N, size_t K,
+                   int splitK)
+{
+    constexpr int    TN = 2 * NT * 16, TM = 2 * RT * 16;
+    constexpr size_t kLoopLds = 2 * (size_t)TN * 256, out_full = tile_stage_bytes<2 * NT, RT, 2>(false), out_part = tile_stage_bytes<NT, RT, 2>(true);
+    constexpr size_t kOut = out_full > out_part ? out_full : out_part, kLds = kLoopLds > kOut ? kLoopLds : kOut;
+    static_assert(kLds <= 160 * 1024, "tile does not fit in LDS");
+    if (M % TM) return FP6MI_ERR_SHAPE;
+    if (kLds > 48 * 1024)
+        if (int rc = allow_dynamic_lds<&gemm_prefill<FM, GS, NT, RT>>(kLds)) return rc;
+    uint32_t units = (uint32_t)((K + 255) / 256), nblocks = (uint32_t)((N + TN - 1) / TN);
+    size_t   wgs = (M / TM) * (size_t)splitK * nblocks;
+    if (wgs > 0x7fffffffu || K > (size_t)1 << 20) return FP6MI_ERR_SHAPE; // (K: 32-bit offsets over TN rows)
+    hipLaunchKernelGGL((gemm_prefill<FM, GS, NT, RT>), dim3((uint32_t)wgs), dim3(4 * kWave), kLds, st, static_cast<const uint8_t *>(W),
+                       static_cast<const half_t *>(sc), static_cast<const uint8_t *>(gexp), static_cast<const half_t *>(B), static_cast<half_t *>(C), ws,
+                       (uint32_t)M, (uint32_t)N, (uint32_t)K, units, (uint32_t)splitK, nblocks);
+    return (int)hipGetLastError();
+}
+// kind 0: gemm_stream (wr == 1, wk = wavefronts per workgroup);  kind 1: gemm_tile (wr x wk wavefronts);  kind 2: gemm_ws (wr arithmetic + wk loading wavefronts),
+// or with wr = wk = 2 gemm_prefill (2 x 2 wavefronts; nt = column tiles of the whole workgroup, rt = row tiles per wavefront)
 template <int FM, bool GS>
 int launch_cfg(const LaunchCfg &c, hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, float *ws, size_t M,
                size_t N, size_t K, int splitK)
@@ -1434,8 +1665,11 @@ int launch_cfg(const LaunchCfg &c, hipStream_t st, const void *W, const void *sc
         // ring depths (2,2): deeper rings on smaller tiles (128 x 64 with (4,2), 128 x 32 and 64 x 64 with (4,3)) measured no faster than
         // gemm_tile at batches 32-64, where the time goes to the partial sums and the second launch, and are not built
 #define FP6MI_CASE(NT, RT, WR, PW) \
-    if (c.nt == NT && c.rt == RT && c.wr == WR && c.wk == PW) return launch_ws<FM, GS, NT, RT, WR, PW, 2, 2>(st, W, sc, gexp, B, C, ws, M, N, K, splitK);
-        FP6MI_CASE(4, 2, 8, 4) FP6MI_CASE(4, 2, 4, 4) FP6MI_CASE(2, 2, 8, 4)
+    if (c.nt == NT && c.rt == RT && c.wr == WR && c.wk == PW) { \
+        if constexpr (WR == 2) return launch_prefill<FM, GS, NT / 2, RT>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
+        else return launch_ws<FM, GS, NT, RT, WR, PW, 2, 2>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
+    }
+        FP6MI_CASE(4, 2, 8, 4) FP6MI_CASE(4, 2, 4, 4) FP6MI_CASE(2, 2, 8, 4) FP6MI_CASE(8, 4, 2, 2)
 #undef FP6MI_CASE
     }
     return FP6MI_ERR_SHAPE;

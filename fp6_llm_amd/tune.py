@@ -44,8 +44,9 @@ COMPILED_TILE = [(1,) + c for c in
                   (4, 4, 2, 1), (4, 4, 2, 2), (8, 2, 4, 1), (8, 2, 2, 1), (4, 2, 8, 1), (4, 2, 8, 2), (2, 2, 8, 1), (2, 2, 8, 2), (8, 2, 8, 1),
                   (4, 1, 8, 2), (4, 1, 8, 1), (4, 1, 4, 2), (2, 1, 2, 4)]]
 
-# kind 2 = wave-specialized tile kernel: (2, n_tiles, row_tiles, arithmetic wavefronts, loading wavefronts)
-COMPILED_WS = [(2, 4, 2, 8, 4), (2, 4, 2, 4, 4), (2, 2, 2, 8, 4)]
+# kind 2 = wave-specialized tile kernel: (2, n_tiles, row_tiles, arithmetic wavefronts, loading wavefronts); with 2 and 2 the prefill kernel
+# (2 x 2 wavefronts, n_tiles of the whole workgroup)
+COMPILED_WS = [(2, 4, 2, 8, 4), (2, 4, 2, 4, 4), (2, 2, 2, 8, 4), (2, 8, 4, 2, 2)]
 
 BLOCK_BYTES = {6: 3072, 5: 2560, 4: 2048}   # one native 16-row x 256-column block per bit width
 

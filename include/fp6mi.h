@@ -136,7 +136,8 @@ int fp6mi_linear_stateless(int E, int Mbits, void *stream, const void *W_ref, co
  *          3, 5, 6 and 7 need not divide M/16: the last workgroup holds the tiles that are left),
  * kind 1 = tile kernel (row_waves x k_waves wavefronts, activations staged in LDS),
  * kind 2 = wave-specialized tile kernel (row_waves arithmetic wavefronts; k_waves = 4 loading wavefronts that move weights and
- *          activations into LDS for them);
+ *          activations into LDS for them); row_waves = k_waves = 2: the prefill kernel (2 x 2 wavefronts, weights straight to
+ *          registers, K <= 2^20);
  * n_tiles = 16-column batch tiles per workgroup, row_tiles = 16-row weight tiles per wavefront.
  * Combinations that are not compiled in, or that do not divide M, return FP6MI_ERR_SHAPE. */
 int fp6mi_linear_native_cfg(int E, int Mbits, void *stream, const void *W_native, const void *scales_f16,

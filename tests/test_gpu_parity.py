@@ -222,6 +222,29 @@ def test_wave_specialized_kernel_edges(E, M, cfg):
         check_close(out.cpu().numpy(), oracle.gemm_f64(wdq, x), "grouped, cfg %s splitK %d" % (cfg, splitK))
 
 
+@pytest.mark.parametrize("E,M", FORMATS)
+@pytest.mark.parametrize("IC", [1088, 1152, 1216, 1280])
+def test_prefill_kernel_stages_zeros_beyond_k(E, M, IC):
+    """The prefill kernel walks K in pairs of 128-column chunks; the part of the last pair that lies beyond K (192, 128, 64 or 0 columns
+    here) must be staged as zeros.  One infinite activation per batch row, in turn at every position that shares an LDS slot with a
+    position beyond K, meets non-zero weights: outputs are infinite where it stands, and a stale copy of it would turn them into NaN."""
+    print("case prefill beyond K", E, M, IC, flush=True)
+    OC, N, cfg = 256, 130, (2, 8, 4, 2, 2)
+    assert cfg in WS_SHAPES
+    codes = np.random.default_rng(IC).integers(1, 1 << (E + M), (OC, IC)).astype(np.uint8)   # no zero weights
+    raw = quant.pack_raw(codes, E, M)
+    sc = np.ones(OC, dtype=np.float16)
+    x = synth.activations(IC, N, IC)
+    last = (IC + 255) // 256 * 256
+    for n in range(0, N, 2):
+        x[n, IC - 1 - (n * 7) % (256 + last - IC)] = np.inf      # the stage of a chunk was last filled 256 columns earlier
+    native, scd, xd = upload(raw, sc, x, E, M)
+    for splitK in (1, 2):
+        y = gemm_capi(E, M, native, scd, xd, OC, splitK, cfg)
+        assert np.isinf(y[0::2]).all(), "splitK %d" % splitK
+        check_close(y[1::2], oracle.gemm_f64(oracle.dequant(raw, sc, E, M), x[1::2]), "IC %d splitK %d" % (IC, splitK))
+
+
 @pytest.mark.parametrize("OC,cfg,N,splitK", [
     (256, (1, 2, 1, 4, 4), 17, 3),     # 4 row blocks x 3 splits = 12 workgroups: four XCDs get two triples, four get one
     (768, (1, 2, 2, 4, 1), 40, 5),     # 6 row blocks x 5 splits x 2 column blocks = 60: XCD boundaries cut row blocks

@@ -254,6 +254,23 @@ def test_measured_table_holds_only_compiled_shapes_and_query_launch_follows_it()
     assert L.fp6mi_query_launch(3, 2, 100, 1, 64, 1, shape) == -2 and L.fp6mi_query_launch(4, 3, 256, 1, 64, 1, shape) == -1
 
 
+@pytest.mark.parametrize("OC,IC,N,splitK,prefill", [
+    (4608, 4544, 777, 1, True),        # 252 workgroups of 128 x 128 (one round) against 126 of 256 x 128
+    (4608, 4544, 777, 2, False),       # a split keeps the measured shapes
+    (28672, 8192, 384, 1, True),       # 672 (three rounds) against 336 (two, of twice the length)
+    (28672, 8192, 512, 1, False),      # a measured problem keeps its measured shape
+    (8192, 8192, 4000, 1, False),      # long prompt whose rows are a power of two apart
+    (8192, 8192, 100, 1, False),       # one column block
+    (15616, 2560, 3854, 1, False),     # long prompt, 15 half rounds for 16
+    (3328, 11904, 3495, 1, True),      # long prompt, 3 for 4
+    (256, 1 << 21, 4096, 1, False),    # K beyond the kernel's 32-bit offsets
+])
+def test_prefill_kernel_rule(OC, IC, N, splitK, prefill):
+    shape = (ctypes.c_int * 5)()
+    assert _lib.lib().fp6mi_query_launch(3, 2, OC, N, IC, splitK, shape) == 0
+    assert (tuple(shape) == (2, 8, 4, 2, 2)) == prefill, tuple(shape)
+
+
 @pytest.mark.parametrize("E,M", FORMATS)
 def test_quantizer(E, M):
     x = 1 + E + M
