@@ -1046,10 +1046,12 @@ __global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, c
     // Positions beyond K (the last block of a K that is no multiple of 256) are given an offset outside the buffer, which reads as
     // zero: no branch, and the same number of transfers to wait for in every chunk.  (The buffer form of the instruction also lets the
     // compiler count the raw codes' loads; behind global_load_lds, which it takes for a flat access, it waits for all of them.)
+    // The whole offset is in the vector operand, which the range check compares with the size as it is.  A scalar offset would be taken
+    // off the size first, and with one row in the buffer and K % 256 == 64 the last half block's lies beyond the size.
     const auto xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(X + (size_t)nbase * K), 0, (int)(xlast + K * 2), 0x00027000);
     auto       transfer = [&](int j, uint32_t h, uint32_t stage) __attribute__((always_inline)) {
-        const uint32_t beyond = h * 128 + xpiece * 8 < K ? 0u : 0xc0000000u, off = (row_offset(j) + xpiece * 16) | beyond;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, (lvoid *)(lds + stage * kStage + (wave + 4 * j) * 1024), 16, off, h * 256, 0, 0);
+        const uint32_t pos = h * 128 + xpiece * 8, off = row_offset(j) + (pos < K ? pos * 2 : 0xc0000000u); // (row offset + 2K < 2^29)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, (lvoid *)(lds + stage * kStage + (wave + 4 * j) * 1024), 16, off, 0, 0, 0);
     };
 
     v8h            b[4][NT];

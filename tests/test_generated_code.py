@@ -1,0 +1,74 @@
+"""Properties of the prefill kernel that hold only if the compiler leaves its memory operations as they are written: they are read off the
+gfx950 instructions of the library that this tree builds.  No GPU is needed."""
+import os
+import re
+import shutil
+import struct
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIBRARY = os.path.join(ROOT, "fp6_llm_amd", "libfp6mi.so")
+OBJDUMP = next((p for p in ("/opt/rocm/llvm/bin/llvm-objdump", shutil.which("llvm-objdump") or "") if os.path.exists(p)), None)
+
+pytestmark = pytest.mark.skipif(OBJDUMP is None, reason="needs llvm-objdump of the ROCm compiler")
+
+
+def code_objects(data):
+    """The gfx950 ELF images in a shared library: every translation unit brings one bundle (magic, count, then per entry
+    offset, size, length of the target's name, name)."""
+    magic, pos = b"__CLANG_OFFLOAD_BUNDLE__", 0
+    while (pos := data.find(magic, pos)) >= 0:
+        at = pos + len(magic) + 8
+        for _ in range(struct.unpack_from("<Q", data, pos + len(magic))[0]):
+            offset, size, length = struct.unpack_from("<QQQ", data, at)
+            if data[at + 24:at + 24 + length].endswith(b"gfx950") and size:
+                yield data[pos + offset:pos + offset + size]
+            at += 24 + length
+        pos += len(magic)
+
+
+@pytest.fixture(scope="module")
+def prefill_kernels(tmp_path_factory):
+    """{symbol: [instruction, ...]} of every gemm_prefill instance."""
+    kernels = {}
+    with open(LIBRARY, "rb") as f:
+        images = list(code_objects(f.read()))
+    for i, image in enumerate(images):
+        path = tmp_path_factory.mktemp("elf") / ("%d.elf" % i)
+        path.write_bytes(image)
+        table = subprocess.run([OBJDUMP, "-t", str(path)], capture_output=True, text=True, check=True).stdout
+        names = sorted({line.split()[-1] for line in table.splitlines() if "gemm_prefill" in line and not line.endswith(".kd")})
+        if not names:
+            continue
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", "--disassemble-symbols=" + ",".join(names), str(path)],
+                              capture_output=True, text=True, check=True).stdout
+        name = None
+        for line in text.splitlines():
+            head = re.match(r"(?:[0-9a-f]+ )?<(\S+)>:$", line.strip())
+            if head:
+                name = head.group(1) if head.group(1) in names else name   # (a label inside a kernel stays part of it)
+                kernels.setdefault(name, [])
+                continue
+            code = line.split("//")[0].strip()
+            if name and code:
+                kernels[name].append(code)
+    assert len(kernels) == 8, sorted(kernels)   # four formats, with and without group exponents
+    return kernels
+
+
+def is_transfer(code):
+    return code.startswith("buffer_load") and code.endswith(" lds")
+
+
+def test_prefill_transfers_have_their_whole_offset_range_checked(prefill_kernels):
+    """A position beyond K reads as zero because its offset lies beyond the buffer's size.  The hardware compares the vector offset
+    with the size less the scalar offset; a scalar offset larger than the size (one row in the buffer and K % 256 == 64) would
+    leave that to the sign of a difference."""
+    for name, code in prefill_kernels.items():
+        transfers = [c for c in code if is_transfer(c)]
+        assert len(transfers) == 24, name       # eight ahead of the loop, eight for each half block
+        for c in transfers:
+            scalar_offset = re.match(r"buffer_load_dwordx4 v\d+, s\[\d+:\d+\], (\S+) offen( offset:\d+)? lds$", c)
+            assert scalar_offset and scalar_offset.group(1) == "0", (name, c)

@@ -245,6 +245,23 @@ def test_prefill_kernel_stages_zeros_beyond_k(E, M, IC):
         check_close(y[1::2], oracle.gemm_f64(oracle.dequant(raw, sc, E, M), x[1::2]), "IC %d splitK %d" % (IC, splitK))
 
 
+@pytest.mark.parametrize("E,M", FORMATS)
+@pytest.mark.parametrize("N", [1, 129, 257])
+@pytest.mark.parametrize("IC", [64, 320, 1088])
+def test_prefill_kernel_single_row_in_the_last_column_block(E, M, N, IC):
+    """One row of activations in a column block and K % 256 == 64: the last half block lies beyond K for every lane, at offsets
+    that start beyond the end of that one-row buffer."""
+    print("case prefill single row", E, M, N, IC, flush=True)
+    OC, cfg = 256, (2, 8, 4, 2, 2)
+    raw, sc, x = synth.uniform_problem(900 + N + IC, OC, IC, N, E, M)
+    native, scd, xd = upload(raw, sc, x, E, M)
+    ref = oracle.gemm_f64(oracle.dequant(raw, sc, E, M), x)
+    for splitK in (1, 2):
+        y = gemm_capi(E, M, native, scd, xd, OC, splitK, cfg)
+        assert np.isfinite(y).all()
+        check_close(y, ref, "IC %d N %d splitK %d" % (IC, N, splitK))
+
+
 @pytest.mark.parametrize("OC,cfg,N,splitK", [
     (256, (1, 2, 1, 4, 4), 17, 3),     # 4 row blocks x 3 splits = 12 workgroups: four XCDs get two triples, four get one
     (768, (1, 2, 2, 4, 1), 40, 5),     # 6 row blocks x 5 splits x 2 column blocks = 60: XCD boundaries cut row blocks
