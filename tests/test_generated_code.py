@@ -62,6 +62,10 @@ def is_transfer(code):
     return code.startswith("buffer_load") and code.endswith(" lds")
 
 
+def is_vector_memory(code):
+    return re.match(r"(buffer|global|flat|scratch)_(load|store|atomic)", code) is not None
+
+
 def test_prefill_transfers_have_their_whole_offset_range_checked(prefill_kernels):
     """A position beyond K reads as zero because its offset lies beyond the buffer's size.  The hardware compares the vector offset
     with the size less the scalar offset; a scalar offset larger than the size (one row in the buffer and K % 256 == 64) would
@@ -72,3 +76,23 @@ def test_prefill_transfers_have_their_whole_offset_range_checked(prefill_kernels
         for c in transfers:
             scalar_offset = re.match(r"buffer_load_dwordx4 v\d+, s\[\d+:\d+\], (\S+) offen( offset:\d+)? lds$", c)
             assert scalar_offset and scalar_offset.group(1) == "0", (name, c)
+
+
+def test_prefill_waits_cover_every_transfer(prefill_kernels):
+    """Before the barrier of a half block a wavefront waits until all but the last n of its vector memory operations are done, n
+    being the number of weight loads it issues after its last transfer.  Were there fewer of those, for instance because two had
+    been merged, the wait would leave transfers open."""
+    for name, code in prefill_kernels.items():
+        counted = 0
+        for i, c in enumerate(code):
+            wait = re.match(r"s_waitcnt vmcnt\((\d+)\)", c)
+            if not wait or int(wait.group(1)) == 0 or code[i + 1] != "s_barrier":
+                continue
+            counted += 1
+            last = max(j for j in range(i) if is_transfer(code[j]))
+            between = code[last + 1:i]
+            assert not any(b.startswith(("s_cbranch", "s_branch", "s_setpc")) for b in between), name
+            assert sum(is_vector_memory(b) for b in between) >= int(wait.group(1)), (name, c)
+            first = max((j for j in range(last) if code[j] == "s_barrier"), default=0)
+            assert sum(is_transfer(b) for b in code[first:i]) >= 8, name
+        assert counted == 2, (name, counted)    # one for each half block
