@@ -239,21 +239,30 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
 
 // Whether gemm_prefill's 128 x 128 tile replaces the shape `c` of another large-batch kernel.  Its workgroups take a CU as long as half a
 // 256 x 128 one does (7 ns per column of K, measured from 64 to 3600 workgroups) and as long as a 256 x 64 one of the same area, so what
-// decides is the number of rounds on the chip.  Over 205 problems (M 1024-57344, K 1024-28672, N 96-4096, three bit widths; time here / time of
-// the shape before):
-//   * 256 x 128: fewer half rounds 0.63-1.00 up to N 2048; as many 0.95-1.00 up to N 1024, 0.99-1.20 above;
-//     beyond N 2048 0.80-0.89 with an eighth fewer and 0.90-1.07 with less gained (3854 columns, 15 half rounds for 16: 1.07);
-//   * 256 x 64: as many rounds or fewer, two at least, 0.83-0.97 up to N 2048 (1.03-1.06 above); a single round 1.02-1.2;
-//   * up to N 144 the second column block is nearly empty (N 128: 1.09, N 135: 1.02, N 166: 0.98);
-//   * beyond N 2048 with rows of a multiple of 8 KB the activation lines crowd the same channels (8192x8192 N 4096: 1.20).
+// decides first is the number of rounds on the chip.  Time here / time of the other shape on 687 problems (three bit widths, no splits,
+// launches in a captured graph; median and range), where the rule takes it:
+//   * from 256 x 128: fewer half rounds 0.67 (0.61-0.78) up to N 1024, 0.82 (0.65-0.87) up to N 2048; as many, N up to 1024, 0.96 (0.89-0.99);
+//     beyond N 2048 an eighth fewer 0.82 (0.73-1.00);
+//   * from 256 x 64, as many rounds and two at least: 0.90 (0.71-1.00) up to N 1024, 0.87 (0.70-0.98) up to N 2048;
+// and where it does not:
+//   * N up to 144, the second column block nearly empty: 256 x 128 0.98 (0.96-1.01), 256 x 64 1.16 (1.01-1.50);
+//   * one round of 256 x 128 with K below 1024: 1.00 (0.96-1.04), prologue and epilogue are most of it;
+//   * from 256 x 64: a single round 1.19 (1.00-1.86), more rounds 1.29 (0.87-1.44) up to N 1024;
+//   * long prompts, where what the activations cost comes in: with K above 8192, N above 3072 and an eighth fewer half rounds 0.97-1.06 (a quarter fewer
+//     0.79-0.98 up to N 3712), N above 4096 with K above 3072 1.00 (0.89-1.12, no line found between the two; up to K 3072 0.92, 0.85-0.96).
+// Faster here on the whole, but not taken over: as many half rounds of 256 x 128 beyond N 1024 (0.92 up to N 2048, 0.94, 0.87-1.11, above), less than an eighth gained
+// beyond N 2048 (0.88, 0.81-1.02), 256 x 64 beyond N 2048 (0.90, 0.74-1.04; with K above 8192 1.08) and rows of a multiple of 8 KB there (256 x 128 0.92,
+// 0.77-1.11; 256 x 64 0.98, 0.91-1.21).
 inline bool prefill_tile_wins(const LaunchCfg &c, size_t M, size_t N, size_t K, int splitK, int cus)
 {
     if (splitK != 1 || N <= 144 || K > (size_t)1 << 20 || (N > 2048 && K % 4096 == 0)) return false;
+    if ((N > 3712 && K > 8192) || (N > 4096 && K > 3072)) return false;
     auto         rounds = [&](size_t rows, size_t cols) { return (M / rows * ((N + cols - 1) / cols) + cus - 1) / cus; };
     const size_t here = rounds(128, 128);
     if (c.kind == 1 && c.nt == 8 && c.rt == 2 && c.wr == 8 && c.wk == 1) {
-        const size_t half = 2 * rounds(256, 128);
-        return N <= 1024 ? here <= half : N <= 2048 ? here < half : 8 * here <= 7 * half;
+        const size_t half = 2 * rounds(256, 128); // never less than `here`
+        if (N <= 1024) return here < half || here > 2 || K >= 1024;
+        return N <= 2048 ? here < half : 8 * here <= (N > 3072 && K > 8192 ? 6 : 7) * half;
     }
     if (c.nt == 4 && c.rt == 2 && c.wr == 8 && (c.kind == 2 || (c.kind == 1 && c.wk == 1))) return rounds(256, 64) >= 2 && here <= rounds(256, 64) && N <= 2048;
     return false;

@@ -264,6 +264,15 @@ def test_measured_table_holds_only_compiled_shapes_and_query_launch_follows_it()
     (15616, 2560, 3854, 1, False),     # long prompt, 15 half rounds for 16
     (3328, 11904, 3495, 1, True),      # long prompt, 3 for 4
     (256, 1 << 21, 4096, 1, False),    # K beyond the kernel's 32-bit offsets
+    (2816, 5504, 6934, 1, False),      # longer prompts than 4096: 1.12 of the time before, 5 half rounds for 6
+    (5888, 9280, 4841, 1, False),      # 1.10, 7 for 8
+    (2304, 1600, 12360, 1, True),      # but short rows: 0.93
+    (7936, 15104, 3537, 1, False),     # long rows from N 3072 on, 7 for 8: 1.03
+    (2816, 10816, 3634, 1, True),      # a quarter fewer: 0.98
+    (2816, 14528, 4049, 1, False),     # the same close to N 4096: 1.01
+    (12032, 64, 343, 1, False),        # one round of 256 x 128 with little K: 1.02
+    (6912, 1024, 800, 1, True),        # from K 1024 on
+    (17152, 64, 793, 1, True),         # two rounds: 0.93
 ])
 def test_prefill_kernel_rule(OC, IC, N, splitK, prefill):
     shape = (ctypes.c_int * 5)()
