@@ -848,9 +848,13 @@ def test_device_quantizer_at_the_edges_of_its_kernels(E, M, dtype, OC, IC):
     top = quant.max_value(E, M)
     mags = quant.magnitudes(E, M)
     mids = torch.from_numpy((mags[1:] + mags[:-1]) / 2)
-    for r, sc in ((0, 0.0123), (5, 2.0 ** -6), (OC - 1, 1.7)):
+    # scales with so few mantissa bits that a midpoint (five of them) times the scale is exact in the weights' type
+    short = {torch.float16: (37 / 32 * 2.0 ** -7, 2.0 ** -6, 53 / 32), torch.bfloat16: (1.25 * 2.0 ** -7, 2.0 ** -6, 1.75),
+             torch.float32: (0.0123, 2.0 ** -6, 1.7)}[dtype]
+    for r, sc in zip((0, 5, OC - 1), short):
         sc = float(np.float16(sc))
         near = (mids * sc).to(dtype)
+        assert (near.double() == mids * sc).all() and float(torch.tensor(top * sc).to(dtype)) == top * sc
         bits = near.view(torch.int32 if dtype == torch.float32 else torch.int16)
         row = torch.cat([near, (bits + 1).view(dtype), (bits - 1).view(dtype)])
         row = torch.cat([row, -row, torch.tensor([top * sc, 0.0, -0.0, float("nan"), float("inf")]).to(dtype)])
@@ -863,6 +867,10 @@ def test_device_quantizer_at_the_edges_of_its_kernels(E, M, dtype, OC, IC):
     for tile in sorted({0, OC // 16 - 1}):
         rows = w[16 * tile:16 * tile + 16].float().numpy().astype(np.float64)
         codes, sc_host = quant.quantize_rowwise(rows, E, M)
+        for r, sc in zip((0, 5, OC - 1), short):
+            if r // 16 == tile:   # the scale comes out as intended, so every midpoint is met exactly, with both signs
+                assert float(sc_host[r - 16 * tile]) == float(np.float16(sc))
+                assert np.isin(np.abs(rows[r - 16 * tile]) / float(np.float16(sc)), mids.numpy()).sum() >= 2 * len(mids)
         assert np.array_equal(scales[16 * tile:16 * tile + 16].cpu().numpy().view(np.uint16), sc_host.view(np.uint16))
         want = fp6.weight_prepacking_native_cpu(E, M, torch.from_numpy(quant.pack_raw(codes, E, M)))
         assert torch.equal(native[per_tile * tile:per_tile * (tile + 1)].cpu(), want)
