@@ -268,6 +268,12 @@ inline bool prefill_tile_wins(const LaunchCfg &c, size_t M, size_t N, size_t K, 
     return false;
 }
 
+// Whether it replaces the shape the table gives for kSplits[i] on 256 CUs.  A problem that was itself measured keeps its shape.
+inline bool prefill_replaces(const TuneAnswer &a, int i, size_t M, size_t N, size_t K)
+{
+    return !a.exact && prefill_tile_wins(a.cfg[i], M, N, K, kSplits[i], 256);
+}
+
 // Launch shape for a given splitK.
 //  N <= 16: stream kernel.  Row tiles per wavefront (rt) reuse the activation registers, so rt grows with M; wavefronts
 //           per workgroup follow the K blocks of one split and the register budget (16 wavefronts leave 128 VGPRs each).
@@ -278,10 +284,7 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
     LaunchCfg c;
     if (const int i = split_index(splitK); cus == 256 && i >= 0) {
         if (const TuneAnswer *a = tune_lookup(xbits, M, N, K)) {
-            if (a->t[i] > 0.f) { // a problem that was itself measured keeps its shape
-                if (!a->exact && prefill_tile_wins(a->cfg[i], M, N, K, splitK, cus)) return LaunchCfg{ 2, 8, 4, 2, 2 };
-                return a->cfg[i];
-            }
+            if (a->t[i] > 0.f) return prefill_replaces(*a, i, M, N, K) ? LaunchCfg{ 2, 8, 4, 2, 2 } : a->cfg[i];
         }
     }
     size_t    tiles = M / 16, units = (K + 255) / 256, per_split = (units + splitK - 1) / splitK;
@@ -532,7 +535,7 @@ int fp6mi_launch_source(int E, int Mb, size_t M, size_t N, size_t K, int splitK)
     const int i = split_index(splitK);
     if (i >= 0)
         if (const TuneAnswer *a = tune_lookup(1 + E + Mb, M, N, K))
-            if (a->t[i] > 0.f) return a->measured ? 0 : 1;
+            if (a->t[i] > 0.f) return prefill_replaces(*a, i, M, N, K) ? 2 : a->measured ? 0 : 1;
     return 2;
 }
 

@@ -157,7 +157,8 @@ int fp6mi_linear_native_grouped_cfg(int E, int Mbits, void *stream, const void *
 int fp6mi_query_launch(int E, int Mbits, size_t M, size_t N, size_t K, int splitK, int *shape);
 /* Where that choice comes from on a 256-CU part: 0 = this (M, K) was measured (at this batch or the next larger measured
  * one), 1 = carried over from measured problems up to a factor 1.5 away in M and in K, 2 = the rules (no measured
- * neighbour, or a splitK the table does not hold).  Negative: FP6MI_ERR_*.  (No counterpart in the reference.) */
+ * neighbour, a splitK the table does not hold, or the prefill kernel in the place of the shape that the table would give: its rows
+ * do not hold that kernel).  Negative: FP6MI_ERR_*.  (No counterpart in the reference.) */
 int fp6mi_launch_source(int E, int Mbits, size_t M, size_t N, size_t K, int splitK);
 
 /* Device-side conversion reference layout -> native layout (both device pointers), run once per weight matrix. */

@@ -591,6 +591,16 @@ def test_launch_source_tells_measured_from_carried_over_from_rules():
     assert b"library version" in L.fp6mi_tuning_info()
 
 
+def test_launch_source_of_problems_the_prefill_rule_takes():
+    """The prefill kernel is in no row of the table: where it runs, a rule has put it there, also on a measured matrix."""
+    L = _lib.lib()
+    shape = (ctypes.c_int * 5)()
+    for OC, IC, N, prefill in ((28672, 8192, 384, True), (28672, 8192, 512, False), (22016, 4096, 511, True), (4608, 4544, 777, True)):
+        assert L.fp6mi_query_launch(3, 2, OC, N, IC, 1, shape) == 0
+        assert (tuple(shape) == (2, 8, 4, 2, 2)) == prefill
+        assert (L.fp6mi_launch_source(3, 2, OC, N, IC, 1) == 2) == prefill
+
+
 def test_cpp_torch_entry_points_carry_the_reference_names():
     """The torch extension defines the reference's six C++ functions (fp6_llm/csrc/fp6_linear.cuh:50-90) and binds them under the
     reference's Python names (fp6_llm/csrc/pybind.cpp:8-15); the CPU ones must give the oracle's bytes."""
