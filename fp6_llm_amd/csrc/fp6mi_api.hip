@@ -239,18 +239,19 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
 
 // Whether gemm_prefill's 128 x 128 tile replaces the shape `c` of another large-batch kernel.  Its workgroups take a CU as long as half a
 // 256 x 128 one does (7 ns per column of K, measured from 64 to 3600 workgroups) and as long as a 256 x 64 one of the same area, so what
-// decides first is the number of rounds on the chip.  Time here / time of the other shape on 687 problems (three bit widths, no splits,
-// launches in a captured graph; median and range), where the rule takes it:
-//   * from 256 x 128: fewer half rounds 0.67 (0.61-0.78) up to N 1024, 0.82 (0.65-0.87) up to N 2048; as many, N up to 1024, 0.96 (0.89-0.99);
-//     beyond N 2048 an eighth fewer 0.82 (0.73-1.00);
-//   * from 256 x 64, as many rounds and two at least: 0.90 (0.71-1.00) up to N 1024, 0.87 (0.70-0.98) up to N 2048;
-// and where it does not:
-//   * N up to 144, the second column block nearly empty: 256 x 128 0.98 (0.96-1.01), 256 x 64 1.16 (1.01-1.50);
-//   * one round of 256 x 128 with K below 1024: 1.00 (0.96-1.04), prologue and epilogue are most of it;
-//   * from 256 x 64: a single round 1.19 (1.00-1.86), more rounds 1.29 (0.87-1.44) up to N 1024;
-//   * long prompts, where what the activations cost comes in: with K above 8192, N above 3072 and an eighth fewer half rounds 0.97-1.06 (a quarter fewer
+// decides first is the number of rounds on the chip.  Time here / time of the other shape (no splits, launches in a captured graph; median and range).
+// Where the rule takes it, on 873 problems (M 2304-56832, K 64-27584, N 150-3867, all formats), with row scales only and with group exponents:
+//   * from 256 x 128, fewer half rounds and K of 320 at least: 0.82 (0.65-0.94) and 0.85 (0.65-0.99) up to N 1024, 0.84 (0.63-0.95) and 0.88 (0.64-0.99) up to
+//     N 2048; beyond, an eighth fewer, 0.84 (0.77-0.98) and 0.86 (0.80-0.97);
+//   * from 256 x 64, as many rounds and two at least: 0.91 (0.77-1.04) and 0.91 (0.78-1.00); above 1 in 21 problems with row scales only and K of 3840 at least.
+// Where it does not, on 217 problems and (*) on 687 of another sweep, row scales only:
+//   * as many half rounds of 256 x 128, N up to 1024: 1.00 (0.92-1.10), with group exponents, whose loads come twice as often per output, 1.05 (0.95-1.19);
+//   * 256 x 128 with K below 320, prologue and epilogue being most of it: 0.99 (0.95-1.05) with fewer half rounds, with group exponents 1.03 (0.99-1.10);
+//   * (*) N up to 144, the second column block nearly empty: 256 x 128 0.98 (0.96-1.01), 256 x 64 1.16 (1.01-1.50);
+//   * (*) from 256 x 64: a single round 1.19 (1.00-1.86), more rounds 1.29 (0.87-1.44) up to N 1024;
+//   * (*) long prompts, where what the activations cost comes in: with K above 8192, N above 3072 and an eighth fewer half rounds 0.97-1.06 (a quarter fewer
 //     0.79-0.98 up to N 3712), N above 4096 with K above 3072 1.00 (0.89-1.12, no line found between the two; up to K 3072 0.92, 0.85-0.96).
-// Faster here on the whole, but not taken over: as many half rounds of 256 x 128 beyond N 1024 (0.92 up to N 2048, 0.94, 0.87-1.11, above), less than an eighth gained
+// (*) Faster here on the whole, but not taken over: as many half rounds of 256 x 128 beyond N 1024 (0.92 up to N 2048, 0.94, 0.87-1.11, above), less than an eighth gained
 // beyond N 2048 (0.88, 0.81-1.02), 256 x 64 beyond N 2048 (0.90, 0.74-1.04; with K above 8192 1.08) and rows of a multiple of 8 KB there (256 x 128 0.92,
 // 0.77-1.11; 256 x 64 0.98, 0.91-1.21).
 inline bool prefill_tile_wins(const LaunchCfg &c, size_t M, size_t N, size_t K, int splitK, int cus)
@@ -261,8 +262,7 @@ inline bool prefill_tile_wins(const LaunchCfg &c, size_t M, size_t N, size_t K, 
     const size_t here = rounds(128, 128);
     if (c.kind == 1 && c.nt == 8 && c.rt == 2 && c.wr == 8 && c.wk == 1) {
         const size_t half = 2 * rounds(256, 128); // never less than `here`
-        if (N <= 1024) return here < half || here > 2 || K >= 1024;
-        return N <= 2048 ? here < half : 8 * here <= (N > 3072 && K > 8192 ? 6 : 7) * half;
+        return K >= 320 && (N <= 2048 ? here < half : 8 * here <= (N > 3072 && K > 8192 ? 6 : 7) * half);
     }
     if (c.nt == 4 && c.rt == 2 && c.wr == 8 && (c.kind == 2 || (c.kind == 1 && c.wk == 1))) return rounds(256, 64) >= 2 && here <= rounds(256, 64) && N <= 2048;
     return false;

@@ -270,9 +270,12 @@ def test_measured_table_holds_only_compiled_shapes_and_query_launch_follows_it()
     (7936, 15104, 3537, 1, False),     # long rows from N 3072 on, 7 for 8: 1.03
     (2816, 10816, 3634, 1, True),      # a quarter fewer: 0.98
     (2816, 14528, 4049, 1, False),     # the same close to N 4096: 1.01
-    (12032, 64, 343, 1, False),        # one round of 256 x 128 with little K: 1.02
-    (6912, 1024, 800, 1, True),        # from K 1024 on
-    (17152, 64, 793, 1, True),         # two rounds: 0.93
+    (12032, 64, 343, 1, False),        # one round of 256 x 128, two half as long: 1.03, with group exponents 1.08
+    (17920, 6016, 218, 1, False),      # the same: 1.07, with group exponents 1.16
+    (26624, 192, 824, 1, False),       # six half rounds for six: 1.10
+    (27648, 192, 1548, 1, False),      # 11 half rounds for 12, but little K: 1.05, with group exponents 1.10
+    (30208, 320, 1724, 1, True),       # from K 320 on (13 for 14): 0.87, 0.90
+    (2304, 5888, 1520, 1, True),       # one half round for two: 0.66
 ])
 def test_prefill_kernel_rule(OC, IC, N, splitK, prefill):
     shape = (ctypes.c_int * 5)()
