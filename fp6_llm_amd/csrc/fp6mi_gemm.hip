@@ -3,8 +3,8 @@
 // exports one table of entry functions (fp6mi::FormatOps) that the C ABI in fp6mi_api.hip dispatches to.
 //
 // Roles taken over from the reference (usyd-fsalab/fp6_llm, paths relative to it):
-//   gemm_stream, gemm_tile, gemm_ws <- QUANT_GEMM_Kernel   fp6_llm/csrc/include/kernel_matmul.cuh:29-191
-//                    (small batches / batches above 16 / large batches: three organisations of the same GEMM)
+//   gemm_stream, gemm_tile, gemm_ws, gemm_prefill <- QUANT_GEMM_Kernel   fp6_llm/csrc/include/kernel_matmul.cuh:29-191
+//                    (small batches / batches above 16 / large batches, the last two: four organisations of the same GEMM)
 //   splitk_reduce <- SplitK_Reduction         fp6_llm/csrc/include/kernel_reduction.cuh:28-47   (in fp6mi_api.hip)
 //   launchers     <- fpx_linear_kernel        fp6_llm/csrc/fp6_linear.cu:44-102
 // The design is not a translation: weights use the native layout described in fp6mi_host.cpp, go from HBM straight
@@ -948,10 +948,11 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
 // operands step by step as its own MFMAs release them.
 // LDS: two stages of [2*NT*16 rows x 256 bytes], piece p of row n (16 bytes) at slot p ^ (n & 15): eight neighbouring columns at one
 // K position then lie in eight different bank groups.
-// 128 x 128 (RT = NT = 4) takes 215-228 registers and 64 KB, two workgroups per CU.  Measured (us, the shape chosen before -> this):
-// FP6 4608x4544 N 777: 59 -> 39, 9984x3328 N 312: 42 -> 29, 28672x8192 N 384: 215 -> 170, N 1024: 446 -> 403; 18944x2432 N 1305: 152 -> 128;
-// FP5 3584x4928 N 3435: 156 -> 125; FP4 6912x4416 N 2563: 194 -> 161.  Where the rounds come out even it is level (8192x8192 N 512: 62.7 both) or
-// behind (N 4096 at K 8192: 484 against 583).  Tiles of 256 x 128 (RT 8, 400+ registers, one wavefront per SIMD: 3-15 % slower than
+// 128 x 128 (RT = NT = 4) takes 197-227 registers and 64 KB, two workgroups per CU.  Measured on problems that the dispatch gives it (us, in turn
+// in captured graphs, the shape it replaces -> this): FP6 4608x4544 N 777: 62.5 -> 40.4, 9984x3328 N 312: 41.4 -> 31.5, 28672x8192 N 384: 222 -> 185,
+// N 1000: 473 -> 401, 18944x2432 N 1305: 154 -> 131; FP5 3584x4928 N 3435: 151 -> 125; FP4 6912x4416 N 2563: 199 -> 160.  Left to the other shapes: where the
+// rounds come out even it is level (8192x8192 N 512: 62.7 both) or behind (N 4096 at K 8192: 484 against 583), and in a single round of 256 x 64 tiles behind
+// (FP5 with group exponents 4608x4544 N 777: 39.5 against 42.8).  Tiles of 256 x 128 (RT 8, 400+ registers, one wavefront per SIMD: 3-15 % slower than
 // gemm_tile's) and 256 x 256 (RT = NT = 8: spills) were left out.
 // ---------------------------------------------------------------------------------------------------------------
 // f(0), ..., f(RT - 1) with the index as a compile-time constant (a body this long is past what `#pragma unroll` takes)
@@ -1282,12 +1283,24 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 //
 // HBM-bound.  Two organisations of the same arithmetic.  quant_fused: one workgroup of eight wavefronts per 16-row tile reads
 // its rows, finds the scales, and converts; the last three (fp32: two) blocks of every wavefront are still in its registers then,
-// the others are read again, latest first, out of L2 or the 256 MB last-level cache.  quant_row_scales + quant_blocks: a workgroup takes
-// a row, then a wavefront a block, and all weights are read twice.  bf16, us, fused / two kernels: 8192x8192 47 / 54 (184 MB, 3.9 TB/s), 4096x4096
-// 12.6 / 17.4, 28672x8192 137 / 199, 1024x1024 4.2 / 6.4, but 2048x8192 20 / 17 and 1024x8192 15 / 11: 64 or 128 workgroups do not pull
-// enough from memory to pay for a second pass over a long row.  The lines where the two meet lie near 192 tiles and K = 3072.  (Held
-// blocks and wavefronts at 8192x8192: 1 / 2 / 3 / 4 blocks on eight wavefronts 54 / 50 / 46 / 50, four wavefronts 54-59, sixteen 50-54.)
-// A conversion in double precision, code by code through a byte array in scratch memory, took 532 us for the first of these.
+// the others are read again, latest first (past L2: 171 MB fetched at 8192x8192 in bf16, 134 MB of weights and a quarter of them twice).
+// quant_row_scales + quant_blocks: a workgroup takes a row, then a wavefront a block, and all weights are read twice.
+// Measured, us, fused / two kernels (e3m2; rotating through more memory than the caches hold):
+//              bf16            bf16 groups     fp16            fp32            fp32 groups
+//   1024x1024    5.0 /   7.2     5.5 /   7.7     4.9 /   7.2     6.2 /   8.4     6.8 /   9.3
+//   1024x3072    7.5 /   8.3     8.5 /   8.9     8.2 /   8.2    11.8 /  11.1    12.9 /  11.9
+//   1024x8192   17.1 /  11.6    20.7 /  12.9    19.5 /  12.0    27.4 /  17.0    30.2 /  17.6
+//   2048x4096   10.8 /  11.9    12.6 /  13.0    12.1 /  12.2    16.2 /  17.2    17.8 /  17.9
+//   2048x8192   19.2 /  16.6    23.0 /  18.6    22.1 /  17.8    33.5 /  28.0    36.6 /  29.1
+//   2560x4096   11.4 /  14.3    13.2 /  15.6    12.7 /  14.6    17.6 /  20.2    19.3 /  21.1
+//   3072x8192   23.1 /  23.0    26.2 /  25.7    25.3 /  24.4    40.7 /  40.3    43.4 /  40.6
+//   4096x4096   13.8 /  18.0    15.6 /  19.8    15.2 /  19.1    23.5 /  28.1    25.2 /  29.1
+//   8192x8192   49.3 /  55.0    58.9 /  59.2    50.4 /  55.5   103.2 /  97.4   109.0 /  98.1
+// Fewer than 192 workgroups do not pull enough from memory to pay for a second pass over a long row.  The line taken (fused from 192 tiles on, or up to
+// K = 3072) was drawn for bf16; on its wrong side stand 2560x4096 (two kernels taken, up to 20 % behind), 3072x8192 (fused taken, up to 7 %), and with
+// fp32 weights 1024x3072 and 8192x8192 (fused taken, up to 11 %).  e2m1 follows e3m2.  (Held blocks and wavefronts at 8192x8192: 1 / 2 / 3 / 4 blocks on
+// eight wavefronts 54 / 50 / 46 / 50, four wavefronts 54-59, sixteen 50-54.)
+// A conversion in double precision, code by code through a byte array in scratch memory, took 532 us at 8192x8192.
 // ---------------------------------------------------------------------------------------------------------------
 struct bf16_t { uint16_t bits; };
 typedef short v2s __attribute__((ext_vector_type(2)));

@@ -26,7 +26,7 @@ class FPxLinear(torch.nn.Module):
         """group_scales: the layer also holds one exponent byte per row and 128 columns (factor 1 until weights are loaded).
         dequant_above: batch size from which forward() dequantizes the weights to a temporary fp16 matrix on the GPU and calls
         the FP16 library GEMM instead (prefill).  The mixed-input kernel wins while the GEMM is bound by weight bytes; from a
-        few thousand rows the FP16 library runs 1.3-1.5 PFLOP/s against its 0.9-1.0, which pays for the dequantization pass
+        few thousand rows the FP16 library runs 1.3-1.5 PFLOP/s against its 0.9-1.2, which pays for the dequantization pass
         (about 30 us at 8192 x 8192).  "auto" (default) = PREFILL_CROSSOVER rows; None never does (the temporary costs 2 bytes
         per weight for the duration of the call); an integer sets the threshold."""
         super().__init__()
