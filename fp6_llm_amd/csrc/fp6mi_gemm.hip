@@ -402,7 +402,7 @@ template <int FM, bool GS> __device__ __forceinline__ void convert_half(const WF
 // ---------------------------------------------------------------------------------------------------------------
 // gemm_tile: GEMM for batches above 16, where every weight must meet many activation columns.
 //   workgroup = WR x WK wavefronts; tile = (WR*RT*16) rows x (NT*16) columns
-//   grid.x enumerates (row block, column block, split) with column blocks of one row block adjacent on one XCD
+//   grid.x enumerates (row block, column block, split), neighbours on one XCD: tile_of
 // The K blocks of a split are walked in chunks of WK blocks.  Per chunk the workgroup stages the activation chunk
 // [WK][NT*16][256] in LDS (double-buffered, filled by fully coalesced 16-byte loads); wavefront (wr, wk) streams the
 // weights of its RT row tiles for K block wk straight from HBM into VGPRs (prefetched one chunk ahead), converts them
@@ -656,6 +656,29 @@ __device__ __forceinline__ void tile_store(const v4f (&acc)[RT][NT], const v4h (
     tile_flush<NT, RT, WR, NTHREADS, OutT>(out, stage, M, N, mb, nbase, tid);
 }
 
+// Workgroup id -> (row block, split, column block).  Ids that are congruent mod 8 run on one XCD and share its L2, so XCD x is given a
+// run of consecutive triples (the column blocks of a row block read the same weights, its splits write partial sums that one
+// reduction workgroup reads): the first (grid mod 8) XCDs take one triple more than the others.
+// Without a split the triples of the large tiles are counted in panels of 1024 rows, down the rows of a panel before the next column block:
+// the 32 or 64 workgroups that an XCD holds then cover about 1024 rows x 512-1024 columns, and what its L2 fetches for them is about
+// as small as it gets (with all the column blocks of one row block first, a long prompt's activations pass by once for every 256 or 512 rows).
+// Measured at FP6 e3m2, us, rows first -> panels: gemm_prefill 8192x8192 N 4096 582 -> 444, 14336x4096 N 3000 334 -> 306, 28672x8192 N 2048 832 -> 787;
+// gemm_ws 28672x8192 N 2048 914 -> 831, 8192x8192 N 4096 503 -> 472; gemm_tile 256 x 128 8192x8192 N 4096 488 -> 460.  Panels of 512, 2048 and 4096
+// rows: within 2 %, and up to 6 % behind.  Level where the grid is a single round (8192x8192 N 512); 128 x 32 tiles lose by 6 % and keep the rows.
+struct TileId { uint32_t mb, split, nb; };
+template <int TM, int TN> __device__ __forceinline__ TileId tile_of(uint32_t splitK, uint32_t nblocks)
+{
+    constexpr uint32_t kPanel = TM * TN >= 128 * 128 ? 1024 / TM : 1; // row blocks per panel
+    const uint32_t     q = gridDim.x >> 3, r = gridDim.x & 7u, x = blockIdx.x & 7u, id = x * q + (x < r ? x : r) + (blockIdx.x >> 3);
+    if (kPanel > 1 && splitK == 1) {
+        const uint32_t mblocks = gridDim.x / nblocks, first = id / (kPanel * nblocks) * kPanel, in = id - first * nblocks;
+        const uint32_t high = mblocks - first < kPanel ? mblocks - first : kPanel; // the last panel may be lower
+        return TileId{ first + in % high, 0, in / high };
+    }
+    const uint32_t rest = id / nblocks;
+    return TileId{ rest / splitK, rest % splitK, id % nblocks };
+}
+
 template <int FM, bool GS, int NT, int RT, int WR, int WK>
 __global__ __launch_bounds__(WR *WK *kWave) void gemm_tile(const uint8_t *__restrict__ W, const half_t *__restrict__ scales,
                                                            const uint8_t *__restrict__ gexp, const half_t *__restrict__ X, half_t *__restrict__ C,
@@ -672,15 +695,8 @@ __global__ __launch_bounds__(WR *WK *kWave) void gemm_tile(const uint8_t *__rest
     const int wr = wave % WR, wk = wave / WR;
     const int col = lane & 15, q = lane >> 4;
 
-    // grid.x -> (row block, split, column block): workgroup ids that are congruent mod 8 run on one XCD and share its L2, so
-    // XCD x is given a run of consecutive triples (the column blocks of a row block read the same weights, its splits write
-    // partial sums that one reduction workgroup reads): the first (gridDim.x mod 8) XCDs take one triple more than the others
-    uint32_t id = blockIdx.x;
-    {
-        const uint32_t q = gridDim.x >> 3, r = gridDim.x & 7u, x = id & 7u;
-        id = x * q + (x < r ? x : r) + (id >> 3);
-    }
-    const uint32_t nb = id % nblocks, rest = id / nblocks, split = rest % splitK, mb = rest / splitK;
+    const TileId   id = tile_of<WR * RT * 16, TN>(splitK, nblocks);
+    const uint32_t mb = id.mb, split = id.split, nb = id.nb;
     const uint32_t nbase = nb * TN, R0 = (mb * WR + wr) * RT; // first row tile of this wavefront
 
     uint32_t u0 = 0, u1 = units;
@@ -757,13 +773,8 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, q = lane >> 4;
 
-    // grid.x -> (row block, split, column block), every XCD a run of consecutive triples: as in gemm_tile
-    uint32_t id = blockIdx.x;
-    {
-        const uint32_t per = gridDim.x >> 3, r = gridDim.x & 7u, x = id & 7u;
-        id = x * per + (x < r ? x : r) + (id >> 3);
-    }
-    const uint32_t nb = id % nblocks, rest = id / nblocks, split = rest % splitK, mb = rest / splitK;
+    const TileId   id = tile_of<WR * RT * 16, NT * 16>(splitK, nblocks);
+    const uint32_t mb = id.mb, split = id.split, nb = id.nb;
     const uint32_t nbase = nb * TN;
     uint32_t       u0 = 0, u1 = units;
     if (splitK > 1) {
@@ -1003,12 +1014,8 @@ __global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, c
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, q = lane >> 4, wr = wave & 1, wc = wave >> 1;
 
-    uint32_t id = blockIdx.x; // -> (row block, split, column block), every XCD a run of consecutive triples: as in gemm_tile
-    {
-        const uint32_t per = gridDim.x >> 3, r = gridDim.x & 7u, x = id & 7u;
-        id = x * per + (x < r ? x : r) + (id >> 3);
-    }
-    const uint32_t nb = id % nblocks, rest = id / nblocks, split = rest % splitK, mb = rest / splitK;
+    const TileId   id = tile_of<2 * RT * 16, TN>(splitK, nblocks);
+    const uint32_t mb = id.mb, split = id.split, nb = id.nb;
     const uint32_t nbase = nb * TN, R0 = (mb * 2 + wr) * RT;
     uint32_t       u0 = 0, u1 = units;
     if (splitK > 1) {
