@@ -410,6 +410,10 @@ template <int FM, bool GS> __device__ __forceinline__ void convert_half(const WF
 // stride is 256+16 halfs (544 bytes): measured on the MI355X, the 16-column x 4-k-group operand read (ds_read_b128) then runs at
 // the conflict-free rate of 7 cycles per wavefront, against 8.8 cycles at 528 bytes and 32 cycles without padding.
 // The WK partial accumulators are summed through LDS at the end (WK > 1), then scaled and stored.
+// Up to about 200 columns the bound is what passes through a CU's vector L1: about 256 lines in flight, an HBM latency of 1 us for the weights and
+// 0.4 us from L2 for the activations, so a column block more costs the weights' way once more, all of them at the latency of the memory that the first asks.
+// Tiles of 48, 80 and 96 columns exist for the batches that the powers of two miss (FP6 e3m2, us, the best of 32, 64 and 128 columns -> 256 x 80 and
+// 256 x 96 here): 28672x8192 N 72 67.3 -> 48.0, N 160 117 -> 81; 8192x28672 N 72 69 -> 49, N 96 68.9 -> 57.9.
 // ---------------------------------------------------------------------------------------------------------------
 
 // One segment of a tile's K range: K blocks [u0, u1) of row block `mb` against the batch columns from `nbase`, accumulated
@@ -1682,16 +1686,19 @@ int launch_cfg(const LaunchCfg &c, hipStream_t st, const void *W, const void *sc
         FP6MI_CASE(2, 1, 4, 4) FP6MI_CASE(2, 2, 4, 4) FP6MI_CASE(2, 2, 4, 2) FP6MI_CASE(2, 2, 4, 1) FP6MI_CASE(2, 4, 4, 1) FP6MI_CASE(2, 4, 4, 2)
         FP6MI_CASE(4, 2, 4, 2) FP6MI_CASE(4, 2, 4, 1) FP6MI_CASE(4, 4, 4, 1) FP6MI_CASE(4, 4, 2, 1) FP6MI_CASE(4, 4, 2, 2)
         FP6MI_CASE(8, 2, 4, 1) FP6MI_CASE(8, 2, 2, 1) FP6MI_CASE(4, 2, 8, 1) FP6MI_CASE(4, 2, 8, 2) FP6MI_CASE(2, 2, 8, 1) FP6MI_CASE(2, 2, 8, 2) FP6MI_CASE(8, 2, 8, 1) FP6MI_CASE(4, 1, 8, 2) FP6MI_CASE(4, 1, 8, 1) FP6MI_CASE(4, 1, 4, 2) FP6MI_CASE(2, 1, 2, 4)
+        FP6MI_CASE(3, 2, 4, 2) FP6MI_CASE(3, 2, 8, 1) FP6MI_CASE(5, 2, 8, 1) FP6MI_CASE(6, 2, 8, 1)
 #undef FP6MI_CASE
     } else if (c.kind == 2) {
-        // ring depths (2,2): deeper rings on smaller tiles (128 x 64 with (4,2), 128 x 32 and 64 x 64 with (4,3)) measured no faster than
-        // gemm_tile at batches 32-64, where the time goes to the partial sums and the second launch, and are not built
+        // ring depths (weights, activations) that LDS holds: 256 rows (2, 2); 128 rows x 48 columns (3, 3), x 64 and x 80 (3, 2), x 96 (2, 2).  With two stages
+        // the memory pipeline runs empty at every barrier: FP6 e3m2, us, (2, 2) -> these: 10240x8192 N 72 in 3 splits 28.1 -> 25.3, 28672x8192 N 72 54.4 -> 48.7,
+        // N 40 46.5 -> 35.2, 8192x28672 N 72 in 4 splits 54.9 -> 49.4.  What they replace there (tiles of 32, 64 and 128 columns of gemm_tile): 28, 67, 46 and 69.
+        // ((3, 3): the block that K cuts comes through registers; its loads are waited for, and with them every transfer before.)
 #define FP6MI_CASE(NT, RT, WR, PW) \
     if (c.nt == NT && c.rt == RT && c.wr == WR && c.wk == PW) { \
         if constexpr (WR == 2) return launch_prefill<FM, GS, NT / 2, RT>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
-        else return launch_ws<FM, GS, NT, RT, WR, PW, 2, 2>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
+        else return launch_ws<FM, GS, NT, RT, WR, PW, WR == 4 && NT < 6 ? 3 : 2, WR == 4 && NT == 3 ? 3 : 2>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
     }
-        FP6MI_CASE(4, 2, 8, 4) FP6MI_CASE(4, 2, 4, 4) FP6MI_CASE(2, 2, 8, 4) FP6MI_CASE(8, 4, 2, 2)
+        FP6MI_CASE(4, 2, 8, 4) FP6MI_CASE(4, 2, 4, 4) FP6MI_CASE(2, 2, 8, 4) FP6MI_CASE(8, 4, 2, 2) FP6MI_CASE(3, 2, 4, 4) FP6MI_CASE(5, 2, 4, 4) FP6MI_CASE(6, 2, 4, 4)
 #undef FP6MI_CASE
     }
     return FP6MI_ERR_SHAPE;

@@ -29,7 +29,7 @@ STREAM_SMALL = [(0, 1, rt, 1, wk) for rt in (1, 2, 3, 4, 5, 6, 7, 8) for wk in (
 STREAM_WIDE = [(0, 2, 1, 1, 8), (0, 2, 2, 1, 4), (0, 2, 3, 1, 4), (0, 2, 3, 1, 8), (0, 2, 4, 1, 4), (0, 2, 4, 1, 8), (0, 2, 5, 1, 4), (0, 2, 5, 1, 8),
                (0, 2, 6, 1, 4), (0, 2, 7, 1, 4), (0, 2, 8, 1, 4)]   # two 16-column tiles per workgroup, batches 17..32
 TILE = [(1, 2, 1, 4, 4), (1, 2, 1, 2, 4), (1, 2, 2, 4, 1), (1, 2, 2, 4, 2), (1, 4, 1, 4, 2), (1, 4, 1, 8, 2), (1, 4, 2, 4, 2), (1, 4, 2, 8, 1),
-        (1, 8, 2, 8, 1)]
+        (1, 8, 2, 8, 1), (1, 3, 2, 4, 2), (1, 3, 2, 8, 1), (1, 5, 2, 8, 1), (1, 6, 2, 8, 1)]
 SPLITS = (1, 2, 3, 4, 6, 8)      # 3 and 6 fill 256 CUs where 80 or 40 row blocks leave a power of two short (M = 10240, 5120)
 FORMAT_OF_BITS = {6: (3, 2), 5: (2, 2), 4: (2, 1)}   # the table is keyed by bit width
 
@@ -42,11 +42,11 @@ COMPILED_STREAM = [(0, nt, rt, 1, wk) for (nt, rt, wk) in
 COMPILED_TILE = [(1,) + c for c in
                  [(2, 1, 4, 4), (2, 2, 4, 4), (2, 2, 4, 2), (2, 2, 4, 1), (2, 4, 4, 1), (2, 4, 4, 2), (4, 2, 4, 2), (4, 2, 4, 1), (4, 4, 4, 1),
                   (4, 4, 2, 1), (4, 4, 2, 2), (8, 2, 4, 1), (8, 2, 2, 1), (4, 2, 8, 1), (4, 2, 8, 2), (2, 2, 8, 1), (2, 2, 8, 2), (8, 2, 8, 1),
-                  (4, 1, 8, 2), (4, 1, 8, 1), (4, 1, 4, 2), (2, 1, 2, 4)]]
+                  (4, 1, 8, 2), (4, 1, 8, 1), (4, 1, 4, 2), (2, 1, 2, 4), (3, 2, 4, 2), (3, 2, 8, 1), (5, 2, 8, 1), (6, 2, 8, 1)]]
 
 # kind 2 = wave-specialized tile kernel: (2, n_tiles, row_tiles, arithmetic wavefronts, loading wavefronts); with 2 and 2 the prefill kernel
 # (2 x 2 wavefronts, n_tiles of the whole workgroup)
-COMPILED_WS = [(2, 4, 2, 8, 4), (2, 4, 2, 4, 4), (2, 2, 2, 8, 4), (2, 8, 4, 2, 2)]
+COMPILED_WS = [(2, 4, 2, 8, 4), (2, 4, 2, 4, 4), (2, 2, 2, 8, 4), (2, 8, 4, 2, 2), (2, 3, 2, 4, 4), (2, 5, 2, 4, 4), (2, 6, 2, 4, 4)]
 
 BLOCK_BYTES = {6: 3072, 5: 2560, 4: 2048}   # one native 16-row x 256-column block per bit width
 
@@ -61,7 +61,7 @@ def shape_compiled_for(cfg, bits):
 GRID_M = [1024, 2048, 3072, 4096, 5120, 6144, 8192, 10240, 11008, 12288, 14336, 16384, 22016, 28672, 32768]
 GRID_K = [2048, 4096, 5120, 8192, 11008, 14336, 28672]
 GRID_N_SMALL = [1, 4, 8, 12, 16]
-GRID_N_LARGE = [24, 32, 48, 64, 96, 128, 256, 512, 1024, 2048]
+GRID_N_LARGE = [24, 32, 48, 64, 80, 96, 128, 160, 192, 256, 320, 512, 1024, 2048]
 MAX_WEIGHTS = 240 * 1000 * 1000   # the grid skips matrices beyond the largest layer of a 70B model (28672 x 8192)
 # Layer shapes (OC, IC) of common decoder models that the grid does not hit: hidden/MLP sizes 2560, 3072, 3584, 5120, 6656,
 # 7168 with their fused QKV and gate+up projections (13B/14B/30B/32B LLaMA- and Qwen-shaped models, 7B Qwen2, Gemma, Phi-3,
@@ -109,7 +109,7 @@ def _all_candidates(OC, IC, BS, bits=6):
             cfgs = cfgs + STREAM_WIDE + STREAM_SMALL   # a tile kernel would have to split K to fill the chip (4096 x 4096 batch 24-64)
         elif BS <= 128 and OC <= 2560:   # the same for matrices of so few rows that even at batch 128 no tile shape fills the chip
             cfgs = cfgs + STREAM_WIDE + STREAM_SMALL
-        if BS >= 96:    # the wave-specialized tiles pay from about 128 columns up (256 x 64 from 256 up on 8192 x 8192)
+        if BS >= 48:    # the wave-specialized tiles: 128 rows from 33 columns up, 256 rows from about 128 up
             cfgs = cfgs + [c for c in COMPILED_WS if c[1] * 16 <= BS]
     units = (IC + 255) // 256
     for cfg in cfgs:
@@ -118,7 +118,7 @@ def _all_candidates(OC, IC, BS, bits=6):
         for sk in SPLITS:
             if sk > units or (cfg[0] == 0 and sk > 1 and OC > 4096):   # the stream kernel splits K inside the workgroup already
                 continue
-            if sk > 1 and (sk * 8 * BS > IC * 0.75 or BS > 512):   # the FP32 partial sums would outweigh the weights themselves
+            if sk > 1 and ((sk * 8 * BS > IC * 0.75 and OC > 2560) or BS > 512):   # the FP32 partial sums would outweigh the weights themselves (with few rows they are small all the same)
                 continue
             yield cfg, sk
 
