@@ -399,6 +399,10 @@ def _sort_forward_args(a, b, c):
 def linear_forward_eXmY_cuda(EXPONENT, MANTISSA, in_feats, weights, scales, splitK=1):
     """Drop-in for fp_eXmY_linear_forward_cuda (fp6_linear.cu:269-313): `weights` is the REFERENCE prepacked layout
     (int32 [OC, IC/32*x] on the GPU).  Its native-layout twin is built by one relayout kernel on first use."""
+    if _ext is not None:
+        out = _ext.linear_forward_any_order(EXPONENT, MANTISSA, in_feats, weights, scales, int(splitK), _native_of)
+        if out is not None:
+            return out
     in_feats, weights, scales = _sort_forward_args(in_feats, weights, scales)
     OC, IC = _weight_shape(weights, EXPONENT, MANTISSA, "weights")
     if weights.device.type != "cuda":

@@ -574,6 +574,31 @@ def test_torch_extension_and_ctypes_binding_agree(monkeypatch):
         check_close(y_ext.cpu().numpy(), oracle.gemm_f64(oracle.dequant(raw, sc, E, M), x), "extension path N=%d" % N)
 
 
+@pytest.mark.parametrize("E,M", FORMATS)
+def test_drop_in_call_through_extension_and_python_agree(E, M, monkeypatch):
+    """Every accepted form of the drop-in call -- the three tensors in any order, strided activations and scales, odd batches, a split -- gives
+    the same bits whether its checks run in the extension or in Python; a refused one is refused by both."""
+    print("case drop-in forms", E, M, flush=True)
+    OC, IC = 256, 320
+    raw, sc, x = synth.uniform_problem(640, OC, IC, 34, E, M)
+    packed = fp6.weight_prepacking_eXmY_cpu(E, M, torch.from_numpy(raw)).to(DEV)
+    scd, xd = torch.from_numpy(sc).to(DEV), torch.from_numpy(x).to(DEV)
+    forms = [((a, b, c), splitK) for xs in (xd[:1], xd[:17], xd[::2], xd.t().contiguous().t(), xd[1:4]) for splitK in (1, 2)
+             for ss in (scd, scd.repeat_interleave(2)[::2]) for a, b, c in ((xs, packed, ss), (packed, ss, xs), (ss, xs, packed))]
+    refused = [(xd[:, :64], packed, scd), (xd, packed, scd[:-1]), (xd.cpu(), packed, scd), (xd, packed, scd.cpu()), (xd[:0], packed, scd),
+               (xd, packed.t().contiguous().t(), scd)]
+    got = []
+    for ext in (fp6._ext, None):
+        monkeypatch.setattr(fp6, "_ext", ext)
+        got.append([fp6.linear_forward_eXmY_cuda(E, M, *args, splitK) for args, splitK in forms])
+        for args in refused:
+            with pytest.raises(ValueError):
+                fp6.linear_forward_eXmY_cuda(E, M, *args)
+        monkeypatch.undo()
+    for i, (y_ext, y_py) in enumerate(zip(*got)):
+        assert torch.equal(y_ext, y_py), i
+
+
 def test_cpp_api_driver():
     """The reference-named C++ API (fp6_llm_amd/csrc/fp6_linear.h) through the command-line driver, in the order the
     reference's C++ test uses it: dequantize, prepack in place, upload, GEMM."""

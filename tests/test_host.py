@@ -187,6 +187,26 @@ def test_python_api_argument_errors():
         fp6.linear_forward_cuda(torch.zeros(1, 64, dtype=torch.float16), t, torch.ones(256, dtype=torch.float16), 1)  # not on GPU
 
 
+def test_drop_in_call_refuses_the_same_arguments_with_and_without_the_extension(monkeypatch):
+    """The drop-in call checks its arguments in the extension where that is built: what is refused, and with which words, is what the
+    Python checks say.  (On the CPU every call ends at the latest at the weights, which have to be on the GPU.)"""
+    if fp6._ext is None:
+        pytest.skip("the torch extension is not built")
+    w, x, sc = torch.zeros(256, 12, dtype=torch.int32), torch.zeros(3, 64, dtype=torch.float16), torch.ones(256, dtype=torch.float16)
+    calls = [(3, 2, x, w, sc), (3, 2, w, sc, x), (2, 2, x, w, sc), (2, 1, sc, x, w), (4, 3, x, w, sc), (2, 3, x[:, :32], w, sc), (3, 2, x.float(), w, sc),
+             (3, 2, x, w, sc.float()), (3, 2, x, w.long(), sc), (3, 2, x, w, w), (3, 2, x, x, sc), (3, 2, x, w, x), (3, 2, x[0], w, sc), (3, 2, x, w, sc[None, None]),
+             (3, 2, x, w[0], sc), (3, 2, x, w[0, 0], sc), (3, 2, x, w[:, :11], sc), (3, 2, x, w.t(), sc), (3, 2, x, None, sc), (3, 2, x, w.numpy(), sc)]
+    for call in calls:
+        said = []
+        for ext in (fp6._ext, None):
+            monkeypatch.setattr(fp6, "_ext", ext)
+            with pytest.raises(Exception) as e:
+                fp6.linear_forward_eXmY_cuda(*call)
+            said.append((type(e.value), str(e.value)))
+        monkeypatch.undo()
+        assert said[0] == said[1], call
+
+
 def test_reference_heuristic_is_kept_verbatim():
     for args in [(4096, 8, 108), (11008, 8, 108), (8192, 512, 256), (256, 1, 108), (28672, 32, 108), (4096, 8, 256)]:
         assert fp6.HeuristicFuntion_SplitK(*args) == oracle.heuristic_splitk(*args)
