@@ -965,8 +965,9 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
 // K position then lie in eight different bank groups.
 // 128 x 128 (RT = NT = 4) takes 197-227 registers and 64 KB, two workgroups per CU.  Measured on problems that the dispatch gives it (us, in turn
 // in captured graphs, the shape it replaces -> this): FP6 4608x4544 N 777: 62.5 -> 40.4, 9984x3328 N 312: 41.4 -> 31.5, 28672x8192 N 384: 222 -> 185,
-// N 1000: 473 -> 401, 18944x2432 N 1305: 154 -> 131; FP5 3584x4928 N 3435: 151 -> 125; FP4 6912x4416 N 2563: 199 -> 160.  Left to the other shapes: where the
-// rounds come out even it is level (8192x8192 N 512: 62.7 both) or behind (N 4096 at K 8192: 484 against 583), and in a single round of 256 x 64 tiles behind
+// N 1000: 473 -> 401, 18944x2432 N 1305: 154 -> 131; FP5 3584x4928 N 3435: 151 -> 125; FP4 6912x4416 N 2563: 199 -> 160.  With tiles counted in panels
+// also where the rounds come out even (FP6 8192x7168 N 1676: 198 -> 184, 16384x13824 N 858: 366 -> 346, 16384x6656 N 2482: 474 -> 437).  Left to the other shapes: up to N 512 with even
+// rounds, where it is level (8192x8192 N 512: 62.7 both), and a single round of 256 x 64 tiles, where it is behind
 // (FP5 with group exponents 4608x4544 N 777: 39.5 against 42.8).  Tiles of 256 x 128 (RT 8, 400+ registers, one wavefront per SIMD: 3-15 % slower than
 // gemm_tile's) and 256 x 256 (RT = NT = 8: spills) were left out.
 // ---------------------------------------------------------------------------------------------------------------
@@ -1293,8 +1294,8 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 // residual turns q into the quotient rounded to odd (truncated, last bit set if inexact), which never sits on a midpoint.
 //
 // HBM-bound.  Two organisations of the same arithmetic.  quant_fused: one workgroup of eight wavefronts per 16-row tile reads
-// its rows, finds the scales, and converts; the last three (fp32: two) blocks of every wavefront are still in its registers then,
-// the others are read again, latest first (past L2: 171 MB fetched at 8192x8192 in bf16, 134 MB of weights and a quarter of them twice).
+// its rows, finds the scales, and converts; the last two blocks of every wavefront are still in its registers then, with 16-bit weights the one
+// before them in LDS, and the others are read again, latest first (8192x8192: a quarter of the weights twice).
 // quant_row_scales + quant_blocks: a workgroup takes a row, then a wavefront a block, and all weights are read twice.
 // Measured, us, fused / two kernels (e3m2; rotating through more memory than the caches hold):
 //              bf16            bf16 groups     fp16            fp32            fp32 groups
@@ -1309,8 +1310,11 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 //   8192x8192   49.3 /  55.0    58.9 /  59.2    50.4 /  55.5   103.2 /  97.4   109.0 /  98.1
 // Fewer than 192 workgroups do not pull enough from memory to pay for a second pass over a long row.  The line taken (fused from 192 tiles on, or up to
 // K = 3072) was drawn for bf16; on its wrong side stand 2560x4096 (two kernels taken, up to 20 % behind), 3072x8192 (fused taken, up to 7 %), and with
-// fp32 weights 1024x3072 and 8192x8192 (fused taken, up to 11 %).  e2m1 follows e3m2.  (Held blocks and wavefronts at 8192x8192: 1 / 2 / 3 / 4 blocks on
-// eight wavefronts 54 / 50 / 46 / 50, four wavefronts 54-59, sixteen 50-54.)
+// fp32 weights 1024x3072 and 8192x8192 (fused taken, up to 11 %).  e2m1 follows e3m2.  (The 16-bit columns of "fused" are those of three blocks in registers
+// and none in LDS.  That takes more than 128 registers with group exponents, and the CU then holds one workgroup; a block in LDS and two in registers leave
+// room for two with either.  us, bf16, before -> now, row scales and group exponents: 4096x4096 13.6 -> 13.2, 15.4 -> 14.9; 8192x7168 34.9 -> 33.8, 44.5 -> 36.6;
+// 8192x8192 49.1 -> 47.6, 57.6 -> 49.6; 28672x4096 61.5 -> 61.0, 87.5 -> 64.3; 8192x28672 178 -> 176, 179 -> 182.  Three in registers and one in LDS, nothing read
+// twice at 8192 columns: 51.4, 53.7 with one workgroup to a CU, 51.9, 56.1 held to 128 registers, which spills.)
 // A conversion in double precision, code by code through a byte array in scratch memory, took 532 us at 8192x8192.
 // ---------------------------------------------------------------------------------------------------------------
 struct bf16_t { uint16_t bits; };
@@ -1464,8 +1468,12 @@ __device__ __forceinline__ void quantize_block(const WeightPiece<T> (&x)[8], flo
     store_native_strings<FM>(str[0], str[1], native + blk * Fmt<FM>::block_bytes, (lane >> 2) + 16 * (lane & 3));
 }
 
+// One block more of every wavefront waits in LDS, where a row has more than KEEP of them a wavefront and the weights 16 bits (64 KB; 32-bit ones would
+// take 128 KB and with it the CU's second workgroup).  It goes there straight from memory, lane l to byte 16 * l of its piece.
+template <typename T, int WAVES> constexpr uint32_t quant_stash_bytes() { return sizeof(T) == 2 ? WAVES * 8 * 1024 : 0; }
+
 template <int FM, typename T, bool GROUPS, int WAVES, int KEEP>
-__global__ __launch_bounds__(WAVES *kWave) void quant_fused(uint8_t *__restrict__ native, half_t *__restrict__ scales, uint8_t *__restrict__ gexp,
+__global__ __launch_bounds__(WAVES *kWave, sizeof(T) == 2 ? WAVES / 2 : 1) void quant_fused(uint8_t *__restrict__ native, half_t *__restrict__ scales, uint8_t *__restrict__ gexp,
                                                             const T *__restrict__ Wf, uint32_t K, uint32_t units)
 {
     __shared__ float  wave_max[WAVES][16];
@@ -1474,11 +1482,24 @@ __global__ __launch_bounds__(WAVES *kWave) void quant_fused(uint8_t *__restrict_
     const uint32_t    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), R = blockIdx.x;
     const T          *w = Wf + (size_t)R * 16 * K;
 
-    // blocks wave, wave + WAVES, ...; the last KEEP of them stay in registers (kept[0] is the very last)
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    typedef __attribute__((address_space(1))) void gvoid;
+    typedef __attribute__((address_space(3))) void lvoid;
+
+    // blocks wave, wave + WAVES, ...; the last KEEP of them stay in registers (kept[0] is the very last), the one before them in LDS
     const uint32_t  mine = wave < units ? (units - wave + WAVES - 1) / WAVES : 0;
     MaxMagnitude<T> mm;
     WeightPiece<T>  kept[KEEP][8];
-    for (uint32_t i = 0; i + KEEP < mine; i++) {
+    constexpr bool  kStash = quant_stash_bytes<T, WAVES>() != 0;
+    const bool      stash = kStash && mine > KEEP;
+    const uint32_t  held = KEEP + (stash ? 1 : 0);
+    uint8_t *const  area = lds + wave * (8 * 1024);
+    if (stash) { // (never the block that K cuts: that is the last one of the row, and the last of its wavefront)
+        const T *p = w + (size_t)(lane >> 2) * K + (size_t)(wave + (mine - 1 - KEEP) * WAVES) * 256 + 8 * (lane & 3);
+#pragma unroll
+        for (int s = 0; s < 8; s++) __builtin_amdgcn_global_load_lds((gvoid *)(p + 32 * s), (lvoid *)(area + s * 1024), 16, 0, 0);
+    }
+    for (uint32_t i = 0; i + held < mine; i++) {
         WeightPiece<T> x[8];
         load_quant_block<T>(x, w, K, wave + i * WAVES, lane);
 #pragma unroll
@@ -1493,6 +1514,18 @@ __global__ __launch_bounds__(WAVES *kWave) void quant_fused(uint8_t *__restrict_
 #pragma unroll
             for (int s = 0; s < 8; s++) mm.add(kept[k][s]);
         }
+    auto stashed = [&](WeightPiece<T>(&x)[8]) {
+        if constexpr (kStash)
+#pragma unroll
+            for (int s = 0; s < 8; s++) x[s].x = *reinterpret_cast<const v4u *>(area + s * 1024 + lane * 16);
+    };
+    if (stash) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the transfers into LDS; the loads above have been waited for
+        WeightPiece<T> x[8];
+        stashed(x);
+#pragma unroll
+        for (int s = 0; s < 8; s++) mm.add(x[s]);
+    }
     float amax = mm.value();
     amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
     amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
@@ -1514,7 +1547,13 @@ __global__ __launch_bounds__(WAVES *kWave) void quant_fused(uint8_t *__restrict_
             const uint32_t U = wave + (mine - 1 - k) * WAVES;
             quantize_block<FM, T, GROUPS>(kept[k], sc, native, gexp, (size_t)R * units + U, K, U, lane);
         }
-    for (uint32_t i = mine > KEEP ? mine - KEEP : 0; i-- > 0;) {
+    if (stash) {
+        WeightPiece<T> x[8];
+        const uint32_t U = wave + (mine - 1 - KEEP) * WAVES;
+        stashed(x);
+        quantize_block<FM, T, GROUPS>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+    }
+    for (uint32_t i = mine > held ? mine - held : 0; i-- > 0;) {
         WeightPiece<T> x[8];
         const uint32_t U = wave + i * WAVES;
         load_quant_block<T>(x, w, K, U, lane);
@@ -1750,28 +1789,25 @@ template <int FM> int op_quantize(void *stream, void *native, void *scales, void
         typedef std::remove_cv_t<std::remove_pointer_t<decltype(typed)>> T;
         constexpr bool GROUPS = decltype(groups_c)::value;
         if (M / 16 >= 192 || K <= 3072) { // (where the two organisations cross: see quant_fused)
-            constexpr int WAVES = 8, KEEP = sizeof(T) == 2 ? 3 : 2;
-            hipLaunchKernelGGL((quant_fused<FM, T, GROUPS, WAVES, KEEP>), dim3((uint32_t)(M / 16)), dim3(WAVES * kWave), 0, st, nat, sc, ge, typed,
+            constexpr int WAVES = 8, KEEP = 2;
+            const uint32_t stash = units > WAVES * KEEP ? quant_stash_bytes<T, WAVES>() : 0; // what some wavefront needs
+            if (stash)
+                if (int rc = allow_dynamic_lds<quant_fused<FM, T, GROUPS, WAVES, KEEP>>(stash)) return rc;
+            hipLaunchKernelGGL((quant_fused<FM, T, GROUPS, WAVES, KEEP>), dim3((uint32_t)(M / 16)), dim3(WAVES * kWave), stash, st, nat, sc, ge, typed,
                                (uint32_t)K, units);
         } else {
             hipLaunchKernelGGL((quant_row_scales<FM, T>), dim3((uint32_t)M), dim3(256), 0, st, sc, typed, (uint32_t)K);
             hipLaunchKernelGGL((quant_blocks<FM, T, GROUPS>), dim3((uint32_t)((blocks + 3) / 4)), dim3(256), 0, st, nat, sc, ge, typed, (uint32_t)M,
                                (uint32_t)K, units);
         }
+        return (int)hipGetLastError();
     };
     auto typed = [&](auto groups_c) {
-        if (dtype == 0)
-            run(static_cast<const half_t *>(weights), groups_c);
-        else if (dtype == 1)
-            run(static_cast<const bf16_t *>(weights), groups_c);
-        else
-            run(static_cast<const float *>(weights), groups_c);
+        if (dtype == 0) return run(static_cast<const half_t *>(weights), groups_c);
+        if (dtype == 1) return run(static_cast<const bf16_t *>(weights), groups_c);
+        return run(static_cast<const float *>(weights), groups_c);
     };
-    if (gexp)
-        typed(std::true_type{});
-    else
-        typed(std::false_type{});
-    return (int)hipGetLastError();
+    return gexp ? typed(std::true_type{}) : typed(std::false_type{});
 }
 
 } // namespace

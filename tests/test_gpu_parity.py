@@ -599,6 +599,26 @@ def test_drop_in_call_through_extension_and_python_agree(E, M, monkeypatch):
         assert torch.equal(y_ext, y_py), i
 
 
+@pytest.mark.parametrize("IC", [4032, 4096, 4160, 6144, 6208, 8192, 8256, 12352])   # 16, 17, 24, 25, 32, 33 and 49 blocks: which wavefronts hold one in LDS
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_fused_quantizer_equals_the_two_kernel_one(IC, dtype):
+    """Many rows take the fused quantizer, 256 rows of this length the two-kernel one: a row's codes do not depend on its neighbours, so the
+    bytes must be the same.  One row holds zeros, one an infinity and a NaN at the ends of a block."""
+    print("case fused quantizer", IC, dtype, flush=True)
+    OC = 3072
+    w = (torch.randn(OC, IC, generator=torch.Generator().manual_seed(IC)) * 0.02).to(dtype)
+    w[5], w[300, 0], w[300, IC - 1] = 0, float("inf"), float("nan")
+    w = w.to(DEV)
+    for E, M in FORMATS:
+        for groups in (False, True):
+            whole = fp6.weight_quantize_native_cuda(E, M, w, groups)
+            for r in range(0, OC, 256):
+                part = fp6.weight_quantize_native_cuda(E, M, w[r:r + 256], groups)
+                for a, b in zip(whole, part):
+                    n = b.numel()
+                    assert torch.equal(a[r // 256 * n:(r // 256 + 1) * n].view(torch.uint8), b.view(torch.uint8)), (E, M, groups, r)
+
+
 def test_cpp_api_driver():
     """The reference-named C++ API (fp6_llm_amd/csrc/fp6_linear.h) through the command-line driver, in the order the
     reference's C++ test uses it: dequantize, prepack in place, upload, GEMM."""
