@@ -244,7 +244,12 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
 //   * from 256 x 128, fewer half rounds and K of 320 at least: 0.82 (0.65-0.94) and 0.85 (0.65-0.99) up to N 1024, 0.84 (0.63-0.95) and 0.88 (0.64-0.99) up to
 //     N 2048; beyond, an eighth fewer, 0.84 (0.77-0.98) and 0.86 (0.80-0.97);
 //   * from 256 x 64, as many rounds and two at least: 0.91 (0.77-1.04) and 0.91 (0.78-1.00); above 1 in 21 problems with row scales only and K of 3840 at least.
-// Where it does not, on 217 problems and (*) on 687 of another sweep, row scales only:
+// Since large tiles are counted in panels, on problems with M 1024-28672, K 1024-28672 (6, 5 and 4 bits; row scales, then group exponents):
+//   * from 256 x 128 between N 512 and 3072 it takes over whatever the rounds: as many half rounds 0.94 (0.83-1.02) on 1160 problems and 0.97 (0.87-1.04) on 368, fewer
+//     0.85 (0.73-0.91) on 249 and 0.88 (0.77-0.94) on 83; rows of a multiple of 8 KB are no exception any more (N above 2048: 0.88, 0.73-1.00, and 0.92, 0.77-1.03);
+//   * from 256 x 64 between N 2048 and 3072: 0.97 (0.87-1.05) on 208 and 0.90 (0.83-0.96) on 73, above 1.02 on 8, all with row scales only.
+// Beyond N 3072 the lines are those of before the panels, and so they are up to N 512 and for K below 1024.
+// Where it did not win before the panels, on 217 problems and (*) on 687 of another sweep, row scales only:
 //   * as many half rounds of 256 x 128, N up to 1024: 1.00 (0.92-1.10), with group exponents, whose loads come twice as often per output, 1.05 (0.95-1.19);
 //   * 256 x 128 with K below 320, prologue and epilogue being most of it: 0.99 (0.95-1.05) with fewer half rounds, with group exponents 1.03 (0.99-1.10);
 //   * (*) N up to 144, the second column block nearly empty: 256 x 128 0.98 (0.96-1.01), 256 x 64 1.16 (1.01-1.50);
@@ -256,15 +261,16 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
 // 0.77-1.11; 256 x 64 0.98, 0.91-1.21).
 inline bool prefill_tile_wins(const LaunchCfg &c, size_t M, size_t N, size_t K, int splitK, int cus)
 {
-    if (splitK != 1 || N <= 144 || K > (size_t)1 << 20 || (N > 2048 && K % 4096 == 0)) return false;
+    if (splitK != 1 || N <= 144 || K > (size_t)1 << 20 || (N > 3072 && K % 4096 == 0)) return false;
     if ((N > 3712 && K > 8192) || (N > 4096 && K > 3072)) return false;
     auto         rounds = [&](size_t rows, size_t cols) { return (M / rows * ((N + cols - 1) / cols) + cus - 1) / cus; };
     const size_t here = rounds(128, 128);
     if (c.kind == 1 && c.nt == 8 && c.rt == 2 && c.wr == 8 && c.wk == 1) {
         const size_t half = 2 * rounds(256, 128); // never less than `here`
+        if (N > 512 && N <= 3072 && K >= 1024) return true;
         return K >= 320 && (N <= 2048 ? here < half : 8 * here <= (N > 3072 && K > 8192 ? 6 : 7) * half);
     }
-    if (c.nt == 4 && c.rt == 2 && c.wr == 8 && (c.kind == 2 || (c.kind == 1 && c.wk == 1))) return rounds(256, 64) >= 2 && here <= rounds(256, 64) && N <= 2048;
+    if (c.nt == 4 && c.rt == 2 && c.wr == 8 && (c.kind == 2 || (c.kind == 1 && c.wk == 1))) return rounds(256, 64) >= 2 && here <= rounds(256, 64) && N <= 3072;
     return false;
 }
 
