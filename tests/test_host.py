@@ -624,6 +624,17 @@ def test_launch_source_of_problems_the_prefill_rule_takes():
         assert (L.fp6mi_launch_source(3, 2, OC, N, IC, 1) == 2) == prefill
 
 
+def test_every_matrix_of_the_table_is_measured_at_every_batch():
+    """A matrix with no row at a batch is answered from its neighbours there: 9216 x 9216 in FP5 was cut into four at 257 to 320 columns, where it and
+    each of its neighbours are fastest unsplit (and four pieces do not fit the static workspace)."""
+    inc = open(os.path.join(os.path.dirname(fp6.__file__), "csrc", "fp6mi_tuning.inc")).read()
+    rows = {tuple(map(int, r)) for r in re.findall(r"^\{(\d+),(\d+),(\d+),(\d+),\{\{", inc, re.M)}
+    matrices, batches = {r[1:3] for r in rows}, {r[3] for r in rows}
+    assert len(rows) == 3 * len(matrices) * len(batches)
+    for N in range(257, 321):
+        assert fp6.heuristic_splitk_mi355x(9216, N, 9216, EXPONENT=2, MANTISSA=2) == 1, N
+
+
 def test_cpp_torch_entry_points_carry_the_reference_names():
     """The torch extension defines the reference's six C++ functions (fp6_llm/csrc/fp6_linear.cuh:50-90) and binds them under the
     reference's Python names (fp6_llm/csrc/pybind.cpp:8-15); the CPU ones must give the oracle's bytes."""
