@@ -29,13 +29,15 @@ from ._lib import Fp6miError  # noqa: F401
 # The native library is loaded on first use (every entry point raises ImportError while it is missing: there is no other
 # path), so that `python -m fp6_llm_amd.build` can import this package before anything is built.  The torch extension links
 # against it and is only tried once it is there.  A library left over from an older source tree (a symbol missing) must not
-# stop the import either, or the build module could not be started to replace it: the first real call reports it.
+# stop the import either, or the build module could not be started to replace it: the first real call reports it.  An extension
+# left over from one is not used.
 _ext = None
 if os.path.exists(_lib.LIB_PATH) and not os.environ.get("FP6MI_NO_TORCH_EXT"):
     try:
         _lib.lib()
         from . import _fp6mi_torch as _ext
-    except (ImportError, OSError, AttributeError):   # extension not built, or a stale library: the ctypes path reports what is wrong
+        _ext.linear_forward_any_order   # the newest of the names used below
+    except (ImportError, OSError, AttributeError):   # extension not built or stale, or a stale library: the ctypes path reports what is wrong
         _ext = None
 
 __all__ = [

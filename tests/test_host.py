@@ -6,6 +6,8 @@ import hashlib
 import json
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -205,6 +207,21 @@ def test_drop_in_call_refuses_the_same_arguments_with_and_without_the_extension(
             said.append((type(e.value), str(e.value)))
         monkeypatch.undo()
         assert said[0] == said[1], call
+
+
+def test_an_extension_of_an_older_tree_is_not_used():
+    """An extension built before the drop-in call moved into it has no linear_forward_any_order: the package then takes its ctypes path."""
+    code = ("import sys, types\n"
+            "old = sys.modules['fp6_llm_amd._fp6mi_torch'] = types.ModuleType('fp6_llm_amd._fp6mi_torch')\n"
+            "old.linear_forward_native = old.clear_workspaces = old.clear_twins = lambda *a: None\n"
+            "import torch, fp6_llm_amd as fp6\n"
+            "w, x, sc = torch.zeros(256, 12, dtype=torch.int32), torch.zeros(3, 64).half(), torch.ones(256).half()\n"
+            "try:\n    fp6.linear_forward_cuda(x, w, sc)\n"
+            "except ValueError as e:\n    assert str(e) == 'weights must be on the GPU', e\n"
+            "fp6.clear_caches()\n"
+            "assert fp6._ext is None\n")
+    env = {k: v for k, v in os.environ.items() if k != "FP6MI_NO_TORCH_EXT"}
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=ROOT, env=env)
 
 
 def test_reference_heuristic_is_kept_verbatim():
