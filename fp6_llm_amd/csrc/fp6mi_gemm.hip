@@ -739,7 +739,7 @@ __global__ __launch_bounds__(WR *WK *kWave) void gemm_tile(const uint8_t *__rest
 //   workgroup = WR arithmetic wavefronts + PW loading wavefronts; tile = (WR*RT*16) rows x (NT*16) columns; same grid as gemm_tile
 // The loading wavefronts move K blocks from memory into LDS without passing through registers (global_load_lds_dwordx4):
 // the tile's weight blocks exactly as they lie in memory (native blocks of raw codes, 16-byte pieces in lane order) and the
-// activation rows of the block.  The arithmetic wavefronts never touch global memory inside the K loop: they read their
+// activation rows of the block.  The arithmetic wavefronts never touch global memory inside the K loop (with 256 rows for group exponents only): they read their
 // weight pieces and their B operands from LDS, convert and run the MFMAs.  In gemm_tile every wavefront does both, a
 // wavefront issues its instructions in order, and the CU's memory pipeline accepts a chunk's loads at its own pace: there
 // the second wavefront of every SIMD starts its MFMAs a third of a K step late, and a block has to arrive within the one
@@ -755,6 +755,13 @@ template <int FM, int NT, int RT, int WR, int SW, int SX> constexpr size_t ws_ri
 {
     return (size_t)SW * WR * RT * Fmt<FM>::block_bytes + (size_t)SX * NT * 16 * 512;
 }
+// Group exponents of 128 rows travel with the weights, in a ring of SW stages behind the activations', 4 bytes a row.  Loaded by the arithmetic
+// wavefronts, one block ahead, they were waited for at the barrier of every block, and the blocks that a ring of three has under way did not help: the
+// shapes that had won without exponents lost up to 28 % with them to those they had replaced.  us, shape before the ring of three / loads in registers /
+// through LDS: e2m1 8704x16192 N 53 29.5 / 38.1 / 29.1; e2m2 5632x10432 N 236 48.7 / 61.8 / 44.6; e2m1 1792x25984 N 672 133.8 / 144.7 / 101.0; over 167
+// problems of N 33 to 946 LDS / registers 0.89 (0.70-1.00).  With 256 rows LDS is full and SW is 2, one block ahead as in registers.
+template <bool GS, int WR> constexpr bool ws_exps_in_lds() { return GS && WR == 4; }
+template <bool GS, int RT, int WR, int SW> constexpr size_t ws_exps_ring_bytes() { return ws_exps_in_lds<GS, WR>() ? (size_t)SW * WR * RT * 64 : 0; }
 
 template <int N> __device__ __forceinline__ void wait_transfers_and_barrier()
 {
@@ -771,6 +778,8 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
     static_assert(SW >= SX && SX >= 2, "weights run at least as far ahead as activations; a stage is filled while another is read");
     constexpr int TN = NT * 16, TILES = WR * RT, NTHREADS = (WR + PW) * kWave;
     constexpr int kBlock = Fmt<FM>::block_bytes, kWStage = TILES * kBlock, kXStage = TN * 512, kXRing = SW * kWStage; // the activation ring follows the weight ring
+    constexpr bool kGLds = ws_exps_in_lds<GS, WR>();
+    constexpr int  kGStage = TILES * 64, kGRing = kXRing + SX * kXStage;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
     asm volatile("" ::"s"(W), "s"(scales), "s"(gexp), "s"(X), "s"(C), "s"(ws), "s"(M), "s"(N), "s"(K), "s"(units), "s"(splitK), "s"(nblocks)); // one batch of argument loads
@@ -807,10 +816,11 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
         static_assert(kWPieces % 64 == 0 && kXPieces % 64 == 0, "a stage is a whole number of 1 KB instructions");
         constexpr int kWInst = kWPieces / 64, kXInst = kXPieces / 64;
         static_assert(kWInst % PW == 0 && kXInst % PW == 0, "every loading wavefront issues the same number of transfers (the waits count them)");
-        constexpr int kWPer = kWInst / PW, kXPer = kXInst / PW;
+        static_assert(!kGLds || TILES * 16 % PW == 0 && TILES * 16 / PW <= 64, "a stage of exponents is one transfer of every loading wavefront");
+        constexpr int kWPer = kWInst / PW, kXPer = kXInst / PW, kGRows = TILES * 16 / PW, kWSteps = kWPer + (kGLds ? 1 : 0);
         // transfers issued after those of block j+1 when step j ends: the later of its two transfers is the activation one, issued
         // SX-2 steps ago and followed there by that step's weight transfers when the weight ring is the deeper one
-        constexpr int kAhead = (SW > SX ? kWPer : 0) + (SX - 2) * (kWPer + kXPer);
+        constexpr int kAhead = (SW > SX ? kWSteps : 0) + (SX - 2) * (kWSteps + kXPer);
         // weight piece P (16 bytes) of a stage = piece P % PB of the block of tile P / PB: a straight copy
         const uint8_t *wsrc[kWPer];
 #pragma unroll
@@ -818,6 +828,8 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
             const uint32_t P = (pw + PW * j) * 64 + lane, tile = P / PB, within = P % PB;
             wsrc[j] = W + ((size_t)(mb * TILES + tile) * units + u0) * kBlock + within * 16;
         }
+        const uint32_t grow = pw * kGRows + (kGLds ? lane % kGRows : 0);
+        const uint8_t *gsrc = kGLds ? gexp + ((size_t)(mb * TILES + grow / 16) * units + u0) * 32 + grow % 16 * 2 : nullptr;
         // activation piece P of a stage = slot P % 32 of row P / 32, which holds piece slot ^ (row & 15) of that batch column's
         // 256 halfs (columns beyond N repeat the last real one: their outputs are never stored)
         const uint8_t *xsrc[kXPer];
@@ -834,6 +846,9 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
 #pragma unroll
             for (int j = 0; j < kWPer; j++)
                 __builtin_amdgcn_global_load_lds((gvoid *)(wsrc[j] + (size_t)k * kBlock), (lvoid *)(st + (pw + PW * j) * 1024), 16, 0, 0);
+            if constexpr (kGLds) // and their exponents: lane l takes the two of row pw * kGRows + l, which LDS receives as 32 bits
+                if (lane < kGRows)
+                    __builtin_amdgcn_global_load_lds((gvoid *)(gsrc + (size_t)k * 32), (lvoid *)(lds + kGRing + slot * kGStage + pw * kGRows * 4), 2, 0, 0);
         };
         auto fetch_x = [&](int k, int slot) { // activations of block k -> stage `slot` of the activation ring
             uint8_t *st = lds + kXRing + slot * kXStage;
@@ -894,11 +909,11 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
         if (nk > 0) {
             uint32_t gnext[RT];
 #pragma unroll
-            for (int r = 0; r < RT; r++) gnext[r] = load_group_exps<GS>(ggroup, (size_t)r * units, lane);
+            for (int r = 0; r < RT; r++) gnext[r] = load_group_exps<GS && !kGLds>(ggroup, (size_t)r * units, lane);
             __syncthreads(); // block 0 has landed
             int wslot = 0, xslot = 0;
             for (int k = 0; k < nk; k++) {
-                const uint8_t *wst = lds + wslot * kWStage, *xst = lds + xslot * kXStage;
+                const uint8_t *wst = lds + wslot * kWStage, *xst = lds + xslot * kXStage, *gst = lds + kGRing + wslot * kGStage;
                 wslot = wslot + 1 == SW ? 0 : wslot + 1;
                 xslot = xslot + 1 == SX ? 0 : xslot + 1;
                 WFrag<FM> wf[RT];
@@ -910,8 +925,8 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
                     wf[r].b = *reinterpret_cast<const v4u *>(b + 1024);
                     if constexpr (Fmt<FM>::bits == 6) wf[r].c = *reinterpret_cast<const v4u *>(b + 2048);
                     if constexpr (Fmt<FM>::bits == 5) wf[r].s = *reinterpret_cast<const v2u *>(wst + (wr * RT + r) * kBlock + 2048 + lane * 8);
-                    g[r] = gnext[r];
-                    if (GS && k + 1 < nk) gnext[r] = load_group_exps<GS>(ggroup, (size_t)r * units + k + 1, lane);
+                    g[r] = kGLds ? *reinterpret_cast<const uint32_t *>(gst + (wr * RT + r) * 64 + col * 4) : gnext[r];
+                    if (GS && !kGLds && k + 1 < nk) gnext[r] = load_group_exps<GS>(ggroup, (size_t)r * units + k + 1, lane);
                 }
                 v8h a0[RT][4], a1[RT][4];
 #pragma unroll
@@ -1658,7 +1673,7 @@ int launch_ws(hipStream_t st, const void *W, const void *sc, const void *gexp, c
               int splitK)
 {
     constexpr int    TN = NT * 16, TM = WR * RT * 16;
-    constexpr size_t kLoopLds = ws_ring_bytes<FM, NT, RT, WR, SW, SX>(), out_max = tile_stage_bytes<NT, RT, WR>(true);
+    constexpr size_t kLoopLds = ws_ring_bytes<FM, NT, RT, WR, SW, SX>() + ws_exps_ring_bytes<GS, RT, WR, SW>(), out_max = tile_stage_bytes<NT, RT, WR>(true);
     constexpr size_t kMaxLds = kLoopLds > out_max ? kLoopLds : out_max;
     static_assert(kMaxLds <= 160 * 1024, "the rings do not fit in LDS");
     static_assert((WR + PW) * kWave <= 1024, "too many wavefronts");

@@ -1,4 +1,4 @@
-"""Properties of the prefill kernel that hold only if the compiler leaves its memory operations as they are written: they are read off the
+"""Properties of the prefill and the wave-specialized kernel that hold only if the compiler leaves its memory operations as they are written: they are read off the
 gfx950 instructions of the library that this tree builds.  No GPU is needed."""
 import os
 import re
@@ -29,9 +29,8 @@ def code_objects(data):
         pos += len(magic)
 
 
-@pytest.fixture(scope="module")
-def prefill_kernels(tmp_path_factory):
-    """{symbol: [instruction, ...]} of every gemm_prefill instance."""
+def instructions(tmp_path_factory, kernel):
+    """{symbol: [instruction, ...]} of every instance of a kernel."""
     kernels = {}
     with open(LIBRARY, "rb") as f:
         images = list(code_objects(f.read()))
@@ -39,7 +38,7 @@ def prefill_kernels(tmp_path_factory):
         path = tmp_path_factory.mktemp("elf") / ("%d.elf" % i)
         path.write_bytes(image)
         table = subprocess.run([OBJDUMP, "-t", str(path)], capture_output=True, text=True, check=True).stdout
-        names = sorted({line.split()[-1] for line in table.splitlines() if "gemm_prefill" in line and not line.endswith(".kd")})
+        names = sorted({line.split()[-1] for line in table.splitlines() if kernel in line and "." not in line.split()[-1]})
         if not names:
             continue
         text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", "--disassemble-symbols=" + ",".join(names), str(path)],
@@ -54,6 +53,13 @@ def prefill_kernels(tmp_path_factory):
             code = line.split("//")[0].strip()
             if name and code:
                 kernels[name].append(code)
+    return kernels
+
+
+@pytest.fixture(scope="module")
+def prefill_kernels(tmp_path_factory):
+    """{symbol: [instruction, ...]} of every gemm_prefill instance."""
+    kernels = instructions(tmp_path_factory, "gemm_prefill")
     assert len(kernels) == 8, sorted(kernels)   # four formats, with and without group exponents
     return kernels
 
@@ -96,3 +102,13 @@ def test_prefill_waits_cover_every_transfer(prefill_kernels):
             first = max((j for j in range(last) if code[j] == "s_barrier"), default=0)
             assert sum(is_transfer(b) for b in code[first:i]) >= 8, name
         assert counted == 2, (name, counted)    # one for each half block
+
+
+def test_wave_specialized_kernels_of_128_rows_hold_no_exponents_in_registers(tmp_path_factory):
+    """The loading wavefronts bring the group exponents of 128 rows as far ahead as the weights.  Loads of the arithmetic wavefronts (one 16-bit load a
+    row tile and K block) were waited for at the barrier of every block, which made what the ring has under way no use."""
+    kernels = {n: code for n, code in instructions(tmp_path_factory, "gemm_ws").items() if re.search(r"gemm_wsILi\d+ELb1ELi\d+ELi\d+ELi4E", n)}
+    assert len(kernels) == 16, sorted(kernels)   # four formats, tiles of 48, 64, 80 and 96 columns
+    for name, code in kernels.items():
+        assert any(c.startswith("global_load_lds_ushort") for c in code), name
+        assert not any(re.match(r"(global|flat|buffer)_load_[us]short", c) for c in code), name

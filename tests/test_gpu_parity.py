@@ -1164,6 +1164,36 @@ def test_grouped_gemm_on_the_256x128_tile(E, M):
     check_close(y[:, rows], oracle.gemm_f64(wdq, x), "grouped, 256x128 tile")
 
 
+@pytest.mark.parametrize("E,M", FORMATS)
+@pytest.mark.parametrize("cfg", [c for c in WS_SHAPES if c[3] == 4])
+def test_grouped_gemm_on_128_rows_of_the_wave_specialized_kernel(E, M, cfg):
+    """Its loading wavefronts move the exponents with the weights, 16 bits at a time (the array is 2-byte aligned only): one to six K blocks, the last one
+    cut or not, in one piece and in splits of none, one and two blocks, over two row blocks.  With factor 1 everywhere the bits are those without exponents."""
+    if not tune_shape_compiled_for(cfg, 1 + E + M):
+        pytest.skip("this shape is not built for this bit width")
+    print("case grouped, 128 rows", E, M, cfg, flush=True)
+    L, OC, N = _lib.lib(), 256, 16 * cfg[1] + 3
+    stream = torch.cuda.current_stream().cuda_stream
+    for IC in (64, 512, 576, 832, 1536):
+        codes, sc, ex = quant.quantize_groupwise(_grouped_weights(OC + IC, OC, IC), E, M)
+        native = fp6.weight_prepacking_native_cpu(E, M, torch.from_numpy(quant.pack_raw(codes, E, M))).to(DEV)
+        packed = fp6.pack_group_exps(torch.from_numpy(ex), OC, IC).to(DEV)
+        gexp = torch.cat([packed.new_zeros(2), packed])[2:]
+        scd, x = torch.from_numpy(sc).to(DEV), synth.activations(IC + 9, N, IC)
+        xd, ref = torch.from_numpy(x).to(DEV), oracle.gemm_f64(oracle.dequant_grouped_from_definition(codes, sc, ex, E, M), x)
+        for splitK in (1, 2, 3):
+            ws = torch.empty(splitK * N * OC, dtype=torch.float32, device=DEV)
+            outs = []
+            for exps in (gexp, torch.full_like(packed, 127)):
+                out = torch.full((N, OC), float("nan"), dtype=torch.float16, device=DEV)
+                rc = L.fp6mi_linear_native_grouped_cfg(E, M, stream, native.data_ptr(), scd.data_ptr(), exps.data_ptr(), xd.data_ptr(), out.data_ptr(), OC, N, IC,
+                                                       ws.data_ptr(), splitK, *cfg)
+                assert rc == 0, L.fp6mi_error_string(rc)
+                outs.append(out.cpu().numpy())
+            check_close(outs[0], ref, "IC %d splitK %d" % (IC, splitK))
+            assert np.array_equal(outs[1], gemm_capi(E, M, native, scd, xd, OC, splitK, cfg)), (IC, splitK)
+
+
 def test_grouped_module_forward_and_prefill_route():
     from fp6_llm_amd import module
     E, M, OC, IC = 2, 1, 512, 1024
