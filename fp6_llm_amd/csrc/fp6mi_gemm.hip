@@ -668,13 +668,21 @@ __device__ __forceinline__ void tile_store(const v4f (&acc)[RT][NT], const v4h (
 // as small as it gets (with all the column blocks of one row block first, a long prompt's activations pass by once for every 256 or 512 rows).
 // Measured at FP6 e3m2, us, rows first -> panels: gemm_prefill 8192x8192 N 4096 582 -> 444, 14336x4096 N 3000 334 -> 306, 28672x8192 N 2048 832 -> 787;
 // gemm_ws 28672x8192 N 2048 914 -> 831, 8192x8192 N 4096 503 -> 472; gemm_tile 256 x 128 8192x8192 N 4096 488 -> 460.  Panels of 512, 2048 and 4096
-// rows: within 2 %, and up to 6 % behind.  Level where the grid is a single round (8192x8192 N 512); 128 x 32 tiles lose by 6 % and keep the rows.
+// rows: within 2 %, and up to 6 % behind.  128 x 32 tiles lose by 6 % and keep the rows.
+// In panels every XCD reads all the weights of a panel, by rows few XCDs read the same ones: activations that stay in an L2 of 4 MB anyway are no
+// reason for it.  Tiles of 256 rows are counted in panels where the activations take more than 2 MB, in a single round of the 256 CUs more than 4 MB and
+// with 128 workgroups at least (a few leave the order no part).  Time in panels / by rows on 440 problems (K 256 to 28288; activations kept and changed from
+// launch to launch), always -> by this rule: gemm_tile 256 x 64 1.02 (0.90-1.19) -> 0.99 (0.90-1.05), 256 x 128 0.99 (0.84-1.10) -> 0.98 (0.84-1.01),
+// gemm_ws 256 x 64 1.00 (0.87-1.11) -> 0.99 (0.87-1.04).  What it leaves to the rows was at most 4 % faster in panels, 1024x256 N 2537 1.18.  gemm_prefill
+// 0.98 (0.64-1.03) always.
 struct TileId { uint32_t mb, split, nb; };
-template <int TM, int TN> __device__ __forceinline__ TileId tile_of(uint32_t splitK, uint32_t nblocks)
+template <int TM, int TN> __device__ __forceinline__ TileId tile_of(uint32_t splitK, uint32_t nblocks, uint32_t N, uint32_t K)
 {
     constexpr uint32_t kPanel = TM * TN >= 128 * 128 ? 1024 / TM : 1; // row blocks per panel
     const uint32_t     q = gridDim.x >> 3, r = gridDim.x & 7u, x = blockIdx.x & 7u, id = x * q + (x < r ? x : r) + (blockIdx.x >> 3);
-    if (kPanel > 1 && splitK == 1) {
+    const uint64_t     X = (uint64_t)N * K * 2; // bytes of the activations
+    const bool         panels = kPanel > 1 && splitK == 1 && (TM < 256 || (gridDim.x > 256 ? X > 2u << 20 : gridDim.x >= 128 && X > 4u << 20));
+    if (panels) {
         const uint32_t mblocks = gridDim.x / nblocks, first = id / (kPanel * nblocks) * kPanel, in = id - first * nblocks;
         const uint32_t high = mblocks - first < kPanel ? mblocks - first : kPanel; // the last panel may be lower
         return TileId{ first + in % high, 0, in / high };
@@ -699,7 +707,7 @@ __global__ __launch_bounds__(WR *WK *kWave) void gemm_tile(const uint8_t *__rest
     const int wr = wave % WR, wk = wave / WR;
     const int col = lane & 15, q = lane >> 4;
 
-    const TileId   id = tile_of<WR * RT * 16, TN>(splitK, nblocks);
+    const TileId   id = tile_of<WR * RT * 16, TN>(splitK, nblocks, N, K);
     const uint32_t mb = id.mb, split = id.split, nb = id.nb;
     const uint32_t nbase = nb * TN, R0 = (mb * WR + wr) * RT; // first row tile of this wavefront
 
@@ -786,7 +794,7 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, q = lane >> 4;
 
-    const TileId   id = tile_of<WR * RT * 16, NT * 16>(splitK, nblocks);
+    const TileId   id = tile_of<WR * RT * 16, NT * 16>(splitK, nblocks, N, K);
     const uint32_t mb = id.mb, split = id.split, nb = id.nb;
     const uint32_t nbase = nb * TN;
     uint32_t       u0 = 0, u1 = units;
@@ -1034,7 +1042,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, c
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, q = lane >> 4, wr = wave & 1, wc = wave >> 1;
 
-    const TileId   id = tile_of<2 * RT * 16, TN>(splitK, nblocks);
+    const TileId   id = tile_of<2 * RT * 16, TN>(splitK, nblocks, N, K);
     const uint32_t mb = id.mb, split = id.split, nb = id.nb;
     const uint32_t nbase = nb * TN, R0 = (mb * 2 + wr) * RT;
     uint32_t       u0 = 0, u1 = units;

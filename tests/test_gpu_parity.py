@@ -301,6 +301,19 @@ def test_large_tiles_counted_in_panels(OC, N, cfg):
     check_close(y, oracle.gemm_f64(oracle.dequant(raw, sc, 3, 2), x), "cfg %s" % (cfg,))
 
 
+@pytest.mark.parametrize("cfg", [(1, 8, 2, 8, 1), (1, 4, 2, 8, 1), (2, 4, 2, 8, 4)])
+def test_tiles_of_256_rows_counted_in_panels(cfg):
+    """They are counted by rows up to 2 MB of activations (4 MB in a single round), as above; here are 4.4 MB in one round of 144 workgroups of 256 x 128
+    and in two of 256 x 64: nine row blocks, the last panel holds one."""
+    print("case panels of 256 rows", cfg, flush=True)
+    OC, IC, N = 2304, 1152, 1930
+    raw, sc, x = synth.uniform_problem(801, OC, IC, N)
+    native, scd, xd = upload(raw, sc, x, 3, 2)
+    y = gemm_capi(3, 2, native, scd, xd, OC, 1, cfg)
+    assert np.isfinite(y).all()
+    check_close(y, oracle.gemm_f64(oracle.dequant(raw, sc, 3, 2), x), "cfg %s" % (cfg,))
+
+
 def test_unsupported_launch_shape_is_rejected():
     raw, sc, x = synth.uniform_problem(1, 256, 256, 4)
     native, scd, xd = upload(raw, sc, x, 3, 2)
