@@ -184,6 +184,19 @@ inline double rounds_on_chip(const TuneCfg &c, size_t M, size_t N, int splitK)
     return std::ceil(wgs / slots);
 }
 
+// What a launch takes however short K is, in 0.02 us: 2 us, and with a split 2 us for the reduction's launch and the partial sums at 8 TB/s, as
+// in tile_estimate_ns.  (Twice a time less the time at twice the K, over the table from 2048 columns on: 3-4 us unsplit, 5-8 us and the partial
+// sums with a split.)  Between 33 and 320 columns the splits are compared with this part carried over as it is and the rest in proportion; the shapes of one split
+// are not.  In proportion to K as a whole, a split's time shrank with the part that does not, and matrices of little K were cut that none of their
+// neighbours gains by: FP4 1280x2304 N 113 in eight (8.5 us, 5.5 unsplit), FP6 2048x3456 N 231 in four (11.0, 8.8), FP5 1536x1408 N 47 in three (5.9, 4.1).
+// Time of the choice / time of the best proposal on 324 matrices off the table, every proposal measured: N 33-80 1.07 before, 1.02 now, N 81-160 1.02 and
+// 1.01, N 161-320 1.03 and 1.02.  Left as they were: up to 32 columns (1.04 and 1.01, but 5 of 87 problems 3-13 % slower), and beyond 320, where the
+// few splits measured are for long K (11520x12800 N 456: 152 us in two pieces, 172 uncut).
+inline double fixed_part(size_t M, size_t N, int splitK)
+{
+    return splitK == 1 ? 100.0 : 200.0 + (double)splitK * M * N * 8.0 / 8e6 / 0.02;
+}
+
 const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
 {
     // a serving loop asks for the same few layer shapes at whatever batch size the scheduler formed: remember answers
@@ -218,18 +231,24 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
     TuneAnswer a = {};
     if (count > 0 && dist[0] == 0.f) count = 1, a.measured = true, a.exact = group->n == N; // measured: nothing to carry over
     const size_t units = (K + 255) / 256;
+    float        of_shape[kNumSplits] = {}; // what the shapes of a split are compared by
     for (int j = 0; j < count; j++) {
         const TuneEntry &e = *near[j];
         const size_t     Me = (size_t)e.m256 * 256, Ke = (size_t)e.k64 * 64, Nq = N > group->n ? N : group->n;
         for (int i = 0; i < kNumSplits; i++) {
             const TuneCfg &c = e.sk[i];
             if (!cfg_fits(c, M) || (size_t)kSplits[i] > units) continue;
-            double t = (double)c.t * (double)K / (double)Ke * (1.0 + 0.15 * dist[j]);
-            t *= rounds_on_chip(c, M, Nq, kSplits[i]) / rounds_on_chip(c, Me, group->n, kSplits[i]);
-            if (a.t[i] == 0.f || (float)t < a.t[i]) {
-                a.t[i] = (float)t;
+            const double rounds = rounds_on_chip(c, M, Nq, kSplits[i]) / rounds_on_chip(c, Me, group->n, kSplits[i]);
+            double       t = (double)c.t * (double)K / (double)Ke * (1.0 + 0.15 * dist[j]);
+            t *= rounds;
+            if (a.t[i] == 0.f || (float)t < of_shape[i]) {
+                of_shape[i] = a.t[i] = (float)t;
                 a.cfg[i] = LaunchCfg{ c.kind, c.nt, c.rt, c.wr, c.wk };
                 a.valid = true;
+                if (!a.measured && N > 32 && N <= 320) {
+                    const double there = std::fmin(fixed_part(Me, group->n, kSplits[i]), 0.8 * c.t), here = std::fmin(fixed_part(M, Nq, kSplits[i]), 0.8 * c.t);
+                    a.t[i] = (float)((here + (c.t - there) * (double)K / (double)Ke * rounds) * (1.0 + 0.15 * dist[j]));
+                }
             }
         }
     }
