@@ -266,18 +266,18 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
 // Since large tiles are counted in panels, on problems with M 1024-28672, K 1024-28672 (6, 5 and 4 bits; row scales, then group exponents):
 //   * from 256 x 128 between N 512 and 3072 it takes over whatever the rounds: as many half rounds 0.94 (0.83-1.02) on 1160 problems and 0.97 (0.87-1.04) on 368, fewer
 //     0.85 (0.73-0.91) on 249 and 0.88 (0.77-0.94) on 83; rows of a multiple of 8 KB are no exception any more (N above 2048: 0.88, 0.73-1.00, and 0.92, 0.77-1.03);
-//   * from 256 x 64 between N 2048 and 3072: 0.97 (0.87-1.05) on 208 and 0.90 (0.83-0.96) on 73, above 1.02 on 8, all with row scales only.
-// Beyond N 3072 the lines are those of before the panels, and so they are up to N 512 and for K below 1024.
+//   * from 256 x 64 between N 2048 and 3072: 0.97 (0.87-1.05) on 208 and 0.90 (0.83-0.96) on 73, above 1.02 on 8, all with row scales only; with K 64-960
+//     0.80 (0.71-0.92) on 64 and 0.81 (0.72-0.94) on 26.
+// Beyond N 3072 the lines are those of before the panels, and so they are up to N 512 and, from 256 x 128, for K below 1024.
 // Where it did not win before the panels, on 217 problems and (*) on 687 of another sweep, row scales only:
-//   * as many half rounds of 256 x 128, N up to 1024: 1.00 (0.92-1.10), with group exponents, whose loads come twice as often per output, 1.05 (0.95-1.19);
 //   * 256 x 128 with K below 320, prologue and epilogue being most of it: 0.99 (0.95-1.05) with fewer half rounds, with group exponents 1.03 (0.99-1.10);
 //   * (*) N up to 144, the second column block nearly empty: 256 x 128 0.98 (0.96-1.01), 256 x 64 1.16 (1.01-1.50);
+//   * as many half rounds of 256 x 128, N up to 1024 (since the panels the line is at 512): 1.00 (0.92-1.10), with group exponents, whose loads come twice as often per output, 1.05 (0.95-1.19);
 //   * (*) from 256 x 64: a single round 1.19 (1.00-1.86), more rounds 1.29 (0.87-1.44) up to N 1024;
 //   * (*) long prompts, where what the activations cost comes in: with K above 8192, N above 3072 and an eighth fewer half rounds 0.97-1.06 (a quarter fewer
 //     0.79-0.98 up to N 3712), N above 4096 with K above 3072 1.00 (0.89-1.12, no line found between the two; up to K 3072 0.92, 0.85-0.96).
-// (*) Faster here on the whole, but not taken over: as many half rounds of 256 x 128 beyond N 1024 (0.92 up to N 2048, 0.94, 0.87-1.11, above), less than an eighth gained
-// beyond N 2048 (0.88, 0.81-1.02), 256 x 64 beyond N 2048 (0.90, 0.74-1.04; with K above 8192 1.08) and rows of a multiple of 8 KB there (256 x 128 0.92,
-// 0.77-1.11; 256 x 64 0.98, 0.91-1.21).
+// (*) Faster there on the whole, but not taken over, beyond N 3072: as many half rounds of 256 x 128 (0.94, 0.87-1.11), less than an eighth gained
+// (0.88, 0.81-1.02), 256 x 64 (0.90, 0.74-1.04; with K above 8192 1.08) and rows of a multiple of 8 KB (256 x 128 0.92, 0.77-1.11; 256 x 64 0.98, 0.91-1.21).
 inline bool prefill_tile_wins(const LaunchCfg &c, size_t M, size_t N, size_t K, int splitK, int cus)
 {
     if (splitK != 1 || N <= 144 || K > (size_t)1 << 20 || (N > 3072 && K % 4096 == 0)) return false;

@@ -667,10 +667,12 @@ __device__ __forceinline__ void tile_store(const v4f (&acc)[RT][NT], const v4h (
 // the 32 or 64 workgroups that an XCD holds then cover about 1024 rows x 512-1024 columns, and what its L2 fetches for them is about
 // as small as it gets (with all the column blocks of one row block first, a long prompt's activations pass by once for every 256 or 512 rows).
 // Measured at FP6 e3m2, us, rows first -> panels: gemm_prefill 8192x8192 N 4096 582 -> 444, 14336x4096 N 3000 334 -> 306, 28672x8192 N 2048 832 -> 787;
-// gemm_ws 28672x8192 N 2048 914 -> 831, 8192x8192 N 4096 503 -> 472; gemm_tile 256 x 128 8192x8192 N 4096 488 -> 460.  Panels of 512, 2048 and 4096
+// gemm_ws 28672x8192 N 2048 914 -> 831, 8192x8192 N 4096 503 -> 472; gemm_tile 256 x 128 8192x8192 N 4096 488 -> 460
+// (forced: the dispatch gives some of these another shape).  What is fetched falls from 2267 to 784 MB (gemm_tile) and 4101 to 1629 (gemm_prefill 28672x8192).  Panels of 512, 2048 and 4096
 // rows: within 2 %, and up to 6 % behind.  128 x 32 tiles lose by 6 % and keep the rows.
 // In panels every XCD reads all the weights of a panel, by rows few XCDs read the same ones: activations that stay in an L2 of 4 MB anyway are no
-// reason for it.  Tiles of 256 rows are counted in panels where the activations take more than 2 MB, in a single round of the 256 CUs more than 4 MB and
+// reason for it (single rounds of 256-row tiles, K up to 1536: 0.8 us longer in panels with weights that come from memory, though less is fetched, 10.3 MB against
+// 14.6 at 1280x768 N 1658; level with weights that the caches hold).  Tiles of 256 rows are counted in panels where the activations take more than 2 MB, in a single round of the 256 CUs more than 4 MB and
 // with 128 workgroups at least (a few leave the order no part).  Time in panels / by rows on 440 problems (K 256 to 28288; activations kept and changed from
 // launch to launch), always -> by this rule: gemm_tile 256 x 64 1.02 (0.90-1.19) -> 0.99 (0.90-1.05), 256 x 128 0.99 (0.84-1.10) -> 0.98 (0.84-1.01),
 // gemm_ws 256 x 64 1.00 (0.87-1.11) -> 0.99 (0.87-1.04).  What it leaves to the rows was at most 4 % faster in panels, 1024x256 N 2537 1.18.  gemm_prefill
@@ -1336,7 +1338,8 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 // fp32 weights 1024x3072 and 8192x8192 (fused taken, up to 11 %).  e2m1 follows e3m2.  (The 16-bit columns of "fused" are those of three blocks in registers
 // and none in LDS.  That takes more than 128 registers with group exponents, and the CU then holds one workgroup; a block in LDS and two in registers leave
 // room for two with either.  us, bf16, before -> now, row scales and group exponents: 4096x4096 13.6 -> 13.2, 15.4 -> 14.9; 8192x7168 34.9 -> 33.8, 44.5 -> 36.6;
-// 8192x8192 49.1 -> 47.6, 57.6 -> 49.6; 28672x4096 61.5 -> 61.0, 87.5 -> 64.3; 8192x28672 178 -> 176, 179 -> 182.  Three in registers and one in LDS, nothing read
+// 8192x8192 49.1 -> 47.6, 57.6 -> 49.6; 28672x4096 61.5 -> 61.0, 87.5 -> 64.3; 8192x28672 178 -> 176, 179 -> 182.  Behind by 1-2 % at 4096x11008 and 3072x2048
+// and, with row scales, by 2-4 % at 28672x8192, where groups gain 20 %.  Three in registers and one in LDS, nothing read
 // twice at 8192 columns: 51.4, 53.7 with one workgroup to a CU, 51.9, 56.1 held to 128 registers, which spills.)
 // A conversion in double precision, code by code through a byte array in scratch memory, took 532 us at 8192x8192.
 // ---------------------------------------------------------------------------------------------------------------

@@ -18,15 +18,16 @@ class FPxLinear(torch.nn.Module):
     the layer is inference-only, like the kernels."""
 
     # Batch size from which dequantize + FP16 library GEMM beats the mixed-input kernel on the MI355X, whatever the matrix: measured
-    # through this module at 4096^2, 8192^2, 28672x8192 and 8192x28672, the route wins by 5-25 % from 3072 rows up, ties at 2048, and
-    # loses below (at 1024 rows by 25-30 %).
+    # through this module at 4096^2, 8192^2, 28672x8192 and 8192x28672, with FP6 and row scales and with FP5 and group exponents, with a bias and without,
+    # kernel time / route time is 0.63-1.00 at 1024 rows, 0.87-1.11 at 2048, 0.94-1.09 at 3072 and 1.10-1.29 at 4096 and 8192 (8192^2 at 4096 rows: 464 us
+    # against 395).
     PREFILL_CROSSOVER = 3072
 
     def __init__(self, in_features, out_features, exponent=3, mantissa=2, bias=None, split_k=None, dequant_above="auto", group_scales=False):
         """group_scales: the layer also holds one exponent byte per row and 128 columns (factor 1 until weights are loaded).
         dequant_above: batch size from which forward() dequantizes the weights to a temporary fp16 matrix on the GPU and calls
         the FP16 library GEMM instead (prefill).  The mixed-input kernel wins while the GEMM is bound by weight bytes; from a
-        few thousand rows the FP16 library runs 1.3-1.5 PFLOP/s against its 0.9-1.2, which pays for the dequantization pass
+        few thousand rows the FP16 library runs 1.3-1.5 PFLOP/s against its 1.1-1.25, which pays for the dequantization pass
         (about 30 us at 8192 x 8192).  "auto" (default) = PREFILL_CROSSOVER rows; None never does (the temporary costs 2 bytes
         per weight for the duration of the call); an integer sets the threshold."""
         super().__init__()

@@ -95,8 +95,10 @@ int fp6mi_linear_native(int E, int Mbits, void *stream, const void *W_native, co
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  Same kernels and results as
  * fp6mi_linear_native; the split-K partial sums go to a static device array of the library,
  * fp6mi_static_workspace_bytes() bytes (32 MiB) per GPU, instead of a caller workspace.  It calls no hipMalloc/hipFree.
- * splitK * M * N floats beyond that size return FP6MI_ERR_TOO_LARGE.  All calls on one GPU share the array: calls with
- * splitK > 1 that overlap in time on one GPU (different streams) race; calls on one stream are ordered.
+ * splitK * M * N floats beyond that size return FP6MI_ERR_TOO_LARGE: a splitK from fp6mi_heuristic_splitk, which is the
+ * fastest with a workspace of any size, may need more, so compare fp6mi_workspace_bytes first (1 always fits).  All calls
+ * on one GPU share the array: calls with splitK > 1 that overlap in time on one GPU (different streams) race; calls on one
+ * stream are ordered.
  * fp6mi_init() looks the array's device address up for the current device ahead of time (the first call on a device does
  * it otherwise); call it once per device outside any stream capture. */
 int    fp6mi_linear_native_static(int E, int Mbits, void *stream, const void *W_native, const void *scales_f16,

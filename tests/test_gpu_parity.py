@@ -290,8 +290,8 @@ def test_split_k_reduction_owns_every_row_once_on_any_grid(OC, cfg, N, splitK):
 @pytest.mark.parametrize("OC,N", [(2304, 333), (1024, 257), (256, 130), (2816, 600)])   # 9, 4, 1 and 11 row blocks of 256 rows
 @pytest.mark.parametrize("cfg", [(1, 8, 2, 8, 1), (1, 4, 2, 8, 1), (2, 4, 2, 8, 4), (2, 8, 4, 2, 2)])
 def test_large_tiles_counted_in_panels(OC, N, cfg):
-    """Without a split the large tiles are counted in panels of 1024 rows: whole panels, a lower last one and a single row block.  The
-    output starts as NaN, so a tile nobody computed would show."""
+    """Without a split the tiles of the prefill kernel are counted in panels of 1024 rows: whole panels, a lower last one and a single row block; those of
+    256 rows by rows at these sizes.  The output starts as NaN, so a tile nobody computed would show."""
     print("case panels", OC, N, cfg, flush=True)
     IC = 320
     raw, sc, x = synth.uniform_problem(700 + OC + N, OC, IC, N)
