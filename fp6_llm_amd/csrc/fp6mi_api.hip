@@ -158,7 +158,7 @@ inline bool cfg_fits(const TuneCfg &c, size_t M) { return c.kind != 255 && (c.ki
 // 16384 and 17920 rows differ by 9 % in size but by a whole round of 64-row workgroups; sweeps off the grid showed that
 // this, not the distance, decides which neighbour's shape is right.  Farther neighbours pay 15 % per octave of distance.
 struct TuneGroup { int xb; size_t n, begin, end; }; // entries [begin, end) of kTune share format and batch (the table is sorted by them)
-struct TuneAnswer { bool valid, measured, exact; LaunchCfg cfg[kNumSplits]; float t[kNumSplits]; }; // index i: splitK = kSplits[i]; t in 0.02 us, 0 = no proposal; measured: this very (M, K) at this or the next larger measured batch; exact: at this batch
+struct TuneAnswer { bool valid, measured, exact; size_t n; LaunchCfg cfg[kNumSplits]; float t[kNumSplits]; }; // index i: splitK = kSplits[i]; t in 0.02 us, 0 = no proposal; measured: this very (M, K) at this or the next larger measured batch; exact: at this batch; n: the measured batch that answers
 
 const std::vector<TuneGroup> &tune_groups()
 {
@@ -229,6 +229,7 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
         }
     }
     TuneAnswer a = {};
+    a.n = group ? group->n : 0;
     if (count > 0 && dist[0] == 0.f) count = 1, a.measured = true, a.exact = group->n == N; // measured: nothing to carry over
     const size_t units = (K + 255) / 256;
     float        of_shape[kNumSplits] = {}; // what the shapes of a split are compared by
@@ -358,10 +359,97 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
     c.nt = t->nt, c.rt = t->rt, c.wr = t->wr, c.wk = t->wk;
     return prefill_tile_wins(c, M, N, K, splitK, cus) ? LaunchCfg{ 2, 8, 4, 2, 2 } : c;
 }
+// ---- gemm_wide: which of its tiles a problem takes, and whether it takes the place of the shape of the table or the rules ----
+// Every tile of gemm_wide is one sum of rounds: its workgroups take the same time, and a CU holds one of eight wavefronts or two of four (two of eight
+// where a wavefront takes at most 128 registers).  So a time is (full rounds) x (fixed + K x rate) + (the last, partly filled round), and a split adds its
+// launch and its partial sums.  The constants are least squares of the relative error over 1050 problems (M 1024-28672, K 1024-28672, N 65-4096, most of them
+// up to 600; 6, 5 and 4 bits; group exponents on 30 %; weights and activations changed from launch to launch, splits 1, 2, 3, 4, 6 and 8): 4-7 % off a single
+// time, the smallest tiles most.  The shape and split that come out smallest are 0.8 % behind the best of these shapes on average, with a constant term, rates
+// and splits only 1.1 %.
+struct WideShape {
+    int   nt, rt, wk, slots;              // column tiles, row tiles per wavefront, K halves; workgroups that 256 CUs hold
+    float full, full_k, full_kg;          // a full round: us, us per column of K, the same with group exponents on top
+    float part, part_k, part_kf, part_kg; // the last round, of at most half the slots where a CU holds two workgroups: us, per column of K, that times its fill, group exponents
+    float k6, k5;                         // either round, per column of K: 6- and 5-bit weights on top of 4-bit ones
+    float base, x_mb, w_mb, out;          // once per launch; per MB of activations, per MB of weights; per million outputs unsplit
+    float split, split_out;               // a split's second launch, and its partial sums per million of them
+};
+constexpr WideShape kWide[] = {
+    { 4, 2, 2, 512, 0.64f, 0.00565f, 0.000445f, 0.779f, 0.0034f, 0.00017f, 0.000127f, 0.000512f, 0.000543f, 1.26f, 0.353f, 0.0607f, 0.85f, 2.89f, 1.35f },
+    { 6, 2, 2, 256, 2.3f, 0.00496f, 0.000302f, 1.35f, 0.004f, 0.000994f, 0.000294f, 0.000379f, 0.000471f, 1.46f, 0.346f, 0.0541f, 0.205f, 2.77f, 0.936f },
+    { 6, 4, 1, 512, 0.f, 0.0145f, 0.000878f, 0.0154f, 0.00811f, 0.000511f, 0.00109f, 0.000564f, 0.000919f, 3.3f, 0.144f, 0.0501f, 0.475f, 3.8f, 1.12f },
+    { 8, 2, 2, 256, 3.11f, 0.00552f, 0.000329f, 1.13f, 0.00458f, 0.00138f, 0.000385f, 0.000557f, 0.000652f, 1.93f, 0.272f, 0.0636f, 0.0816f, 2.61f, 1.11f },
+    { 8, 4, 1, 512, 0.f, 0.0187f, 0.000715f, 0.434f, 0.00994f, 0.000692f, 0.00107f, 0.0006f, 0.00103f, 3.6f, 0.119f, 0.0321f, 0.458f, 3.81f, 1.15f },
+    { 8, 4, 2, 256, 3.85f, 0.0102f, 0.000388f, 2.21f, 0.00798f, 0.00154f, 0.000812f, 0.000575f, 0.000692f, 3.05f, 0.119f, 0.021f, 0.325f, 3.17f, 1.19f },
+};
+
+inline float wide_estimate(const WideShape &w, int xbits, size_t M, size_t N, size_t K, int splitK, bool groups)
+{
+    const size_t units = (K + 255) / 256, kc = (units + splitK - 1) / splitK * 256;
+    const size_t wgs = M / (64u * w.rt) * ((N + 16 * w.nt - 1) / (16 * w.nt)) * splitK;
+    size_t       full = wgs / w.slots, rest = wgs % w.slots;
+    if (w.slots == 512 && rest > 256) full++, rest = 0;
+    const float k = (float)kc, kf = k * (xbits == 6 ? w.k6 : xbits == 5 ? w.k5 : 0.f), out = (float)M * (float)N * 1e-6f;
+    float       t = w.base + w.x_mb * (float)N * (float)K * 2e-6f + w.w_mb * (float)M * (float)K * (float)xbits * 0.125e-6f;
+    t += (float)full * (w.full + k * (w.full_k + (groups ? w.full_kg : 0.f)) + kf);
+    if (rest) t += w.part + k * (w.part_k + w.part_kf * (float)rest / 256.f + (groups ? w.part_kg : 0.f)) + kf;
+    return t + (splitK > 1 ? w.split + w.split_out * (float)splitK * out : w.out * out);
+}
+
+// the fastest of the shapes for a given split, and its time in us; 0 where none fits
+inline float wide_best(LaunchCfg &c, int xbits, size_t M, size_t N, size_t K, int splitK, bool groups)
+{
+    float best = 0.f;
+    if (N <= 96 || K > (size_t)1 << 20 || (size_t)splitK > (K + 255) / 256) return best;
+    for (const WideShape &w : kWide) {
+        const float t = wide_estimate(w, xbits, M, N, K, splitK, groups);
+        if (best == 0.f || t < best) best = t, c = LaunchCfg{ 2, w.nt, w.rt, 4, w.wk };
+    }
+    return best;
+}
+
+// us that the table expects of a split on 256 CUs; 0 for none.  A row's time is that of the measured batch, which the query rounds up to: what this batch
+// saves in rounds of the chip is taken off the part of it that is not fixed.
+inline float narrow_estimate(const TuneAnswer *a, size_t M, size_t N, int splitK)
+{
+    const int i = split_index(splitK);
+    if (!a || i < 0 || a->t[i] <= 0.f) return 0.f;
+    if (N <= 96) return a->t[i] * 0.02f; // (where nothing else is compared with it)
+    const LaunchCfg &c = a->cfg[i];
+    const TuneCfg    tc = { (uint8_t)c.kind, (uint8_t)c.nt, (uint8_t)c.rt, (uint8_t)c.wr, (uint8_t)c.wk, 0 };
+    const float      t = a->t[i] * 0.02f, fixed = std::fmin((float)fixed_part(M, N, splitK) * 0.02f, 0.8f * t);
+    return fixed + (t - fixed) * (float)(rounds_on_chip(tc, M, N, splitK) / rounds_on_chip(tc, M, a->n > N ? a->n : N, splitK));
+}
+
+// Whether gemm_wide, expected to take t us, takes the place of the table's shape, expected to take `narrow` (0: not in the table's reach, K below 1366 for
+// the most part; there it is a matter of the outputs, of which the rules' smaller tiles serve few better: 1536x1216 N 258 5.4 us against 7.3,
+// 3072x1024 N 2867 26.0 against 22.5).  Time after / before on 849 problems drawn as above, the split chosen anew: N 97-160 1.00 (0.75-1.01), N 161-256 0.98
+// (0.80-1.07), N 257-400 0.90 (0.50-1.13), N 401-640 0.84 (0.48-1.03), beyond 0.83 (0.46-1.06); N 65-96 1.00, not worth it.  The margins are what the two
+// estimates are off where the kernels are close, and allow for the table's, which is low, where they are not: without them 40 of these problems were more than
+// 2 % slower, with them 5.
+inline bool wide_replaces(float t, float narrow, size_t M, size_t N)
+{
+    if (t <= 0.f) return false;
+    if (narrow <= 0.f) return M * N >= (size_t)1 << 20;
+    return t < narrow * (N <= 400 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
+}
+
+// The launch shape of a call: gemm_wide's, or that of the table and the rules (which fp6mi_query_launch reports)
+inline LaunchCfg final_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, bool groups, int cus)
+{
+    LaunchCfg wide;
+    if (cus == 256 && N > 96)
+        if (const float t = wide_best(wide, xbits, M, N, K, splitK, groups); t > 0.f) {
+            const float narrow = narrow_estimate(tune_lookup(xbits, M, N, K), M, N, splitK);
+            if (wide_replaces(t, groups ? 1.06f * narrow : narrow, M, N)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
+        }
+    return pick_cfg(xbits, M, N, K, splitK, cus);
+}
+
 int linear_native(const fp6mi::FormatOps &ops, hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, size_t M, size_t N, size_t K, float *ws,
                   int splitK, const LaunchCfg *forced)
 {
-    LaunchCfg c = forced ? *forced : pick_cfg(ops.bits, M, N, K, splitK, current_device_cus());
+    LaunchCfg c = forced ? *forced : final_cfg(ops.bits, M, N, K, splitK, gexp != nullptr, current_device_cus());
     if (c.kind == 0 && !(c.rt & (c.rt - 1)) && (M / 16) % c.rt) return FP6MI_ERR_SHAPE; // (3, 5, 6, 7 tiles per workgroup end in a workgroup with fewer)
     int rc = ops.gemm(c, st, W, sc, gexp, B, C, ws, M, N, K, splitK);
     if (rc != 0) return rc;
@@ -418,7 +506,7 @@ const char *fp6mi_tuning_info(void)
         ;
 }
 
-int fp6mi_version(void) { return 137; } // 137: group exponents of 128 rows through LDS in the wave-specialized kernel, panels of 256-row tiles only for activations beyond L2; 136: tiles of 48, 80 and 96 columns, deeper rings in the wave-specialized kernel of 128 rows, panels; 135: prefill kernel (launch kind 2 with 2 x 2 wavefronts), relayout and quantizer kernels rewritten, the other GEMM kernels unchanged; 134: three row tiles per workgroup in the small-batch kernel (any M: the last workgroup takes what is left), no other kernel changed; 133: wave-specialized tile kernel (launch kind 2) for large batches; 132: split-K reduction runs on the XCD that wrote the partial sums, every grid size gets XCD-contiguous tiles; 131: tile kernel stores through LDS; 130: small-batch kernel loads activations as whole rows and turns them into operand order through LDS
+int fp6mi_version(void) { return 138; } // 138: gemm_wide (launch kind 2 with four rows of one or two wavefronts) in the place of larger tiles from 97 columns on, the other kernels unchanged; 137: group exponents of 128 rows through LDS in the wave-specialized kernel, panels of 256-row tiles only for activations beyond L2; 136: tiles of 48, 80 and 96 columns, deeper rings in the wave-specialized kernel of 128 rows, panels; 135: prefill kernel (launch kind 2 with 2 x 2 wavefronts), relayout and quantizer kernels rewritten, the other GEMM kernels unchanged; 134: three row tiles per workgroup in the small-batch kernel (any M: the last workgroup takes what is left), no other kernel changed; 133: wave-specialized tile kernel (launch kind 2) for large batches; 132: split-K reduction runs on the XCD that wrote the partial sums, every grid size gets XCD-contiguous tiles; 131: tile kernel stores through LDS; 130: small-batch kernel loads activations as whole rows and turns them into operand order through LDS
 
 int fp6mi_prepack_ref(int E, int Mb, void *packed, const void *raw, size_t M, size_t K) { return fp6mi::prepack_ref(E, Mb, packed, raw, M, K); }
 int fp6mi_unpack_ref(int E, int Mb, void *raw, const void *packed, size_t M, size_t K) { return fp6mi::unpack_ref(E, Mb, raw, packed, M, K); }
@@ -458,16 +546,20 @@ static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus
 {
     if (M == 0 || N == 0 || K == 0 || num_cus <= 0) return 1;
     size_t units = (K + 255) / 256;
-    if (num_cus == 256) { // a measured neighbour knows better than any model: take its fastest split (3 % hysteresis towards fewer splits)
-        if (const TuneAnswer *a = tune_lookup(xbits, M, N, K)) {
-            int   best_s = 0;
-            float best_t = 0.f;
-            for (int i = 0; i < kNumSplits; i++) {
-                if (a->t[i] == 0.f) continue;
-                if (best_s == 0 || a->t[i] * 1.03f < best_t) { best_s = kSplits[i]; best_t = a->t[i]; }
-            }
-            if (best_s) return best_s;
+    if (num_cus == 256) { // the fastest split by the times of measured neighbours, or of gemm_wide where it takes their place (3 % hysteresis towards fewer splits)
+        const TuneAnswer *a = tune_lookup(xbits, M, N, K);
+        int               best_s = 0, wide_s = 0;
+        float             best_t = 0.f, wide_t = 0.f;
+        auto              better = [](int s, float t, int &best_s, float &best_t) {
+            if (t > 0.f && (best_s == 0 || t * 1.03f < best_t)) best_s = s, best_t = t;
+        };
+        for (int s : kSplits) {
+            LaunchCfg wide;
+            better(s, narrow_estimate(a, M, N, s), best_s, best_t);
+            better(s, wide_best(wide, xbits, M, N, K, s, false), wide_s, wide_t);
         }
+        if (wide_replaces(wide_t, best_t, M, N)) return wide_s;
+        if (best_s) return best_s;
     }
     if (N > 16) {
         int    best_s = 1;
@@ -571,6 +663,14 @@ int fp6mi_query_launch(int E, int Mb, size_t M, size_t N, size_t K, int splitK, 
     if (M == 0 || M % 256 || K == 0 || K % 64 || N == 0) return FP6MI_ERR_SHAPE;
     if (splitK < 1) return FP6MI_ERR_SPLITK;
     LaunchCfg c = pick_cfg(1 + E + Mb, M, N, K, splitK, current_device_cus()); // the count the launch path uses (256 where no device answers)
+    shape[0] = c.kind, shape[1] = c.nt, shape[2] = c.rt, shape[3] = c.wr, shape[4] = c.wk;
+    return FP6MI_OK;
+}
+
+int fp6mi_query_kernel(int E, int Mb, size_t M, size_t N, size_t K, int splitK, int grouped, int *shape)
+{
+    if (int rc = fp6mi_query_launch(E, Mb, M, N, K, splitK, shape); rc != FP6MI_OK) return rc;
+    LaunchCfg c = final_cfg(1 + E + Mb, M, N, K, splitK, grouped != 0, current_device_cus());
     shape[0] = c.kind, shape[1] = c.nt, shape[2] = c.rt, shape[3] = c.wr, shape[4] = c.wk;
     return FP6MI_OK;
 }

@@ -616,18 +616,19 @@ typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 template <int NT, int RT, int WR> constexpr size_t tile_stage_bytes(bool partial) { return (size_t)NT * 16 * (WR * RT * 16 * (partial ? 4 : 2) + 16); }
 
 // first half: a wavefront that holds results scales them and parks them in the stage
-template <int FM, int NT, int RT, int WR, typename OutT>
+// (column tiles T0 .. T1-1 of it)
+template <int FM, int NT, int RT, int WR, typename OutT, int T0 = 0, int T1 = NT>
 __device__ __forceinline__ void tile_park(const v4f (&acc)[RT][NT], const v4h (&sc4)[RT], uint8_t *stage, int wr, int col, int q)
 {
     constexpr int TM = WR * RT * 16, kStride = TM * (int)sizeof(OutT) + 16;
 #pragma unroll
     for (int r = 0; r < RT; r++)
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
+        for (int t = T0; t < T1; t++) {
             v4f v;
 #pragma unroll
             for (int i = 0; i < 4; i++) v[i] = acc[r][t][i] * ((float)sc4[r][i] * Fmt<FM>::post_scale);
-            uint8_t *dst = stage + (16 * t + col) * kStride + ((wr * RT + r) * 16 + 4 * q) * (int)sizeof(OutT);
+            uint8_t *dst = stage + (16 * (t - T0) + col) * kStride + ((wr * RT + r) * 16 + 4 * q) * (int)sizeof(OutT);
             if constexpr (sizeof(OutT) == 2)
                 *reinterpret_cast<v4h *>(dst) = (v4h){ (half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3] };
             else
@@ -1185,6 +1186,225 @@ __global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, c
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// gemm_wide: the tile GEMM of large batches, wavefronts one below the other across the whole width of the tile.
+//   workgroup = 4 x WK wavefronts; tile = (4*RT*16) rows x (NT*16) columns, (RT*16) x (NT*16) of it per wavefront; grid as gemm_tile
+// A chip full of MFMAs is held by its power, not by its clock: registers only, 16x16x32 MFMAs of random halfs run at 1.84-1.93 GHz = 1.73-1.96 PFLOP/s
+// (32x32x16 ones at 1.72 GHz = 1.74), with one conversion for every 16 of them 1.70, for every 8 1.54.  What a GEMM gets is then a matter of what
+// it does beside them: conversions (64 cycles each, in which the SIMD starts no MFMA), operand reads from LDS, bytes from L2.  Here
+//   * a converted fragment meets all NT column tiles: NT = 8 has one conversion per 32 MFMAs, where gemm_prefill, gemm_ws and 256 x 64 tiles have one per 16;
+//   * a B operand read feeds RT row tiles: 4 in the 256-row tiles, where gemm_tile and gemm_ws have 2;
+//   * no wavefront loads weights that another one loads, and 256 x 128 outputs share each byte of both operands.
+// Weights go memory -> registers, activations memory -> LDS as in gemm_prefill.  K is walked in chunks of 128 columns (half a block), two stages in LDS,
+// one barrier a chunk.  A chunk is eight half steps of RT * NT / 2 MFMAs, the B operands of the next half step being read meanwhile (across the barrier
+// too).  All RT row tiles are converted at the top of a chunk; 256 x 128 then fills the register file (254-256), and the next raw codes are asked for when
+// half of the converted fragments are used up.  With fewer outputs a second set of raw codes is a chunk and a half ahead.
+// WK = 2 is for problems that do not fill the chip with two workgroups of four wavefronts to a CU: the second four take the other half of every K block (its
+// odd chunks), with stages of their own, and hand their sums over through LDS at the end.
+// Measured, us (FP6 e3m2, the best of gemm_tile 256 x 128, gemm_prefill and gemm_ws 256 x 64 -> here): 28672x8192 N 2048 759 -> 645 (1.49 PFLOP/s),
+// 8192x8192 N 4096 453 -> 381, N 1024 116 -> 109, N 512 60.3 -> 57.9 (WK 2); 11008x4096 N 1500 132 -> 110 (256 x 96), 4096x4096 N 1024 30.5 -> 28.9; FP5 with
+// group exponents 4608x4544 N 777 38.3 -> 33.1, 8192x8192 N 1024 114 -> 103.  One card to another differs by 4 %.
+// Tried and left out (28672x8192 N 2048 / 8192x8192 N 512): s_setprio around the MFMAs (+ 0.5 %), no scheduling fence between half steps (+ 0.5 %, spills with
+// group exponents), non-temporal weights (+ 5 %), panels of 2048 rows (level), conversions of two row tiles' quarters at once (level; with group exponents + 10 %),
+// WK 2 there (+ 4 %); a ring of four stages of 64 columns (level / + 1 %: what is in flight is not the bound, a kernel that only transfers the second one's
+// bytes takes 36 us).
+// ---------------------------------------------------------------------------------------------------------------
+template <int FM, bool GS, int NT, int RT, int WK>
+__global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X,
+                                                            half_t *__restrict__ C, float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
+                                                            uint32_t units, uint32_t splitK, uint32_t nblocks)
+{
+    constexpr int TM = 4 * RT * 16, TN = NT * 16, kStage = TN * 256, NH = NT / 2, NTHREADS = 4 * WK * kWave;
+    constexpr int kDma = TN / 16; // transfers of 1 KB (four rows) per wavefront and chunk
+    // loads a wavefront issues for certain after its last transfer of a chunk and before the chunk's barrier
+    constexpr int kRawLoads = (Fmt<FM>::bits == 4 ? 1 : 2) + (GS ? 1 : 0), kAfterDma = RT * kRawLoads;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, q = lane >> 4, wr = wave & 3, wk = WK == 1 ? 0 : wave >> 2;
+
+    const TileId   id = tile_of<TM, TN>(splitK, nblocks, N, K);
+    const uint32_t mb = id.mb, split = id.split, nb = id.nb;
+    const uint32_t nbase = nb * TN, R0 = (mb * 4 + wr) * RT;
+    uint32_t       u0 = 0, u1 = units;
+    if (splitK > 1) {
+        const uint32_t avg = units / splitK, extra = units % splitK;
+        u0 = split * avg + (split < extra ? split : extra);
+        u1 = u0 + avg + (split < extra ? 1u : 0u);
+    }
+
+    v4f acc[RT][NT];
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[r][t] = (v4f){ 0.f, 0.f, 0.f, 0.f };
+
+    // raw codes: scalar offsets into one buffer per wavefront (its RT row tiles), so that no address takes vector registers
+    const uint32_t tile_stride = units * Fmt<FM>::block_bytes; // 32 bits: the launcher bounds K
+    const auto     wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W + (size_t)R0 * tile_stride), 0, (int)(RT * tile_stride), 0x00027000);
+    const auto     gbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(GS ? gexp + (size_t)R0 * units * 32 : W), 0, (int)(RT * units * 32), 0x00027000);
+    constexpr int  kSets = RT * NT < 32 ? 2 : 1; // sets of raw codes: two where registers allow, which are then asked for a chunk and a half ahead
+    RawHalf        raw[kSets][RT];
+    auto           load_raw = [&](auto half_c, RawHalf (&raw)[RT], int r, uint32_t u) __attribute__((always_inline)) { // pieces as in load_raw_half
+        constexpr int  H = decltype(half_c)::value, kPiece = Fmt<FM>::bits == 6 ? 2048 : 1024;
+        const uint32_t at = r * tile_stride + u * Fmt<FM>::block_bytes;
+        raw[r].p = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16 + H * kPiece, at, 0));
+        if constexpr (Fmt<FM>::bits == 6) raw[r].s = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(wbuf, lane * 16 + 1024 + 8 * H, at, 0));
+        if constexpr (Fmt<FM>::bits == 5) raw[r].s[0] = __builtin_amdgcn_raw_buffer_load_b32(wbuf, lane * 8 + 2048 + 4 * H, at, 0);
+        if constexpr (GS) raw[r].g = __builtin_amdgcn_raw_buffer_load_b8(gbuf, 2 * col + H, (r * units + u) * 32, 0);
+    };
+
+    // transfers of activations: as in gemm_prefill
+    typedef __attribute__((address_space(3))) void lvoid;
+    uint8_t *const xstage = lds + wk * 2 * kStage;
+    const uint32_t xrow0 = 4 * wr + q, xpiece = (lane & 15) ^ xrow0; // xrow0 < 16
+    const uint32_t xoff0 = xrow0 * K * 2, xlast = (N - nbase < (uint32_t)TN ? N - 1 - nbase : TN - 1) * K * 2; // 32 bits: the launcher bounds K
+    auto           row_offset = [&](int j) __attribute__((always_inline)) {
+        uint32_t o = xoff0;
+        asm volatile("" : "+v"(o));
+        o += (uint32_t)j * 32u * K;
+        return o < xlast ? o : xlast;
+    };
+    const auto xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(X + (size_t)nbase * K), 0, (int)(xlast + K * 2), 0x00027000);
+    auto       transfer = [&](int j, uint32_t h, uint32_t stage) __attribute__((always_inline)) {
+        const uint32_t pos = h * 128 + xpiece * 8, off = row_offset(j) + (pos < K ? pos * 2 : 0xc0000000u); // (row offset + 2K < 2^29)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, (lvoid *)(xstage + stage * kStage + (wr + 4 * j) * 1024), 16, off, 0, 0, 0);
+    };
+
+    // B operands: half the column tiles of one MFMA step at a time, in two sets; half step i of a chunk is step i / 2, column tiles from NH * (i % 2) on
+    v8h            b[2][NH];
+    const uint8_t *xread = xstage + col * 256;
+    auto           read_b = [&](int i, uint32_t stage) __attribute__((always_inline)) {
+        const uint8_t *p = xread + stage * kStage + (((4 * (i >> 1) + q) ^ col) * 16) + (i & 1) * NH * 16 * 256;
+#pragma unroll
+        for (int t = 0; t < NH; t++) b[i & 1][t] = *reinterpret_cast<const v8h *>(p + t * 16 * 256);
+    };
+
+    // Chunk h (half H of a block) from stage `st`; its B operands of half step 0 are in b, its raw codes in (or on the way to) set `st` of raw.  The
+    // next chunk of this wavefront is h + WK.  (LAST: a last odd one of two K halves, which fetches nothing.  No other copy of the code is special: after
+    // the last chunk another one is fetched and not used.)
+    v32h a[RT];
+    auto chunk = [&](auto half_c, auto next_c, uint32_t h, auto st_c, auto last_c) __attribute__((always_inline)) {
+        constexpr bool LAST = decltype(last_c)::value;
+        constexpr int  H = decltype(half_c)::value, st = decltype(st_c)::value, set = kSets == 2 ? st : 0;
+        const uint32_t hx = h + WK < 2 * u1 ? h + WK : h, hr = h + kSets * WK, u_raw = hr < 2 * u1 ? hr >> 1 : u1 - 1;
+        sections<8>([&](auto i_c) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_c)::value;
+            if constexpr (i == 0) {
+#pragma unroll
+                for (int r = 0; r < RT; r++) a[r] = convert_raw_half<FM, GS, H>(raw[set][r]);
+            }
+            if constexpr (i == 4 && !LAST) { // (half of the converted fragments are used up: their registers hold these)
+#pragma unroll
+                for (int r = 0; r < RT; r++) load_raw(std::conditional_t<kSets == 2, decltype(half_c), decltype(next_c)>{}, raw[set], r, u_raw);
+            }
+            if constexpr (i < 4 && !LAST) {
+#pragma unroll
+                for (int j = i * kDma / 4; j < (i + 1) * kDma / 4; j++) transfer(j, hx, st ^ 1);
+            }
+            if constexpr (i == 7 && LAST) {
+                wait_transfers_and_barrier<0>();
+            } else if constexpr (i == 7) { // the next chunk's activations have landed, for every wavefront
+                wait_transfers_and_barrier<kAfterDma>();
+                __builtin_amdgcn_sched_barrier(0);
+                read_b(0, st ^ 1);
+            } else {
+                read_b(i + 1, st);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < NH; t++)
+#pragma unroll
+                for (int r = 0; r < RT; r++)
+                    acc[r][(i & 1) * NH + t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(slice8(a[r], i >> 1), b[i & 1][t], acc[r][(i & 1) * NH + t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+
+    typedef std::integral_constant<int, 0> Half0;
+    typedef std::integral_constant<int, 1> Half1;
+    if (u0 < u1) { // (more splits than K blocks leave some empty: their partial sums are zeros)
+        auto fill = [&](auto half_c, auto next_c) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < kDma; j++) transfer(j, 2 * u0 + decltype(half_c)::value, 0);
+#pragma unroll
+            for (int r = 0; r < RT; r++) load_raw(half_c, raw[0], r, u0);
+            if constexpr (kSets == 2) {
+#pragma unroll
+                for (int r = 0; r < RT; r++) load_raw(next_c, raw[kSets - 1], r, WK == 1 ? u0 : u0 + 1 < u1 ? u0 + 1 : u0);
+            }
+            wait_transfers_and_barrier<0>();
+            read_b(0, 0);
+        };
+        if constexpr (WK == 1) {
+            fill(Half0{}, Half1{});
+            for (uint32_t u = u0; u < u1; u++) {
+                chunk(Half0{}, Half1{}, 2 * u, Half0{}, std::false_type{});
+                chunk(Half1{}, Half0{}, 2 * u + 1, Half1{}, std::false_type{});
+            }
+        } else {
+            // (every wavefront passes the same number of barriers)
+            auto run = [&](auto half_c) __attribute__((always_inline)) {
+                constexpr int H = decltype(half_c)::value;
+                fill(half_c, half_c);
+                uint32_t u = u0;
+                for (; u + 2 <= u1; u += 2) {
+                    chunk(half_c, half_c, 2 * u + H, Half0{}, std::false_type{});
+                    chunk(half_c, half_c, 2 * u + 2 + H, Half1{}, std::false_type{});
+                }
+                if (u < u1) chunk(half_c, half_c, 2 * u + H, Half0{}, std::true_type{});
+            };
+            if (wk == 0)
+                run(Half0{});
+            else
+                run(Half1{});
+        }
+    }
+    wait_transfers_and_barrier<0>(); // nothing is on its way to LDS any more, and nobody reads operands
+
+    // output: as in the other tile kernels, through LDS; the row scales are asked for here, one round trip at the end of a long K loop
+    v4h sc4[RT];
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        const half_t *p = scales + (R0 + r) * 16 + 4 * q;
+        sc4[r] = (v4h){ p[0], p[1], p[2], p[3] };
+    }
+    if constexpr (WK == 2) { // each half of the wavefronts hands the other one's half of the columns over: [half][wr][r][t][lane]
+        float *red = reinterpret_cast<float *>(lds);
+        auto   at = [&](int half, int r, int t) { return reinterpret_cast<v4f *>(red + ((((half * 4 + wr) * RT + r) * NH + t) * 64 + lane) * 4); };
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+            for (int t = 0; t < NH; t++) *at(wk ^ 1, r, t) = wk == 0 ? acc[r][NH + t] : acc[r][t];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+            for (int t = 0; t < NH; t++) acc[r][t] = (wk == 0 ? acc[r][t] : acc[r][NH + t]) + *at(wk, r, t);
+        __syncthreads();
+    }
+    if (splitK == 1) {
+        constexpr int kCols = WK == 2 ? NH : NT; // column tiles that a wavefront holds results of
+        tile_park<FM, NT, RT, 4, half_t, 0, kCols>(acc, sc4, lds + (size_t)wk * NH * 16 * (TM * 2 + 16), wr, col, q);
+        __syncthreads();
+        tile_flush<NT, RT, 4, NTHREADS, half_t>(C, lds, M, N, mb, nbase, tid);
+    } else {
+        // fp32 partial sums in two turns, one half of the columns each: both at once take more LDS than the K loop
+        float *out = ws + (size_t)split * N * M;
+        if (WK == 1 || wk == 0) tile_park<FM, NT, RT, 4, float, 0, NH>(acc, sc4, lds, wr, col, q);
+        __syncthreads();
+        tile_flush<NH, RT, 4, NTHREADS, float>(out, lds, M, N, mb, nbase, tid);
+        __syncthreads();
+        if constexpr (WK == 1) {
+            tile_park<FM, NT, RT, 4, float, NH, NT>(acc, sc4, lds, wr, col, q);
+        } else {
+            if (wk == 1) tile_park<FM, NT, RT, 4, float, 0, NH>(acc, sc4, lds, wr, col, q);
+        }
+        __syncthreads();
+        tile_flush<NH, RT, 4, NTHREADS, float>(out, lds, M, N, mb, nbase + NH * 16, tid);
+    }
+}
+
 // Native layout -> fp16 [M,K], with the GEMM's own conversion code.  One lane per (row tile, K block, lane) triple.
 template <int FM, bool GS>
 __global__ __launch_bounds__(256) void dequant_native(half_t *__restrict__ out, const uint8_t *__restrict__ W, const half_t *__restrict__ scales,
@@ -1725,6 +1945,26 @@ int launch_prefill(hipStream_t st, const void *W, const void *sc, const void *ge
                        (uint32_t)M, (uint32_t)N, (uint32_t)K, units, (uint32_t)splitK, nblocks);
     return (int)hipGetLastError();
 }
+template <int FM, bool GS, int NT, int RT, int WK>
+int launch_wide(hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, float *ws, size_t M, size_t N, size_t K,
+                int splitK)
+{
+    constexpr int    TN = NT * 16, TM = 4 * RT * 16;
+    constexpr size_t kLoopLds = WK * 2 * (size_t)TN * 256, out_full = tile_stage_bytes<NT, RT, 4>(false), out_part = tile_stage_bytes<NT / 2, RT, 4>(true);
+    constexpr size_t kSums = WK == 2 ? (size_t)TM * TN * 4 : 0, kOut = out_full > out_part ? out_full : out_part, kMore = kOut > kSums ? kOut : kSums;
+    constexpr size_t kLds = kLoopLds > kMore ? kLoopLds : kMore;
+    static_assert(kLds <= 160 * 1024 / (3 - WK), "two workgroups of four wavefronts or one of eight do not fit in LDS");
+    if (M % TM) return FP6MI_ERR_SHAPE;
+    if (kLds > 48 * 1024)
+        if (int rc = allow_dynamic_lds<&gemm_wide<FM, GS, NT, RT, WK>>(kLds)) return rc;
+    uint32_t units = (uint32_t)((K + 255) / 256), nblocks = (uint32_t)((N + TN - 1) / TN);
+    size_t   wgs = (M / TM) * (size_t)splitK * nblocks;
+    if (wgs > 0x7fffffffu || K > (size_t)1 << 20) return FP6MI_ERR_SHAPE; // (K: 32-bit offsets over TN rows)
+    hipLaunchKernelGGL((gemm_wide<FM, GS, NT, RT, WK>), dim3((uint32_t)wgs), dim3(4 * WK * kWave), kLds, st, static_cast<const uint8_t *>(W),
+                       static_cast<const half_t *>(sc), static_cast<const uint8_t *>(gexp), static_cast<const half_t *>(B), static_cast<half_t *>(C), ws,
+                       (uint32_t)M, (uint32_t)N, (uint32_t)K, units, (uint32_t)splitK, nblocks);
+    return (int)hipGetLastError();
+}
 // kind 0: gemm_stream (wr == 1, wk = wavefronts per workgroup);  kind 1: gemm_tile (wr x wk wavefronts);  kind 2: gemm_ws (wr arithmetic + wk loading wavefronts),
 // or with wr = wk = 2 gemm_prefill (2 x 2 wavefronts; nt = column tiles of the whole workgroup, rt = row tiles per wavefront)
 template <int FM, bool GS>
@@ -1761,9 +2001,10 @@ int launch_cfg(const LaunchCfg &c, hipStream_t st, const void *W, const void *sc
 #define FP6MI_CASE(NT, RT, WR, PW) \
     if (c.nt == NT && c.rt == RT && c.wr == WR && c.wk == PW) { \
         if constexpr (WR == 2) return launch_prefill<FM, GS, NT / 2, RT>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
+        else if constexpr (PW <= 2) return launch_wide<FM, GS, NT, RT, PW>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
         else return launch_ws<FM, GS, NT, RT, WR, PW, WR == 4 && NT < 6 ? 3 : 2, WR == 4 && NT == 3 ? 3 : 2>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
     }
-        FP6MI_CASE(4, 2, 8, 4) FP6MI_CASE(4, 2, 4, 4) FP6MI_CASE(2, 2, 8, 4) FP6MI_CASE(8, 4, 2, 2) FP6MI_CASE(3, 2, 4, 4) FP6MI_CASE(5, 2, 4, 4) FP6MI_CASE(6, 2, 4, 4)
+        FP6MI_CASE(4, 2, 8, 4) FP6MI_CASE(4, 2, 4, 4) FP6MI_CASE(2, 2, 8, 4) FP6MI_CASE(8, 4, 2, 2) FP6MI_CASE(3, 2, 4, 4) FP6MI_CASE(5, 2, 4, 4) FP6MI_CASE(6, 2, 4, 4) FP6MI_CASE(8, 4, 4, 1) FP6MI_CASE(8, 4, 4, 2) FP6MI_CASE(6, 4, 4, 1) FP6MI_CASE(8, 2, 4, 2) FP6MI_CASE(6, 2, 4, 2) FP6MI_CASE(4, 2, 4, 2)
 #undef FP6MI_CASE
     }
     return FP6MI_ERR_SHAPE;

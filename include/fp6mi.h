@@ -162,6 +162,9 @@ int fp6mi_query_launch(int E, int Mbits, size_t M, size_t N, size_t K, int split
  * neighbour, a splitK the table does not hold, or the prefill kernel in the place of the shape that the table would give: its rows
  * do not hold that kernel).  Negative: FP6MI_ERR_*.  (No counterpart in the reference.) */
 int fp6mi_launch_source(int E, int Mbits, size_t M, size_t N, size_t K, int splitK);
+/* The two above report the table and the rules.  From 97 columns on a call is run by gemm_wide instead (launch kind 2 with row_waves 4 and k_waves 1 or 2)
+ * where that is expected to be faster: this is the shape that a call launches (grouped: 1 with group exponents).  (No counterpart in the reference.) */
+int fp6mi_query_kernel(int E, int Mbits, size_t M, size_t N, size_t K, int splitK, int grouped, int *shape);
 
 /* Device-side conversion reference layout -> native layout (both device pointers), run once per weight matrix. */
 int fp6mi_relayout_ref_to_native_gpu(int E, int Mbits, void *stream, void *native_dev, const void *packed_ref_dev,

@@ -314,6 +314,69 @@ def test_tiles_of_256_rows_counted_in_panels(cfg):
     check_close(y, oracle.gemm_f64(oracle.dequant(raw, sc, 3, 2), x), "cfg %s" % (cfg,))
 
 
+WIDE_SHAPES = [c for c in WS_SHAPES if c[3] == 4 and c[4] <= 2]
+
+
+@pytest.mark.parametrize("E,M", FORMATS)
+@pytest.mark.parametrize("IC", [64, 320, 1088, 1152, 1216, 1280, 1536])
+def test_wide_kernel_at_the_edges_of_k_and_n(E, M, IC):
+    """The wide kernel walks K in chunks of 128 columns, with two K halves in the odd and even ones: one block, an odd number of them and an even one, the
+    last cut after 64, 128 and 192 columns; one batch row in the last column block; splits that leave a workgroup a block or none.  Infinite
+    activations stand where a stage was last filled before what lies beyond K: a stale copy of one would meet the padding's zero weights and give NaN."""
+    print("case wide edges", E, M, IC, flush=True)
+    OC = 256
+    codes = np.random.default_rng(IC).integers(1, 1 << (E + M), (OC, IC)).astype(np.uint8)   # no zero weights
+    raw, sc = quant.pack_raw(codes, E, M), np.ones(OC, dtype=np.float16)
+    last = (IC + 255) // 256 * 256
+    for cfg in WIDE_SHAPES:
+        for N in (1, 16 * cfg[1] + 1):
+            x = synth.activations(IC, N, IC)
+            x[::2, :] = np.abs(x[::2, :])
+            for n in range(0, N, 2):
+                x[n, max(0, IC - 1 - (n * 7) % (256 + last - IC))] = np.inf
+            native, scd, xd = upload(raw, sc, x, E, M)
+            ref = oracle.gemm_f64(oracle.dequant(raw, sc, E, M), x[1::2]) if N > 1 else None
+            for splitK in (1, 2, 7):
+                y = gemm_capi(E, M, native, scd, xd, OC, splitK, cfg)
+                assert np.isinf(y[0::2]).all(), (cfg, N, splitK)
+                if N > 1:
+                    check_close(y[1::2], ref, "cfg %s N %d splitK %d" % (cfg, N, splitK))
+
+
+@pytest.mark.parametrize("E,M", FORMATS)
+@pytest.mark.parametrize("cfg", WIDE_SHAPES)
+def test_wide_kernel_with_group_exponents(E, M, cfg):
+    """Group exponents in the wide kernel, nine K blocks (the last cut), one round of panels and a split."""
+    OC, IC, N = 512, 2176, 16 * cfg[1] + 5
+    codes, sc, ex = quant.quantize_groupwise(_grouped_weights(91, OC, IC), E, M)
+    native = fp6.weight_prepacking_native_cpu(E, M, torch.from_numpy(quant.pack_raw(codes, E, M))).to(DEV)
+    gexp = fp6.pack_group_exps(torch.from_numpy(ex), OC, IC).to(DEV)
+    scd = torch.from_numpy(sc).to(DEV)
+    x = synth.activations(92, N, IC)
+    xd = torch.from_numpy(x).to(DEV)
+    ref = oracle.gemm_f64(oracle.dequant_grouped_from_definition(codes, sc, ex, E, M), x)
+    for splitK in (1, 2):
+        y = torch.full((N, OC), float("nan"), dtype=torch.float16, device=DEV)
+        ws = torch.empty(splitK * N * OC, dtype=torch.float32, device=DEV)
+        rc = _lib.lib().fp6mi_linear_native_grouped_cfg(E, M, torch.cuda.current_stream().cuda_stream, native.data_ptr(), scd.data_ptr(), gexp.data_ptr(),
+                                                        xd.data_ptr(), y.data_ptr(), OC, N, IC, ws.data_ptr(), splitK, *cfg)
+        assert rc == 0
+        check_close(y.cpu().numpy(), ref, "cfg %s splitK %d" % (cfg, splitK))
+
+
+@pytest.mark.parametrize("OC,IC,N", [(2304, 1152, 1930), (2816, 320, 600), (256, 320, 4096)])
+def test_wide_kernel_tiles_cover_the_output(OC, IC, N):
+    """Counted by rows and in panels, the last of them lower, and one row block against many column blocks.  The output starts as NaN."""
+    raw, sc, x = synth.uniform_problem(802 + OC, OC, IC, N)
+    native, scd, xd = upload(raw, sc, x, 3, 2)
+    ref = oracle.gemm_f64(oracle.dequant(raw, sc, 3, 2), x)
+    for cfg in WIDE_SHAPES:
+        print("case wide tiles", OC, IC, N, cfg, flush=True)
+        y = gemm_capi(3, 2, native, scd, xd, OC, 1, cfg)
+        assert np.isfinite(y).all()
+        check_close(y, ref, "cfg %s" % (cfg,))
+
+
 def test_unsupported_launch_shape_is_rejected():
     raw, sc, x = synth.uniform_problem(1, 256, 256, 4)
     native, scd, xd = upload(raw, sc, x, 3, 2)

@@ -641,6 +641,32 @@ def test_launch_source_of_problems_the_prefill_rule_takes():
         assert (L.fp6mi_launch_source(3, 2, OC, N, IC, 1) == 2) == prefill
 
 
+def test_wide_kernel_takes_the_place_of_larger_tiles():
+    """fp6mi_query_kernel is what a call launches: the table's shape or the rules' up to 96 columns, where K is beyond the wide kernel's 32-bit offsets and where
+    the problem is small; a compiled shape that divides the rows everywhere."""
+    from fp6_llm_amd import tune
+    L = _lib.lib()
+    base, shape = (ctypes.c_int * 5)(), (ctypes.c_int * 5)()
+    compiled = set(tune.COMPILED_STREAM + tune.COMPILED_TILE + tune.COMPILED_WS)
+    rng = np.random.default_rng(11)
+    seen = set()
+    for _ in range(2000):
+        E, M = FORMATS[rng.integers(len(FORMATS))]
+        OC, IC, N = 256 * int(2 ** rng.uniform(0, 7.5)), 64 * int(2 ** rng.uniform(0, 9)), int(2 ** rng.uniform(0, 13.5))
+        for splitK in {1, int(rng.integers(1, 12)), fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M)}:
+            for grouped in (0, 1):
+                assert L.fp6mi_query_launch(E, M, OC, N, IC, splitK, base) == 0 and L.fp6mi_query_kernel(E, M, OC, N, IC, splitK, grouped, shape) == 0
+                s = tuple(shape)
+                wide = s[0] == 2 and s[3] == 4 and s[4] <= 2
+                assert s in compiled and (s[0] == 0 or OC % tune.tile_rows(s) == 0)
+                assert (wide and N > 96 and splitK <= (IC + 255) // 256) or s == tuple(base)
+                seen.add(s)
+    assert {(2, 8, 4, 4, 1), (2, 8, 4, 4, 2), (2, 6, 4, 4, 1), (2, 8, 2, 4, 2), (2, 6, 2, 4, 2), (2, 4, 2, 4, 2)} <= seen
+    for OC, IC, N, wide in ((8192, 8192, 96, False), (1536, 1216, 258, False), (28672, 8192, 2048, True), (8192, 1 << 21, 2048, False)):
+        assert L.fp6mi_query_kernel(3, 2, OC, N, IC, 1, 0, shape) == 0 and (shape[0] == 2 and shape[3] == 4 and shape[4] <= 2) == wide
+    assert L.fp6mi_query_kernel(3, 2, 100, 1, 64, 1, 0, shape) == -2 and L.fp6mi_query_kernel(4, 3, 256, 1, 64, 1, 0, shape) == -1
+
+
 def test_every_matrix_of_the_table_is_measured_at_every_batch():
     """A matrix with no row at a batch is answered from its neighbours there: 9216 x 9216 in FP5 was cut into four at 257 to 320 columns, where it and
     each of its neighbours are fastest unsplit (and four pieces do not fit the static workspace)."""
