@@ -1538,36 +1538,41 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 // its side.  A 24-bit w can be as near as 2^-24, where q might round onto the midpoint: for fp32 weights the sign of a second
 // residual turns q into the quotient rounded to odd (truncated, last bit set if inexact), which never sits on a midpoint.
 //
-// HBM-bound.  Two organisations of the same arithmetic.  quant_fused: one workgroup of eight wavefronts per 16-row tile reads
+// HBM-bound but for its arithmetic, which does not hide: a chip's worth of workgroups loads, finds its maxima and converts in step.  Clamps, NaN tests and
+// sign handling made that 10 operations a weight (17 us of 46 at 8192x8192); they are left to a second pass of the wavefronts that have met an Inf, a NaN or a
+// scale that is no normal number, the others take 5 (quantize_string's PLAIN).  us, e3m2, before -> now, row scales and group exponents: bf16 8192x8192
+// 45.9 -> 41.9, 49.6 -> 44.0; 3072x8192 23.5 -> 18.9, 26.1 -> 20.7; 28672x8192 141 -> 136, 142 -> 137; 8192x28672 176 -> 165, 183 -> 176; fp16 8192x8192
+// 47.1 -> 43.1, 51.6 -> 45.2; fp32 8192x8192 95.2 -> 87.6, 98.7 -> 91.9.
+//
+// Two organisations of the same arithmetic.  quant_fused: one workgroup of eight wavefronts per 16-row tile reads
 // its rows, finds the scales, and converts; the last two blocks of every wavefront are still in its registers then, with 16-bit weights the one
 // before them in LDS, and the others are read again, latest first (8192x8192: a quarter of the weights twice).
 // quant_row_scales + quant_blocks: a workgroup takes a row, then a wavefront a block, and all weights are read twice.
-// Measured, us, fused / two kernels (e3m2; rotating through more memory than the caches hold):
-//              bf16            bf16 groups     fp16            fp32            fp32 groups
-//   1024x1024    5.0 /   7.2     5.5 /   7.7     4.9 /   7.2     6.2 /   8.4     6.8 /   9.3
-//   1024x3072    7.5 /   8.3     8.5 /   8.9     8.2 /   8.2    11.8 /  11.1    12.9 /  11.9
-//   1024x8192   17.1 /  11.6    20.7 /  12.9    19.5 /  12.0    27.4 /  17.0    30.2 /  17.6
-//   2048x4096   10.8 /  11.9    12.6 /  13.0    12.1 /  12.2    16.2 /  17.2    17.8 /  17.9
-//   2048x8192   19.2 /  16.6    23.0 /  18.6    22.1 /  17.8    33.5 /  28.0    36.6 /  29.1
-//   2560x4096   11.4 /  14.3    13.2 /  15.6    12.7 /  14.6    17.6 /  20.2    19.3 /  21.1
-//   3072x8192   23.1 /  23.0    26.2 /  25.7    25.3 /  24.4    40.7 /  40.3    43.4 /  40.6
-//   4096x4096   13.8 /  18.0    15.6 /  19.8    15.2 /  19.1    23.5 /  28.1    25.2 /  29.1
-//   8192x8192   49.3 /  55.0    58.9 /  59.2    50.4 /  55.5   103.2 /  97.4   109.0 /  98.1
-// Fewer than 192 workgroups do not pull enough from memory to pay for a second pass over a long row.  The line taken (fused from 192 tiles on, or up to
-// K = 3072) was drawn for bf16; on its wrong side stand 2560x4096 (two kernels taken, up to 20 % behind), 3072x8192 (fused taken, up to 7 %), and with
-// fp32 weights 1024x3072 and 8192x8192 (fused taken, up to 11 %).  e2m1 follows e3m2.  (The 16-bit columns of "fused" are those of three blocks in registers
-// and none in LDS.  That takes more than 128 registers with group exponents, and the CU then holds one workgroup; a block in LDS and two in registers leave
-// room for two with either.  us, bf16, before -> now, row scales and group exponents: 4096x4096 13.6 -> 13.2, 15.4 -> 14.9; 8192x7168 34.9 -> 33.8, 44.5 -> 36.6;
-// 8192x8192 49.1 -> 47.6, 57.6 -> 49.6; 28672x4096 61.5 -> 61.0, 87.5 -> 64.3; 8192x28672 178 -> 176, 179 -> 182.  Behind by 1-2 % at 4096x11008 and 3072x2048
-// and, with row scales, by 2-4 % at 28672x8192, where groups gain 20 %.  Three in registers and one in LDS, nothing read
-// twice at 8192 columns: 51.4, 53.7 with one workgroup to a CU, 51.9, 56.1 held to 128 registers, which spills.)
+// Measured, us, e3m2, fused / two kernels (replayed from a graph, through more memory than the caches hold):
+//               bf16            bf16 groups     fp32            fp32 groups
+//   1024x3072     6.4 /   7.9     7.4 /   8.2     9.9 /  10.1    10.8 /  10.4
+//   1024x4096     7.6 /   8.3     9.2 /   8.6    11.4 /  11.1    12.5 /  11.5
+//   1536x4096     8.0 /   9.9     9.6 /  10.4    12.9 /  13.9    14.1 /  14.2
+//   2048x4096     8.9 /  11.0    10.2 /  11.5    14.3 /  16.5    15.5 /  16.9
+//   2048x6144    12.3 /  13.5    13.9 /  14.1    20.2 /  22.3    22.1 /  23.0
+//   2048x8192    15.6 /  16.2    18.9 /  16.6    26.9 /  26.9    29.6 /  27.7
+//   2560x8192    16.8 /  19.3    19.6 /  19.7    30.6 /  33.4    32.4 /  33.7
+//   2816x16384   36.0 /  37.3    40.0 /  37.9    65.4 /  68.7    69.2 /  68.6
+//   4096x8192    23.1 /  28.7    24.8 /  29.5    47.7 /  50.1    49.2 /  50.6
+//   8192x8192    42.9 /  52.7    45.0 /  52.7    93.3 /  95.2    98.6 /  94.6
+//   4096x28672   85.8 /  89.4    89.9 /  89.6   164 / 180       168 / 180
+//  16384x4096    37.2 /  53.6    38.8 /  53.7    72.2 /  93.6    76.1 /  93.8
+// Few workgroups do not pull enough from memory to pay for a second pass over a long row: fused from 160 tiles on, and below that up to K = 3072 or three
+// times the rows.  On the wrong side of that line group exponents of 2816x16384 (6 %) and, in fp32, 8192x8192 (4 %) and 1024x3072 (4 %).
+// (A block of every wavefront in LDS and two in registers leave room for two workgroups to a CU.  Three in registers and one in LDS, nothing read
+// twice at 8192 columns, were slower with one workgroup to a CU, and held to 128 registers they spill.)
 // A conversion in double precision, code by code through a byte array in scratch memory, took 532 us at 8192x8192.
 // ---------------------------------------------------------------------------------------------------------------
 struct bf16_t { uint16_t bits; };
 typedef short v2s __attribute__((ext_vector_type(2)));
 
-// Eight consecutive weights as loaded, their widening, and a running maximum of their magnitudes that lets NaN and Inf pass by: magnitude
-// bits order like the values, and adding the distance of the exponent field's top to the sign bit makes Inf and NaN negative.
+// Eight consecutive weights as loaded, their widening, and a running maximum of their magnitudes: magnitude bits order like the values, with Inf and NaN above
+// all others.  A wavefront that has met one of these (`special`) goes over its weights once more with `add_finite`, which lets them pass by.
 template <typename T> struct WeightPiece {
     v4u x;
     __device__ __forceinline__ void load(const T *p) { x = *reinterpret_cast<const v4u *>(p); }
@@ -1588,33 +1593,50 @@ template <> struct WeightPiece<float> {
     __device__ __forceinline__ float value(int j) const { return __builtin_bit_cast(float, j < 4 ? x[j] : y[j - 4]); }
 };
 template <typename T> struct MaxMagnitude {
-    static constexpr short kLift = std::is_same<T, bf16_t>::value ? 0x0080 : 0x0400; // 0x8000 - the bits of infinity
-    v2s m = { kLift, kLift };
+    typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+    static constexpr uint16_t kInf = std::is_same<T, bf16_t>::value ? 0x7F80 : 0x7C00;
+    v2us                      m = { 0, 0 };
     __device__ __forceinline__ void add(const WeightPiece<T> &p)
     {
 #pragma unroll
-        for (int i = 0; i < 4; i++) m = __builtin_elementwise_max(m, __builtin_bit_cast(v2s, p.x[i] & 0x7FFF7FFFu) + (v2s){ kLift, kLift });
+        for (int i = 0; i < 4; i++) m = __builtin_elementwise_max(m, __builtin_bit_cast(v2us, p.x[i] & 0x7FFF7FFFu));
     }
-    __device__ __forceinline__ float value() const
-    {
-        const uint16_t b = (uint16_t)((m[0] > m[1] ? m[0] : m[1]) - kLift);
-        if constexpr (std::is_same<T, bf16_t>::value)
-            return __builtin_bit_cast(float, (uint32_t)b << 16);
-        else
-            return (float)__builtin_bit_cast(half_t, b);
-    }
-};
-template <> struct MaxMagnitude<float> {
-    int m = 0x00800000;
-    __device__ __forceinline__ void add(const WeightPiece<float> &p)
+    __device__ __forceinline__ void add_finite(const WeightPiece<T> &p)
     {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            m = max(m, (int)((p.x[i] & 0x7FFFFFFFu) + 0x00800000u));
-            m = max(m, (int)((p.y[i] & 0x7FFFFFFFu) + 0x00800000u));
+            const v2us a = __builtin_bit_cast(v2us, p.x[i] & 0x7FFF7FFFu);
+            m = __builtin_elementwise_max(m, (v2us){ a[0] < kInf ? a[0] : (uint16_t)0, a[1] < kInf ? a[1] : (uint16_t)0 });
         }
     }
-    __device__ __forceinline__ float value() const { return __builtin_bit_cast(float, m - 0x00800000); }
+    __device__ __forceinline__ uint16_t top() const { return m[0] > m[1] ? m[0] : m[1]; }
+    __device__ __forceinline__ bool     special() const { return top() >= kInf; }
+    __device__ __forceinline__ float    value() const
+    {
+        if constexpr (std::is_same<T, bf16_t>::value)
+            return __builtin_bit_cast(float, (uint32_t)top() << 16);
+        else
+            return (float)__builtin_bit_cast(half_t, top());
+    }
+};
+template <> struct MaxMagnitude<float> {
+    static constexpr uint32_t kInf = 0x7F800000u;
+    uint32_t                  m = 0;
+    __device__ __forceinline__ void add(const WeightPiece<float> &p)
+    {
+#pragma unroll
+        for (int i = 0; i < 4; i++) m = max(m, max(p.x[i] & 0x7FFFFFFFu, p.y[i] & 0x7FFFFFFFu));
+    }
+    __device__ __forceinline__ void add_finite(const WeightPiece<float> &p)
+    {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint32_t a = (i < 4 ? p.x[i & 3] : p.y[i & 3]) & 0x7FFFFFFFu;
+            m = max(m, a < kInf ? a : 0u);
+        }
+    }
+    __device__ __forceinline__ bool  special() const { return m >= kInf; }
+    __device__ __forceinline__ float value() const { return __builtin_bit_cast(float, m); }
 };
 
 // round-to-nearest-even of a non-negative double to fp16 without passing through float (no double rounding)
@@ -1633,33 +1655,54 @@ template <int FM> __device__ __forceinline__ half_t row_scale(float amax)
     return (float)sc == 0.f ? (half_t)1.0f : sc;
 }
 
+// FP4's coarser grid (steps of 1/2 below 2, 1 below 4, 2 above), on which values are exact in the fields
+__device__ __forceinline__ float fp4_grid(float q)
+{
+    const float magic = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, __builtin_fmaxf(__builtin_fabsf(q), 1.f)) & 0x7F800000u) * 6291456.f; // 1.5 * 2^23 steps
+    return (q + magic) - magic;
+}
+
 // The 32 weights of one field string (four pieces of eight) against the scale f -> their 6-bit fields.
-template <int FM, typename T> __device__ __forceinline__ v6u quantize_string(const WeightPiece<T> *p, float f)
+// PLAIN: the weights are finite and the row's scale is a normal fp16 number, so that no quotient is beyond the largest code by more than the rounding of the
+// scale (2^-11, which rounds to that code), and the arithmetic carries signs by itself: the residual is taken as q * f - w, whose exact zero leaves a
+// quotient of -0 alone.  Three operations a 16-bit weight instead of eight.
+template <int FM, typename T, bool PLAIN> __device__ __forceinline__ v6u quantize_string(const WeightPiece<T> *p, float f)
 {
     typedef float v16f __attribute__((ext_vector_type(16)));
     // the fields of FP5 hold a quarter of the value (its grid up to 7 is the e3m2 grid up to 1.75, times 4)
     constexpr float top = (float)Fmt<FM>::max_value / Fmt<FM>::post_scale, kInf = __builtin_inff();
     f *= Fmt<FM>::post_scale;
-    const bool  overflown = f == kInf; // a row whose scale left fp16: finite weights become zeros
+    const bool  overflown = !PLAIN && f == kInf; // a row whose scale left fp16: finite weights become zeros
     const float rf = overflown ? 0.f : 1.0f / f, fd = overflown ? 0.f : f, limit = overflown ? 3.4028234663852886e38f : kInf;
     v16f        even, odd;
 #pragma unroll
     for (int i = 0; i < 32; i++) {
-        const float w = p[i >> 3].value(i & 7), a = __builtin_fabsf(w);
-        float       q = __builtin_fminf(a * rf, 2.f * top);
-        q = __builtin_fminf(__builtin_fmaf(__builtin_fmaf(-q, fd, a), rf, q), top);
-        if constexpr (std::is_same<T, float>::value) {
-            const float r = __builtin_fmaf(-q, fd, a);
-            uint32_t    u = __builtin_bit_cast(uint32_t, q);
-            if (r < 0.f) u -= 1;
-            if (r != 0.f) u |= 1;
-            q = __builtin_bit_cast(float, u);
+        const float w = p[i >> 3].value(i & 7);
+        float       q;
+        if constexpr (PLAIN) {
+            q = w * rf;
+            q = __builtin_fmaf(-__builtin_fmaf(q, fd, -w), rf, q);
+            if constexpr (std::is_same<T, float>::value) {
+                const float r = __builtin_fmaf(-q, fd, w);
+                uint32_t    u = __builtin_bit_cast(uint32_t, q);
+                if ((int)(__builtin_bit_cast(uint32_t, r) ^ u) < 0) u -= 1;
+                q = r != 0.f ? __builtin_bit_cast(float, u | 1u) : q;
+            }
+            if constexpr (Fmt<FM>::bits == 4) q = __builtin_copysignf(fp4_grid(q), w);
+        } else {
+            const float a = __builtin_fabsf(w);
+            q = __builtin_fminf(a * rf, 2.f * top);
+            q = __builtin_fminf(__builtin_fmaf(__builtin_fmaf(-q, fd, a), rf, q), top);
+            if constexpr (std::is_same<T, float>::value) {
+                const float r = __builtin_fmaf(-q, fd, a);
+                uint32_t    u = __builtin_bit_cast(uint32_t, q);
+                if (r < 0.f) u -= 1;
+                if (r != 0.f) u |= 1;
+                q = __builtin_bit_cast(float, u);
+            }
+            if constexpr (Fmt<FM>::bits == 4) q = fp4_grid(q);
+            q = a <= limit ? __builtin_copysignf(q, w) : 0.f; // NaN: +0
         }
-        if constexpr (Fmt<FM>::bits == 4) { // to the coarser grid first (steps of 1/2 below 2, 1 below 4, 2 above): exact in the fields then
-            const float magic = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, __builtin_fmaxf(q, 1.f)) & 0x7F800000u) * 6291456.f; // 1.5 * 2^23 steps
-            q = (q + magic) - magic;
-        }
-        q = a <= limit ? __builtin_copysignf(q, w) : 0.f; // NaN: +0
         if (i & 1)
             odd[i >> 1] = q;
         else
@@ -1670,6 +1713,8 @@ template <int FM, typename T> __device__ __forceinline__ v6u quantize_string(con
     else
         return __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(even, odd, 1.0f);
 }
+// (wave-uniform) whether every row of a wavefront's block has a scale of the PLAIN kind
+__device__ __forceinline__ bool plain_scales(float sc) { return __all(sc >= 6.103515625e-5f && sc < __builtin_inff()); }
 
 // A lane of the quantizer is (m = l/4, p = l%4): the four lanes of a row read 64 or 128 consecutive bytes, and its codes go to the places
 // of lane (m, q = p) of the native block.  w points at the tile's first row.
@@ -1677,17 +1722,20 @@ template <typename T> __device__ __forceinline__ void load_quant_block(WeightPie
 {
     const T *p = w + (size_t)(lane >> 2) * K + (size_t)U * 256 + 8 * (lane & 3);
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
-        if (U * 256 + 32 * s < K) // uniform: K is a multiple of 64
-            x[s].load(p + 32 * s);
-        else
-            x[s].zero();
+    for (int s = 0; s < 8; s++) x[s].zero();
+    if (U * 256 + 256 <= K) { // (uniform) one branch for all but the block that K cuts
+#pragma unroll
+        for (int s = 0; s < 8; s++) x[s].load(p + 32 * s);
+    } else {
+#pragma unroll
+        for (int s = 0; s < 6; s += 2) // K is a multiple of 64
+            if (U * 256 + 32 * s < K) x[s].load(p + 32 * s), x[s + 1].load(p + 32 * s + 32);
     }
 }
 // GROUPS: every group of 128 columns of a row also gets the smallest factor 2^k, -15 <= k <= 0, that still holds its largest
 // magnitude, stored as the byte 127 + k, and its codes are chosen against scale * 2^k.  max_value * scale has at most 14 significant bits, so
 // comparing amax with it (by exponent, then by mantissa) decides like the double quotient amax / scale against max_value * 2^k.
-template <int FM, typename T, bool GROUPS>
+template <int FM, typename T, bool GROUPS, bool PLAIN>
 __device__ __forceinline__ void quantize_block(const WeightPiece<T> (&x)[8], float sc, uint8_t *native, uint8_t *gexp, size_t blk, uint32_t K, uint32_t U, int lane)
 {
     v6u str[2];
@@ -1697,7 +1745,12 @@ __device__ __forceinline__ void quantize_block(const WeightPiece<T> (&x)[8], flo
         if constexpr (GROUPS) {
             MaxMagnitude<T> mm;
 #pragma unroll
-            for (int s = 0; s < 4; s++) mm.add(x[4 * h + s]);
+            for (int s = 0; s < 4; s++) {
+                if constexpr (PLAIN)
+                    mm.add(x[4 * h + s]);
+                else
+                    mm.add_finite(x[4 * h + s]);
+            }
             float amax = mm.value();
             amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
             amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
@@ -1709,7 +1762,8 @@ __device__ __forceinline__ void quantize_block(const WeightPiece<T> (&x)[8], flo
             f = ldexpf(sc, k);
             if ((lane & 3) == 0) gexp[(blk * 16 + (lane >> 2)) * 2 + h] = (uint8_t)(127 + k);
         }
-        str[h] = quantize_string<FM, T>(x + 4 * h, f);
+        str[h] = quantize_string<FM, T, PLAIN>(x + 4 * h, f);
+        __builtin_amdgcn_sched_barrier(0); // one string's 32 quotients at a time
     }
     store_native_strings<FM>(str[0], str[1], native + blk * Fmt<FM>::block_bytes, (lane >> 2) + 16 * (lane & 3));
 }
@@ -1772,6 +1826,17 @@ __global__ __launch_bounds__(WAVES *kWave, sizeof(T) == 2 ? WAVES / 2 : 1) void 
 #pragma unroll
         for (int s = 0; s < 8; s++) mm.add(x[s]);
     }
+    const bool special = __any(mm.special());
+    if (special) { // Inf or NaN among this wavefront's weights: once more, without them
+        mm = MaxMagnitude<T>{};
+#pragma unroll 1
+        for (uint32_t i = 0; i < mine; i++) {
+            WeightPiece<T> x[8];
+            load_quant_block<T>(x, w, K, wave + i * WAVES, lane);
+#pragma unroll
+            for (int s = 0; s < 8; s++) mm.add_finite(x[s]);
+        }
+    }
     float amax = mm.value();
     amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
     amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
@@ -1791,19 +1856,27 @@ __global__ __launch_bounds__(WAVES *kWave, sizeof(T) == 2 ? WAVES / 2 : 1) void 
     for (int k = 0; k < KEEP; k++)
         if ((uint32_t)k < mine) {
             const uint32_t U = wave + (mine - 1 - k) * WAVES;
-            quantize_block<FM, T, GROUPS>(kept[k], sc, native, gexp, (size_t)R * units + U, K, U, lane);
+            quantize_block<FM, T, GROUPS, true>(kept[k], sc, native, gexp, (size_t)R * units + U, K, U, lane);
         }
     if (stash) {
         WeightPiece<T> x[8];
         const uint32_t U = wave + (mine - 1 - KEEP) * WAVES;
         stashed(x);
-        quantize_block<FM, T, GROUPS>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+        quantize_block<FM, T, GROUPS, true>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
     }
     for (uint32_t i = mine > held ? mine - held : 0; i-- > 0;) {
         WeightPiece<T> x[8];
         const uint32_t U = wave + i * WAVES;
         load_quant_block<T>(x, w, K, U, lane);
-        quantize_block<FM, T, GROUPS>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+        quantize_block<FM, T, GROUPS, true>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+    }
+    if (special || !plain_scales(sc)) { // again over what was just written (last, where nothing is held any more: before the fast pass it would spill)
+#pragma unroll 1
+        for (uint32_t U = wave; U < units; U += WAVES) {
+            WeightPiece<T> x[8];
+            load_quant_block<T>(x, w, K, U, lane);
+            quantize_block<FM, T, GROUPS, false>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+        }
     }
 }
 
@@ -1818,6 +1891,14 @@ __global__ __launch_bounds__(256) void quant_row_scales(half_t *__restrict__ sca
         WeightPiece<T> x;
         x.load(p + k);
         mm.add(x);
+    }
+    if (__any(mm.special())) { // Inf or NaN: once more, without them
+        mm = MaxMagnitude<T>{};
+        for (uint32_t k = threadIdx.x * 8; k < K; k += 2048) {
+            WeightPiece<T> x;
+            x.load(p + k);
+            mm.add_finite(x);
+        }
     }
     float amax = mm.value();
 #pragma unroll
@@ -1837,7 +1918,14 @@ __global__ __launch_bounds__(256) void quant_blocks(uint8_t *__restrict__ native
     const uint32_t R = blk / units, U = blk % units;
     WeightPiece<T> x[8];
     load_quant_block<T>(x, Wf + (size_t)R * 16 * K, K, U, lane);
-    quantize_block<FM, T, GROUPS>(x, (float)scales[R * 16 + (lane >> 2)], native, gexp, blk, K, U, lane);
+    const float     sc = (float)scales[R * 16 + (lane >> 2)];
+    MaxMagnitude<T> mm;
+#pragma unroll
+    for (int s = 0; s < 8; s++) mm.add(x[s]);
+    if (!__any(mm.special()) && plain_scales(sc))
+        quantize_block<FM, T, GROUPS, true>(x, sc, native, gexp, blk, K, U, lane);
+    else
+        quantize_block<FM, T, GROUPS, false>(x, sc, native, gexp, blk, K, U, lane);
 }
 // ------------------------------------------------------------------------------------------------ launch helpers
 
@@ -2055,7 +2143,7 @@ template <int FM> int op_quantize(void *stream, void *native, void *scales, void
     auto           run = [&](auto *typed, auto groups_c) {
         typedef std::remove_cv_t<std::remove_pointer_t<decltype(typed)>> T;
         constexpr bool GROUPS = decltype(groups_c)::value;
-        if (M / 16 >= 192 || K <= 3072) { // (where the two organisations cross: see quant_fused)
+        if (M / 16 >= 160 || K <= 3072 || K <= M * 3) { // (where the two organisations cross: see quant_fused)
             constexpr int WAVES = 8, KEEP = 2;
             const uint32_t stash = units > WAVES * KEEP ? quant_stash_bytes<T, WAVES>() : 0; // what some wavefront needs
             if (stash)

@@ -675,6 +675,34 @@ def test_drop_in_call_through_extension_and_python_agree(E, M, monkeypatch):
         assert torch.equal(y_ext, y_py), i
 
 
+@pytest.mark.parametrize("E,M", FORMATS)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("OC,IC", [(32, 64), (32, 2880), (32, 4416), (2560, 4416)])
+def test_device_quantizer_mixes_its_two_conversions(E, M, dtype, OC, IC):
+    """Wavefronts that meet an Inf, a NaN or a scale that is no normal fp16 number convert with clamps and tests, their neighbours in the same rows
+    without: one special block among plain ones (first, last, cut by K), tiles with subnormal, zero and overflown scales, zeros of both signs."""
+    print("case quantizer conversions", E, M, dtype, OC, IC, flush=True)
+    w = (torch.randn(OC, IC, generator=torch.Generator().manual_seed(IC)) * 0.02)
+    w[3, ::7], w[3, 1::7] = -0.0, 0.0
+    w[1, 0], w[2, IC - 1], w[4, IC // 2] = float("-inf"), float("nan"), float("inf")
+    w[OC - 16:] *= 2.0 ** -14 if dtype == torch.float16 else 2.0 ** -20                     # subnormal scales, some of them 2^-24 or 0
+    w[OC - 1] = (w[OC - 1].abs() + 0.5) * (6e4 if dtype == torch.float16 else 1e7)            # the largest scales of the type; beyond fp16 where it can be
+    w = w.to(dtype)
+    native, scales = fp6.weight_quantize_native_cuda(E, M, w.to(DEV))
+    native_g, scales_g, gexp = fp6.weight_quantize_native_cuda(E, M, w.to(DEV), group_scales=True)
+    per_tile, per_gexp = native.numel() // (OC // 16), gexp.numel() // (OC // 16)
+    for tile in (0, OC // 16 - 1):
+        rows = w[16 * tile:16 * tile + 16].float().numpy().astype(np.float64)
+        codes, sc_host = quant.quantize_rowwise(rows, E, M)
+        codes_g, _, ex = quant.quantize_groupwise(rows, E, M)
+        for sc in (scales, scales_g):
+            assert np.array_equal(sc[16 * tile:16 * tile + 16].cpu().numpy().view(np.uint16), sc_host.view(np.uint16))
+        for got, c in ((native, codes), (native_g, codes_g)):
+            want = fp6.weight_prepacking_native_cpu(E, M, torch.from_numpy(quant.pack_raw(c, E, M)))
+            assert torch.equal(got[per_tile * tile:per_tile * (tile + 1)].cpu(), want)
+        assert torch.equal(gexp[per_gexp * tile:per_gexp * (tile + 1)].cpu(), fp6.pack_group_exps(torch.from_numpy(ex), 16, IC))
+
+
 @pytest.mark.parametrize("IC", [4032, 4096, 4160, 6144, 6208, 8192, 8256, 12352])   # 16, 17, 24, 25, 32, 33 and 49 blocks: which wavefronts hold one in LDS
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_fused_quantizer_equals_the_two_kernel_one(IC, dtype):
