@@ -36,7 +36,8 @@ if os.path.exists(_lib.LIB_PATH) and not os.environ.get("FP6MI_NO_TORCH_EXT"):
     try:
         _lib.lib()
         from . import _fp6mi_torch as _ext
-        _ext.linear_forward_any_order   # the newest of the names used below
+        if "bias" not in (_ext.linear_forward_native.__doc__ or ""):   # the newest of the names and arguments used below
+            raise ImportError("the extension was built from an older tree")
     except (ImportError, OSError, AttributeError):   # extension not built or stale, or a stale library: the ctypes path reports what is wrong
         _ext = None
 
@@ -298,11 +299,12 @@ def _workspace(device, stream, nbytes):
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # the current stream's handle without building a Stream object
 
 
-def linear_forward_native(EXPONENT, MANTISSA, in_feats, native_weight, scales, OC, splitK=1, out=None, workspace=None, group_exps=None):
-    """out[B, OC] = in_feats[B, IC] @ dequant(W)^T with W in the native layout.  Enqueued on the current stream.
-    group_exps: the tensor of pack_group_exps on the same GPU for weights with per-group exponents, else None."""
+def linear_forward_native(EXPONENT, MANTISSA, in_feats, native_weight, scales, OC, splitK=1, out=None, workspace=None, group_exps=None, bias=None):
+    """out[B, OC] = in_feats[B, IC] @ dequant(W)^T (+ bias) with W in the native layout.  Enqueued on the current stream.
+    group_exps: the tensor of pack_group_exps on the same GPU for weights with per-group exponents, else None.
+    bias: contiguous float16 [OC] on the same GPU, added to the float32 sums before the one rounding, else None."""
     if _ext is not None:
-        return _ext.linear_forward_native(EXPONENT, MANTISSA, in_feats, native_weight, scales, OC, int(splitK), out, workspace, group_exps)
+        return _ext.linear_forward_native(EXPONENT, MANTISSA, in_feats, native_weight, scales, OC, int(splitK), out, workspace, group_exps, bias)
     _bits(EXPONENT, MANTISSA)
     if in_feats.dtype != torch.float16 or in_feats.dim() != 2:
         raise ValueError("in_feats must be a 2-D float16 tensor [B, IC]")
@@ -329,6 +331,8 @@ def linear_forward_native(EXPONENT, MANTISSA, in_feats, native_weight, scales, O
         out = torch.empty((B, OC), dtype=torch.float16, device=dev)
     elif out.shape != (B, OC) or out.dtype != torch.float16 or not out.is_contiguous() or out.device != dev:
         raise ValueError("out must be a contiguous float16 [B, OC] tensor on the same GPU")
+    if bias is not None and (bias.dtype != torch.float16 or bias.shape != (OC,) or not bias.is_contiguous() or bias.device != dev):
+        raise ValueError("bias must be a contiguous float16 [OC] tensor on the same GPU")
     L = _lib.lib()
     switch = dev.index is not None and dev.index != torch.cuda.current_device()
     if switch:
@@ -344,11 +348,16 @@ def linear_forward_native(EXPONENT, MANTISSA, in_feats, native_weight, scales, O
             elif workspace.dtype != torch.float32 or workspace.numel() * 4 < need or workspace.device != dev:
                 raise ValueError("workspace must be a float32 GPU tensor with at least splitK*B*OC elements")
             ws_ptr = workspace.data_ptr()
-        if group_exps is None:
+        if group_exps is not None:
+            _check_group_exps(group_exps, OC, IC, dev)
+        if bias is not None:
+            rc = L.fp6mi_linear_native_bias(EXPONENT, MANTISSA, stream, native_weight.data_ptr(), sc.data_ptr(),
+                                            None if group_exps is None else group_exps.data_ptr(), bias.data_ptr(), x.data_ptr(), out.data_ptr(),
+                                            OC, B, IC, ws_ptr, splitK)
+        elif group_exps is None:
             rc = L.fp6mi_linear_native(EXPONENT, MANTISSA, stream, native_weight.data_ptr(), sc.data_ptr(), x.data_ptr(),
                                        out.data_ptr(), OC, B, IC, ws_ptr, splitK)
         else:
-            _check_group_exps(group_exps, OC, IC, dev)
             rc = L.fp6mi_linear_native_grouped(EXPONENT, MANTISSA, stream, native_weight.data_ptr(), sc.data_ptr(), group_exps.data_ptr(),
                                                x.data_ptr(), out.data_ptr(), OC, B, IC, ws_ptr, splitK)
     finally:

@@ -22,9 +22,12 @@ typedef float    v4f __attribute__((ext_vector_type(4)));
 
 using fp6mi::LaunchCfg;
 
-// C[i] = fp16_rn(sum over splits, in split order, of ws[s][i]) for the four outputs from index i.
-__device__ __forceinline__ void reduce_four(half_t *__restrict__ C, const float *__restrict__ ws, size_t MN, int splitK, size_t i)
+// C[i] = fp16_rn(sum over splits, in split order, of ws[s][i] + bias) for the four outputs from index i.  bias: of the first of them
+template <bool BIAS> __device__ __forceinline__ void reduce_four(half_t *__restrict__ C, const float *__restrict__ ws, size_t MN, int splitK, size_t i, const half_t *bias)
 {
+    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+    v4h b;
+    if constexpr (BIAS) b = (v4h){ bias[0], bias[1], bias[2], bias[3] }; // (any 2-byte boundary)
     v4f sum = { 0.f, 0.f, 0.f, 0.f };
     // up to eight loads in flight instead of one round trip to memory per split; the order of the sum is unchanged.  The
     // remainder after the groups of eight is one group of its exact size (a 3 done as 2 + 1 would be two round trips).
@@ -48,16 +51,21 @@ __device__ __forceinline__ void reduce_four(half_t *__restrict__ C, const float 
     case 1: chunk(std::integral_constant<int, 1>{}, s); break;
     default: break;
     }
-    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+    if constexpr (BIAS) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) sum[k] += (float)b[k];
+    }
     v4h o = { (half_t)sum[0], (half_t)sum[1], (half_t)sum[2], (half_t)sum[3] };
     *reinterpret_cast<v4h *>(C + i) = o;
 }
 
 // four outputs per thread, in the order of the output
-__global__ __launch_bounds__(256) void splitk_reduce(half_t *__restrict__ C, const float *__restrict__ ws, size_t MN, int splitK)
+template <bool BIAS>
+__global__ __launch_bounds__(256) void splitk_reduce(half_t *__restrict__ C, const float *__restrict__ ws, size_t MN, int splitK, const half_t *__restrict__ bias,
+                                                     uint32_t M)
 {
     const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i < MN) reduce_four(C, ws, MN, splitK, i);
+    if (i < MN) reduce_four<BIAS>(C, ws, MN, splitK, i, BIAS ? bias + i % M : nullptr);
 }
 
 // The same sums with the workgroups placed where the partial sums were written.  gemm_tile hands XCD x (workgroup ids
@@ -67,8 +75,9 @@ __global__ __launch_bounds__(256) void splitk_reduce(half_t *__restrict__ C, con
 // XCD produced, for every batch column: its loads hit the L2 that the partial sums were written through, where the
 // output-order kernel above finds most of them behind another XCD's L2 (measured: 4 MB written by one kernel are read by
 // the next in 0.7 us from the writer's XCD and in 2.6 us from another).
+template <bool BIAS>
 __global__ __launch_bounds__(256) void splitk_reduce_by_xcd(half_t *__restrict__ C, const float *__restrict__ ws, uint32_t M, uint32_t N, int splitK,
-                                                             uint32_t tile_rows, uint32_t q, uint32_t r, uint32_t per_block)
+                                                             uint32_t tile_rows, uint32_t q, uint32_t r, uint32_t per_block, const half_t *__restrict__ bias)
 {
     const uint32_t x = blockIdx.x & 7u, j = blockIdx.x >> 3;
     const uint32_t s0 = x * q + (x < r ? x : r), s1 = (x + 1) * q + (x + 1 < r ? x + 1 : r);
@@ -76,7 +85,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_by_xcd(half_t *__restrict__
     const uint32_t g = j * 256 + threadIdx.x;
     if (g >= quads * N) return;
     const uint32_t n = g / quads, m = lo + (g - n * quads) * 4;
-    reduce_four(C, ws, (size_t)M * N, splitK, (size_t)n * M + m);
+    reduce_four<BIAS>(C, ws, (size_t)M * N, splitK, (size_t)n * M + m, BIAS ? bias + m : nullptr);
 }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -446,12 +455,12 @@ inline LaunchCfg final_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, 
     return pick_cfg(xbits, M, N, K, splitK, cus);
 }
 
-int linear_native(const fp6mi::FormatOps &ops, hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, size_t M, size_t N, size_t K, float *ws,
+int linear_native(const fp6mi::FormatOps &ops, hipStream_t st, const void *W, const void *sc, const void *gexp, const void *bias, const void *B, void *C, size_t M, size_t N, size_t K, float *ws,
                   int splitK, const LaunchCfg *forced)
 {
     LaunchCfg c = forced ? *forced : final_cfg(ops.bits, M, N, K, splitK, gexp != nullptr, current_device_cus());
     if (c.kind == 0 && !(c.rt & (c.rt - 1)) && (M / 16) % c.rt) return FP6MI_ERR_SHAPE; // (3, 5, 6, 7 tiles per workgroup end in a workgroup with fewer)
-    int rc = ops.gemm(c, st, W, sc, gexp, B, C, ws, M, N, K, splitK);
+    int rc = ops.gemm(c, st, W, sc, gexp, B, C, splitK > 1 ? ws : static_cast<float *>(const_cast<void *>(bias)), M, N, K, splitK); // (a workspace given without a split is no bias)
     if (rc != 0) return rc;
     if (splitK > 1) {
         size_t MN = M * N; // M % 256 == 0, so MN % 4 == 0
@@ -467,10 +476,10 @@ int linear_native(const fp6mi::FormatOps &ops, hipStream_t st, const void *W, co
                 most = rows > most ? rows : most;
             }
             const size_t per_xcd = (most / 4 * N + 255) / 256;
-            hipLaunchKernelGGL(splitk_reduce_by_xcd, dim3((uint32_t)(per_xcd * 8)), dim3(256), 0, st, static_cast<half_t *>(C), ws, (uint32_t)M, (uint32_t)N,
-                               splitK, (uint32_t)tile_rows, q, r, per_block);
+            hipLaunchKernelGGL(bias ? splitk_reduce_by_xcd<true> : splitk_reduce_by_xcd<false>, dim3((uint32_t)(per_xcd * 8)), dim3(256), 0, st, static_cast<half_t *>(C), ws, (uint32_t)M, (uint32_t)N,
+                               splitK, (uint32_t)tile_rows, q, r, per_block, static_cast<const half_t *>(bias));
         } else {
-            hipLaunchKernelGGL(splitk_reduce, dim3((uint32_t)((MN / 4 + 255) / 256)), dim3(256), 0, st, static_cast<half_t *>(C), ws, MN, splitK);
+            hipLaunchKernelGGL(bias ? splitk_reduce<true> : splitk_reduce<false>, dim3((uint32_t)((MN / 4 + 255) / 256)), dim3(256), 0, st, static_cast<half_t *>(C), ws, MN, splitK, static_cast<const half_t *>(bias), (uint32_t)M);
         }
         rc = (int)hipGetLastError();
     }
@@ -492,7 +501,7 @@ const char *fp6mi_error_string(int code)
     case FP6MI_ERR_NULL: return "a required pointer is NULL";
     case FP6MI_ERR_WORKSPACE: return "splitK > 1 needs a workspace of splitK*M*N floats";
     case FP6MI_ERR_SPLITK: return "splitK must be >= 1";
-    case FP6MI_ERR_ALIGN: return "weights, activations, output and workspace must be 16-byte aligned (scales: 2-byte, group exponents: 2-byte)";
+    case FP6MI_ERR_ALIGN: return "weights, activations, output and workspace must be 16-byte aligned (scales, group exponents, bias: 2-byte)";
     case FP6MI_ERR_TOO_LARGE: return "splitK*M*N floats exceed the library's static workspace (fp6mi_static_workspace_bytes)";
     case FP6MI_ERR_CAPTURE: return "the stream is being captured and this call would have to allocate: convert the weights first (fp6mi_relayout_ref_to_native_gpu) or make the first call outside the capture";
     default: return code > 0 ? hipGetErrorString((hipError_t)code) : "unknown fp6mi error";
@@ -506,7 +515,7 @@ const char *fp6mi_tuning_info(void)
         ;
 }
 
-int fp6mi_version(void) { return 138; } // 138: gemm_wide (launch kind 2 with four rows of one or two wavefronts) in the place of larger tiles from 97 columns on, the other kernels unchanged; 137: group exponents of 128 rows through LDS in the wave-specialized kernel, panels of 256-row tiles only for activations beyond L2; 136: tiles of 48, 80 and 96 columns, deeper rings in the wave-specialized kernel of 128 rows, panels; 135: prefill kernel (launch kind 2 with 2 x 2 wavefronts), relayout and quantizer kernels rewritten, the other GEMM kernels unchanged; 134: three row tiles per workgroup in the small-batch kernel (any M: the last workgroup takes what is left), no other kernel changed; 133: wave-specialized tile kernel (launch kind 2) for large batches; 132: split-K reduction runs on the XCD that wrote the partial sums, every grid size gets XCD-contiguous tiles; 131: tile kernel stores through LDS; 130: small-batch kernel loads activations as whole rows and turns them into operand order through LDS
+int fp6mi_version(void) { return 139; } // 139: a bias in the epilogues of the GEMM kernels, the quantizer's arithmetic; 138: gemm_wide (launch kind 2 with four rows of one or two wavefronts) in the place of larger tiles from 97 columns on, the other kernels unchanged; 137: group exponents of 128 rows through LDS in the wave-specialized kernel, panels of 256-row tiles only for activations beyond L2; 136: tiles of 48, 80 and 96 columns, deeper rings in the wave-specialized kernel of 128 rows, panels; 135: prefill kernel (launch kind 2 with 2 x 2 wavefronts), relayout and quantizer kernels rewritten, the other GEMM kernels unchanged; 134: three row tiles per workgroup in the small-batch kernel (any M: the last workgroup takes what is left), no other kernel changed; 133: wave-specialized tile kernel (launch kind 2) for large batches; 132: split-K reduction runs on the XCD that wrote the partial sums, every grid size gets XCD-contiguous tiles; 131: tile kernel stores through LDS; 130: small-batch kernel loads activations as whole rows and turns them into operand order through LDS
 
 int fp6mi_prepack_ref(int E, int Mb, void *packed, const void *raw, size_t M, size_t K) { return fp6mi::prepack_ref(E, Mb, packed, raw, M, K); }
 int fp6mi_unpack_ref(int E, int Mb, void *raw, const void *packed, size_t M, size_t K) { return fp6mi::unpack_ref(E, Mb, raw, packed, M, K); }
@@ -608,7 +617,7 @@ int fp6mi_linear_native(int E, int Mb, void *stream, const void *W, const void *
     int rc = check_gemm_args(E, Mb, W, sc, B, C, M, N, K, ws, splitK);
     if (rc != FP6MI_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, nullptr, B, C, M, N, K, ws, splitK, nullptr);
+    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, nullptr, nullptr, B, C, M, N, K, ws, splitK, nullptr);
 }
 
 int fp6mi_linear_native_grouped(int E, int Mb, void *stream, const void *W, const void *sc, const void *group_exps, const void *B, void *C, size_t M,
@@ -619,7 +628,18 @@ int fp6mi_linear_native_grouped(int E, int Mb, void *stream, const void *W, cons
     if (!group_exps) return FP6MI_ERR_NULL;
     if (reinterpret_cast<uintptr_t>(group_exps) & 1u) return FP6MI_ERR_ALIGN;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, group_exps, B, C, M, N, K, ws, splitK, nullptr);
+    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, group_exps, nullptr, B, C, M, N, K, ws, splitK, nullptr);
+}
+
+int fp6mi_linear_native_bias(int E, int Mb, void *stream, const void *W, const void *sc, const void *group_exps, const void *bias, const void *B, void *C, size_t M,
+                             size_t N, size_t K, float *ws, int splitK)
+{
+    int rc = check_gemm_args(E, Mb, W, sc, B, C, M, N, K, ws, splitK);
+    if (rc != FP6MI_OK) return rc;
+    if (!bias) return FP6MI_ERR_NULL;
+    if ((reinterpret_cast<uintptr_t>(group_exps) & 1u) || (reinterpret_cast<uintptr_t>(bias) & 1u)) return FP6MI_ERR_ALIGN;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, group_exps, bias, B, C, M, N, K, ws, splitK, nullptr);
 }
 
 int fp6mi_linear_native_cfg(int E, int Mb, void *stream, const void *W, const void *sc, const void *B, void *C, size_t M, size_t N, size_t K,
@@ -629,7 +649,7 @@ int fp6mi_linear_native_cfg(int E, int Mb, void *stream, const void *W, const vo
     if (rc != FP6MI_OK) return rc;
     LaunchCfg   c = { kind, n_tiles, row_tiles, row_waves, k_waves };
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, nullptr, B, C, M, N, K, ws, splitK, &c);
+    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, nullptr, nullptr, B, C, M, N, K, ws, splitK, &c);
 }
 
 int fp6mi_linear_native_grouped_cfg(int E, int Mb, void *stream, const void *W, const void *sc, const void *group_exps, const void *B, void *C, size_t M,
@@ -641,7 +661,7 @@ int fp6mi_linear_native_grouped_cfg(int E, int Mb, void *stream, const void *W, 
     if (reinterpret_cast<uintptr_t>(group_exps) & 1u) return FP6MI_ERR_ALIGN;
     LaunchCfg   c = { kind, n_tiles, row_tiles, row_waves, k_waves };
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, group_exps, B, C, M, N, K, ws, splitK, &c);
+    return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, group_exps, nullptr, B, C, M, N, K, ws, splitK, &c);
 }
 
 int fp6mi_launch_source(int E, int Mb, size_t M, size_t N, size_t K, int splitK)
@@ -721,7 +741,7 @@ int fp6mi_linear_native_static(int E, int Mb, void *stream, const void *W, const
     }
     int rc = check_gemm_args(E, Mb, W, sc, B, C, M, N, K, ws, splitK);
     if (rc != FP6MI_OK) return rc;
-    return linear_native(*fp6mi::ops_for(E, Mb), static_cast<hipStream_t>(stream), W, sc, nullptr, B, C, M, N, K, ws, splitK, nullptr);
+    return linear_native(*fp6mi::ops_for(E, Mb), static_cast<hipStream_t>(stream), W, sc, nullptr, nullptr, B, C, M, N, K, ws, splitK, nullptr);
 }
 
 // ---- drop-in entry on REFERENCE-layout weights: native twins are made on first sight of a weight pointer and kept ----

@@ -161,6 +161,12 @@ template <int FM, bool GS> __device__ __forceinline__ void convert(const WFrag<F
     }
 }
 
+// `ws` of the GEMM kernels: the partial sums where K is split (splitk_reduce adds a bias then), else an fp16 bias [M] on any 2-byte boundary or null, which
+// the epilogue adds to the float32 sums.  gemm_stream has instances of its own for it: a branch in the epilogue that no launch took cost it 0.04-0.1 us (1 % of
+// 4096x4096 N 8).  Instead of an addition behind the GEMM, us, e3m2, replayed: 4096x4096 N 1 6.1 -> 4.4, N 8 7.6 -> 5.0; 8192x8192 N 16 15.7 -> 12.9,
+// N 72 25.9 -> 22.1; 28672x8192 N 2048 680 -> 657.
+template <typename P> __device__ __forceinline__ const half_t *bias_of(P ws) { return reinterpret_cast<const half_t *>(ws); }
+
 // ---------------------------------------------------------------------------------------------------------------
 // gemm_stream: weight-bandwidth-bound GEMM for small batches.
 //   grid  = (M/(16*RT) row groups, splitK, ceil(N / (16*NT)))      block = WAVES wavefronts
@@ -192,7 +198,7 @@ __host__ __device__ constexpr uint32_t stream_wave_bytes(int rows, int RT, int N
     return (uint32_t)(rows * kXsRowBytes > RT * NT * 1024 ? rows * kXsRowBytes : RT * NT * 1024);
 }
 
-template <int FM, bool GS, int NT, int RT, int WAVES, bool SPLIT>
+template <int FM, bool GS, int NT, int RT, int WAVES, bool SPLIT, bool BIAS>
 __global__ __launch_bounds__(WAVES *kWave) void gemm_stream(const uint8_t *__restrict__ W, const half_t *__restrict__ scales,
                                                             const uint8_t *__restrict__ gexp, const half_t *__restrict__ X, half_t *__restrict__ C,
                                                             float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
@@ -368,6 +374,14 @@ __global__ __launch_bounds__(WAVES *kWave) void gemm_stream(const uint8_t *__res
     for (int r = 0; r < RT; r++)
 #pragma unroll
         for (int t = 0; t < NT; t++) *reinterpret_cast<v4f *>(mine + (r * NT + t) * 1024 + lane * 16) = acc[r][t];
+    half_t my_bias[BIAS ? kOutPerThread : 1];
+    if constexpr (BIAS) { // (under the wait for the other wavefronts)
+#pragma unroll
+        for (int j = 0; j < kOutPerThread; j++) {
+            const int e = threadIdx.x + j * WAVES * kWave;
+            my_bias[j] = bias_of(ws)[(R0 + real(e < RT * NT * 256 ? (e >> 8) / NT : 0)) * 16 + (e & 15)];
+        }
+    }
     __syncthreads();
 
 #pragma unroll
@@ -383,6 +397,7 @@ __global__ __launch_bounds__(WAVES *kWave) void gemm_stream(const uint8_t *__res
         uint32_t ng = nbase + 16 * t + n, mg = (R0 + r) * 16 + mm;
         if (ng < N && (!kRagged || (uint32_t)r <= rlast)) {
             float v = sum * ((float)my_scale[j] * Fmt<FM>::post_scale);
+            if constexpr (BIAS) v += (float)my_bias[j];
             if constexpr (!SPLIT)
                 C[(size_t)ng * M + mg] = (half_t)v;
             else
@@ -616,18 +631,29 @@ typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 template <int NT, int RT, int WR> constexpr size_t tile_stage_bytes(bool partial) { return (size_t)NT * 16 * (WR * RT * 16 * (partial ? 4 : 2) + 16); }
 
 // first half: a wavefront that holds results scales them and parks them in the stage
-// (column tiles T0 .. T1-1 of it)
+// (column tiles T0 .. T1-1 of it).  bias: of the tile's first row, or null; added before the one rounding to fp16
 template <int FM, int NT, int RT, int WR, typename OutT, int T0 = 0, int T1 = NT>
-__device__ __forceinline__ void tile_park(const v4f (&acc)[RT][NT], const v4h (&sc4)[RT], uint8_t *stage, int wr, int col, int q)
+__device__ __forceinline__ void tile_park(const v4f (&acc)[RT][NT], const v4h (&sc4)[RT], uint8_t *stage, int wr, int col, int q, const half_t *bias = nullptr)
 {
     constexpr int TM = WR * RT * 16, kStride = TM * (int)sizeof(OutT) + 16;
+    v4h           b4[RT] = {};
+    if (sizeof(OutT) == 2 && bias) {
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const half_t *p = bias + (wr * RT + r) * 16 + 4 * q;
+            b4[r] = (v4h){ p[0], p[1], p[2], p[3] };
+        }
+    }
 #pragma unroll
     for (int r = 0; r < RT; r++)
 #pragma unroll
         for (int t = T0; t < T1; t++) {
             v4f v;
 #pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = acc[r][t][i] * ((float)sc4[r][i] * Fmt<FM>::post_scale);
+            for (int i = 0; i < 4; i++) {
+                v[i] = acc[r][t][i] * ((float)sc4[r][i] * Fmt<FM>::post_scale);
+                if constexpr (sizeof(OutT) == 2) v[i] += (float)b4[r][i]; // (one instruction with the scaling)
+            }
             uint8_t *dst = stage + (16 * (t - T0) + col) * kStride + ((wr * RT + r) * 16 + 4 * q) * (int)sizeof(OutT);
             if constexpr (sizeof(OutT) == 2)
                 *reinterpret_cast<v4h *>(dst) = (v4h){ (half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3] };
@@ -654,9 +680,9 @@ __device__ __forceinline__ void tile_flush(OutT *__restrict__ out, const uint8_t
 
 template <int FM, int NT, int RT, int WR, int NTHREADS, typename OutT>
 __device__ __forceinline__ void tile_store(const v4f (&acc)[RT][NT], const v4h (&sc4)[RT], OutT *__restrict__ out, uint8_t *stage, bool holds_results,
-                                           uint32_t M, uint32_t N, uint32_t mb, uint32_t nbase, int tid, int wr, int col, int q)
+                                           uint32_t M, uint32_t N, uint32_t mb, uint32_t nbase, int tid, int wr, int col, int q, const half_t *bias)
 {
-    if (holds_results) tile_park<FM, NT, RT, WR, OutT>(acc, sc4, stage, wr, col, q);
+    if (holds_results) tile_park<FM, NT, RT, WR, OutT>(acc, sc4, stage, wr, col, q, bias);
     __syncthreads();
     tile_flush<NT, RT, WR, NTHREADS, OutT>(out, stage, M, N, mb, nbase, tid);
 }
@@ -740,9 +766,9 @@ __global__ __launch_bounds__(WR *WK *kWave) void gemm_tile(const uint8_t *__rest
     if (WK > 1) __syncthreads();
     uint8_t *stage = lds;
     if (splitK == 1)
-        tile_store<FM, NT, RT, WR, NTHREADS>(acc, sc4, C, stage, wk == 0, M, N, mb, nbase, tid, wr, col, q);
+        tile_store<FM, NT, RT, WR, NTHREADS>(acc, sc4, C, stage, wk == 0, M, N, mb, nbase, tid, wr, col, q, ws ? bias_of(ws) + mb * (WR * RT * 16) : nullptr);
     else
-        tile_store<FM, NT, RT, WR, NTHREADS>(acc, sc4, ws + (size_t)split * N * M, stage, wk == 0, M, N, mb, nbase, tid, wr, col, q);
+        tile_store<FM, NT, RT, WR, NTHREADS>(acc, sc4, ws + (size_t)split * N * M, stage, wk == 0, M, N, mb, nbase, tid, wr, col, q, nullptr);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -965,7 +991,7 @@ __global__ __launch_bounds__((WR + PW) * kWave) void gemm_ws(const uint8_t *__re
     // every wavefront has passed the last barrier of the K loop: the rings are free, the output tile is parked there
     uint8_t *stage = lds;
     if (splitK == 1) {
-        if (wave < WR) tile_park<FM, NT, RT, WR, half_t>(acc, sc4, stage, wave, col, q);
+        if (wave < WR) tile_park<FM, NT, RT, WR, half_t>(acc, sc4, stage, wave, col, q, ws ? bias_of(ws) + mb * (WR * RT * 16) : nullptr);
         __syncthreads();
         tile_flush<NT, RT, WR, NTHREADS, half_t>(C, stage, M, N, mb, nbase, tid);
     } else {
@@ -1170,7 +1196,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, c
         sc4[r] = (v4h){ p[0], p[1], p[2], p[3] };
     }
     if (splitK == 1) {
-        tile_park<FM, NT, RT, 2, half_t>(acc, sc4, lds + (size_t)wc * NT * 16 * (2 * RT * 16 * 2 + 16), wr, col, q);
+        tile_park<FM, NT, RT, 2, half_t>(acc, sc4, lds + (size_t)wc * NT * 16 * (2 * RT * 16 * 2 + 16), wr, col, q, ws ? bias_of(ws) + mb * (2 * RT * 16) : nullptr);
         __syncthreads();
         tile_flush<2 * NT, RT, 2, 4 * kWave, half_t>(C, lds, M, N, mb, nbase, tid);
     } else {
@@ -1385,7 +1411,7 @@ __global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(
     }
     if (splitK == 1) {
         constexpr int kCols = WK == 2 ? NH : NT; // column tiles that a wavefront holds results of
-        tile_park<FM, NT, RT, 4, half_t, 0, kCols>(acc, sc4, lds + (size_t)wk * NH * 16 * (TM * 2 + 16), wr, col, q);
+        tile_park<FM, NT, RT, 4, half_t, 0, kCols>(acc, sc4, lds + (size_t)wk * NH * 16 * (TM * 2 + 16), wr, col, q, ws ? bias_of(ws) + mb * TM : nullptr);
         __syncthreads();
         tile_flush<NT, RT, 4, NTHREADS, half_t>(C, lds, M, N, mb, nbase, tid);
     } else {
@@ -1962,8 +1988,10 @@ int launch_stream(hipStream_t st, const void *W, const void *sc, const void *gex
                            (uint32_t)K, units, (uint32_t)splitK);
         return (int)hipGetLastError();
     };
-    if (splitK > 1) return go(std::integral_constant<decltype(&gemm_stream<FM, GS, NT, RT, WAVES, true>), &gemm_stream<FM, GS, NT, RT, WAVES, true>>{});
-    return go(std::integral_constant<decltype(&gemm_stream<FM, GS, NT, RT, WAVES, false>), &gemm_stream<FM, GS, NT, RT, WAVES, false>>{});
+    typedef decltype(&gemm_stream<FM, GS, NT, RT, WAVES, false, false>) Kernel;
+    if (splitK > 1) return go(std::integral_constant<Kernel, &gemm_stream<FM, GS, NT, RT, WAVES, true, false>>{});
+    if (ws) return go(std::integral_constant<Kernel, &gemm_stream<FM, GS, NT, RT, WAVES, false, true>>{});
+    return go(std::integral_constant<Kernel, &gemm_stream<FM, GS, NT, RT, WAVES, false, false>>{});
 }
 
 template <int FM, bool GS, int NT, int RT, int WR, int WK>
@@ -2100,7 +2128,7 @@ int launch_cfg(const LaunchCfg &c, hipStream_t st, const void *W, const void *sc
 
 // ------------------------------------------------------------------------------------------------ entry functions of this format
 // (arguments are checked by the C ABI before it comes here)
-// gexp: group exponents in their native layout, or null for none
+// gexp: group exponents in their native layout, or null for none; ws: see bias_of
 template <int FM>
 int op_gemm(const LaunchCfg &c, void *stream, const void *W, const void *sc, const void *gexp, const void *B, void *C, float *ws, size_t M,
             size_t N, size_t K, int splitK)

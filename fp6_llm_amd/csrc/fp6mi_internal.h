@@ -18,7 +18,7 @@ inline bool supported(int E, int Mbits) { return (E == 3 && Mbits == 2) || (E ==
 struct LaunchCfg { int kind, nt, rt, wr, wk; };
 struct FormatOps {
     int bits;
-    // gexp: group exponents in their native layout (one byte per row and 128 columns), or null
+    // gexp: group exponents in their native layout (one byte per row and 128 columns), or null; ws: the partial sums with a split, else an fp16 bias [M] or null
     int (*gemm)(const LaunchCfg &c, void *stream, const void *W, const void *sc, const void *gexp, const void *B, void *C, float *ws, size_t M,
                 size_t N, size_t K, int splitK);
     int (*relayout)(void *stream, void *native, const void *packed_ref, size_t M, size_t K);

@@ -42,10 +42,10 @@ at::Tensor workspace_for(const at::Device &dev, void *stream, int64_t floats)
     return it->second;
 }
 
-// out[B, OC] = in_feats[B, IC] @ dequant(W)^T with W in the native layout, enqueued on the current stream of in_feats' device.
+// out[B, OC] = in_feats[B, IC] @ dequant(W)^T (+ bias) with W in the native layout, enqueued on the current stream of in_feats' device.
 at::Tensor linear_forward_native(int64_t E, int64_t Mb, const at::Tensor &in_feats, const at::Tensor &native_weight, const at::Tensor &scales,
                                  int64_t OC, int64_t splitK, const c10::optional<at::Tensor> &out_opt, const c10::optional<at::Tensor> &ws_opt,
-                                 const c10::optional<at::Tensor> &gexp_opt)
+                                 const c10::optional<at::Tensor> &gexp_opt, const c10::optional<at::Tensor> &bias_opt)
 {
     const bool known = (E == 3 && Mb == 2) || (E == 2 && Mb >= 1 && Mb <= 3);
     if (!known) bad("unsupported format: EXPONENT=" + std::to_string(E) + ", MANTISSA=" + std::to_string(Mb) + " (only e3m2, e2m2, e2m3 and e2m1)");
@@ -68,6 +68,8 @@ at::Tensor linear_forward_native(int64_t E, int64_t Mb, const at::Tensor &in_fea
         if (out.dim() != 2 || out.size(0) != B || out.size(1) != OC || out.scalar_type() != at::kHalf || !out.is_contiguous() || out.device() != dev)
             bad("out must be a contiguous float16 [B, OC] tensor on the same GPU");
     }
+    if (bias_opt.has_value() && (bias_opt->scalar_type() != at::kHalf || bias_opt->dim() != 1 || bias_opt->size(0) != OC || !bias_opt->is_contiguous() || bias_opt->device() != dev))
+        bad("bias must be a contiguous float16 [OC] tensor on the same GPU");
     c10::hip::HIPGuard guard(dev.index());
     if (!out_opt.has_value()) out = at::empty({ B, OC }, at::TensorOptions().dtype(at::kHalf).device(dev));
     void  *stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
@@ -84,17 +86,23 @@ at::Tensor linear_forward_native(int64_t E, int64_t Mb, const at::Tensor &in_fea
         }
         ws_ptr = ws.data_ptr<float>();
     }
-    int rc;
+    const void *gexp = nullptr;
     if (gexp_opt.has_value()) { // per-group exponents in the kernels' own order (fp6mi_pack_group_exps)
         const at::Tensor &g = *gexp_opt;
         if (g.scalar_type() != at::kByte || g.device() != dev || !g.is_contiguous() || g.numel() != (int64_t)fp6mi_group_exps_bytes((size_t)OC, (size_t)IC))
             bad("group_exps must be the contiguous uint8 tensor of pack_group_exps(exps, OC, IC) on the weights' GPU");
-        rc = fp6mi_linear_native_grouped((int)E, (int)Mb, stream, native_weight.data_ptr(), sc.data_ptr(), g.data_ptr(), x.data_ptr(), out.data_ptr(),
+        gexp = g.data_ptr();
+    }
+    int rc;
+    if (bias_opt.has_value())
+        rc = fp6mi_linear_native_bias((int)E, (int)Mb, stream, native_weight.data_ptr(), sc.data_ptr(), gexp, bias_opt->data_ptr(), x.data_ptr(), out.data_ptr(),
+                                      (size_t)OC, (size_t)B, (size_t)IC, ws_ptr, (int)splitK);
+    else if (gexp)
+        rc = fp6mi_linear_native_grouped((int)E, (int)Mb, stream, native_weight.data_ptr(), sc.data_ptr(), gexp, x.data_ptr(), out.data_ptr(),
                                          (size_t)OC, (size_t)B, (size_t)IC, ws_ptr, (int)splitK);
-    } else {
+    else
         rc = fp6mi_linear_native((int)E, (int)Mb, stream, native_weight.data_ptr(), sc.data_ptr(), x.data_ptr(), out.data_ptr(), (size_t)OC, (size_t)B,
                                  (size_t)IC, ws_ptr, (int)splitK);
-    }
     if (rc != 0) throw std::runtime_error(std::string("fp6mi_linear_native: ") + fp6mi_error_string(rc));
     return out;
 }
@@ -210,7 +218,7 @@ torch::Tensor fp_eXmY_linear_forward_cuda(int EXPONENT, int MANTISSA, torch::Ten
     if (_in_feats.dim() != 2 || _in_feats.size(1) != IC) bad("in_feats must be [B, IC] with the weights' IC");
     if (OC % 256 != 0 || IC % 64 != 0) bad("need OC % 256 == 0, IC % 64 == 0");
     at::Tensor native = native_twin_of(_weights, EXPONENT, MANTISSA, OC, IC);
-    return linear_forward_native(EXPONENT, MANTISSA, _in_feats, native, _scales, OC, splitK, c10::nullopt, c10::nullopt, c10::nullopt);
+    return linear_forward_native(EXPONENT, MANTISSA, _in_feats, native, _scales, OC, splitK, c10::nullopt, c10::nullopt, c10::nullopt, c10::nullopt);
 }
 // fp6_llm/csrc/fp6_linear.cu:161-201
 torch::Tensor fp6_linear_forward_cuda(torch::Tensor _in_feats, torch::Tensor _weights, torch::Tensor _scales, int splitK)
@@ -245,7 +253,7 @@ pybind11::object linear_forward_any_order(int64_t E, int64_t Mb, pybind11::handl
     if (!w.is_contiguous()) bad("weights must be contiguous");
     const pybind11::object native = twin_of(args[weights], E, Mb);
     return pybind11::cast(linear_forward_native(E, Mb, x, pybind11::cast<at::Tensor>(native), THPVariable_Unpack(args[scales].ptr()), OC, splitK, c10::nullopt, c10::nullopt,
-                                                c10::nullopt));
+                                                c10::nullopt, c10::nullopt));
 }
 
 void clear_twins()
@@ -260,7 +268,7 @@ PYBIND11_MODULE(_fp6mi_torch, m)
     m.doc() = "torch tensors -> fp6mi C ABI";
     m.def("linear_forward_native", &linear_forward_native, pybind11::arg("EXPONENT"), pybind11::arg("MANTISSA"), pybind11::arg("in_feats"),
           pybind11::arg("native_weight"), pybind11::arg("scales"), pybind11::arg("OC"), pybind11::arg("splitK") = 1, pybind11::arg("out") = pybind11::none(),
-          pybind11::arg("workspace") = pybind11::none(), pybind11::arg("group_exps") = pybind11::none());
+          pybind11::arg("workspace") = pybind11::none(), pybind11::arg("group_exps") = pybind11::none(), pybind11::arg("bias") = pybind11::none());
     m.def("linear_forward_any_order", &linear_forward_any_order);
     m.def("clear_workspaces", &clear_workspaces);
     m.def("clear_twins", &clear_twins);

@@ -118,6 +118,14 @@ class FPxLinear(torch.nn.Module):
             m.group_exps = torch.cat([l.group_exps for l in layers])
         return m
 
+    def _bias_in_kernel(self, x2):
+        """Whether the kernels add the bias (to their float32 sums; otherwise a torch addition follows): a plain fp16 vector on the GPU that nothing
+        differentiates or maps over."""
+        b = self.bias
+        return (type(b) in (torch.Tensor, torch.nn.Parameter) and b.dtype == torch.float16 and b.shape == (self.out_features,) and b.is_contiguous()
+                and b.device == x2.device and not (b.requires_grad and torch.is_grad_enabled())
+                and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0)
+
     def forward(self, x):
         lead = x.shape[:-1]
         x2 = x.reshape(-1, self.in_features)
@@ -136,8 +144,10 @@ class FPxLinear(torch.nn.Module):
             sk = self._split_cache.get(x2.shape[0])
             if sk is None:
                 sk = self._split_cache[x2.shape[0]] = heuristic_splitk_mi355x(self.out_features, x2.shape[0], self.in_features, MI355X_CUS, self.exponent, self.mantissa)
-        y = linear_forward_native(self.exponent, self.mantissa, x2, self.weight_native, self.scales, self.out_features, sk, None, None, self.group_exps)
-        if self.bias is not None:
+        fused = self.bias is not None and self._bias_in_kernel(x2)
+        y = linear_forward_native(self.exponent, self.mantissa, x2, self.weight_native, self.scales, self.out_features, sk, None, None, self.group_exps,
+                                  self.bias if fused else None)
+        if self.bias is not None and not fused:
             y = y + self.bias
         return y.reshape(*lead, self.out_features)
 

@@ -201,6 +201,10 @@ int fp6mi_dequant_grouped(int E, int Mbits, void *out_f16, const void *raw, size
 int fp6mi_linear_native_grouped(int E, int Mbits, void *stream, const void *W_native, const void *scales_f16,
                                 const void *group_exps_native, const void *B_f16, void *C_f16, size_t M, size_t N, size_t K,
                                 float *workspace, int splitK);
+/* C = fp16_rn(B @ dequant(W)^T + bias): either of the above with fp16 bias[M] (device pointer, 2-byte aligned) added to the FP32 sums
+ * before the one rounding.  group_exps_native may be NULL. */
+int fp6mi_linear_native_bias(int E, int Mbits, void *stream, const void *W_native, const void *scales_f16, const void *group_exps_native,
+                             const void *bias_f16, const void *B_f16, void *C_f16, size_t M, size_t N, size_t K, float *workspace, int splitK);
 int fp6mi_dequant_native_grouped_gpu(int E, int Mbits, void *stream, void *out_f16_dev, const void *W_native_dev,
                                      const void *scales_f16_dev, const void *group_exps_native_dev, size_t M, size_t K);
 /* fp6mi_quantize_native_gpu that also chooses the group exponents: per group the smallest 2^(b-127), 112 <= b <= 127, that

@@ -1054,6 +1054,34 @@ def test_device_quantizer_rejects_bad_arguments():
         fp6.weight_quantize_native_cuda(3, 2, torch.zeros(256, 128, dtype=torch.float16))
 
 
+@pytest.mark.parametrize("E,M,OC,IC,BS,splitK", [
+    (3, 2, 256, 256, 1, 1), (2, 3, 256, 320, 7, 1), (2, 2, 1536, 576, 16, 1), (2, 1, 1792, 1728, 3, 2), (3, 2, 5120, 512, 12, 1), (3, 2, 4096, 1024, 24, 1),   # gemm_stream
+    (2, 2, 256, 256, 19, 1), (3, 2, 256, 640, 17, 2), (3, 2, 11008, 1600, 36, 1), (2, 2, 1792, 4224, 66, 8),                                                    # gemm_tile, gemm_ws
+    (2, 2, 512, 256, 2113, 1), (3, 2, 768, 5696, 212, 8), (2, 3, 1024, 320, 200, 4), (2, 2, 23296, 2304, 493, 1)])                                              # gemm_wide, gemm_prefill
+@pytest.mark.parametrize("groups", [False, True])
+def test_bias_in_the_epilogues(E, M, OC, IC, BS, splitK, groups):
+    """Every kernel's epilogue and both reductions add a bias (on a 2-byte boundary) to the float32 sums: the result is within half an fp16 step of the
+    sum in float64 plus what IC float32 additions may lose, and a bias of zeros changes no bit."""
+    print("case bias", E, M, OC, IC, BS, splitK, groups, flush=True)
+    gen = torch.Generator().manual_seed(OC + IC + BS)
+    native, sc, *rest = fp6.weight_quantize_native_cuda(E, M, (torch.randn(OC, IC, generator=gen) * 0.02).half().to(DEV), groups)
+    exps = rest[0] if rest else None
+    x = torch.randn(BS, IC, generator=gen).half().to(DEV)
+    bias = torch.randn(OC + 1, generator=gen).half().to(DEV)[1:]
+    run = lambda b: fp6.linear_forward_native(E, M, x, native, sc, OC, splitK, group_exps=exps, bias=b)   # noqa: E731
+    plain, zeros, y = run(None), run(torch.zeros_like(bias)), run(bias).double()
+    assert torch.equal(plain, zeros)
+    w = fp6.weight_dequant_native_cuda(E, M, native, sc, OC, IC, exps).double()   # (rounded to fp16: the kernels scale the sums instead)
+    want = x.double() @ w.t() + bias.double()
+    allowed = want.abs() * 2.0 ** -11 + (x.double().abs() @ w.abs().t()) * (2.0 ** -11 + IC * 2.0 ** -24) + 2.0 ** -24
+    assert ((y - want).abs() <= allowed).all()
+    assert (y - plain.double() - bias.double()).abs().max() <= 2.0 ** -10 * max(float(y.abs().max()), float(plain.abs().max()))
+    with pytest.raises(ValueError):
+        run(bias[:-1])
+    with pytest.raises(ValueError):
+        run(bias.float())
+
+
 def test_module_prefill_route_dequantizes_and_matches():
     from fp6_llm_amd import module
     w = torch.from_numpy(synth.normal(53, (256, 512))).half()

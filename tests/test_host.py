@@ -712,3 +712,25 @@ def test_cpp_torch_entry_points_carry_the_reference_names():
         ext.weight_prepacking_eXmY_cpu(4, 3, torch.zeros((256, 16), dtype=torch.int32))  # a format nobody has
     with pytest.raises(ValueError):
         ext.weight_dequant_cpu(torch.zeros((256, 12), dtype=torch.int32), torch.zeros(255, dtype=torch.float16))
+
+
+def test_which_biases_the_kernels_add():
+    """A plain fp16 vector beside the input; whatever autograd, a transform or another type has a part in stays a torch addition."""
+    from torch.autograd import forward_ad
+    from fp6_llm_amd.module import FPxLinear
+    layer, x = FPxLinear(64, 256), torch.zeros(1, 64, dtype=torch.float16)
+    assert not layer._bias_in_kernel(x)   # none
+    half = torch.ones(256, dtype=torch.float16)
+    for bias, want in ((half, True), (half.float(), False), (half[:1], False), (torch.ones(512, dtype=torch.float16)[::2], False), (half[None], False)):
+        layer.bias = bias
+        assert layer._bias_in_kernel(x) is want
+    layer.bias = half.clone().requires_grad_()
+    assert not layer._bias_in_kernel(x)
+    with torch.no_grad():
+        assert layer._bias_in_kernel(x)
+    layer.bias = half
+    with forward_ad.dual_level():
+        assert not layer._bias_in_kernel(x)
+    seen = []
+    torch.func.vmap(lambda z: (z, seen.append(layer._bias_in_kernel(x)))[0])(torch.zeros(2))
+    assert seen == [False]
