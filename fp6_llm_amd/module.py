@@ -13,25 +13,29 @@ from . import (MI355X_CUS, group_exps_bytes, heuristic_splitk_mi355x, linear_for
 _MAGIC = b"FP6MI\x00\x01\x00"   # name, NUL, layout version 1, reserved
 
 
+class _AutoRows(int):
+    """FPxLinear.dequant_above as "auto" leaves it: a number set by the user is a plain int and is taken as it stands."""
+
+
 class FPxLinear(torch.nn.Module):
     """y = x @ dequant(W)^T (+ bias) with W held in the native gfx950 layout.  Weights are buffers, not parameters:
     the layer is inference-only, like the kernels."""
 
-    # Batch size from which dequantize + FP16 library GEMM beats the mixed-input kernel on the MI355X, whatever the matrix: measured
-    # through this module at 4096^2, 8192^2, 28672x8192 and 8192x28672, with FP6 and row scales and with FP5 and group exponents, with a bias and without,
-    # kernel time / route time is 0.63-1.00 at 1024 rows, 0.87-1.11 at 2048, 0.94-1.09 at 3072 and 1.10-1.29 at 4096 and 8192 (8192^2 at 4096 rows: 464 us
-    # against 395).
+    # dequant_above="auto": below PREFILL_CROSSOVER rows the mixed-input kernels always run.  From there on the choice is by measurement, and since the wide
+    # tiles it falls on them up to LIBRARY_ROWS.  Measured through this module at 4096^2, 8192^2, 28672x8192, 8192x28672, 11008x4096, 1024x8192, 1024^2, 4608x4544
+    # and 2560x18944, FP6 with row scales and FP5 with group exponents, kernel time / time of dequantization + FP16 library GEMM: 0.33-0.99 at 3072 rows,
+    # 0.35-1.06 at 4096, 0.40-0.99 at 4100, 0.44-1.07 at 6144, 0.51-1.06 at 8192, 0.73-1.03 at 16384, 0.85-1.10 at 32768 (8192^2 at 4096 rows 369 us against
+    # 394, at 16384 1465 against 1464); with a bias, which the kernels add by themselves, 0.29-1.03 at 4096 and 0.58-0.96 at 16384.
     PREFILL_CROSSOVER = 3072
+    LIBRARY_ROWS = 32768
 
     def __init__(self, in_features, out_features, exponent=3, mantissa=2, bias=None, split_k=None, dequant_above="auto", group_scales=False):
         """group_scales: the layer also holds one exponent byte per row and 128 columns (factor 1 until weights are loaded).
         dequant_above: batch size from which forward() dequantizes the weights to a temporary fp16 matrix on the GPU and calls
-        the FP16 library GEMM instead (prefill).  The mixed-input kernel wins while the GEMM is bound by weight bytes; from a
-        few thousand rows the FP16 library runs 1.3-1.5 PFLOP/s against its 1.1-1.25, which pays for the dequantization pass
-        (about 30 us at 8192 x 8192).  "auto" (default) = PREFILL_CROSSOVER rows; None never does (the temporary costs 2 bytes
-        per weight for the duration of the call); an integer sets the threshold."""
+        the FP16 library GEMM instead (the temporary costs 2 bytes per weight for the duration of the call).  "auto" (default) leaves
+        it to the measurements above, from PREFILL_CROSSOVER rows on; None never does; an integer sets the threshold."""
         super().__init__()
-        self.dequant_above = self.PREFILL_CROSSOVER if dequant_above == "auto" else dequant_above
+        self.dequant_above = _AutoRows(self.PREFILL_CROSSOVER) if dequant_above == "auto" else dequant_above
         if out_features % 256 or in_features % 64:
             raise ValueError("FPxLinear needs out_features %% 256 == 0 and in_features %% 64 == 0")
         self.in_features, self.out_features = in_features, out_features
@@ -131,7 +135,10 @@ class FPxLinear(torch.nn.Module):
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype != torch.float16:
             x2 = x2.half()
-        if self.dequant_above is not None and x2.shape[0] >= self.dequant_above:
+        rows = self.dequant_above
+        if type(rows) is _AutoRows:
+            rows = max(rows, self.LIBRARY_ROWS)
+        if rows is not None and x2.shape[0] >= rows:
             w16 = weight_dequant_native_cuda(self.exponent, self.mantissa, self.weight_native, self.scales, self.out_features, self.in_features,
                                              self.group_exps)
             y = torch.nn.functional.linear(x2, w16)

@@ -734,3 +734,18 @@ def test_which_biases_the_kernels_add():
     seen = []
     torch.func.vmap(lambda z: (z, seen.append(layer._bias_in_kernel(x)))[0])(torch.zeros(2))
     assert seen == [False]
+
+
+@pytest.mark.parametrize("above,rows,library", [("auto", 3072, False), ("auto", 32767, False), ("auto", 32768, True), (3072, 3072, True), (3072, 3071, False), (None, 32768, False)])
+def test_which_route_a_long_prompt_takes(monkeypatch, above, rows, library):
+    """dequant_above: "auto" keeps the mixed-input kernels up to 32768 rows, a number of the user's own is taken as it stands, also when it is set later."""
+    import copy
+    from fp6_llm_amd import module
+    monkeypatch.setattr(module, "weight_dequant_native_cuda", lambda *a: torch.full((256, 64), 2.0, dtype=torch.float16))
+    monkeypatch.setattr(module, "linear_forward_native", lambda E, M, x, *a: torch.full((x.shape[0], 256), -1.0, dtype=torch.float16))
+    layer = module.FPxLinear(64, 256, dequant_above=above)
+    later = module.FPxLinear(64, 256)
+    later.dequant_above = 3072 if above == 3072 else layer.dequant_above
+    x = torch.ones(rows, 64, dtype=torch.float16)
+    for l in (layer, later, copy.deepcopy(layer)):
+        assert float(l(x)[0, 0]) == (128.0 if library else -1.0)
