@@ -13,6 +13,14 @@ from . import (MI355X_CUS, group_exps_bytes, heuristic_splitk_mi355x, linear_for
 _MAGIC = b"FP6MI\x00\x01\x00"   # name, NUL, layout version 1, reserved
 
 
+def _values_only(t):
+    """Whether nothing but t's values counts in what is done with it: no derivative, transform, trace, subclass or dispatch mode has a part in it, which a kernel
+    that is handed t's address would pass by."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and not (t.requires_grad and torch.is_grad_enabled())
+            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0 and not torch.jit.is_tracing() and not t.is_neg())
+
+
 class _AutoRows(int):
     """FPxLinear.dequant_above as "auto" leaves it: a number set by the user is a plain int and is taken as it stands."""
 
@@ -126,9 +134,14 @@ class FPxLinear(torch.nn.Module):
         """Whether the kernels add the bias (to their float32 sums; otherwise a torch addition follows): a plain fp16 vector on the GPU that nothing
         differentiates or maps over."""
         b = self.bias
-        return (type(b) in (torch.Tensor, torch.nn.Parameter) and b.dtype == torch.float16 and b.shape == (self.out_features,) and b.is_contiguous()
-                and b.device == x2.device and not (b.requires_grad and torch.is_grad_enabled())
-                and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0)
+        return (b is not None and _values_only(b) and b.dtype == torch.float16 and b.shape == (self.out_features,) and b.is_contiguous() and b.device == x2.device)
+
+    def _kernels_take(self, x2):
+        """Whether a long prompt can leave torch.nn.functional.linear for the mixed-input kernels and nothing is lost: they are no part of an autograd graph, a
+        trace or a transform, give fp16 whatever autocast would, and read contiguous rows at a 16-byte boundary."""
+        kind = x2.device.type
+        return (_values_only(x2) and (not torch.is_autocast_enabled(kind) or torch.get_autocast_dtype(kind) == torch.float16)
+                and (not x2.is_contiguous() or x2.data_ptr() % 16 == 0))
 
     def forward(self, x):
         lead = x.shape[:-1]
@@ -136,7 +149,7 @@ class FPxLinear(torch.nn.Module):
         if x2.dtype != torch.float16:
             x2 = x2.half()
         rows = self.dequant_above
-        if type(rows) is _AutoRows:
+        if type(rows) is _AutoRows and x2.shape[0] >= rows and self._kernels_take(x2):
             rows = max(rows, self.LIBRARY_ROWS)
         if rows is not None and x2.shape[0] >= rows:
             w16 = weight_dequant_native_cuda(self.exponent, self.mantissa, self.weight_native, self.scales, self.out_features, self.in_features,

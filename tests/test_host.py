@@ -749,3 +749,62 @@ def test_which_route_a_long_prompt_takes(monkeypatch, above, rows, library):
     x = torch.ones(rows, 64, dtype=torch.float16)
     for l in (layer, later, copy.deepcopy(layer)):
         assert float(l(x)[0, 0]) == (128.0 if library else -1.0)
+
+
+def _long_prompt_stubs(monkeypatch):
+    """FPxLinear's two routes without a GPU: the kernels answer -1 and are no part of any graph, dequantized weights are all 2."""
+    from fp6_llm_amd import module
+    monkeypatch.setattr(module, "weight_dequant_native_cuda", lambda *a: torch.full((256, 64), 2.0, dtype=torch.float16))
+    monkeypatch.setattr(module, "linear_forward_native", lambda E, M, x, *a: torch.full((x.shape[0], 256), -1.0, dtype=torch.float16))
+    return module
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_long_prompts_that_something_follows_keep_the_library_route(monkeypatch, bias):
+    """From 3072 rows on an input that is differentiated (backward, forward mode, torch.func), mapped over, traced, seen by a dispatch mode or a subclass, cast by
+    autocast or off a 16-byte boundary goes through torch.nn.functional.linear, as it always did."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+    module = _long_prompt_stubs(monkeypatch)
+    layer = module.FPxLinear(64, 256, bias=torch.ones(256, dtype=torch.float16) if bias else None)
+    want, kernels = 128.0 + bias, -1.0 + bias
+    monkeypatch.setattr(module.FPxLinear, "_bias_in_kernel", lambda self, x2: False)
+    x = torch.ones(3072, 64, dtype=torch.float16)
+    assert float(layer(x)[0, 0]) == kernels and float(layer(x[:, None, :])[0, 0, 0]) == kernels
+
+    g = x.clone().requires_grad_()
+    (g.sum() + layer(g).sum(dtype=torch.float32)).backward()
+    assert torch.equal(g.grad, torch.full_like(x, 513.0))                     # 1 + 256 * 2
+    f = torch.ones(3072, 64, requires_grad=True)                              # (float32: cast to fp16 on the way in)
+    layer(f).sum(dtype=torch.float32).backward()
+    assert torch.equal(f.grad, torch.full_like(f, 512.0))
+    with torch.no_grad():
+        assert float(layer(g)[0, 0]) == kernels
+    with forward_ad.dual_level():
+        y = forward_ad.unpack_dual(layer(forward_ad.make_dual(x, x)))
+        assert float(y.tangent[0, 0]) == 128.0 and float(y.primal[0, 0]) == want
+    assert float(torch.func.vmap(layer)(x[None])[0, 0, 0]) == want
+    assert float(torch.func.grad(lambda z: layer(z).sum(dtype=torch.float32))(x)[0, 0]) == 512.0
+    traced = torch.jit.trace(layer.forward, (x,), check_trace=False)
+    assert float(traced(2 * x)[0, 0]) == 256.0 + bias
+
+    class Seen(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+    with Seen():
+        assert float(layer(x)[0, 0]) == want
+    assert any("mm" in n for n in Seen.names)
+
+    class Sub(torch.Tensor):
+        pass
+    assert type(layer(x.as_subclass(Sub))) is Sub
+    with torch.autocast("cpu", torch.bfloat16):
+        y = layer(x)
+    assert float(y[0, 0]) == want and (y.dtype == torch.bfloat16 or bias)
+    off = torch.ones(3072 * 64 + 1, dtype=torch.float16)[1:].view(3072, 64)
+    assert off.data_ptr() % 16 and float(layer(off)[0, 0]) == want
+    neg = torch._neg_view(x)
+    assert float(layer(neg)[0, 0]) == -128.0 + bias
