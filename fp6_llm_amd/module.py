@@ -13,12 +13,16 @@ from . import (MI355X_CUS, group_exps_bytes, heuristic_splitk_mi355x, linear_for
 _MAGIC = b"FP6MI\x00\x01\x00"   # name, NUL, layout version 1, reserved
 
 
+_peek_transform = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", None)
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
+
+
 def _values_only(t):
     """Whether nothing but t's values counts in what is done with it: no derivative, transform, trace, subclass or dispatch mode has a part in it, which a kernel
-    that is handed t's address would pass by."""
+    that is handed t's address would pass by.  (A torch that lacks one of the names asked here is taken to have one of these active.)"""
     return (type(t) in (torch.Tensor, torch.nn.Parameter) and not (t.requires_grad and torch.is_grad_enabled())
-            and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
-            and torch._C._len_torch_dispatch_stack() == 0 and not torch.jit.is_tracing() and not t.is_neg())
+            and _peek_transform is not None and _peek_transform() is None and getattr(torch.autograd.forward_ad, "_current_level", 0) < 0
+            and _dispatch_modes is not None and _dispatch_modes() == 0 and not torch.jit.is_tracing() and not t.is_neg())
 
 
 class _AutoRows(int):

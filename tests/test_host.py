@@ -808,3 +808,17 @@ def test_long_prompts_that_something_follows_keep_the_library_route(monkeypatch,
     assert off.data_ptr() % 16 and float(layer(off)[0, 0]) == want
     neg = torch._neg_view(x)
     assert float(layer(neg)[0, 0]) == -128.0 + bias
+
+
+def test_a_torch_without_the_private_names_keeps_the_torch_operations(monkeypatch):
+    """Whether a transform or a mode is active is asked by names of torch's own that another version may lack: then nothing is passed by."""
+    module = _long_prompt_stubs(monkeypatch)
+    layer, x = module.FPxLinear(64, 256, bias=torch.ones(256, dtype=torch.float16)), torch.ones(3072, 64, dtype=torch.float16)
+    assert layer._bias_in_kernel(x) and layer._kernels_take(x)
+    for owner, name in ((module, "_peek_transform"), (module, "_dispatch_modes")):
+        with monkeypatch.context() as m:
+            m.setattr(owner, name, None)
+            assert not layer._bias_in_kernel(x) and not layer._kernels_take(x) and float(layer(x)[0, 0]) == 129.0
+    with monkeypatch.context() as m:
+        m.delattr(torch.autograd.forward_ad, "_current_level")
+        assert not layer._bias_in_kernel(x) and not layer._kernels_take(x) and float(layer(x)[0, 0]) == 129.0
