@@ -26,28 +26,33 @@ def _values_only(t):
 
 
 class _AutoRows(int):
-    """FPxLinear.dequant_above as "auto" leaves it: a number set by the user is a plain int and is taken as it stands."""
+    """What dequant_above reads under "auto": the number of rows, and "auto" again for a module that it is assigned to.  (Modules that library version 139
+    pickled whole hold one.)"""
+
+
+_CROSSOVER, _CROSSOVER_LIBRARY = 32768, 3072   # FPxLinear.PREFILL_CROSSOVER as it is shipped, and the one without the wide tiles
 
 
 class FPxLinear(torch.nn.Module):
     """y = x @ dequant(W)^T (+ bias) with W held in the native gfx950 layout.  Weights are buffers, not parameters:
     the layer is inference-only, like the kernels."""
 
-    # dequant_above="auto": below PREFILL_CROSSOVER rows the mixed-input kernels always run.  From there on the choice is by measurement, and since the wide
-    # tiles it falls on them up to LIBRARY_ROWS.  Measured through this module at 4096^2, 8192^2, 28672x8192, 8192x28672, 11008x4096, 1024x8192, 1024^2, 4608x4544
-    # and 2560x18944, FP6 with row scales and FP5 with group exponents, kernel time / time of dequantization + FP16 library GEMM: 0.33-0.99 at 3072 rows,
-    # 0.35-1.06 at 4096, 0.40-0.99 at 4100, 0.44-1.07 at 6144, 0.51-1.06 at 8192, 0.73-1.03 at 16384, 0.85-1.10 at 32768 (8192^2 at 4096 rows 369 us against
-    # 394, at 16384 1465 against 1464); with a bias, which the kernels add by themselves, 0.29-1.03 at 4096 and 0.58-0.96 at 16384.
-    PREFILL_CROSSOVER = 3072
-    LIBRARY_ROWS = 32768
+    # Batch size from which dequantize + FP16 library GEMM is no slower than the mixed-input kernels, measured through this module at 4096^2, 8192^2, 28672x8192,
+    # 8192x28672, 11008x4096, 1024x8192, 1024^2, 4608x4544 and 2560x18944, FP6 with row scales and FP5 with group exponents.  Kernel time / time of dequantization +
+    # library GEMM: 0.33-0.99 at 3072 rows, 0.35-1.06 at 4096, 0.40-0.99 at 4100, 0.44-1.07 at 6144, 0.51-1.06 at 8192, 0.73-1.03 at 16384, 0.85-1.10 at 32768
+    # (8192^2 at 4096 rows 369 us against 394, at 16384 1465 against 1464); with a bias, which the kernels add by themselves, 0.29-1.03 at 4096 and 0.58-0.96 at
+    # 16384.  That is with the wide tiles, so on 256 CUs and with K up to 2^20; without them the two cross at 3072 rows.
+    PREFILL_CROSSOVER = _CROSSOVER
 
     def __init__(self, in_features, out_features, exponent=3, mantissa=2, bias=None, split_k=None, dequant_above="auto", group_scales=False):
         """group_scales: the layer also holds one exponent byte per row and 128 columns (factor 1 until weights are loaded).
         dequant_above: batch size from which forward() dequantizes the weights to a temporary fp16 matrix on the GPU and calls
-        the FP16 library GEMM instead (the temporary costs 2 bytes per weight for the duration of the call).  "auto" (default) leaves
-        it to the measurements above, from PREFILL_CROSSOVER rows on; None never does; an integer sets the threshold."""
+        the FP16 library GEMM instead (the temporary costs 2 bytes per weight for the duration of the call).  None never does; an
+        integer sets the threshold; "auto" (default) is PREFILL_CROSSOVER rows, or 3072 where the wide tiles do not run.  Under "auto" an
+        input of 3072 rows or more that the kernels cannot take as it is (_kernels_take: one that requires a gradient, say) also goes through
+        the library.  A module that a version up to 138 pickled whole holds the number that "auto" was then, 3072."""
         super().__init__()
-        self.dequant_above = _AutoRows(self.PREFILL_CROSSOVER) if dequant_above == "auto" else dequant_above
+        self.dequant_above = dequant_above
         if out_features % 256 or in_features % 64:
             raise ValueError("FPxLinear needs out_features %% 256 == 0 and in_features %% 64 == 0")
         self.in_features, self.out_features = in_features, out_features
@@ -134,6 +139,28 @@ class FPxLinear(torch.nn.Module):
             m.group_exps = torch.cat([l.group_exps for l in layers])
         return m
 
+    def _wide_tiles(self, device):
+        return self.in_features <= 1 << 20 and (device.type != "cuda" or torch.cuda.get_device_properties(device).multi_processor_count == MI355X_CUS)
+
+    @property
+    def dequant_above(self):
+        """Rows from which forward() dequantizes an input that the kernels could take, on the weights' device; None: never."""
+        if not self._auto:
+            return self._rows
+        return _AutoRows(self._rows if self._wide_tiles(self.weight_native.device) else _CROSSOVER_LIBRARY)
+
+    @dequant_above.setter
+    def dequant_above(self, rows):
+        if isinstance(rows, str) and rows == "auto":   # (a subclass or a program with a PREFILL_CROSSOVER of its own means that number, whatever the device)
+            rows = _AutoRows(_CROSSOVER) if self.PREFILL_CROSSOVER == _CROSSOVER else self.PREFILL_CROSSOVER
+        self._auto = type(rows) is _AutoRows
+        self._rows = _CROSSOVER if self._auto else rows
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        if "dequant_above" in self.__dict__:   # pickled whole when it was a plain attribute
+            self.dequant_above = self.__dict__.pop("dequant_above")
+
     def _bias_in_kernel(self, x2):
         """Whether the kernels add the bias (to their float32 sums; otherwise a torch addition follows): a plain fp16 vector on the GPU that nothing
         differentiates or maps over."""
@@ -142,9 +169,9 @@ class FPxLinear(torch.nn.Module):
 
     def _kernels_take(self, x2):
         """Whether a long prompt can leave torch.nn.functional.linear for the mixed-input kernels and nothing is lost: they are no part of an autograd graph, a
-        trace or a transform, give fp16 whatever autocast would, and read contiguous rows at a 16-byte boundary."""
+        trace or a transform, give fp16 whatever autocast would, and read contiguous rows at a 16-byte boundary; and only the wide tiles are faster."""
         kind = x2.device.type
-        return (_values_only(x2) and (not torch.is_autocast_enabled(kind) or torch.get_autocast_dtype(kind) == torch.float16)
+        return (self._wide_tiles(x2.device) and _values_only(x2) and (not torch.is_autocast_enabled(kind) or torch.get_autocast_dtype(kind) == torch.float16)
                 and (not x2.is_contiguous() or x2.data_ptr() % 16 == 0))
 
     def forward(self, x):
@@ -152,10 +179,8 @@ class FPxLinear(torch.nn.Module):
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype != torch.float16:
             x2 = x2.half()
-        rows = self.dequant_above
-        if type(rows) is _AutoRows and x2.shape[0] >= rows and self._kernels_take(x2):
-            rows = max(rows, self.LIBRARY_ROWS)
-        if rows is not None and x2.shape[0] >= rows:
+        rows, n = self._rows, x2.shape[0]
+        if rows is not None and (n >= rows or (self._auto and n >= _CROSSOVER_LIBRARY and not self._kernels_take(x2))):
             w16 = weight_dequant_native_cuda(self.exponent, self.mantissa, self.weight_native, self.scales, self.out_features, self.in_features,
                                              self.group_exps)
             y = torch.nn.functional.linear(x2, w16)
@@ -165,9 +190,9 @@ class FPxLinear(torch.nn.Module):
             return y.reshape(*lead, self.out_features)
         sk = self.split_k
         if not sk:   # the heuristic's answer per batch size is remembered: the layer is called once per token
-            sk = self._split_cache.get(x2.shape[0])
+            sk = self._split_cache.get(n)
             if sk is None:
-                sk = self._split_cache[x2.shape[0]] = heuristic_splitk_mi355x(self.out_features, x2.shape[0], self.in_features, MI355X_CUS, self.exponent, self.mantissa)
+                sk = self._split_cache[n] = heuristic_splitk_mi355x(self.out_features, n, self.in_features, MI355X_CUS, self.exponent, self.mantissa)
         fused = self.bias is not None and self._bias_in_kernel(x2)
         y = linear_forward_native(self.exponent, self.mantissa, x2, self.weight_native, self.scales, self.out_features, sk, None, None, self.group_exps,
                                   self.bias if fused else None)

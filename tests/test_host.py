@@ -822,3 +822,54 @@ def test_a_torch_without_the_private_names_keeps_the_torch_operations(monkeypatc
     with monkeypatch.context() as m:
         m.delattr(torch.autograd.forward_ad, "_current_level")
         assert not layer._bias_in_kernel(x) and not layer._kernels_take(x) and float(layer(x)[0, 0]) == 129.0
+
+
+def test_dequant_above_says_what_it_does(monkeypatch):
+    """The number that is read is the number of rows from which weights are dequantized: "auto" reads PREFILL_CROSSOVER, which a subclass may lower, or 3072
+    where the wide tiles do not run; whole modules pickled before it was a property keep their route."""
+    import copy
+    import pickle
+    import types
+    module = _long_prompt_stubs(monkeypatch)
+    x = torch.ones(33000, 64, dtype=torch.float16)
+
+    def library_from(layer, rows):
+        assert layer.dequant_above == rows
+        assert float(layer(x[:rows])[0, 0]) == 128.0 and float(layer(x[:rows - 1])[0, 0]) == -1.0
+    def layer_is_auto(layer):   # what requires a gradient still gets it
+        return layer(x[:3072].clone().requires_grad_()).requires_grad
+    plain = module.FPxLinear(64, 256)
+    assert plain.dequant_above == module.FPxLinear.PREFILL_CROSSOVER
+    for layer in (plain, copy.deepcopy(plain), pickle.loads(pickle.dumps(plain))):
+        library_from(layer, 32768)
+    for rows in (7, 3072, 32768):
+        library_from(module.FPxLinear(64, 256, dequant_above=rows), rows)
+        plain.dequant_above = rows
+        library_from(plain, rows)
+    assert not layer_is_auto(plain)
+    for auto in ("auto", module.FPxLinear(64, 256).dequant_above):
+        plain.dequant_above = auto
+        library_from(plain, 32768)
+        assert layer_is_auto(plain)
+    plain.dequant_above = None
+    assert plain.dequant_above is None and float(plain(x)[0, 0]) == -1.0
+
+    for rows in (100, 3072, 5000):
+        monkeypatch.setattr(module.FPxLinear, "PREFILL_CROSSOVER", rows)
+        library_from(module.FPxLinear(64, 256), rows)
+    monkeypatch.setattr(module.FPxLinear, "PREFILL_CROSSOVER", 32768)
+    monkeypatch.setattr(module.FPxLinear, "_wide_tiles", lambda self, device: False)
+    library_from(module.FPxLinear(64, 256), 3072)
+    monkeypatch.undo()
+    _long_prompt_stubs(monkeypatch)
+    part = module.FPxLinear(64, 256)
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: types.SimpleNamespace(multi_processor_count=32))
+    assert not part._wide_tiles(torch.device("cuda:0")) and part._wide_tiles(torch.device("cpu"))
+    assert not module.FPxLinear((1 << 20) + 64, 256)._wide_tiles(torch.device("cpu"))
+
+    # the state of a whole module as earlier versions pickled it
+    for held, rows in ((3072, 3072), (module._AutoRows(3072), 32768), (512, 512)):
+        state = {k: v for k, v in module.FPxLinear(64, 256).__dict__.items() if k not in ("_auto", "_rows")}
+        old = module.FPxLinear.__new__(module.FPxLinear)
+        old.__setstate__(dict(state, dequant_above=held))
+        library_from(old, rows)
