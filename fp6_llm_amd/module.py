@@ -45,7 +45,8 @@ class FPxLinear(torch.nn.Module):
     PREFILL_CROSSOVER = _CROSSOVER
 
     def __init__(self, in_features, out_features, exponent=3, mantissa=2, bias=None, split_k=None, dequant_above="auto", group_scales=False):
-        """group_scales: the layer also holds one exponent byte per row and 128 columns (factor 1 until weights are loaded).
+        """split_k: number of pieces of K, None for the heuristic's choice; under dequant_above="auto" it holds for less than 3072 rows.
+        group_scales: the layer also holds one exponent byte per row and 128 columns (factor 1 until weights are loaded).
         dequant_above: batch size from which forward() dequantizes the weights to a temporary fp16 matrix on the GPU and calls
         the FP16 library GEMM instead (the temporary costs 2 bytes per weight for the duration of the call).  None never does; an
         integer sets the threshold; "auto" (default) is PREFILL_CROSSOVER rows, or 3072 where the wide tiles do not run.  Under "auto" an
@@ -189,7 +190,8 @@ class FPxLinear(torch.nn.Module):
                 y = y + self.bias
             return y.reshape(*lead, self.out_features)
         sk = self.split_k
-        if not sk:   # the heuristic's answer per batch size is remembered: the layer is called once per token
+        if not sk or (self._auto and n >= _CROSSOVER_LIBRARY):   # the heuristic's answer per batch size is remembered: the layer is called once per token
+            # (split_k is for the batches up to 3071 rows; the partial sums of a long prompt would take gigabytes)
             sk = self._split_cache.get(n)
             if sk is None:
                 sk = self._split_cache[n] = heuristic_splitk_mi355x(self.out_features, n, self.in_features, MI355X_CUS, self.exponent, self.mantissa)

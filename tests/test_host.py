@@ -873,3 +873,16 @@ def test_dequant_above_says_what_it_does(monkeypatch):
         old = module.FPxLinear.__new__(module.FPxLinear)
         old.__setstate__(dict(state, dequant_above=held))
         library_from(old, rows)
+
+
+def test_a_split_for_decoding_is_not_taken_for_long_prompts(monkeypatch):
+    """split_k=4 of 28672 features would keep 15 GB of partial sums for 32767 rows; under "auto" long prompts take the heuristic's split, as they took none
+    before they ran on the kernels.  With a threshold of the user's own, or none, the split holds for all rows that the kernels get."""
+    module = _long_prompt_stubs(monkeypatch)
+    splits = []
+    monkeypatch.setattr(module, "linear_forward_native", lambda E, M, x, w, s, OC, sk, *a: (splits.append(sk), torch.zeros(x.shape[0], OC, dtype=torch.float16))[1])
+    monkeypatch.setattr(module, "heuristic_splitk_mi355x", lambda *a: 77)
+    x = torch.ones(32767, 64, dtype=torch.float16)
+    for above, rows, want in (("auto", 1, 4), ("auto", 3071, 4), ("auto", 3072, 77), ("auto", 32767, 77), (None, 3072, 4), (4000, 3999, 4)):
+        module.FPxLinear(64, 256, split_k=4, dequant_above=above)(x[:rows])
+        assert splits.pop() == want, (above, rows)
