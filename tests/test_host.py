@@ -886,3 +886,14 @@ def test_a_split_for_decoding_is_not_taken_for_long_prompts(monkeypatch):
     for above, rows, want in (("auto", 1, 4), ("auto", 3071, 4), ("auto", 3072, 77), ("auto", 32767, 77), (None, 3072, 4), (4000, 3999, 4)):
         module.FPxLinear(64, 256, split_k=4, dequant_above=above)(x[:rows])
         assert splits.pop() == want, (above, rows)
+
+
+def test_a_call_reads_every_buffer_once(monkeypatch):
+    """A read of a buffer is a call of nn.Module.__getattr__, half a microsecond beside kernels of four: a forward pass without a bias takes four."""
+    module = _long_prompt_stubs(monkeypatch)
+    layer, x, names = module.FPxLinear(64, 256), torch.ones(8, 64, dtype=torch.float16), []
+    layer(x)
+    found = torch.nn.Module.__getattr__
+    monkeypatch.setattr(module.FPxLinear, "__getattr__", lambda self, name: (names.append(name), found(self, name))[1], raising=False)
+    layer(x)
+    assert sorted(names) == ["bias", "group_exps", "scales", "weight_native"]
