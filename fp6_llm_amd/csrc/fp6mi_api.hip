@@ -443,14 +443,30 @@ inline bool wide_replaces(float t, float narrow, size_t M, size_t N)
     return t < narrow * (N <= 400 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
 }
 
-// The launch shape of a call: gemm_wide's, or that of the table and the rules (which fp6mi_query_launch reports)
+// The fastest split of the table's (3 % hysteresis towards fewer pieces) and its time in us; 0 where it holds none
+inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N)
+{
+    float best = 0.f;
+    split = 0;
+    for (int s : kSplits)
+        if (const float t = narrow_estimate(a, M, N, s); t > 0.f && (split == 0 || t * 1.03f < best)) split = s, best = t;
+    return best;
+}
+// The launch shape of a call: gemm_wide's, or that of the table and the rules.  A split that the table does not hold for a problem it does hold (in other
+// splits) is compared with the fastest of those, as the heuristic, which knows no group exponents, does before it answers with one: of what the rules would
+// launch there neither has a time.  60 problems whose split the rules launched until then (1280x2624 N 525 in four, say), time / time before gemm_wide: 0.74 (0.39-1.03), 0.77
+// (0.37-1.26) by the rules.
 inline LaunchCfg final_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, bool groups, int cus)
 {
     LaunchCfg wide;
     if (cus == 256 && N > 96)
         if (const float t = wide_best(wide, xbits, M, N, K, splitK, groups); t > 0.f) {
-            const float narrow = narrow_estimate(tune_lookup(xbits, M, N, K), M, N, splitK);
-            if (wide_replaces(t, groups ? 1.06f * narrow : narrow, M, N)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
+            const TuneAnswer *a = tune_lookup(xbits, M, N, K);
+            const float       here = narrow_estimate(a, M, N, splitK);
+            if (wide_replaces(t, groups ? 1.06f * here : here, M, N)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
+            LaunchCfg other;
+            int       split;
+            if (here <= 0.f && wide_replaces(groups ? wide_best(other, xbits, M, N, K, splitK, false) : t, best_narrow(split, a, M, N), M, N)) return wide;
         }
     return pick_cfg(xbits, M, N, K, splitK, cus);
 }
@@ -556,18 +572,14 @@ static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus
     if (M == 0 || N == 0 || K == 0 || num_cus <= 0) return 1;
     size_t units = (K + 255) / 256;
     if (num_cus == 256) { // the fastest split by the times of measured neighbours, or of gemm_wide where it takes their place (3 % hysteresis towards fewer splits)
-        const TuneAnswer *a = tune_lookup(xbits, M, N, K);
-        int               best_s = 0, wide_s = 0;
-        float             best_t = 0.f, wide_t = 0.f;
-        auto              better = [](int s, float t, int &best_s, float &best_t) {
-            if (t > 0.f && (best_s == 0 || t * 1.03f < best_t)) best_s = s, best_t = t;
-        };
+        int               best_s, wide_s = 0;
+        const float       best_t = best_narrow(best_s, tune_lookup(xbits, M, N, K), M, N);
+        float             wide_t = 0.f;
         for (int s : kSplits) {
             LaunchCfg wide;
-            better(s, narrow_estimate(a, M, N, s), best_s, best_t);
-            better(s, wide_best(wide, xbits, M, N, K, s, false), wide_s, wide_t);
+            if (const float t = wide_best(wide, xbits, M, N, K, s, false); t > 0.f && (wide_s == 0 || t * 1.03f < wide_t)) wide_s = s, wide_t = t;
         }
-        if (wide_replaces(wide_t, best_t, M, N)) return wide_s;
+        if (wide_replaces(wide_t, best_t, M, N)) return wide_s; // (final_cfg launches gemm_wide then)
         if (best_s) return best_s;
     }
     if (N > 16) {

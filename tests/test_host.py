@@ -897,3 +897,25 @@ def test_a_call_reads_every_buffer_once(monkeypatch):
     monkeypatch.setattr(module.FPxLinear, "__getattr__", lambda self, name: (names.append(name), found(self, name))[1], raising=False)
     layer(x)
     assert sorted(names) == ["bias", "group_exps", "scales", "weight_native"]
+
+
+def test_a_split_of_the_heuristics_is_launched_by_what_it_was_chosen_for():
+    """From 97 columns on the heuristic's split is launched by gemm_wide or by the table's shape for that very split; the rules launch one only where the table
+    holds no split of the problem.  1024x8192 N 600 was cut in three for gemm_wide and launched with a tile of the rules, whose time nothing had compared."""
+    L = _lib.lib()
+    shape = (ctypes.c_int * 5)()
+    rng = np.random.default_rng(12)
+    problems = [(3, 2, 1024, 8192, 600), (3, 2, 1024, 8192, 800), (3, 2, 2048, 8192, 500), (3, 2, 1280, 2624, 525)]
+    for _ in range(4000):
+        problems.append((*FORMATS[rng.integers(len(FORMATS))], 256 * int(2 ** rng.uniform(0, 7)), 64 * int(2 ** rng.uniform(0, 9)), int(2 ** rng.uniform(6.6, 12))))
+    cut = 0
+    for E, M, OC, IC, N in problems:
+        split = fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M)
+        for grouped in (0, 1):
+            assert L.fp6mi_query_kernel(E, M, OC, N, IC, split, grouped, shape) == 0
+            if shape[0] == 2 and ((shape[3] == 4 and shape[4] <= 2) or shape[3] == 2):   # gemm_wide, or gemm_prefill in the place of a shape of the table's
+                cut += split > 1
+                continue
+            if L.fp6mi_launch_source(E, M, OC, N, IC, split) == 2:
+                assert all(L.fp6mi_launch_source(E, M, OC, N, IC, s) == 2 for s in (1, 2, 3, 4, 6, 8)), (E, M, OC, IC, N, split, tuple(shape))
+    assert cut > 100
