@@ -50,6 +50,7 @@ __all__ = [
 ]
 
 MI355X_CUS = 256
+SPLIT_WORKSPACE_BYTES = 96 << 20   # as much as the measured table's own splits take, up to 28672 rows
 
 
 # ----------------------------------------------------------------------------------------------------------------
@@ -71,8 +72,10 @@ def HeuristicFuntion_SplitK(M, N, Num_GPU_SMs):
 def heuristic_splitk_mi355x(M, N, K, num_cus=MI355X_CUS, EXPONENT=3, MANTISSA=2):
     """Split-K for this engine's kernels: K is already split across the wavefronts of a workgroup, so a split across
     workgroups (second launch + FP32 workspace traffic) only pays when M/16 workgroups cannot occupy the chip.  The answer
-    comes from the table measured for the format's bit width where the problem is near a measured one."""
-    return _lib.lib().fp6mi_heuristic_splitk_format(EXPONENT, MANTISSA, M, N, K, num_cus)
+    comes from the table measured for the format's bit width where the problem is near a measured one.  Its partial sums
+    (splitK*N*M floats) are kept per stream; those of a split that is not in the table take at most
+    SPLIT_WORKSPACE_BYTES."""
+    return _lib.lib().fp6mi_heuristic_splitk_within(EXPONENT, MANTISSA, M, N, K, num_cus, SPLIT_WORKSPACE_BYTES)
 
 
 # ----------------------------------------------------------------------------------------------------------------

@@ -443,13 +443,17 @@ inline bool wide_replaces(float t, float narrow, size_t M, size_t N)
     return t < narrow * (N <= 400 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
 }
 
-// The fastest split of the table's (3 % hysteresis towards fewer pieces) and its time in us; 0 where it holds none
-inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N)
+// The fastest split of the table's (3 % hysteresis towards fewer pieces) and its time in us; 0 where it holds none.  One that takes more than ws_bytes has to be
+// the faster by the table's times as they stand too, which were what decided before narrow_estimate.
+inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N, size_t ws_bytes)
 {
     float best = 0.f;
     split = 0;
     for (int s : kSplits)
-        if (const float t = narrow_estimate(a, M, N, s); t > 0.f && (split == 0 || t * 1.03f < best)) split = s, best = t;
+        if (const float t = narrow_estimate(a, M, N, s); t > 0.f && (split == 0 || t * 1.03f < best)) {
+            if (split && fp6mi_workspace_bytes(M, N, s) > ws_bytes && a->t[split_index(s)] * 1.03f >= a->t[split_index(split)]) continue;
+            split = s, best = t;
+        }
     return best;
 }
 // The launch shape of a call: gemm_wide's, or that of the table and the rules.  A split that the table does not hold for a problem it does hold (in other
@@ -466,7 +470,7 @@ inline LaunchCfg final_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, 
             if (wide_replaces(t, groups ? 1.06f * here : here, M, N)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
             LaunchCfg other;
             int       split;
-            if (here <= 0.f && wide_replaces(groups ? wide_best(other, xbits, M, N, K, splitK, false) : t, best_narrow(split, a, M, N), M, N)) return wide;
+            if (here <= 0.f && wide_replaces(groups ? wide_best(other, xbits, M, N, K, splitK, false) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N)) return wide;
         }
     return pick_cfg(xbits, M, N, K, splitK, cus);
 }
@@ -558,25 +562,36 @@ size_t fp6mi_workspace_bytes(size_t M, size_t N, int splitK) { return splitK > 1
 // chip cannot beat HBM, and a split costs a second launch plus writing and re-reading the FP32 partial sums; K is
 // already split inside the workgroup, so a split rarely pays.  Larger batches (tile kernel): as much of the wanted K
 // parallelism as keeps the FP32 partial-sum traffic (8 bytes per output per split) under half of the weight bytes.
-static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus);
+//
+// ws_bytes: what a split chosen for gemm_wide may take.  Its model asked for up to 370 MB where the table's splits take up to 99 (M up to 28672), and for more than
+// the static workspace on 3.3 % of sizes of 98 to 4096 columns where it had taken them before.  On 60 of those, time / time before gemm_wide: 0.83 with any workspace, 0.84 held to 32 MiB.
+constexpr size_t kStaticWsFloats = (size_t)8 << 20; // the static workspace: 32 MiB per GPU, held from the first use of the library on that GPU until the process ends
 
-int fp6mi_heuristic_splitk(size_t M, size_t N, size_t K, int num_cus) { return heuristic_splitk(6, M, N, K, num_cus); }
+static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus, size_t ws_bytes);
+
+int fp6mi_heuristic_splitk(size_t M, size_t N, size_t K, int num_cus) { return heuristic_splitk(6, M, N, K, num_cus, kStaticWsFloats * sizeof(float)); }
 
 int fp6mi_heuristic_splitk_format(int E, int Mb, size_t M, size_t N, size_t K, int num_cus)
 {
-    return heuristic_splitk(fp6mi::supported(E, Mb) ? 1 + E + Mb : 6, M, N, K, num_cus);
+    return fp6mi_heuristic_splitk_within(E, Mb, M, N, K, num_cus, kStaticWsFloats * sizeof(float));
 }
 
-static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus)
+int fp6mi_heuristic_splitk_within(int E, int Mb, size_t M, size_t N, size_t K, int num_cus, size_t ws_bytes)
+{
+    return heuristic_splitk(fp6mi::supported(E, Mb) ? 1 + E + Mb : 6, M, N, K, num_cus, ws_bytes);
+}
+
+static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus, size_t ws_bytes)
 {
     if (M == 0 || N == 0 || K == 0 || num_cus <= 0) return 1;
     size_t units = (K + 255) / 256;
     if (num_cus == 256) { // the fastest split by the times of measured neighbours, or of gemm_wide where it takes their place (3 % hysteresis towards fewer splits)
         int               best_s, wide_s = 0;
-        const float       best_t = best_narrow(best_s, tune_lookup(xbits, M, N, K), M, N);
+        const float       best_t = best_narrow(best_s, tune_lookup(xbits, M, N, K), M, N, ws_bytes);
         float             wide_t = 0.f;
         for (int s : kSplits) {
             LaunchCfg wide;
+            if (fp6mi_workspace_bytes(M, N, s) > ws_bytes) break;
             if (const float t = wide_best(wide, xbits, M, N, K, s, false); t > 0.f && (wide_s == 0 || t * 1.03f < wide_t)) wide_s = s, wide_t = t;
         }
         if (wide_replaces(wide_t, best_t, M, N)) return wide_s; // (final_cfg launches gemm_wide then)
@@ -709,7 +724,6 @@ int fp6mi_query_kernel(int E, int Mb, size_t M, size_t N, size_t K, int splitK, 
 
 // ---- allocation-free variant of fp6mi_linear_native: the split-K workspace is a static device array of the library ----
 namespace {
-constexpr size_t kStaticWsFloats = (size_t)8 << 20; // 32 MiB per GPU, held from the first use of the library on that GPU until the process ends
 __device__ __align__(256) float g_static_ws[kStaticWsFloats];
 
 // Device address of g_static_ws on the current device (every GPU holds its own copy of the array at its own address); asked

@@ -75,6 +75,9 @@ int    fp6mi_unpack_native(int E, int Mbits, void *raw, const void *native, size
 int fp6mi_heuristic_splitk(size_t M, size_t N, size_t K, int num_cus);
 /* The same for a given weight format (the measured table is per bit width; the function above answers for FP6). */
 int fp6mi_heuristic_splitk_format(int E, int Mbits, size_t M, size_t N, size_t K, int num_cus);
+/* The same for callers that lend a workspace of their own: from 97 columns on a split that is not one of the measured table may take up to workspace_bytes
+ * of it; the two above hold those to the static workspace (fp6mi_static_workspace_bytes).  The table's splits take up to 99 MB for M up to 28672. */
+int fp6mi_heuristic_splitk_within(int E, int Mbits, size_t M, size_t N, size_t K, int num_cus, size_t workspace_bytes);
 
 /* Bytes of the split-K workspace the GEMM entry points need: splitK*M*N floats (fp6_llm/csrc/fp6_linear.cuh:17),
  * 0 when splitK == 1. */
@@ -95,8 +98,8 @@ int fp6mi_linear_native(int E, int Mbits, void *stream, const void *W_native, co
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  Same kernels and results as
  * fp6mi_linear_native; the split-K partial sums go to a static device array of the library,
  * fp6mi_static_workspace_bytes() bytes (32 MiB) per GPU, instead of a caller workspace.  It calls no hipMalloc/hipFree.
- * splitK * M * N floats beyond that size return FP6MI_ERR_TOO_LARGE: a splitK from fp6mi_heuristic_splitk, which is the
- * fastest with a workspace of any size, may need more, so compare fp6mi_workspace_bytes first (1 always fits).  All calls
+ * splitK * M * N floats beyond that size return FP6MI_ERR_TOO_LARGE: a splitK from fp6mi_heuristic_splitk may
+ * still need more where the measured table holds one, so compare fp6mi_workspace_bytes first (1 always fits).  All calls
  * on one GPU share the array: calls with splitK > 1 that overlap in time on one GPU (different streams) race; calls on one
  * stream are ordered.
  * fp6mi_init() looks the array's device address up for the current device ahead of time (the first call on a device does

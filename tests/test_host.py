@@ -919,3 +919,27 @@ def test_a_split_of_the_heuristics_is_launched_by_what_it_was_chosen_for():
             if L.fp6mi_launch_source(E, M, OC, N, IC, split) == 2:
                 assert all(L.fp6mi_launch_source(E, M, OC, N, IC, s) == 2 for s in (1, 2, 3, 4, 6, 8)), (E, M, OC, IC, N, split, tuple(shape))
     assert cut > 100
+
+
+def test_splits_stay_within_the_workspaces_they_are_chosen_for():
+    """Where gemm_wide took the table's place the heuristic asked for up to 370 MB of partial sums, and ordinary prompts for more than the static workspace holds
+    (which the table had left uncut).  The C heuristic's splits fit that one, but for the few that the table itself holds; Python's stay under 96 MiB, and are
+    also taken by the workspace that the C answer fits into."""
+    L = _lib.lib()
+    static = L.fp6mi_static_workspace_bytes()
+    for OC, IC, N in ((8192, 28672, 512), (8192, 8192, 600), (5120, 8192, 800), (4096, 14336, 700), (5120, 21952, 896), (6912, 27712, 257), (1280, 24384, 1117)):
+        for E, M in ((3, 2), (2, 2)):
+            assert L.fp6mi_workspace_bytes(OC, N, L.fp6mi_heuristic_splitk_format(E, M, OC, N, IC, 256)) <= static, (OC, IC, N)
+    for OC, IC, N in ((13568, 24704, 364), (12800, 28288, 365), (12544, 25664, 355)):   # the table's choice once its times are scaled to N, not before
+        assert L.fp6mi_workspace_bytes(OC, N, L.fp6mi_heuristic_splitk(OC, N, IC, 256)) <= static, (OC, IC, N)
+    rng = np.random.default_rng(13)
+    most, beyond, fewer = 0, 0, 0
+    for _ in range(20000):
+        E, M = FORMATS[rng.integers(len(FORMATS))]
+        OC, IC, N = 256 * int(2 ** rng.uniform(0, 6.8)), 64 * int(2 ** rng.uniform(2, 8.8)), int(2 ** rng.uniform(6.6, 15))
+        c, py = L.fp6mi_heuristic_splitk_format(E, M, OC, N, IC, 256), fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M)
+        most, beyond = max(most, L.fp6mi_workspace_bytes(OC, N, py)), beyond + (L.fp6mi_workspace_bytes(OC, N, c) > static)
+        fewer += c != py
+        assert c == py or L.fp6mi_workspace_bytes(OC, N, py) > static or c > py
+        assert c == L.fp6mi_heuristic_splitk_within(E, M, OC, N, IC, 256, static)
+    assert most <= fp6.SPLIT_WORKSPACE_BYTES and beyond <= 20000 // 100 and fewer > 100
