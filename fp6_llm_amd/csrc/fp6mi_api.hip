@@ -436,11 +436,13 @@ inline float narrow_estimate(const TuneAnswer *a, size_t M, size_t N, int splitK
 // (0.80-1.07), N 257-400 0.90 (0.50-1.13), N 401-640 0.84 (0.48-1.03), beyond 0.83 (0.46-1.06); N 65-96 1.00, not worth it.  The margins are what the two
 // estimates are off where the kernels are close, and allow for the table's, which is low, where they are not: without them 40 of these problems were more than
 // 2 % slower, with them 5.
-inline bool wide_replaces(float t, float narrow, size_t M, size_t N)
+// The tile of 64 columns has the smallest margin whatever N is: on 175 problems beyond N 640 it took with 1.15 (1024x6144 N 1848, 2560x19904 N 3224) it was 1.00
+// (0.56-1.28), 71 of them over 1.02; with 0.9 it takes 44 of them at 0.91 and 4 are over 1.02 (9472x17024 N 1984 in FP4 1.28, the others up to 1.06); on 34 problems of N 401-640 as good as with 0.95, 1 over 1.02 for 5.
+inline bool wide_replaces(const LaunchCfg &wide, float t, float narrow, size_t M, size_t N)
 {
     if (t <= 0.f) return false;
     if (narrow <= 0.f) return M * N >= (size_t)1 << 20;
-    return t < narrow * (N <= 400 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
+    return t < narrow * (N <= 400 || wide.nt == 4 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
 }
 
 // The fastest split of the table's (3 % hysteresis towards fewer pieces) and its time in us; 0 where it holds none.  One that takes more than ws_bytes has to be
@@ -467,10 +469,10 @@ inline LaunchCfg final_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, 
         if (const float t = wide_best(wide, xbits, M, N, K, splitK, groups); t > 0.f) {
             const TuneAnswer *a = tune_lookup(xbits, M, N, K);
             const float       here = narrow_estimate(a, M, N, splitK);
-            if (wide_replaces(t, groups ? 1.06f * here : here, M, N)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
-            LaunchCfg other;
+            if (wide_replaces(wide, t, groups ? 1.06f * here : here, M, N)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
+            LaunchCfg ungrouped = wide;
             int       split;
-            if (here <= 0.f && wide_replaces(groups ? wide_best(other, xbits, M, N, K, splitK, false) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N)) return wide;
+            if (here <= 0.f && wide_replaces(ungrouped, groups ? wide_best(ungrouped, xbits, M, N, K, splitK, false) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N)) return wide;
         }
     return pick_cfg(xbits, M, N, K, splitK, cus);
 }
@@ -589,12 +591,13 @@ static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus
         int               best_s, wide_s = 0;
         const float       best_t = best_narrow(best_s, tune_lookup(xbits, M, N, K), M, N, ws_bytes);
         float             wide_t = 0.f;
+        LaunchCfg         wide = {};
         for (int s : kSplits) {
-            LaunchCfg wide;
+            LaunchCfg c;
             if (fp6mi_workspace_bytes(M, N, s) > ws_bytes) break;
-            if (const float t = wide_best(wide, xbits, M, N, K, s, false); t > 0.f && (wide_s == 0 || t * 1.03f < wide_t)) wide_s = s, wide_t = t;
+            if (const float t = wide_best(c, xbits, M, N, K, s, false); t > 0.f && (wide_s == 0 || t * 1.03f < wide_t)) wide_s = s, wide_t = t, wide = c;
         }
-        if (wide_replaces(wide_t, best_t, M, N)) return wide_s; // (final_cfg launches gemm_wide then)
+        if (wide_replaces(wide, wide_t, best_t, M, N)) return wide_s; // (final_cfg launches gemm_wide then)
         if (best_s) return best_s;
     }
     if (N > 16) {

@@ -943,3 +943,14 @@ def test_splits_stay_within_the_workspaces_they_are_chosen_for():
         assert c == py or L.fp6mi_workspace_bytes(OC, N, py) > static or c > py
         assert c == L.fp6mi_heuristic_splitk_within(E, M, OC, N, IC, 256, static)
     assert most <= fp6.SPLIT_WORKSPACE_BYTES and beyond <= 20000 // 100 and fewer > 100
+
+
+@pytest.mark.parametrize("E,M,OC,IC,N,grouped,wide", [
+    (2, 2, 1024, 6144, 1848, 0, False), (2, 1, 2560, 19904, 3224, 0, False), (2, 2, 1536, 14336, 691, 0, False), (3, 2, 1024, 16000, 774, 0, False),
+    (2, 2, 768, 5504, 2310, 0, False), (2, 2, 1792, 28288, 807, 1, False), (2, 2, 2048, 2304, 616, 0, False),   # 1.11 to 1.24 with 64-column tiles
+    (3, 2, 4608, 2816, 545, 0, True), (3, 2, 512, 8960, 2877, 0, True), (3, 2, 5632, 4096, 1000, 0, True)])
+def test_where_the_wide_kernel_does_not_pay(E, M, OC, IC, N, grouped, wide):
+    """Problems on which gemm_wide took 1.05 to 1.24 of the time of the shape whose place it took, unsplit, and some beside them where it takes less."""
+    shape = (ctypes.c_int * 5)()
+    assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, 1, grouped, shape) == 0
+    assert (shape[0] == 2 and shape[3] == 4 and shape[4] <= 2) == wide, tuple(shape)
