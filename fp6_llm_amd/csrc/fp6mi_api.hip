@@ -437,11 +437,13 @@ inline float narrow_estimate(const TuneAnswer *a, size_t M, size_t N, int splitK
 // estimates are off where the kernels are close, and allow for the table's, which is low, where they are not: without them 40 of these problems were more than
 // 2 % slower, with them 5.
 // The tile of 64 columns has the smallest margin whatever N is: on 175 problems beyond N 640 it took with 1.15 (1024x6144 N 1848, 2560x19904 N 3224) it was 1.00
-// (0.56-1.28), 71 of them over 1.02; with 0.9 it takes 44 of them at 0.91 and 4 are over 1.02 (9472x17024 N 1984 in FP4 1.28, the others up to 1.06); on 34 problems of N 401-640 as good as with 0.95, 1 over 1.02 for 5.
-inline bool wide_replaces(const LaunchCfg &wide, float t, float narrow, size_t M, size_t N)
+// (0.56-1.28), 71 of them over 1.02; with 0.9 it takes 44 of them at 0.91 and 4 are over 1.02 (9472x17024 N 1984 in FP4 1.28, the others up to 1.03); on 34 problems of N 401-640 as good as with 0.95, 1 over 1.02 for 5.
+// Out of the table's reach K up to 512 takes 2^22 outputs: 23 problems below that took 1.02 of the time of the rules' tiles (0.90-1.22: 5632x256 N 325 4.9 us -> 5.9);
+// of the 177 others, 0.87 (0.63-1.09), 8 are over 1.02.
+inline bool wide_replaces(const LaunchCfg &wide, float t, float narrow, size_t M, size_t N, size_t K)
 {
     if (t <= 0.f) return false;
-    if (narrow <= 0.f) return M * N >= (size_t)1 << 20;
+    if (narrow <= 0.f) return M * N >= (size_t)1 << (K <= 512 ? 22 : 20);
     return t < narrow * (N <= 400 || wide.nt == 4 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
 }
 
@@ -469,10 +471,10 @@ inline LaunchCfg final_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, 
         if (const float t = wide_best(wide, xbits, M, N, K, splitK, groups); t > 0.f) {
             const TuneAnswer *a = tune_lookup(xbits, M, N, K);
             const float       here = narrow_estimate(a, M, N, splitK);
-            if (wide_replaces(wide, t, groups ? 1.06f * here : here, M, N)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
+            if (wide_replaces(wide, t, groups ? 1.06f * here : here, M, N, K)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
             LaunchCfg ungrouped = wide;
             int       split;
-            if (here <= 0.f && wide_replaces(ungrouped, groups ? wide_best(ungrouped, xbits, M, N, K, splitK, false) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N)) return wide;
+            if (here <= 0.f && wide_replaces(ungrouped, groups ? wide_best(ungrouped, xbits, M, N, K, splitK, false) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N, K)) return wide;
         }
     return pick_cfg(xbits, M, N, K, splitK, cus);
 }
@@ -597,7 +599,7 @@ static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus
             if (fp6mi_workspace_bytes(M, N, s) > ws_bytes) break;
             if (const float t = wide_best(c, xbits, M, N, K, s, false); t > 0.f && (wide_s == 0 || t * 1.03f < wide_t)) wide_s = s, wide_t = t, wide = c;
         }
-        if (wide_replaces(wide, wide_t, best_t, M, N)) return wide_s; // (final_cfg launches gemm_wide then)
+        if (wide_replaces(wide, wide_t, best_t, M, N, K)) return wide_s; // (final_cfg launches gemm_wide then)
         if (best_s) return best_s;
     }
     if (N > 16) {

@@ -948,7 +948,9 @@ def test_splits_stay_within_the_workspaces_they_are_chosen_for():
 @pytest.mark.parametrize("E,M,OC,IC,N,grouped,wide", [
     (2, 2, 1024, 6144, 1848, 0, False), (2, 1, 2560, 19904, 3224, 0, False), (2, 2, 1536, 14336, 691, 0, False), (3, 2, 1024, 16000, 774, 0, False),
     (2, 2, 768, 5504, 2310, 0, False), (2, 2, 1792, 28288, 807, 1, False), (2, 2, 2048, 2304, 616, 0, False),   # 1.11 to 1.24 with 64-column tiles
-    (3, 2, 4608, 2816, 545, 0, True), (3, 2, 512, 8960, 2877, 0, True), (3, 2, 5632, 4096, 1000, 0, True)])
+    (3, 2, 5632, 256, 325, 0, False), (2, 1, 512, 256, 2951, 0, False), (3, 2, 21504, 384, 172, 1, False), (3, 2, 14336, 512, 220, 0, False),         # 1.05 to 1.22 with little K
+    (3, 2, 4608, 2816, 545, 0, True), (3, 2, 512, 8960, 2877, 0, True), (3, 2, 5632, 4096, 1000, 0, True), (3, 2, 4096, 960, 609, 0, True),
+    (2, 2, 28672, 512, 500, 0, True)])
 def test_where_the_wide_kernel_does_not_pay(E, M, OC, IC, N, grouped, wide):
     """Problems on which gemm_wide took 1.05 to 1.24 of the time of the shape whose place it took, unsplit, and some beside them where it takes less."""
     shape = (ctypes.c_int * 5)()
