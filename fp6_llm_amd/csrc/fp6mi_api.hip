@@ -696,11 +696,18 @@ int fp6mi_linear_native_grouped_cfg(int E, int Mb, void *stream, const void *W, 
     return linear_native(*fp6mi::ops_for(E, Mb), st, W, sc, group_exps, nullptr, B, C, M, N, K, ws, splitK, &c);
 }
 
-int fp6mi_launch_source(int E, int Mb, size_t M, size_t N, size_t K, int splitK)
+static int query_args(int E, int Mb, size_t M, size_t N, size_t K, int splitK)
 {
     if (!fp6mi::supported(E, Mb)) return FP6MI_ERR_FORMAT;
     if (M == 0 || M % 256 || K == 0 || K % 64 || N == 0) return FP6MI_ERR_SHAPE;
-    if (splitK < 1) return FP6MI_ERR_SPLITK;
+    return splitK < 1 ? FP6MI_ERR_SPLITK : FP6MI_OK;
+}
+static void write_shape(int *shape, const LaunchCfg &c) { shape[0] = c.kind, shape[1] = c.nt, shape[2] = c.rt, shape[3] = c.wr, shape[4] = c.wk; }
+
+int fp6mi_query_table(int E, int Mb, size_t M, size_t N, size_t K, int splitK, int *shape)
+{
+    if (int rc = query_args(E, Mb, M, N, K, splitK); rc != FP6MI_OK) return rc;
+    if (shape) write_shape(shape, pick_cfg(1 + E + Mb, M, N, K, splitK, current_device_cus())); // the count the launch path uses (256 where no device answers)
     const int i = split_index(splitK);
     if (i >= 0)
         if (const TuneAnswer *a = tune_lookup(1 + E + Mb, M, N, K))
@@ -708,23 +715,22 @@ int fp6mi_launch_source(int E, int Mb, size_t M, size_t N, size_t K, int splitK)
     return 2;
 }
 
-int fp6mi_query_launch(int E, int Mb, size_t M, size_t N, size_t K, int splitK, int *shape)
+int fp6mi_query_kernel(int E, int Mb, size_t M, size_t N, size_t K, int splitK, int grouped, int *shape)
 {
-    if (!fp6mi::supported(E, Mb)) return FP6MI_ERR_FORMAT;
+    if (int rc = query_args(E, Mb, M, N, K, splitK); rc != FP6MI_OK) return rc;
     if (!shape) return FP6MI_ERR_NULL;
-    if (M == 0 || M % 256 || K == 0 || K % 64 || N == 0) return FP6MI_ERR_SHAPE;
-    if (splitK < 1) return FP6MI_ERR_SPLITK;
-    LaunchCfg c = pick_cfg(1 + E + Mb, M, N, K, splitK, current_device_cus()); // the count the launch path uses (256 where no device answers)
-    shape[0] = c.kind, shape[1] = c.nt, shape[2] = c.rt, shape[3] = c.wr, shape[4] = c.wk;
+    write_shape(shape, final_cfg(1 + E + Mb, M, N, K, splitK, grouped != 0, current_device_cus()));
     return FP6MI_OK;
 }
 
-int fp6mi_query_kernel(int E, int Mb, size_t M, size_t N, size_t K, int splitK, int grouped, int *shape)
+int fp6mi_query_launch(int E, int Mb, size_t M, size_t N, size_t K, int splitK, int *shape) { return fp6mi_query_kernel(E, Mb, M, N, K, splitK, 0, shape); }
+
+int fp6mi_launch_source(int E, int Mb, size_t M, size_t N, size_t K, int splitK)
 {
-    if (int rc = fp6mi_query_launch(E, Mb, M, N, K, splitK, shape); rc != FP6MI_OK) return rc;
-    LaunchCfg c = final_cfg(1 + E + Mb, M, N, K, splitK, grouped != 0, current_device_cus());
-    shape[0] = c.kind, shape[1] = c.nt, shape[2] = c.rt, shape[3] = c.wr, shape[4] = c.wk;
-    return FP6MI_OK;
+    int        shape[5];
+    const int  rc = fp6mi_query_launch(E, Mb, M, N, K, splitK, shape);
+    const bool wide = rc == FP6MI_OK && shape[0] == 2 && shape[3] == 4 && shape[4] <= 2; // gemm_wide
+    return rc != FP6MI_OK ? rc : wide ? 2 : fp6mi_query_table(E, Mb, M, N, K, splitK, nullptr);
 }
 
 // ---- allocation-free variant of fp6mi_linear_native: the split-K workspace is a static device array of the library ----

@@ -157,17 +157,20 @@ int fp6mi_linear_native_grouped_cfg(int E, int Mbits, void *stream, const void *
 /* Which kernel shape fp6mi_linear_native would launch for this problem: shape[0..4] = kind, n_tiles, row_tiles,
  * row_waves, k_waves, with the meaning they have in fp6mi_linear_native_cfg.  Pure host code, no GPU needed.  The
  * choice comes from a table measured on the MI355X (python -m fp6_llm_amd.tune) where the problem is near a measured
- * one, else from a rule; it plays the part of the reference's compile-time TilingConfig dispatch
+ * one, else from a rule; from 97 columns on gemm_wide (kind 2 with row_waves 4 and k_waves 1 or 2) takes the place of that
+ * shape where a model of its time says so.  It plays the part of the reference's compile-time TilingConfig dispatch
  * (fp6_llm/csrc/fp6_linear.cu:61-81). */
 int fp6mi_query_launch(int E, int Mbits, size_t M, size_t N, size_t K, int splitK, int *shape);
-/* Where that choice comes from on a 256-CU part: 0 = this (M, K) was measured (at this batch or the next larger measured
- * one), 1 = carried over from measured problems up to a factor 1.5 away in M and in K, 2 = the rules (no measured
- * neighbour, a splitK the table does not hold, or the prefill kernel in the place of the shape that the table would give: its rows
- * do not hold that kernel).  Negative: FP6MI_ERR_*.  (No counterpart in the reference.) */
-int fp6mi_launch_source(int E, int Mbits, size_t M, size_t N, size_t K, int splitK);
-/* The two above report the table and the rules.  From 97 columns on a call is run by gemm_wide instead (launch kind 2 with row_waves 4 and k_waves 1 or 2)
- * where that is expected to be faster: this is the shape that a call launches (grouped: 1 with group exponents).  (No counterpart in the reference.) */
+/* The same with grouped = 1 for fp6mi_linear_native_grouped: group exponents count in gemm_wide's model.  (No counterpart in the reference.) */
 int fp6mi_query_kernel(int E, int Mbits, size_t M, size_t N, size_t K, int splitK, int grouped, int *shape);
+/* Where fp6mi_query_launch's choice comes from on a 256-CU part: 0 = this (M, K) was measured (at this batch or the next larger measured
+ * one), 1 = carried over from measured problems up to a factor 1.5 away in M and in K, 2 = the rules (no measured
+ * neighbour, a splitK the table does not hold, or gemm_wide or the prefill kernel in the place of the shape that the table would give: its
+ * rows do not hold those kernels).  Negative: FP6MI_ERR_*.  (No counterpart in the reference.) */
+int fp6mi_launch_source(int E, int Mbits, size_t M, size_t N, size_t K, int splitK);
+/* The two for the table and the rules alone, before gemm_wide is considered: returns the source and, unless shape is NULL, writes the
+ * shape.  (For the table's own tests and tools; no counterpart in the reference.) */
+int fp6mi_query_table(int E, int Mbits, size_t M, size_t N, size_t K, int splitK, int *shape);
 
 /* Device-side conversion reference layout -> native layout (both device pointers), run once per weight matrix. */
 int fp6mi_relayout_ref_to_native_gpu(int E, int Mbits, void *stream, void *native_dev, const void *packed_ref_dev,

@@ -281,8 +281,11 @@ def test_measured_table_holds_only_compiled_shapes_and_query_launch_follows_it()
                 continue
             assert v[:5] in compiled, (xb, OC, IC, BS, v)
             assert v[0] == 0 or OC % tune.tile_rows(v[:5]) == 0      # (the stream kernel's last workgroup holds what is left of the row tiles)
-            assert L.fp6mi_query_launch(E, Mb, OC, BS, IC, tune.SPLITS[i], shape) == 0
+            assert L.fp6mi_query_table(E, Mb, OC, BS, IC, tune.SPLITS[i], shape) == 0
             assert tuple(shape) == v[:5], (xb, OC, IC, BS, tune.SPLITS[i], tuple(shape), v)
+            assert L.fp6mi_query_launch(E, Mb, OC, BS, IC, tune.SPLITS[i], shape) == 0
+            wide = BS > 96 and shape[0] == 2 and shape[3] == 4 and shape[4] <= 2
+            assert (wide or tuple(shape) == v[:5]) and L.fp6mi_launch_source(E, Mb, OC, BS, IC, tune.SPLITS[i]) == (2 if wide else 0)
     # any legal problem gets a compiled shape that divides its rows, measured neighbour or not
     for (OC, IC, BS, sk) in [(256, 64, 1, 1), (768, 1088, 3, 2), (4352, 4160, 8, 1), (9984, 3008, 40, 3), (65536, 16384, 700, 1), (512, 64, 17, 1)]:
         for (E, Mb) in FORMATS:
@@ -316,7 +319,7 @@ def test_measured_table_holds_only_compiled_shapes_and_query_launch_follows_it()
 ])
 def test_prefill_kernel_rule(OC, IC, N, splitK, prefill):
     shape = (ctypes.c_int * 5)()
-    assert _lib.lib().fp6mi_query_launch(3, 2, OC, N, IC, splitK, shape) == 0
+    assert _lib.lib().fp6mi_query_table(3, 2, OC, N, IC, splitK, shape) >= 0
     assert (tuple(shape) == (2, 8, 4, 2, 2)) == prefill, tuple(shape)
 
 
@@ -636,9 +639,8 @@ def test_launch_source_of_problems_the_prefill_rule_takes():
     L = _lib.lib()
     shape = (ctypes.c_int * 5)()
     for OC, IC, N, prefill in ((28672, 8192, 384, True), (28672, 8192, 512, False), (22016, 4096, 511, True), (4608, 4544, 777, True)):
-        assert L.fp6mi_query_launch(3, 2, OC, N, IC, 1, shape) == 0
+        assert (L.fp6mi_query_table(3, 2, OC, N, IC, 1, shape) == 2) == prefill
         assert (tuple(shape) == (2, 8, 4, 2, 2)) == prefill
-        assert (L.fp6mi_launch_source(3, 2, OC, N, IC, 1) == 2) == prefill
 
 
 def test_wide_kernel_takes_the_place_of_larger_tiles():
@@ -655,11 +657,15 @@ def test_wide_kernel_takes_the_place_of_larger_tiles():
         OC, IC, N = 256 * int(2 ** rng.uniform(0, 7.5)), 64 * int(2 ** rng.uniform(0, 9)), int(2 ** rng.uniform(0, 13.5))
         for splitK in {1, int(rng.integers(1, 12)), fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M)}:
             for grouped in (0, 1):
-                assert L.fp6mi_query_launch(E, M, OC, N, IC, splitK, base) == 0 and L.fp6mi_query_kernel(E, M, OC, N, IC, splitK, grouped, shape) == 0
+                source = L.fp6mi_query_table(E, M, OC, N, IC, splitK, base)
+                assert source >= 0 and L.fp6mi_query_kernel(E, M, OC, N, IC, splitK, grouped, shape) == 0
                 s = tuple(shape)
                 wide = s[0] == 2 and s[3] == 4 and s[4] <= 2
                 assert s in compiled and (s[0] == 0 or OC % tune.tile_rows(s) == 0)
                 assert (wide and N > 96 and splitK <= (IC + 255) // 256) or s == tuple(base)
+                if not grouped:   # the other two queries say the same
+                    assert L.fp6mi_query_launch(E, M, OC, N, IC, splitK, base) == 0 and tuple(base) == s
+                    assert L.fp6mi_launch_source(E, M, OC, N, IC, splitK) == (2 if wide else source)
                 seen.add(s)
     assert {(2, 8, 4, 4, 1), (2, 8, 4, 4, 2), (2, 6, 4, 4, 1), (2, 8, 2, 4, 2), (2, 6, 2, 4, 2), (2, 4, 2, 4, 2)} <= seen
     for OC, IC, N, wide in ((8192, 8192, 96, False), (1536, 1216, 258, False), (28672, 8192, 2048, True), (8192, 1 << 21, 2048, False)):
@@ -916,8 +922,8 @@ def test_a_split_of_the_heuristics_is_launched_by_what_it_was_chosen_for():
             if shape[0] == 2 and ((shape[3] == 4 and shape[4] <= 2) or shape[3] == 2):   # gemm_wide, or gemm_prefill in the place of a shape of the table's
                 cut += split > 1
                 continue
-            if L.fp6mi_launch_source(E, M, OC, N, IC, split) == 2:
-                assert all(L.fp6mi_launch_source(E, M, OC, N, IC, s) == 2 for s in (1, 2, 3, 4, 6, 8)), (E, M, OC, IC, N, split, tuple(shape))
+            if L.fp6mi_query_table(E, M, OC, N, IC, split, None) == 2:
+                assert all(L.fp6mi_query_table(E, M, OC, N, IC, s, None) == 2 for s in (1, 2, 3, 4, 6, 8)), (E, M, OC, IC, N, split, tuple(shape))
     assert cut > 100
 
 
