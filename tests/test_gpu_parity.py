@@ -948,7 +948,7 @@ def test_random_shapes_through_the_automatic_launch_choice(E, M):
         native, scd, xd = upload(raw, sc, x, E, M)
         y = gemm_capi(E, M, native, scd, xd, OC, splitK)
         check_close(y, oracle.gemm_f64(oracle.dequant(raw, sc, E, M), x), "random %d: %dx%d N=%d splitK=%d" % (case, OC, IC, N, splitK))
-        assert L.fp6mi_query_launch(E, M, OC, N, IC, splitK, shape) == 0
+        assert L.fp6mi_query_launch(E, M, OC, N, IC, splitK, shape) == 0   # (what gemm_capi has launched)
         seen.add(tuple(shape))
     assert len(seen) >= 5   # the cases really spread over several kernel shapes
 
@@ -1054,15 +1054,27 @@ def test_device_quantizer_rejects_bad_arguments():
         fp6.weight_quantize_native_cuda(3, 2, torch.zeros(256, 128, dtype=torch.float16))
 
 
-@pytest.mark.parametrize("E,M,OC,IC,BS,splitK", [
-    (3, 2, 256, 256, 1, 1), (2, 3, 256, 320, 7, 1), (2, 2, 1536, 576, 16, 1), (2, 1, 1792, 1728, 3, 2), (3, 2, 5120, 512, 12, 1), (3, 2, 4096, 1024, 24, 1),   # gemm_stream
-    (2, 2, 256, 256, 19, 1), (3, 2, 256, 640, 17, 2), (3, 2, 11008, 1600, 36, 1), (2, 2, 1792, 4224, 66, 8),                                                    # gemm_tile, gemm_ws
-    (2, 2, 512, 256, 2113, 1), (3, 2, 768, 5696, 212, 8), (2, 3, 1024, 320, 200, 4), (2, 2, 23296, 2304, 493, 1)])                                              # gemm_wide, gemm_prefill
+@pytest.mark.parametrize("E,M,OC,IC,BS,splitK,shape", [
+    # gemm_stream
+    (3, 2, 256, 256, 1, 1, (0, 1, 1, 1, 4)), (2, 3, 256, 320, 7, 1, (0, 1, 1, 1, 4)), (2, 2, 1536, 576, 16, 1, (0, 1, 1, 1, 4)), (2, 1, 1792, 1728, 3, 2, (0, 1, 1, 1, 8)),
+    (3, 2, 5120, 512, 12, 1, (0, 1, 2, 1, 4)),
+    # gemm_tile
+    (3, 2, 4096, 1024, 24, 1, (1, 2, 1, 4, 4)), (2, 2, 256, 256, 19, 1, (1, 2, 2, 4, 1)), (3, 2, 256, 640, 17, 2, (1, 2, 2, 4, 2)), (2, 3, 1024, 320, 200, 4, (1, 2, 2, 4, 1)),
+    (2, 2, 512, 256, 2113, 1, (1, 2, 2, 4, 1)),
+    # gemm_ws, gemm_prefill
+    (3, 2, 11008, 1600, 36, 1, (2, 3, 2, 4, 4)), (2, 2, 1792, 4224, 66, 8, (2, 3, 2, 4, 4)), (3, 2, 768, 1472, 536, 1, (2, 2, 2, 8, 4)), (2, 2, 23296, 2304, 493, 1, (2, 8, 4, 2, 2)),
+    # gemm_wide, each tile unsplit, then in pieces
+    (2, 1, 1280, 1472, 389, 1, (2, 4, 2, 4, 2)), (2, 2, 3328, 640, 577, 1, (2, 6, 2, 4, 2)), (3, 2, 8192, 576, 290, 1, (2, 8, 2, 4, 2)), (2, 1, 2560, 64, 1641, 1, (2, 6, 4, 4, 1)),
+    (3, 2, 22784, 64, 194, 1, (2, 8, 4, 4, 1)), (2, 2, 22528, 320, 199, 1, (2, 8, 4, 4, 2)),
+    (3, 2, 768, 5696, 212, 8, (2, 4, 2, 4, 2)), (2, 1, 2304, 1664, 287, 3, (2, 6, 2, 4, 2)), (2, 1, 1024, 640, 1099, 3, (2, 8, 2, 4, 2)), (2, 3, 1280, 832, 1105, 3, (2, 6, 4, 4, 1)),
+    (2, 3, 1536, 960, 1363, 3, (2, 8, 4, 4, 1)), (2, 2, 1536, 1088, 1392, 3, (2, 8, 4, 4, 2))])
 @pytest.mark.parametrize("groups", [False, True])
-def test_bias_in_the_epilogues(E, M, OC, IC, BS, splitK, groups):
+def test_bias_in_the_epilogues(E, M, OC, IC, BS, splitK, shape, groups):
     """Every kernel's epilogue and both reductions add a bias (on a 2-byte boundary) to the float32 sums: the result is within half an fp16 step of the
     sum in float64 plus what IC float32 additions may lose, and a bias of zeros changes no bit."""
     print("case bias", E, M, OC, IC, BS, splitK, groups, flush=True)
+    launched = (ctypes.c_int * 5)()
+    assert _lib.lib().fp6mi_query_kernel(E, M, OC, BS, IC, splitK, groups, launched) == 0 and tuple(launched) == shape
     gen = torch.Generator().manual_seed(OC + IC + BS)
     native, sc, *rest = fp6.weight_quantize_native_cuda(E, M, (torch.randn(OC, IC, generator=gen) * 0.02).half().to(DEV), groups)
     exps = rest[0] if rest else None
@@ -1280,17 +1292,21 @@ def test_grouped_gemm_on_the_256x128_tile(E, M):
     """A prefill-sized batch: the 256 x 128 tile, which spreads its loads (the group exponents among them) over the MFMA steps;
     K = 1088 ends in a quarter-full K block.  Checked on a sample of rows against the definition."""
     OC, IC, BS = 2048, 1088, 4096
-    shape = (ctypes.c_int * 5)()
-    assert _lib.lib().fp6mi_query_launch(E, M, OC, BS, IC, 1, shape) == 0 and tuple(shape) == (1, 8, 2, 8, 1)
+    cfg, L, stream = (1, 8, 2, 8, 1), _lib.lib(), torch.cuda.current_stream().cuda_stream   # (launched by its shape: the dispatch takes gemm_wide for such a batch)
     codes, sc, ex = quant.quantize_groupwise(_grouped_weights(77, OC, IC), E, M)
     native = fp6.weight_prepacking_native_cpu(E, M, torch.from_numpy(quant.pack_raw(codes, E, M))).to(DEV)
     gexp = fp6.pack_group_exps(torch.from_numpy(ex), OC, IC).to(DEV)
     scd = torch.from_numpy(sc).to(DEV)
     x = synth.activations(78, BS, IC)
     xd = torch.from_numpy(x).to(DEV)
-    y = fp6.linear_forward_native(E, M, xd, native, scd, OC, 1, group_exps=gexp).cpu().numpy()
-    y_plain = fp6.linear_forward_native(E, M, xd, native, scd, OC, 1, group_exps=torch.full_like(gexp, 127))
-    assert torch.equal(y_plain, fp6.linear_forward_native(E, M, xd, native, scd, OC, 1))
+
+    def run(exps):
+        out = torch.full((BS, OC), float("nan"), dtype=torch.float16, device=DEV)
+        rc = L.fp6mi_linear_native_grouped_cfg(E, M, stream, native.data_ptr(), scd.data_ptr(), exps.data_ptr(), xd.data_ptr(), out.data_ptr(), OC, BS, IC, None, 1, *cfg)
+        assert rc == 0, L.fp6mi_error_string(rc)
+        return out.cpu().numpy()
+    y = run(gexp)
+    assert np.array_equal(run(torch.full_like(gexp, 127)), gemm_capi(E, M, native, scd, xd, OC, 1, cfg))
     rows = np.sort(np.random.default_rng(6).choice(OC, 192, replace=False))
     wdq = oracle.dequant_grouped_from_definition(codes[rows], sc[rows], ex[rows], E, M)
     check_close(y[:, rows], oracle.gemm_f64(wdq, x), "grouped, 256x128 tile")
