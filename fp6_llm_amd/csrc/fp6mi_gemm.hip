@@ -1565,7 +1565,7 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 // residual turns q into the quotient rounded to odd (truncated, last bit set if inexact), which never sits on a midpoint.
 //
 // HBM-bound but for its arithmetic, which does not hide: a chip's worth of workgroups loads, finds its maxima and converts in step.  Clamps, NaN tests and
-// sign handling made that 10 operations a weight (17 us of 46 at 8192x8192); they are left to a second pass of the wavefronts that have met an Inf, a NaN or a
+// sign handling made that 10 operations a weight (17 us of 46 at 8192x8192); they are left to the wavefronts that have met an Inf, a NaN or a
 // scale that is no normal number, the others take 5 (quantize_string's PLAIN).  us, e3m2, before -> now, row scales and group exponents: bf16 8192x8192
 // 45.9 -> 41.9, 49.6 -> 44.0; 3072x8192 23.5 -> 18.9, 26.1 -> 20.7; 28672x8192 141 -> 136, 142 -> 137; 8192x28672 176 -> 165, 183 -> 176; fp16 8192x8192
 // 47.1 -> 43.1, 51.6 -> 45.2; fp32 8192x8192 95.2 -> 87.6, 98.7 -> 91.9.
@@ -1878,31 +1878,37 @@ __global__ __launch_bounds__(WAVES *kWave, sizeof(T) == 2 ? WAVES / 2 : 1) void 
     }
     __syncthreads();
     const float sc = (float)tile_scale[lane >> 2];
+    // Both arithmetics at every block, chosen before it: a slow pass of its own over all blocks, behind the fast one, cost a wavefront a second reading of its weights
+    // where one row of 16 has a scale below 2^-14.  us, e3m2, such a row in every tile, before the two arithmetics / with that pass / now: bf16 8192x8192
+    // 45.8 / 65.4 / 45.4, 28672x4096 63.1 / 104 / 64.9; fp32 8192x8192 101 / 144 / 98.5; a NaN in every tile, bf16 8192x8192 45.9 / 51.4 / 46.5.
+    const bool plain = !special && plain_scales(sc); // (uniform)
+    auto       convert = [&](const WeightPiece<T>(&x)[8], uint32_t U) __attribute__((always_inline)) {
+        if (plain) {
+            quantize_block<FM, T, GROUPS, true>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+        } else if constexpr (GROUPS || sizeof(T) != 2) {
+            quantize_block<FM, T, GROUPS, false>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+        } else { // (opaque copies: what both would widen alike is kept from being widened ahead of the branch, into registers that the held blocks need)
+            WeightPiece<T> y[8];
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                y[s] = x[s];
+                asm volatile("" : "+v"(y[s].x));
+            }
+            quantize_block<FM, T, GROUPS, false>(y, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+        }
+    };
 #pragma unroll
     for (int k = 0; k < KEEP; k++)
-        if ((uint32_t)k < mine) {
-            const uint32_t U = wave + (mine - 1 - k) * WAVES;
-            quantize_block<FM, T, GROUPS, true>(kept[k], sc, native, gexp, (size_t)R * units + U, K, U, lane);
-        }
+        if ((uint32_t)k < mine) convert(kept[k], wave + (mine - 1 - k) * WAVES);
     if (stash) {
         WeightPiece<T> x[8];
-        const uint32_t U = wave + (mine - 1 - KEEP) * WAVES;
         stashed(x);
-        quantize_block<FM, T, GROUPS, true>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
+        convert(x, wave + (mine - 1 - KEEP) * WAVES);
     }
     for (uint32_t i = mine > held ? mine - held : 0; i-- > 0;) {
         WeightPiece<T> x[8];
-        const uint32_t U = wave + i * WAVES;
-        load_quant_block<T>(x, w, K, U, lane);
-        quantize_block<FM, T, GROUPS, true>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
-    }
-    if (special || !plain_scales(sc)) { // again over what was just written (last, where nothing is held any more: before the fast pass it would spill)
-#pragma unroll 1
-        for (uint32_t U = wave; U < units; U += WAVES) {
-            WeightPiece<T> x[8];
-            load_quant_block<T>(x, w, K, U, lane);
-            quantize_block<FM, T, GROUPS, false>(x, sc, native, gexp, (size_t)R * units + U, K, U, lane);
-        }
+        load_quant_block<T>(x, w, K, wave + i * WAVES, lane);
+        convert(x, wave + i * WAVES);
     }
 }
 

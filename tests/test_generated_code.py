@@ -135,3 +135,21 @@ def test_wave_specialized_kernels_of_128_rows_hold_no_exponents_in_registers(tmp
     for name, code in kernels.items():
         assert any(c.startswith("global_load_lds_ushort") for c in code), name
         assert not any(re.match(r"(global|flat|buffer)_load_[us]short", c) for c in code), name
+
+
+def test_quantizer_chooses_its_arithmetic_before_a_block(tmp_path_factory):
+    """quant_fused holds both arithmetics at each place where it converts a block (two strings each).  The general one once followed the fast one in a pass
+    of its own, so that a row with a subnormal scale had its tile read and converted twice.  Registers that do not suffice go to scratch memory in the
+    general one alone: between two conversions of the fast one there is no scratch access."""
+    kernels = instructions(tmp_path_factory, "quant_fused")
+    assert len(kernels) == 24, sorted(kernels)   # four formats, three types of weights, with and without group exponents
+    for name, code in kernels.items():
+        conversions = [i for i, c in enumerate(code) if c.startswith("v_cvt_scalef32_2xpk16")]
+        places = 3 if "ILi" in name and re.search(r"ELi8ELi2E", name) and "EfLb" in name else 4   # two blocks in registers, one in LDS (16-bit weights), the others
+        assert len(conversions) == places * 2 * 2, (name, len(conversions))
+        scratch = [i for i, c in enumerate(code) if c.startswith("scratch")]
+        assert len(scratch) <= 8, name
+        for i in scratch:   # the conversion that follows a store or stands around a reload has the general arithmetic's clamps ahead of it
+            after = next(j for j in conversions if j > i)
+            before = max([j for j in conversions if j < i], default=max(0, after - 400))
+            assert sum(c.startswith("v_min") for c in code[before:after]) >= 16, (name, i)
