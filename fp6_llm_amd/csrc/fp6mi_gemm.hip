@@ -162,8 +162,9 @@ template <int FM, bool GS> __device__ __forceinline__ void convert(const WFrag<F
 }
 
 // `ws` of the GEMM kernels: the partial sums where K is split (splitk_reduce adds a bias then), else an fp16 bias [M] on any 2-byte boundary or null, which
-// the epilogue adds to the float32 sums.  gemm_stream has instances of its own for it: a branch in the epilogue that no launch took cost it 0.04-0.1 us (1 % of
-// 4096x4096 N 8).  Instead of an addition behind the GEMM, us, e3m2, replayed: 4096x4096 N 1 6.1 -> 4.4, N 8 7.6 -> 5.0; 8192x8192 N 16 15.7 -> 12.9,
+// the epilogue adds to the float32 sums.  gemm_stream and gemm_tile have instances of their own for it: a branch in the epilogue that no launch took cost the one 0.04-0.1 us (1 % of
+// 4096x4096 N 8), the other a register or two, in some instances spilled, and 0.2-0.5 % of calls of 5 us.  The kernels of larger tiles branch (gemm_ws +0.0-0.6 % on calls of
+// 9-20 us, as much as two builds of the same instructions differ by).  Instead of an addition behind the GEMM, us, e3m2, replayed: 4096x4096 N 1 6.1 -> 4.4, N 8 7.6 -> 5.0; 8192x8192 N 16 15.7 -> 12.9,
 // N 72 25.9 -> 22.1; 28672x8192 N 2048 680 -> 657.
 template <typename P> __device__ __forceinline__ const half_t *bias_of(P ws) { return reinterpret_cast<const half_t *>(ws); }
 
@@ -720,7 +721,7 @@ template <int TM, int TN> __device__ __forceinline__ TileId tile_of(uint32_t spl
     return TileId{ rest / splitK, rest % splitK, id % nblocks };
 }
 
-template <int FM, bool GS, int NT, int RT, int WR, int WK>
+template <int FM, bool GS, int NT, int RT, int WR, int WK, bool BIAS>
 __global__ __launch_bounds__(WR *WK *kWave) void gemm_tile(const uint8_t *__restrict__ W, const half_t *__restrict__ scales,
                                                            const uint8_t *__restrict__ gexp, const half_t *__restrict__ X, half_t *__restrict__ C,
                                                            float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
@@ -765,8 +766,8 @@ __global__ __launch_bounds__(WR *WK *kWave) void gemm_tile(const uint8_t *__rest
     // the output tile is parked where the partial sums of the K wavefronts met: everybody has read those first
     if (WK > 1) __syncthreads();
     uint8_t *stage = lds;
-    if (splitK == 1)
-        tile_store<FM, NT, RT, WR, NTHREADS>(acc, sc4, C, stage, wk == 0, M, N, mb, nbase, tid, wr, col, q, ws ? bias_of(ws) + mb * (WR * RT * 16) : nullptr);
+    if (BIAS || splitK == 1) // (a split's bias is added by the reduction)
+        tile_store<FM, NT, RT, WR, NTHREADS>(acc, sc4, C, stage, wk == 0, M, N, mb, nbase, tid, wr, col, q, BIAS ? bias_of(ws) + mb * (WR * RT * 16) : nullptr);
     else
         tile_store<FM, NT, RT, WR, NTHREADS>(acc, sc4, ws + (size_t)split * N * M, stage, wk == 0, M, N, mb, nbase, tid, wr, col, q, nullptr);
 }
@@ -2011,15 +2012,21 @@ int launch_tile(hipStream_t st, const void *W, const void *sc, const void *gexp,
     static_assert(kMaxLds <= 160 * 1024, "tile does not fit in LDS");
     const size_t out_bytes = tile_stage_bytes<NT, RT, WR>(splitK > 1), lds_bytes = kLoopLds > out_bytes ? kLoopLds : out_bytes;
     if (M % TM) return FP6MI_ERR_SHAPE;
-    if (kMaxLds > 48 * 1024)
-        if (int rc = allow_dynamic_lds<&gemm_tile<FM, GS, NT, RT, WR, WK>>(kMaxLds)) return rc;
     uint32_t units = (uint32_t)((K + 255) / 256), nblocks = (uint32_t)((N + TN - 1) / TN);
     size_t   wgs = (M / TM) * (size_t)splitK * nblocks;
     if (wgs > 0x7fffffffu) return FP6MI_ERR_SHAPE;
-    hipLaunchKernelGGL((gemm_tile<FM, GS, NT, RT, WR, WK>), dim3((uint32_t)wgs), dim3(WR * WK * kWave), lds_bytes, st,
-                       static_cast<const uint8_t *>(W), static_cast<const half_t *>(sc), static_cast<const uint8_t *>(gexp), static_cast<const half_t *>(B),
-                       static_cast<half_t *>(C), ws, (uint32_t)M, (uint32_t)N, (uint32_t)K, units, (uint32_t)splitK, nblocks);
-    return (int)hipGetLastError();
+    auto go = [&](auto kernel_c) -> int {
+        constexpr auto kernel = decltype(kernel_c)::value;
+        if (kMaxLds > 48 * 1024)
+            if (int rc = allow_dynamic_lds<kernel>(kMaxLds)) return rc;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)wgs), dim3(WR * WK * kWave), lds_bytes, st, static_cast<const uint8_t *>(W), static_cast<const half_t *>(sc),
+                           static_cast<const uint8_t *>(gexp), static_cast<const half_t *>(B), static_cast<half_t *>(C), ws, (uint32_t)M, (uint32_t)N, (uint32_t)K,
+                           units, (uint32_t)splitK, nblocks);
+        return (int)hipGetLastError();
+    };
+    typedef decltype(&gemm_tile<FM, GS, NT, RT, WR, WK, false>) Kernel;
+    if (ws && splitK == 1) return go(std::integral_constant<Kernel, &gemm_tile<FM, GS, NT, RT, WR, WK, true>>{});
+    return go(std::integral_constant<Kernel, &gemm_tile<FM, GS, NT, RT, WR, WK, false>>{});
 }
 template <int FM, bool GS, int NT, int RT, int WR, int PW, int SW, int SX>
 int launch_ws(hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, float *ws, size_t M, size_t N, size_t K,
