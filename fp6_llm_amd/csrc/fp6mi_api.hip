@@ -432,10 +432,10 @@ inline float narrow_estimate(const TuneAnswer *a, size_t M, size_t N, int splitK
 
 // Whether gemm_wide, expected to take t us, takes the place of the table's shape, expected to take `narrow` (0: not in the table's reach, K below 1366 for
 // the most part; there it is a matter of the outputs, of which the rules' smaller tiles serve few better: 1536x1216 N 258 5.4 us against 7.3,
-// 3072x1024 N 2867 26.0 against 22.5).  Time after / before on 849 problems drawn as above, the split chosen anew: N 97-160 1.00 (0.75-1.01), N 161-256 0.98
-// (0.80-1.07), N 257-400 0.90 (0.50-1.13), N 401-640 0.84 (0.48-1.03), beyond 0.83 (0.46-1.06); N 65-96 1.00, not worth it.  The margins are what the two
-// estimates are off where the kernels are close, and allow for the table's, which is low, where they are not: without them 40 of these problems were more than
-// 2 % slower, with them 5.
+// 3072x1024 N 2867 26.0 against 22.5).  Time after / before on 500 problems that no line was drawn on (M and K 1024-28672, group exponents on 30 %, the split chosen anew):
+// N 97-160 0.99 (0.84-1.03), N 161-256 0.98 (0.81-1.07), N 257-400 0.91 (0.60-1.02), N 401-640 0.85 (0.50-1.01), beyond 0.84 (0.36-1.04), 5 of all over 1.02 (16640x2752
+// N 186 with group exponents 1.07); N 65-96 1.00, not worth it.  The margins are what the two estimates are off where the kernels are close, and allow for the
+// table's, which is low, where they are not: of 849 problems that they were drawn on 40 were over 1.02 without them, 5 with them.
 // The tile of 64 columns has the smallest margin whatever N is: on 175 problems beyond N 640 it took with 1.15 (1024x6144 N 1848, 2560x19904 N 3224) it was 1.00
 // (0.56-1.28), 71 of them over 1.02; with 0.9 it takes 44 of them at 0.91 and 4 are over 1.02 (9472x17024 N 1984 in FP4 1.28, the others up to 1.03); on 34 problems of N 401-640 as good as with 0.95, 1 over 1.02 for 5.
 // Out of the table's reach K up to 512 takes 2^22 outputs: 23 problems below that took 1.02 of the time of the rules' tiles (0.90-1.22: 5632x256 N 325 4.9 us -> 5.9);
@@ -539,7 +539,7 @@ const char *fp6mi_tuning_info(void)
         ;
 }
 
-int fp6mi_version(void) { return 139; } // 139: a bias in the epilogues of the GEMM kernels, the quantizer's arithmetic; 138: gemm_wide (launch kind 2 with four rows of one or two wavefronts) in the place of larger tiles from 97 columns on, the other kernels unchanged; 137: group exponents of 128 rows through LDS in the wave-specialized kernel, panels of 256-row tiles only for activations beyond L2; 136: tiles of 48, 80 and 96 columns, deeper rings in the wave-specialized kernel of 128 rows, panels; 135: prefill kernel (launch kind 2 with 2 x 2 wavefronts), relayout and quantizer kernels rewritten, the other GEMM kernels unchanged; 134: three row tiles per workgroup in the small-batch kernel (any M: the last workgroup takes what is left), no other kernel changed; 133: wave-specialized tile kernel (launch kind 2) for large batches; 132: split-K reduction runs on the XCD that wrote the partial sums, every grid size gets XCD-contiguous tiles; 131: tile kernel stores through LDS; 130: small-batch kernel loads activations as whole rows and turns them into operand order through LDS
+int fp6mi_version(void) { return 140; } // 140: where gemm_wide is taken and with which splits, instances of gemm_tile for a bias, the quantizer chooses its arithmetic before a block; 139: a bias in the epilogues of the GEMM kernels, the quantizer's arithmetic; 138: gemm_wide (launch kind 2 with four rows of one or two wavefronts) in the place of larger tiles from 97 columns on, the other kernels unchanged; 137: group exponents of 128 rows through LDS in the wave-specialized kernel, panels of 256-row tiles only for activations beyond L2; 136: tiles of 48, 80 and 96 columns, deeper rings in the wave-specialized kernel of 128 rows, panels; 135: prefill kernel (launch kind 2 with 2 x 2 wavefronts), relayout and quantizer kernels rewritten, the other GEMM kernels unchanged; 134: three row tiles per workgroup in the small-batch kernel (any M: the last workgroup takes what is left), no other kernel changed; 133: wave-specialized tile kernel (launch kind 2) for large batches; 132: split-K reduction runs on the XCD that wrote the partial sums, every grid size gets XCD-contiguous tiles; 131: tile kernel stores through LDS; 130: small-batch kernel loads activations as whole rows and turns them into operand order through LDS
 
 int fp6mi_prepack_ref(int E, int Mb, void *packed, const void *raw, size_t M, size_t K) { return fp6mi::prepack_ref(E, Mb, packed, raw, M, K); }
 int fp6mi_unpack_ref(int E, int Mb, void *raw, const void *packed, size_t M, size_t K) { return fp6mi::unpack_ref(E, Mb, raw, packed, M, K); }

@@ -1216,8 +1216,9 @@ __global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, c
 // ---------------------------------------------------------------------------------------------------------------
 // gemm_wide: the tile GEMM of large batches, wavefronts one below the other across the whole width of the tile.
 //   workgroup = 4 x WK wavefronts; tile = (4*RT*16) rows x (NT*16) columns, (RT*16) x (NT*16) of it per wavefront; grid as gemm_tile
-// A chip full of MFMAs is held by its power, not by its clock: registers only, 16x16x32 MFMAs of random halfs run at 1.84-1.93 GHz = 1.73-1.96 PFLOP/s
-// (32x32x16 ones at 1.72 GHz = 1.74), with one conversion for every 16 of them 1.70, for every 8 1.54.  What a GEMM gets is then a matter of what
+// A chip full of MFMAs is held by its power, not by its clock: registers only, 16x16x32 MFMAs of zeros run at 2.39 GHz = 2.47 PFLOP/s, of random halfs at 1.78-1.93 GHz =
+// 1.73-1.96, with one conversion for every 32 of them 1.79 PFLOP/s, for every 16 1.65, for every 8 1.38 (32x32x16 ones of random halfs at 1.56-1.73 GHz); and in 28672x8192
+// N 2048 gemm_tile keeps the MFMAs busy for 0.57 of its cycles at 2.0 GHz, gemm_prefill 0.64 at 1.75, this kernel 0.75 at 1.57.  What a GEMM gets is then a matter of what
 // it does beside them: conversions (64 cycles each, in which the SIMD starts no MFMA), operand reads from LDS, bytes from L2.  Here
 //   * a converted fragment meets all NT column tiles: NT = 8 has one conversion per 32 MFMAs, where gemm_prefill, gemm_ws and 256 x 64 tiles have one per 16;
 //   * a B operand read feeds RT row tiles: 4 in the 256-row tiles, where gemm_tile and gemm_ws have 2;
@@ -1590,7 +1591,7 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 //   4096x28672   85.8 /  89.4    89.9 /  89.6   164 / 180       168 / 180
 //  16384x4096    37.2 /  53.6    38.8 /  53.7    72.2 /  93.6    76.1 /  93.8
 // Few workgroups do not pull enough from memory to pay for a second pass over a long row: fused from 160 tiles on, and below that up to K = 3072 or three
-// times the rows.  On the wrong side of that line group exponents of 2816x16384 (6 %) and, in fp32, 8192x8192 (4 %) and 1024x3072 (4 %).
+// times the rows.  On the wrong side of that line bf16 of 1024x4096 (9 %) and 2048x8192 (4 %), group exponents of 2816x16384 (6 %) and, in fp32 with them, 8192x8192 (4 %) and 1024x3072 (4 %).
 // (A block of every wavefront in LDS and two in registers leave room for two workgroups to a CU.  Three in registers and one in LDS, nothing read
 // twice at 8192 columns, were slower with one workgroup to a CU, and held to 128 registers they spill.)
 // A conversion in double precision, code by code through a byte array in scratch memory, took 532 us at 8192x8192.
@@ -2095,7 +2096,7 @@ int launch_wide(hipStream_t st, const void *W, const void *sc, const void *gexp,
     return (int)hipGetLastError();
 }
 // kind 0: gemm_stream (wr == 1, wk = wavefronts per workgroup);  kind 1: gemm_tile (wr x wk wavefronts);  kind 2: gemm_ws (wr arithmetic + wk loading wavefronts),
-// or with wr = wk = 2 gemm_prefill (2 x 2 wavefronts; nt = column tiles of the whole workgroup, rt = row tiles per wavefront)
+// with wr = wk = 2 gemm_prefill (2 x 2 wavefronts; nt = column tiles of the whole workgroup, rt = row tiles per wavefront), with wr = 4 and wk = 1 or 2 gemm_wide (wk: parts of K)
 template <int FM, bool GS>
 int launch_cfg(const LaunchCfg &c, hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, float *ws, size_t M,
                size_t N, size_t K, int splitK)

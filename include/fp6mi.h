@@ -142,7 +142,8 @@ int fp6mi_linear_stateless(int E, int Mbits, void *stream, const void *W_ref, co
  * kind 1 = tile kernel (row_waves x k_waves wavefronts, activations staged in LDS),
  * kind 2 = wave-specialized tile kernel (row_waves arithmetic wavefronts; k_waves = 4 loading wavefronts that move weights and
  *          activations into LDS for them); row_waves = k_waves = 2: the prefill kernel (2 x 2 wavefronts, weights straight to
- *          registers, K <= 2^20);
+ *          registers, K <= 2^20); row_waves = 4 with k_waves = 1 or 2: the wide kernel (4 wavefronts one below the other for all of a K
+ *          block or for each half of it, K <= 2^20);
  * n_tiles = 16-column batch tiles per workgroup, row_tiles = 16-row weight tiles per wavefront.
  * Combinations that are not compiled in, or that do not divide M, return FP6MI_ERR_SHAPE. */
 int fp6mi_linear_native_cfg(int E, int Mbits, void *stream, const void *W_native, const void *scales_f16,
