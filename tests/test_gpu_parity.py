@@ -1057,7 +1057,7 @@ def test_device_quantizer_rejects_bad_arguments():
 @pytest.mark.parametrize("E,M,OC,IC,BS,splitK,shape", [
     # gemm_stream
     (3, 2, 256, 256, 1, 1, (0, 1, 1, 1, 4)), (2, 3, 256, 320, 7, 1, (0, 1, 1, 1, 4)), (2, 2, 1536, 576, 16, 1, (0, 1, 1, 1, 4)), (2, 1, 1792, 1728, 3, 2, (0, 1, 1, 1, 8)),
-    (3, 2, 5120, 512, 12, 1, (0, 1, 2, 1, 4)),
+    (3, 2, 5120, 512, 12, 1, (0, 1, 2, 1, 4)), (3, 2, 10496, 512, 8, 1, (0, 1, 3, 1, 4)), (3, 2, 28160, 320, 9, 1, (0, 1, 7, 1, 4)), (3, 2, 11008, 4096, 24, 1, (0, 2, 3, 1, 8)),
     # gemm_tile
     (3, 2, 4096, 1024, 24, 1, (1, 2, 1, 4, 4)), (2, 2, 256, 256, 19, 1, (1, 2, 2, 4, 1)), (3, 2, 256, 640, 17, 2, (1, 2, 2, 4, 2)), (2, 3, 1024, 320, 200, 4, (1, 2, 2, 4, 1)),
     (2, 2, 512, 256, 2113, 1, (1, 2, 2, 4, 1)),
