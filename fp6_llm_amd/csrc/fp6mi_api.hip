@@ -375,6 +375,11 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
 // up to 600; 6, 5 and 4 bits; group exponents on 30 %; weights and activations changed from launch to launch, splits 1, 2, 3, 4, 6 and 8): 4-7 % off a single
 // time, the smallest tiles most.  The shape and split that come out smallest are 0.8 % behind the best of these shapes on average, with a constant term, rates
 // and splits only 1.1 %.
+// gemm_span's tiles (odd widths, and 256 x 96 with the halves of K side by side) were fitted later, to 252 problems of N 97-1500 on which all twelve were measured (4-5 %
+// off; what group exponents cost was taken from their neighbours).  They are asked from K 1024 up to N 3072, what lies beyond not having been measured (128 x 48 up to N 600:
+// beyond, shapes of the table whose place it took were up to 11 % ahead of it), and have to be 2.5 % ahead of gemm_wide's, with a split or K below 1536 4 %: on those
+// problems 118 of 250 choices fell to them at a margin of 2 %, time / time of gemm_wide's best 0.93, 3 over 1.02; without a margin 150, 0.94, 7 over 1.02 and up to 1.11.
+// On 260 problems that no line was drawn on (N 97-4096, group exponents on 30 %) 69 calls changed: 0.94 (0.79-1.02) of the time before, with group exponents 0.93.
 struct WideShape {
     int   nt, rt, wk, slots;              // column tiles, row tiles per wavefront, K halves; workgroups that 256 CUs hold
     float full, full_k, full_kg;          // a full round: us, us per column of K, the same with group exponents on top
@@ -384,9 +389,15 @@ struct WideShape {
     float split, split_out;               // a split's second launch, and its partial sums per million of them
 };
 constexpr WideShape kWide[] = {
+    { 3, 2, 2, 512, 0.f, 0.00481f, 0.0004f, 0.419f, 0.00315f, 0.000117f, 0.00013f, 0.000505f, 0.000437f, 1.77f, 0.262f, 0.0942f, 0.879f, 2.29f, 1.69f },
     { 4, 2, 2, 512, 0.64f, 0.00565f, 0.000445f, 0.779f, 0.0034f, 0.00017f, 0.000127f, 0.000512f, 0.000543f, 1.26f, 0.353f, 0.0607f, 0.85f, 2.89f, 1.35f },
+    { 5, 2, 2, 256, 0.818f, 0.00446f, 0.0003f, 1.59f, 0.00369f, 0.000268f, 0.0002f, 0.000214f, 0.000416f, 1.55f, 0.303f, 0.0898f, 0.462f, 1.89f, 1.59f },
+    { 5, 4, 2, 256, 1.71f, 0.00656f, 0.000388f, 1.76f, 0.00553f, 0.000671f, 0.000812f, 0.000938f, 0.000901f, 2.78f, 0.074f, 0.0772f, 0.627f, 2.98f, 1.47f },
     { 6, 2, 2, 256, 2.3f, 0.00496f, 0.000302f, 1.35f, 0.004f, 0.000994f, 0.000294f, 0.000379f, 0.000471f, 1.46f, 0.346f, 0.0541f, 0.205f, 2.77f, 0.936f },
     { 6, 4, 1, 512, 0.f, 0.0145f, 0.000878f, 0.0154f, 0.00811f, 0.000511f, 0.00109f, 0.000564f, 0.000919f, 3.3f, 0.144f, 0.0501f, 0.475f, 3.8f, 1.12f },
+    { 6, 4, 2, 256, 3.7f, 0.00801f, 0.000388f, 4.22f, 0.00596f, 0.00166f, 0.000812f, 0.000649f, 0.000689f, 1.73f, 0.0414f, 0.0428f, 0.288f, 2.95f, 1.19f },
+    { 7, 2, 2, 256, 1.9f, 0.00514f, 0.000315f, 2.78f, 0.00393f, 0.000609f, 0.00034f, 0.000385f, 0.000465f, 1.09f, 0.374f, 0.0979f, 0.328f, 1.87f, 1.37f },
+    { 7, 4, 2, 256, 3.24f, 0.00918f, 0.000388f, 4.28f, 0.00669f, 0.00179f, 0.000812f, 0.000591f, 0.000692f, 1.68f, 0.0537f, 0.0378f, 0.299f, 3.07f, 1.2f },
     { 8, 2, 2, 256, 3.11f, 0.00552f, 0.000329f, 1.13f, 0.00458f, 0.00138f, 0.000385f, 0.000557f, 0.000652f, 1.93f, 0.272f, 0.0636f, 0.0816f, 2.61f, 1.11f },
     { 8, 4, 1, 512, 0.f, 0.0187f, 0.000715f, 0.434f, 0.00994f, 0.000692f, 0.00107f, 0.0006f, 0.00103f, 3.6f, 0.119f, 0.0321f, 0.458f, 3.81f, 1.15f },
     { 8, 4, 2, 256, 3.85f, 0.0102f, 0.000388f, 2.21f, 0.00798f, 0.00154f, 0.000812f, 0.000575f, 0.000692f, 3.05f, 0.119f, 0.021f, 0.325f, 3.17f, 1.19f },
@@ -411,7 +422,9 @@ inline float wide_best(LaunchCfg &c, int xbits, size_t M, size_t N, size_t K, in
     float best = 0.f;
     if (N <= 96 || K > (size_t)1 << 20 || (size_t)splitK > (K + 255) / 256) return best;
     for (const WideShape &w : kWide) {
-        const float t = wide_estimate(w, xbits, M, N, K, splitK, groups);
+        const bool  span = w.nt % 2 || (w.nt == 6 && w.rt == 4 && w.wk == 2); // gemm_span's: see kWide
+        const float t = wide_estimate(w, xbits, M, N, K, splitK, groups) * (!span ? 1.f : splitK > 1 || K < 1536 ? 1.04f : 1.025f);
+        if (span && (K < 1024 || N > (w.nt == 3 ? 600 : 3072))) continue;
         if (best == 0.f || t < best) best = t, c = LaunchCfg{ 2, w.nt, w.rt, 4, w.wk };
     }
     return best;
@@ -444,7 +457,7 @@ inline bool wide_replaces(const LaunchCfg &wide, float t, float narrow, size_t M
 {
     if (t <= 0.f) return false;
     if (narrow <= 0.f) return M * N >= (size_t)1 << (K <= 512 ? 22 : 20);
-    return t < narrow * (N <= 400 || wide.nt == 4 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
+    return t < narrow * (N <= 400 || wide.nt <= 5 && wide.rt == 2 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
 }
 
 // The fastest split of the table's (3 % hysteresis towards fewer pieces) and its time in us; 0 where it holds none.  One that takes more than ws_bytes has to be

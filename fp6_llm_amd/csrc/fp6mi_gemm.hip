@@ -3,8 +3,8 @@
 // exports one table of entry functions (fp6mi::FormatOps) that the C ABI in fp6mi_api.hip dispatches to.
 //
 // Roles taken over from the reference (usyd-fsalab/fp6_llm, paths relative to it):
-//   gemm_stream, gemm_tile, gemm_ws, gemm_prefill <- QUANT_GEMM_Kernel   fp6_llm/csrc/include/kernel_matmul.cuh:29-191
-//                    (small batches / batches above 16 / large batches, the last two: four organisations of the same GEMM)
+//   gemm_stream, gemm_tile, gemm_ws, gemm_prefill, gemm_wide, gemm_span <- QUANT_GEMM_Kernel   fp6_llm/csrc/include/kernel_matmul.cuh:29-191
+//                    (small batches / batches above 16 / large batches, the last four: five organisations of the same GEMM)
 //   splitk_reduce <- SplitK_Reduction         fp6_llm/csrc/include/kernel_reduction.cuh:28-47   (in fp6mi_api.hip)
 //   launchers     <- fpx_linear_kernel        fp6_llm/csrc/fp6_linear.cu:44-102
 // The design is not a translation: weights use the native layout described in fp6mi_host.cpp, go from HBM straight
@@ -1238,11 +1238,11 @@ __global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, c
 // bytes takes 36 us).
 // ---------------------------------------------------------------------------------------------------------------
 template <int FM, bool GS, int NT, int RT, int WK>
-__global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X,
-                                                            half_t *__restrict__ C, float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
-                                                            uint32_t units, uint32_t splitK, uint32_t nblocks)
+__device__ __forceinline__ void wide_tile(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X, half_t *__restrict__ C,
+                                          float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K, uint32_t units, uint32_t splitK, uint32_t nblocks)
 {
-    constexpr int TM = 4 * RT * 16, TN = NT * 16, kStage = TN * 256, NH = NT / 2, NTHREADS = 4 * WK * kWave;
+    constexpr int TM = 4 * RT * 16, TN = NT * 16, kStage = TN * 256, NTHREADS = 4 * WK * kWave;
+    constexpr int NA = (NT + 1) / 2, NB = NT / 2; // column tiles of the first and of the second half step
     constexpr int kDma = TN / 16; // transfers of 1 KB (four rows) per wavefront and chunk
     // loads a wavefront issues for certain after its last transfer of a chunk and before the chunk's barrier
     constexpr int kRawLoads = (Fmt<FM>::bits == 4 ? 1 : 2) + (GS ? 1 : 0), kAfterDma = RT * kRawLoads;
@@ -1271,7 +1271,7 @@ __global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(
     const uint32_t tile_stride = units * Fmt<FM>::block_bytes; // 32 bits: the launcher bounds K
     const auto     wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W + (size_t)R0 * tile_stride), 0, (int)(RT * tile_stride), 0x00027000);
     const auto     gbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(GS ? gexp + (size_t)R0 * units * 32 : W), 0, (int)(RT * units * 32), 0x00027000);
-    constexpr int  kSets = RT * NT < 32 ? 2 : 1; // sets of raw codes: two where registers allow, which are then asked for a chunk and a half ahead
+    constexpr int  kSets = RT * NT < 28 ? 2 : 1; // sets of raw codes: two where registers allow, which are then asked for a chunk and a half ahead
     RawHalf        raw[kSets][RT];
     auto           load_raw = [&](auto half_c, RawHalf (&raw)[RT], int r, uint32_t u) __attribute__((always_inline)) { // pieces as in load_raw_half
         constexpr int  H = decltype(half_c)::value, kPiece = Fmt<FM>::bits == 6 ? 2048 : 1024;
@@ -1299,13 +1299,13 @@ __global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, (lvoid *)(xstage + stage * kStage + (wr + 4 * j) * 1024), 16, off, 0, 0, 0);
     };
 
-    // B operands: half the column tiles of one MFMA step at a time, in two sets; half step i of a chunk is step i / 2, column tiles from NH * (i % 2) on
-    v8h            b[2][NH];
+    // B operands: half the column tiles of one MFMA step at a time, in two sets; half step i of a chunk is step i / 2, column tiles from NA * (i % 2) on
+    v8h            b[2][NA];
     const uint8_t *xread = xstage + col * 256;
     auto           read_b = [&](int i, uint32_t stage) __attribute__((always_inline)) {
-        const uint8_t *p = xread + stage * kStage + (((4 * (i >> 1) + q) ^ col) * 16) + (i & 1) * NH * 16 * 256;
+        const uint8_t *p = xread + stage * kStage + (((4 * (i >> 1) + q) ^ col) * 16) + (i & 1) * NA * 16 * 256;
 #pragma unroll
-        for (int t = 0; t < NH; t++) b[i & 1][t] = *reinterpret_cast<const v8h *>(p + t * 16 * 256);
+        for (int t = 0; t < (i & 1 ? NB : NA); t++) b[i & 1][t] = *reinterpret_cast<const v8h *>(p + t * 16 * 256);
     };
 
     // Chunk h (half H of a block) from stage `st`; its B operands of half step 0 are in b, its raw codes in (or on the way to) set `st` of raw.  The
@@ -1341,10 +1341,10 @@ __global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int t = 0; t < NH; t++)
+            for (int t = 0; t < (i & 1 ? NB : NA); t++)
 #pragma unroll
                 for (int r = 0; r < RT; r++)
-                    acc[r][(i & 1) * NH + t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(slice8(a[r], i >> 1), b[i & 1][t], acc[r][(i & 1) * NH + t], 0, 0, 0);
+                    acc[r][(i & 1) * NA + t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(slice8(a[r], i >> 1), b[i & 1][t], acc[r][(i & 1) * NA + t], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         });
     };
@@ -1399,38 +1399,72 @@ __global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(
     }
     if constexpr (WK == 2) { // each half of the wavefronts hands the other one's half of the columns over: [half][wr][r][t][lane]
         float *red = reinterpret_cast<float *>(lds);
-        auto   at = [&](int half, int r, int t) { return reinterpret_cast<v4f *>(red + ((((half * 4 + wr) * RT + r) * NH + t) * 64 + lane) * 4); };
+        auto   at = [&](int half, int r, int t) { return reinterpret_cast<v4f *>(red + ((((half * 4 + wr) * RT + r) * NA + t) * 64 + lane) * 4); };
 #pragma unroll
         for (int r = 0; r < RT; r++)
 #pragma unroll
-            for (int t = 0; t < NH; t++) *at(wk ^ 1, r, t) = wk == 0 ? acc[r][NH + t] : acc[r][t];
+            for (int t = 0; t < NA; t++)
+                if (t < NB || wk == 1) *at(wk ^ 1, r, t) = wk == 0 ? acc[r][NA + (t < NB ? t : 0)] : acc[r][t];
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < RT; r++)
 #pragma unroll
-            for (int t = 0; t < NH; t++) acc[r][t] = (wk == 0 ? acc[r][t] : acc[r][NH + t]) + *at(wk, r, t);
+            for (int t = 0; t < NA; t++)
+                if (t < NB || wk == 0) acc[r][t] = (wk == 0 ? acc[r][t] : acc[r][NA + (t < NB ? t : 0)]) + *at(wk, r, t);
         __syncthreads();
     }
     if (splitK == 1) {
-        constexpr int kCols = WK == 2 ? NH : NT; // column tiles that a wavefront holds results of
-        tile_park<FM, NT, RT, 4, half_t, 0, kCols>(acc, sc4, lds + (size_t)wk * NH * 16 * (TM * 2 + 16), wr, col, q, ws ? bias_of(ws) + mb * TM : nullptr);
+        const half_t *bias = ws ? bias_of(ws) + mb * TM : nullptr;
+        if constexpr (WK == 1) {
+            tile_park<FM, NT, RT, 4, half_t>(acc, sc4, lds, wr, col, q, bias);
+        } else if constexpr (NA == NB) { // (the column tiles that a wavefront holds results of)
+            tile_park<FM, NT, RT, 4, half_t, 0, NA>(acc, sc4, lds + (size_t)wk * NA * 16 * (TM * 2 + 16), wr, col, q, bias);
+        } else {
+            if (wk == 0)
+                tile_park<FM, NT, RT, 4, half_t, 0, NA>(acc, sc4, lds, wr, col, q, bias);
+            else
+                tile_park<FM, NT, RT, 4, half_t, 0, NB>(acc, sc4, lds + (size_t)NA * 16 * (TM * 2 + 16), wr, col, q, bias);
+        }
         __syncthreads();
         tile_flush<NT, RT, 4, NTHREADS, half_t>(C, lds, M, N, mb, nbase, tid);
     } else {
         // fp32 partial sums in two turns, one half of the columns each: both at once take more LDS than the K loop
         float *out = ws + (size_t)split * N * M;
-        if (WK == 1 || wk == 0) tile_park<FM, NT, RT, 4, float, 0, NH>(acc, sc4, lds, wr, col, q);
+        if (WK == 1 || wk == 0) tile_park<FM, NT, RT, 4, float, 0, NA>(acc, sc4, lds, wr, col, q);
         __syncthreads();
-        tile_flush<NH, RT, 4, NTHREADS, float>(out, lds, M, N, mb, nbase, tid);
+        tile_flush<NA, RT, 4, NTHREADS, float>(out, lds, M, N, mb, nbase, tid);
         __syncthreads();
         if constexpr (WK == 1) {
-            tile_park<FM, NT, RT, 4, float, NH, NT>(acc, sc4, lds, wr, col, q);
+            tile_park<FM, NT, RT, 4, float, NA, NT>(acc, sc4, lds, wr, col, q);
         } else {
-            if (wk == 1) tile_park<FM, NT, RT, 4, float, 0, NH>(acc, sc4, lds, wr, col, q);
+            if (wk == 1) tile_park<FM, NT, RT, 4, float, 0, NB>(acc, sc4, lds, wr, col, q);
         }
         __syncthreads();
-        tile_flush<NH, RT, 4, NTHREADS, float>(out, lds, M, N, mb, nbase + NH * 16, tid);
+        tile_flush<NB, RT, 4, NTHREADS, float>(out, lds, M, N, mb, nbase + NA * 16, tid);
     }
+}
+
+template <int FM, bool GS, int NT, int RT, int WK>
+__global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X,
+                                                            half_t *__restrict__ C, float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
+                                                            uint32_t units, uint32_t splitK, uint32_t nblocks)
+{
+    wide_tile<FM, GS, NT, RT, WK>(W, scales, gexp, X, C, ws, M, N, K, units, splitK, nblocks);
+}
+
+// gemm_span: the same organisation with the tile widths between gemm_wide's: 128 x 48, 128 x 80, 128 x 112, 256 x 80 and 256 x 112, and 256 x 96 with the halves of K
+// side by side, all of eight wavefronts.  What bounds a GEMM of some hundred columns is the same as there, and on top of it what the tile grid adds: columns that no tile
+// is full of (777 columns are 7 tiles of 128 or of 112), a last round of few workgroups, and CUs with a single workgroup of four wavefronts.  A half step holds (NT + 1) / 2
+// column tiles, the other one NT / 2.  Measured, us, the best there was -> here: e2m2 with group exponents 4608x4544 N 777 35.2 -> 32.3 (128 x 112), e2m1 20736x4992 N 142
+// 41.5 -> 35.6 (128 x 48), e2m2 3584x3200 N 1293 36.5 -> 31.7 and e3m2 17408x7168 N 196 72.0 -> 64.0 (256 x 80), 8192x4992 N 445 39.3 -> 35.5 (128 x 112), e2m2 4864x5632
+// N 1067 60.6 -> 54.8 (256 x 96).  Left out: 256 x 48, 256 x 64, 256 x 80 and 256 x 112 of four wavefronts and 256 x 48, 256 x 64 of eight (0.4 % over all problems
+// measured), and the same tiles for 33 to 96 columns (88 problems, the best of them with what there is: 0.990).
+template <int FM, bool GS, int NT, int RT, int WK>
+__global__ __launch_bounds__(4 * WK *kWave, RT == 2 && NT <= 4 ? 4 : 2) void gemm_span(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X,
+                                                            half_t *__restrict__ C, float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
+                                                            uint32_t units, uint32_t splitK, uint32_t nblocks)
+{
+    wide_tile<FM, GS, NT, RT, WK>(W, scales, gexp, X, C, ws, M, N, K, units, splitK, nblocks);
 }
 
 // Native layout -> fp16 [M,K], with the GEMM's own conversion code.  One lane per (row tile, K block, lane) triple.
@@ -2080,23 +2114,30 @@ int launch_wide(hipStream_t st, const void *W, const void *sc, const void *gexp,
                 int splitK)
 {
     constexpr int    TN = NT * 16, TM = 4 * RT * 16;
-    constexpr size_t kLoopLds = WK * 2 * (size_t)TN * 256, out_full = tile_stage_bytes<NT, RT, 4>(false), out_part = tile_stage_bytes<NT / 2, RT, 4>(true);
-    constexpr size_t kSums = WK == 2 ? (size_t)TM * TN * 4 : 0, kOut = out_full > out_part ? out_full : out_part, kMore = kOut > kSums ? kOut : kSums;
+    constexpr size_t kLoopLds = WK * 2 * (size_t)TN * 256, out_full = tile_stage_bytes<NT, RT, 4>(false), out_part = tile_stage_bytes<(NT + 1) / 2, RT, 4>(true);
+    constexpr size_t kSums = WK == 2 ? (size_t)TM * ((NT + 1) / 2) * 128 : 0, kOut = out_full > out_part ? out_full : out_part, kMore = kOut > kSums ? kOut : kSums;
     constexpr size_t kLds = kLoopLds > kMore ? kLoopLds : kMore;
     static_assert(kLds <= 160 * 1024 / (3 - WK), "two workgroups of four wavefronts or one of eight do not fit in LDS");
     if (M % TM) return FP6MI_ERR_SHAPE;
+    constexpr bool kSpan = NT % 2 == 1 || (NT == 6 && RT == 4 && WK == 2);
+    constexpr auto kernel = [] {
+        if constexpr (kSpan)
+            return &gemm_span<FM, GS, NT, RT, WK>;
+        else
+            return &gemm_wide<FM, GS, NT, RT, WK>;
+    }();
     if (kLds > 48 * 1024)
-        if (int rc = allow_dynamic_lds<&gemm_wide<FM, GS, NT, RT, WK>>(kLds)) return rc;
+        if (int rc = allow_dynamic_lds<kernel>(kLds)) return rc;
     uint32_t units = (uint32_t)((K + 255) / 256), nblocks = (uint32_t)((N + TN - 1) / TN);
     size_t   wgs = (M / TM) * (size_t)splitK * nblocks;
     if (wgs > 0x7fffffffu || K > (size_t)1 << 20) return FP6MI_ERR_SHAPE; // (K: 32-bit offsets over TN rows)
-    hipLaunchKernelGGL((gemm_wide<FM, GS, NT, RT, WK>), dim3((uint32_t)wgs), dim3(4 * WK * kWave), kLds, st, static_cast<const uint8_t *>(W),
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)wgs), dim3(4 * WK * kWave), kLds, st, static_cast<const uint8_t *>(W),
                        static_cast<const half_t *>(sc), static_cast<const uint8_t *>(gexp), static_cast<const half_t *>(B), static_cast<half_t *>(C), ws,
                        (uint32_t)M, (uint32_t)N, (uint32_t)K, units, (uint32_t)splitK, nblocks);
     return (int)hipGetLastError();
 }
 // kind 0: gemm_stream (wr == 1, wk = wavefronts per workgroup);  kind 1: gemm_tile (wr x wk wavefronts);  kind 2: gemm_ws (wr arithmetic + wk loading wavefronts),
-// with wr = wk = 2 gemm_prefill (2 x 2 wavefronts; nt = column tiles of the whole workgroup, rt = row tiles per wavefront), with wr = 4 and wk = 1 or 2 gemm_wide (wk: parts of K)
+// with wr = wk = 2 gemm_prefill (2 x 2 wavefronts; nt = column tiles of the whole workgroup, rt = row tiles per wavefront), with wr = 4 and wk = 1 or 2 gemm_wide or gemm_span (wk: parts of K)
 template <int FM, bool GS>
 int launch_cfg(const LaunchCfg &c, hipStream_t st, const void *W, const void *sc, const void *gexp, const void *B, void *C, float *ws, size_t M,
                size_t N, size_t K, int splitK)
@@ -2135,6 +2176,7 @@ int launch_cfg(const LaunchCfg &c, hipStream_t st, const void *W, const void *sc
         else return launch_ws<FM, GS, NT, RT, WR, PW, WR == 4 && NT < 6 ? 3 : 2, WR == 4 && NT == 3 ? 3 : 2>(st, W, sc, gexp, B, C, ws, M, N, K, splitK); \
     }
         FP6MI_CASE(4, 2, 8, 4) FP6MI_CASE(4, 2, 4, 4) FP6MI_CASE(2, 2, 8, 4) FP6MI_CASE(8, 4, 2, 2) FP6MI_CASE(3, 2, 4, 4) FP6MI_CASE(5, 2, 4, 4) FP6MI_CASE(6, 2, 4, 4) FP6MI_CASE(8, 4, 4, 1) FP6MI_CASE(8, 4, 4, 2) FP6MI_CASE(6, 4, 4, 1) FP6MI_CASE(8, 2, 4, 2) FP6MI_CASE(6, 2, 4, 2) FP6MI_CASE(4, 2, 4, 2)
+        FP6MI_CASE(3, 2, 4, 2) FP6MI_CASE(5, 2, 4, 2) FP6MI_CASE(7, 2, 4, 2) FP6MI_CASE(5, 4, 4, 2) FP6MI_CASE(6, 4, 4, 2) FP6MI_CASE(7, 4, 4, 2)
 #undef FP6MI_CASE
     }
     return FP6MI_ERR_SHAPE;

@@ -45,9 +45,10 @@ COMPILED_TILE = [(1,) + c for c in
                   (4, 1, 8, 2), (4, 1, 8, 1), (4, 1, 4, 2), (2, 1, 2, 4), (3, 2, 4, 2), (3, 2, 8, 1), (5, 2, 8, 1), (6, 2, 8, 1)]]
 
 # kind 2 = wave-specialized tile kernel: (2, n_tiles, row_tiles, arithmetic wavefronts, loading wavefronts); with 2 and 2 the prefill kernel
-# (2 x 2 wavefronts, n_tiles of the whole workgroup), with 4 and 1 or 2 the wide kernel (4 wavefronts, one below the other, for each of one or two halves of K)
+# (2 x 2 wavefronts, n_tiles of the whole workgroup), with 4 and 1 or 2 the wide kernel and its widths in between, gemm_span (4 wavefronts, one below the other, for each of one or two halves of K)
 COMPILED_WS = [(2, 4, 2, 8, 4), (2, 4, 2, 4, 4), (2, 2, 2, 8, 4), (2, 8, 4, 2, 2), (2, 3, 2, 4, 4), (2, 5, 2, 4, 4), (2, 6, 2, 4, 4),
-               (2, 8, 4, 4, 1), (2, 8, 4, 4, 2), (2, 6, 4, 4, 1), (2, 8, 2, 4, 2), (2, 6, 2, 4, 2), (2, 4, 2, 4, 2)]
+               (2, 8, 4, 4, 1), (2, 8, 4, 4, 2), (2, 6, 4, 4, 1), (2, 8, 2, 4, 2), (2, 6, 2, 4, 2), (2, 4, 2, 4, 2),
+               (2, 3, 2, 4, 2), (2, 5, 2, 4, 2), (2, 7, 2, 4, 2), (2, 5, 4, 4, 2), (2, 6, 4, 4, 2), (2, 7, 4, 4, 2)]
 
 BLOCK_BYTES = {6: 3072, 5: 2560, 4: 2048}   # one native 16-row x 256-column block per bit width
 

@@ -127,6 +127,28 @@ def test_wide_kernel_waits_cover_every_transfer(tmp_path_factory):
         assert counted == 2 * WK, (name, counted)
 
 
+def test_span_kernel_waits_cover_every_transfer(tmp_path_factory):
+    """The wide kernel's waits at the widths in between, where the transfers of a chunk do not divide evenly over the half steps."""
+    kernels = instructions(tmp_path_factory, "gemm_span")
+    assert len(kernels) == 48, sorted(kernels)   # four formats, with and without group exponents, six tiles
+    for name, code in kernels.items():
+        FM, GS, NT, RT, WK = map(int, re.search(r"gemm_spanILi(\d+)ELb([01])ELi(\d+)ELi(\d+)ELi(\d+)E", name).groups())
+        loads = RT * ((1 if FM == 21 else 2) + GS)
+        counted = 0
+        for i, c in enumerate(code):
+            wait = re.match(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)", c)
+            if not wait or int(wait.group(1)) != loads or code[i + 1] != "s_barrier":
+                continue
+            counted += 1
+            last = max(j for j in range(i) if is_transfer(code[j]))
+            between = code[last + 1:i]
+            assert not any(b.startswith(("s_cbranch", "s_branch", "s_setpc")) for b in between), name
+            assert sum(is_vector_memory(b) and not b.startswith("scratch") for b in between) >= loads, (name, c)
+            first = max(j for j in range(last) if code[j] == "s_barrier")
+            assert sum(is_transfer(b) for b in code[first:i]) == NT, (name, i)
+        assert counted == 2 * WK, (name, counted)
+
+
 def test_wave_specialized_kernels_of_128_rows_hold_no_exponents_in_registers(tmp_path_factory):
     """The loading wavefronts bring the group exponents of 128 rows as far ahead as the weights.  Loads of the arithmetic wavefronts (one 16-bit load a
     row tile and K block) were waited for at the barrier of every block, which made what the ring has under way no use."""
