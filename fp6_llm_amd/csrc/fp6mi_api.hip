@@ -309,10 +309,14 @@ inline bool prefill_replaces(const TuneAnswer &a, int i, size_t M, size_t N, siz
     return !a.exact && prefill_tile_wins(a.cfg[i], M, N, K, kSplits[i], 256);
 }
 
+// K up to which a split never pays, by the rules: its launch and partial sums (3 us and more) against at most five and a half K blocks.  On 440 problems off the table with
+// K 64-1472 and N 17-500 the best split was 1 every time.
+constexpr size_t kLittleK = 1408;
+
 // Launch shape for a given splitK.
 //  N <= 16: stream kernel.  Row tiles per wavefront (rt) reuse the activation registers, so rt grows with M; wavefronts
 //           per workgroup follow the K blocks of one split and the register budget (16 wavefronts leave 128 VGPRs each).
-//  N > 16:  tile kernel, 128 rows x 32 or 64 columns, with the K parallelism that splitK leaves open given to the
+//  N > 16:  stream kernel where K and the outputs are few, else tile kernel, 128 rows x 32 or 64 columns, with the K parallelism that splitK leaves open given to the
 //           wavefronts of the workgroup (at most what its LDS holds).
 inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, int cus)
 {
@@ -360,6 +364,17 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
         if (c.rt == 4 && c.wk == 16) c.wk = 8; // not compiled: 16 wavefronts leave too few registers for four row tiles
         (void)xbits;
         return c;
+    }
+    // Little K, few outputs: the stream kernel over several column blocks, whose workgroups are many and done when their few K blocks are.  Per CU w workgroups of 16 x 16
+    // outputs; time here / the rules' tile unsplit / the best of all shapes, on 190 problems (M 256-28672, N 17-500): two and three K blocks up to w = 8 0.64 and 1.01 (up to
+    // 1.17 of the tile's beyond); from five on w up to 3 0.53-0.70 and 1.00-1.03, up to 4 0.75-0.79 and 1.02, up to 6 0.90-0.97 and 1.00-1.06, and beyond it the tiles are level
+    // or ahead.  On 200 other problems (K 256-1472, M from 512, group exponents on 30 %) 95 calls changed: 0.65 (0.39-1.00) of the time before, of 200 with K from 1024 83: 0.66 (0.41-1.03).  us, before -> here: e2m1 1280x1216 N 21
+    // 6.7 -> 3.2, e2m2 3584x1088 N 20 7.2 -> 3.8, 2304x1088 N 31 7.8 -> 3.9, e3m2 3328x1344 N 41 6.5 -> 4.9.  (A single K block leaves all wavefronts but one idle;
+    // four of them stay with the tiles of four K wavefronts, which take them in one chunk: 0.74 here.)
+    const size_t columns = (N + 15) / 16, wgs = tiles * columns, some = (size_t)cus;
+    if (splitK == 1 && K <= kLittleK && units > 1 && units != 4 && wgs <= (units < 4 ? 8 : 6) * some) {
+        if (units < 4) return LaunchCfg{ 0, 1, wgs < 3 * some ? 1 : 2, 1, 4 };
+        return LaunchCfg{ 0, 1, wgs <= some ? 1 : wgs > 2 * some && (tiles + 2) / 3 * columns <= some ? 3 : 2, 1, wgs <= 4 * some ? 8 : 4 };
     }
     c.kind = 1;
     const TileShape *t = nullptr;
@@ -618,6 +633,7 @@ static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus
     if (N > 16) {
         int    best_s = 1;
         double best_ns = 1e30;
+        if (K <= kLittleK) return 1;
         for (int sp = 1; sp <= 8 && (size_t)sp <= units; sp *= 2) {
             if (sp > 1 && (double)sp * 8.0 * (double)N > 0.75 * (double)K) break; // partial sums would outweigh the weights
             double ns = tile_estimate_ns(M, N, K, sp, num_cus, nullptr);

@@ -377,6 +377,22 @@ def test_wide_kernel_tiles_cover_the_output(OC, IC, N):
         check_close(y, ref, "cfg %s" % (cfg,))
 
 
+@pytest.mark.parametrize("E,M,OC,IC,N", [(3, 2, 1280, 1216, 21), (2, 2, 512, 1344, 379), (2, 1, 4096, 1152, 33), (2, 3, 2304, 320, 65), (3, 2, 256, 1088, 500), (2, 2, 4096, 576, 127)])
+@pytest.mark.parametrize("groups", [False, True])
+def test_stream_kernel_over_many_column_blocks_of_little_k(E, M, OC, IC, N, groups):
+    """What the rules launch for little K: five K blocks or fewer on up to eight wavefronts, the last cut, one to three row tiles (768 and 4096 rows
+    leave a short last workgroup), up to 32 column blocks, the last with 1 to 16 columns."""
+    shape = (ctypes.c_int * 5)()
+    assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, 1, groups, shape) == 0 and shape[0] == 0
+    codes, sc, ex = quant.quantize_groupwise(_grouped_weights(OC + N, OC, IC), E, M)
+    raw = quant.pack_raw(codes, E, M)
+    x = synth.activations(N, N, IC)
+    ref = oracle.gemm_f64(oracle.dequant_grouped_from_definition(codes, sc, ex, E, M) if groups else oracle.dequant(raw, sc, E, M), x)
+    native, scd, xd = upload(raw, sc, x, E, M)
+    y = fp6.linear_forward_native(E, M, xd, native, scd, OC, 1, group_exps=fp6.pack_group_exps(torch.from_numpy(ex), OC, IC).to(DEV) if groups else None)
+    check_close(y.cpu().numpy(), ref, "little K")
+
+
 def test_unsupported_launch_shape_is_rejected():
     raw, sc, x = synth.uniform_problem(1, 256, 256, 4)
     native, scd, xd = upload(raw, sc, x, 3, 2)

@@ -962,3 +962,15 @@ def test_where_the_wide_kernel_does_not_pay(E, M, OC, IC, N, grouped, wide):
     shape = (ctypes.c_int * 5)()
     assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, 1, grouped, shape) == 0
     assert (shape[0] == 2 and shape[3] == 4 and shape[4] <= 2) == wide, tuple(shape)
+
+
+@pytest.mark.parametrize("OC,IC,N,shape", [
+    (1280, 1216, 21, (0, 1, 1, 1, 8)), (4096, 1152, 20, (0, 1, 2, 1, 8)), (4096, 1152, 33, (0, 1, 3, 1, 8)), (4096, 1152, 49, (0, 1, 2, 1, 8)), (4096, 1152, 65, (0, 1, 2, 1, 4)),
+    (4096, 1152, 96, (0, 1, 2, 1, 4)), (4096, 320, 32, (0, 1, 1, 1, 4)), (4096, 320, 48, (0, 1, 2, 1, 4)), (4096, 768, 128, (0, 1, 2, 1, 4)), (512, 1344, 384, (0, 1, 3, 1, 8)),
+    (4096, 1152, 97, None), (4096, 320, 129, None), (4096, 256, 20, None), (4096, 1024, 24, None)])   # more outputs, a single K block, four of them: tiles
+def test_little_k_takes_the_stream_kernel_unsplit(OC, IC, N, shape):
+    """Up to K 1408 the rules never split, and give few outputs to the stream kernel; its shapes on both sides of each line."""
+    got = (ctypes.c_int * 5)()
+    assert fp6.heuristic_splitk_mi355x(OC, N, IC) == 1
+    assert _lib.lib().fp6mi_query_table(3, 2, OC, N, IC, 1, got) == 2
+    assert tuple(got) == shape if shape else got[0] == 1
