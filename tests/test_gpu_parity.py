@@ -377,7 +377,7 @@ def test_wide_kernel_tiles_cover_the_output(OC, IC, N):
         check_close(y, ref, "cfg %s" % (cfg,))
 
 
-@pytest.mark.parametrize("E,M,OC,IC,N", [(3, 2, 1280, 1216, 21), (2, 2, 512, 1344, 379), (2, 1, 4096, 1152, 33), (2, 3, 2304, 320, 65), (3, 2, 256, 1088, 500), (2, 2, 4096, 576, 127)])
+@pytest.mark.parametrize("E,M,OC,IC,N", [(3, 2, 1280, 1216, 21), (2, 2, 768, 1344, 251), (2, 1, 2304, 1152, 70), (2, 3, 2304, 320, 65), (3, 2, 256, 1088, 500), (2, 2, 4096, 576, 127)])
 @pytest.mark.parametrize("groups", [False, True])
 def test_stream_kernel_over_many_column_blocks_of_little_k(E, M, OC, IC, N, groups):
     """What the rules launch for little K: five K blocks or fewer on up to eight wavefronts, the last cut, one to three row tiles (768 and 4096 rows

@@ -965,8 +965,8 @@ def test_where_the_wide_kernel_does_not_pay(E, M, OC, IC, N, grouped, wide):
 
 
 @pytest.mark.parametrize("OC,IC,N,shape", [
-    (1280, 1216, 21, (0, 1, 1, 1, 8)), (4096, 1152, 20, (0, 1, 2, 1, 8)), (4096, 1152, 33, (0, 1, 3, 1, 8)), (4096, 1152, 49, (0, 1, 2, 1, 8)), (4096, 1152, 65, (0, 1, 2, 1, 4)),
-    (4096, 1152, 96, (0, 1, 2, 1, 4)), (4096, 320, 32, (0, 1, 1, 1, 4)), (4096, 320, 48, (0, 1, 2, 1, 4)), (4096, 768, 128, (0, 1, 2, 1, 4)), (512, 1344, 384, (0, 1, 3, 1, 8)),
+    (1280, 1216, 21, (0, 1, 1, 1, 8)), (4096, 1152, 20, (0, 1, 2, 1, 8)), (2304, 1152, 70, (0, 1, 3, 1, 8)), (4096, 1152, 33, (0, 1, 2, 1, 8)), (4096, 1152, 49, (0, 1, 2, 1, 8)), (4096, 1152, 65, (0, 1, 2, 1, 4)),
+    (4096, 1152, 96, (0, 1, 2, 1, 4)), (4096, 320, 32, (0, 1, 1, 1, 4)), (4096, 320, 48, (0, 1, 2, 1, 4)), (4096, 768, 128, (0, 1, 2, 1, 4)), (768, 1344, 256, (0, 1, 3, 1, 8)),
     (4096, 1152, 97, None), (4096, 320, 129, None), (4096, 256, 20, None), (4096, 1024, 24, None)])   # more outputs, a single K block, four of them: tiles
 def test_little_k_takes_the_stream_kernel_unsplit(OC, IC, N, shape):
     """Up to K 1408 the rules never split, and give few outputs to the stream kernel; its shapes on both sides of each line."""
