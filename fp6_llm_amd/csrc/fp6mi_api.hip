@@ -392,9 +392,11 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
 // and splits only 1.1 %.
 // gemm_span's tiles (odd widths, and 256 x 96 with the halves of K side by side) were fitted later, to 252 problems of N 97-1500 on which all twelve were measured (4-5 %
 // off; what group exponents cost was taken from their neighbours).  They are asked from K 1024 up to N 3072, what lies beyond not having been measured (128 x 48 up to N 600:
-// beyond, shapes of the table whose place it took were up to 11 % ahead of it), and have to be 2.5 % ahead of gemm_wide's, with a split or K below 1536 4 %: on those
+// beyond, shapes of the table whose place it took were up to 11 % ahead of it), and have to be 2.5 % ahead of gemm_wide's, with a split or K below 1536 4 %, and
+// with a last round more than three quarters full 3 % more for a split and for 128 x 112, which take that much longer there than their rows say (e3m2 2048x2176 N 1635 18.2 us, with
+// 128 x 128 17.0; 1792x26048 N 1048 in three 107, with 256 x 128 in four 99): on those
 // problems 118 of 250 choices fell to them at a margin of 2 %, time / time of gemm_wide's best 0.93, 3 over 1.02; without a margin 150, 0.94, 7 over 1.02 and up to 1.11.
-// On 260 problems that no line was drawn on (N 97-4096, group exponents on 30 %) 69 calls changed: 0.94 (0.79-1.02) of the time before, with group exponents 0.93.
+// On 300 problems that no line was drawn on (N 97-3500, group exponents on 30 %) 76 calls changed: 0.94 (0.87-1.01) of the time before, with group exponents the same.
 struct WideShape {
     int   nt, rt, wk, slots;              // column tiles, row tiles per wavefront, K halves; workgroups that 256 CUs hold
     float full, full_k, full_kg;          // a full round: us, us per column of K, the same with group exponents on top
@@ -437,8 +439,12 @@ inline float wide_best(LaunchCfg &c, int xbits, size_t M, size_t N, size_t K, in
     float best = 0.f;
     if (N <= 96 || K > (size_t)1 << 20 || (size_t)splitK > (K + 255) / 256) return best;
     for (const WideShape &w : kWide) {
-        const bool  span = w.nt % 2 || (w.nt == 6 && w.rt == 4 && w.wk == 2); // gemm_span's: see kWide
-        const float t = wide_estimate(w, xbits, M, N, K, splitK, groups) * (!span ? 1.f : splitK > 1 || K < 1536 ? 1.04f : 1.025f);
+        const bool span = w.nt % 2 || (w.nt == 6 && w.rt == 4 && w.wk == 2); // gemm_span's: see kWide
+        float      t = wide_estimate(w, xbits, M, N, K, splitK, groups);
+        if (span) {
+            const size_t last = M / (64u * w.rt) * ((N + 16 * w.nt - 1) / (16 * w.nt)) * splitK % w.slots; // workgroups of the last round, 0 for a full one
+            t *= (splitK > 1 || K < 1536 ? 1.04f : 1.025f) + ((splitK > 1 || (w.nt == 7 && w.rt == 2)) && (last == 0 || 4 * last >= 3 * (size_t)w.slots) ? 0.03f : 0.f);
+        }
         if (span && (K < 1024 || N > (w.nt == 3 ? 600 : 3072))) continue;
         if (best == 0.f || t < best) best = t, c = LaunchCfg{ 2, w.nt, w.rt, 4, w.wk };
     }
