@@ -12,7 +12,7 @@ plus what the gfx950 engine adds: the native weight layout (``weight_prepacking_
 
 Everything is computed by ``libfp6mi.so`` (C ABI in include/fp6mi.h).  The per-call GEMM path goes through a small torch
 C++ extension over that ABI (``_fp6mi_torch``, csrc/torch_binding.cpp) when it is built, else through ctypes -- the same
-library and kernels either way (``FP6MI_NO_TORCH_EXT=1`` forces ctypes); everything else uses ctypes.  Torch only owns
+library and kernels either way (``FP6MI_NO_TORCH_EXT=1`` forces ctypes), and so does the preparation of weights on the GPU; everything else uses ctypes.  Torch only owns
 memory and streams.  Where the reference aborts the process (assert / exit) these functions raise ``ValueError`` /
 ``RuntimeError`` instead.
 """
@@ -36,7 +36,7 @@ if os.path.exists(_lib.LIB_PATH) and not os.environ.get("FP6MI_NO_TORCH_EXT"):
     try:
         _lib.lib()
         from . import _fp6mi_torch as _ext
-        if "bias" not in (_ext.linear_forward_native.__doc__ or ""):   # the newest of the names and arguments used below
+        if "bias" not in (_ext.linear_forward_native.__doc__ or "") or not hasattr(_ext, "weight_quantize_native"):   # the newest of the names and arguments used below
             raise ImportError("the extension was built from an older tree")
     except (ImportError, OSError, AttributeError):   # extension not built or stale, or a stale library: the ctypes path reports what is wrong
         _ext = None
@@ -165,6 +165,10 @@ def weight_prepacking_native_cpu(EXPONENT, MANTISSA, fpx_tensor):
 def to_native(packed_tensor, EXPONENT=3, MANTISSA=2):
     """Reference-layout weights (output of weight_prepacking*_cpu, on CPU or GPU) -> native layout on the same device.
     On a GPU the conversion is one kernel on the current stream."""
+    if _ext is not None:
+        out = _ext.to_native(packed_tensor, EXPONENT, MANTISSA)
+        if out is not None:
+            return out
     OC, IC = _weight_shape(packed_tensor, EXPONENT, MANTISSA, "packed_tensor")
     src = packed_tensor.contiguous()
     out = torch.empty(native_bytes(EXPONENT, MANTISSA, OC, IC) // 4, dtype=torch.int32, device=src.device)
@@ -220,6 +224,10 @@ def _check_group_exps(group_exps, OC, IC, dev):
 def weight_dequant_native_cuda(EXPONENT, MANTISSA, native_weight, fp16_scale, OC, IC, group_exps=None):
     """Native-layout weights on the GPU -> fp16 [OC, IC] with the GEMM's own in-register conversion (bit-exact to
     weight_dequant_eXmY_cpu of the same weights; with group_exps, to weight_dequant_grouped_cpu)."""
+    if _ext is not None:
+        out = _ext.weight_dequant_native(EXPONENT, MANTISSA, native_weight, fp16_scale, OC, IC, group_exps)
+        if out is not None:
+            return out
     _bits(EXPONENT, MANTISSA)
     if native_weight.device.type != "cuda" or fp16_scale.device != native_weight.device:
         raise ValueError("native_weight and fp16_scale must be on the same GPU")
@@ -248,6 +256,10 @@ def weight_quantize_native_cuda(EXPONENT, MANTISSA, weight, group_scales=False):
     bits as quant.quantize_rowwise + quant.pack_raw + weight_prepacking_native_cpu on the host, without leaving the device.
     group_scales=True also chooses a power-of-two factor per row and 128 columns and returns (native, scales, group_exps),
     the same bits as quant.quantize_groupwise + pack_group_exps."""
+    if _ext is not None:
+        out = _ext.weight_quantize_native(EXPONENT, MANTISSA, weight, bool(group_scales))
+        if out is not None:
+            return out
     _bits(EXPONENT, MANTISSA)
     if weight.device.type != "cuda" or weight.dim() != 2 or weight.dtype not in _QUANT_DTYPES:
         raise ValueError("weight must be a 2-D fp16, bf16 or fp32 tensor on the GPU")

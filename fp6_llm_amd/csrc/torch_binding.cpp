@@ -261,6 +261,96 @@ void clear_twins()
     std::lock_guard<std::mutex> lock(g_twin_mutex);
     g_twin_cache.clear();
 }
+
+// ---- the package's weight preparation on the GPU: to_native, weight_dequant_native_cuda and weight_quantize_native_cuda, their checks in their order ----
+// Each is one kernel of 2 to 10 us for a matrix of 1024 to 4096 rows, and took 10.6 us a call with checks, allocations, device guard and ctypes in Python,
+// so that everything up to about 20 million weights was bound by the host; here 4.8-5.3 us, of which the launch is 2.3.  None where an argument is no plain GPU tensor:
+// the package then goes its own way, which says what is wrong.
+void raise_status(int rc, const char *where)
+{
+    if (rc != 0) pybind11::module_::import("fp6_llm_amd._lib").attr("check")(rc, where); // raises Fp6miError
+}
+const at::Tensor *gpu_tensor(pybind11::handle h)
+{
+    if (!THPVariable_CheckExact(h.ptr())) return nullptr; // (a subclass may have a say in what is asked of it)
+    const at::Tensor &t = THPVariable_Unpack(h.ptr());
+    return t.is_cuda() ? &t : nullptr;
+}
+at::Tensor native_buffer(int64_t E, int64_t Mb, int64_t OC, int64_t IC, const at::Device &dev)
+{
+    const int64_t n = (int64_t)fp6mi_native_bytes((int)E, (int)Mb, (size_t)OC, (size_t)IC);
+    if (n == 0) bad("native layout needs OC % 16 == 0, IC % 64 == 0 and a supported format");
+    return at::empty({ n / 4 }, at::TensorOptions().dtype(at::kInt).device(dev));
+}
+at::Tensor group_exps_buffer(int64_t OC, int64_t IC, const at::Device &dev)
+{
+    const int64_t n = (int64_t)fp6mi_group_exps_bytes((size_t)OC, (size_t)IC);
+    if (n == 0) bad("group exponents need OC % 16 == 0 and IC % 64 == 0");
+    return at::empty({ n }, at::TensorOptions().dtype(at::kByte).device(dev));
+}
+
+pybind11::object to_native(pybind11::handle packed, int64_t E, int64_t Mb)
+{
+    const at::Tensor *t = gpu_tensor(packed);
+    if (!t) return pybind11::none();
+    const auto [OC, IC] = weight_shape(*t, E, Mb, "packed_tensor");
+    const at::Tensor   src = t->contiguous();
+    const at::Device   dev = src.device();
+    c10::hip::HIPGuard guard(dev.index());
+    const at::Tensor   out = native_buffer(E, Mb, OC, IC, dev);
+    raise_status(fp6mi_relayout_ref_to_native_gpu((int)E, (int)Mb, c10::hip::getCurrentHIPStream(dev.index()).stream(), out.data_ptr(), src.data_ptr(), (size_t)OC, (size_t)IC),
+                 "fp6mi_relayout_ref_to_native_gpu");
+    return pybind11::cast(out);
+}
+
+pybind11::object weight_dequant_native(int64_t E, int64_t Mb, pybind11::handle native, pybind11::handle scales, int64_t OC, int64_t IC, pybind11::handle group_exps)
+{
+    const at::Tensor *w = gpu_tensor(native), *s = gpu_tensor(scales), *gexp = group_exps.is_none() ? nullptr : gpu_tensor(group_exps);
+    if (!w || !s || (!gexp && !group_exps.is_none()) || OC < 0 || IC < 0) return pybind11::none();
+    check_format(E, Mb);
+    const at::Device dev = w->device();
+    if (s->device() != dev) bad("native_weight and fp16_scale must be on the same GPU");
+    static const int kBlockBytes[] = { 2048, 2560, 3072 }; // 4, 5 and 6 bits
+    if ((int64_t)w->numel() * (int64_t)w->element_size() != OC / 16 * ((IC + 255) / 256) * kBlockBytes[E + Mb - 3])
+        bad("native_weight has the wrong size for OC=" + std::to_string(OC) + " IC=" + std::to_string(IC));
+    c10::hip::HIPGuard guard(dev.index());
+    const at::Tensor   out = at::empty({ OC, IC }, at::TensorOptions().dtype(at::kHalf).device(dev)), sc = s->contiguous();
+    void              *stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+    if (!gexp) {
+        raise_status(fp6mi_dequant_native_gpu((int)E, (int)Mb, stream, out.data_ptr(), w->data_ptr(), sc.data_ptr(), (size_t)OC, (size_t)IC), "fp6mi_dequant_native_gpu");
+    } else {
+        if (gexp->scalar_type() != at::kByte || gexp->device() != dev || !gexp->is_contiguous() || gexp->numel() != OC / 16 * ((IC + 255) / 256) * 32)
+            bad("group_exps must be the contiguous uint8 tensor of pack_group_exps(exps, OC, IC) on the weights' GPU");
+        raise_status(fp6mi_dequant_native_grouped_gpu((int)E, (int)Mb, stream, out.data_ptr(), w->data_ptr(), sc.data_ptr(), gexp->data_ptr(), (size_t)OC, (size_t)IC),
+                     "fp6mi_dequant_native_grouped_gpu");
+    }
+    return pybind11::cast(out);
+}
+
+pybind11::object weight_quantize_native(int64_t E, int64_t Mb, pybind11::handle weight, bool group_scales)
+{
+    const at::Tensor *t = gpu_tensor(weight);
+    if (!t) return pybind11::none();
+    check_format(E, Mb);
+    const at::ScalarType type = t->scalar_type();
+    if (t->dim() != 2 || (type != at::kHalf && type != at::kBFloat16 && type != at::kFloat)) bad("weight must be a 2-D fp16, bf16 or fp32 tensor on the GPU");
+    const int64_t OC = t->size(0), IC = t->size(1);
+    if (OC % 16 || IC % 64) bad("weight_quantize_native_cuda needs OC % 16 == 0 and IC % 64 == 0, got [" + std::to_string(OC) + ", " + std::to_string(IC) + "]");
+    const at::Tensor   w = t->contiguous();
+    const at::Device   dev = w.device();
+    const int          dtype = type == at::kHalf ? 0 : type == at::kBFloat16 ? 1 : 2;
+    c10::hip::HIPGuard guard(dev.index());
+    const at::Tensor   native = native_buffer(E, Mb, OC, IC, dev), scales = at::empty({ OC }, at::TensorOptions().dtype(at::kHalf).device(dev));
+    void              *stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+    if (group_scales) {
+        const at::Tensor gexp = group_exps_buffer(OC, IC, dev);
+        raise_status(fp6mi_quantize_native_grouped_gpu((int)E, (int)Mb, stream, native.data_ptr(), scales.data_ptr(), gexp.data_ptr(), w.data_ptr(), dtype, (size_t)OC, (size_t)IC),
+                     "fp6mi_quantize_native_grouped_gpu");
+        return pybind11::make_tuple(native, scales, gexp);
+    }
+    raise_status(fp6mi_quantize_native_gpu((int)E, (int)Mb, stream, native.data_ptr(), scales.data_ptr(), w.data_ptr(), dtype, (size_t)OC, (size_t)IC), "fp6mi_quantize_native_gpu");
+    return pybind11::make_tuple(native, scales);
+}
 } // namespace
 
 PYBIND11_MODULE(_fp6mi_torch, m)
@@ -272,6 +362,9 @@ PYBIND11_MODULE(_fp6mi_torch, m)
     m.def("linear_forward_any_order", &linear_forward_any_order);
     m.def("clear_workspaces", &clear_workspaces);
     m.def("clear_twins", &clear_twins);
+    m.def("to_native", &to_native);
+    m.def("weight_dequant_native", &weight_dequant_native);
+    m.def("weight_quantize_native", &weight_quantize_native);
     // the reference's bindings, name for name (fp6_llm/csrc/pybind.cpp:8-15)
     m.def("linear_forward_cuda", &fp6_linear_forward_cuda, "Computes FP6-FP16 GEMM.", pybind11::arg("in_feats"), pybind11::arg("weights"),
           pybind11::arg("scales"), pybind11::arg("splitK") = 1);

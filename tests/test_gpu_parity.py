@@ -667,6 +667,56 @@ def test_torch_extension_and_ctypes_binding_agree(monkeypatch):
 
 
 @pytest.mark.parametrize("E,M", FORMATS)
+def test_weight_preparation_through_extension_and_python_agree(E, M, monkeypatch):
+    """Every accepted form of to_native, the quantizer and the dequantizer -- strided, offset and Parameter inputs, three types, with and without group
+    exponents, rows that are no multiple of 256, on a second stream, under capture -- gives the same bits whether it runs in the extension or in Python,
+    and what one refuses the other refuses with the same kind of error."""
+    print("case preparation forms", E, M, flush=True)
+    OC, IC, x = 256, 320, 1 + E + M
+    gen = torch.Generator().manual_seed(E + 8 * M)
+    packed = torch.randint(-2 ** 31, 2 ** 31 - 1, (OC, IC // 32 * x), generator=gen, dtype=torch.int64).to(torch.int32).to(DEV)
+    w = (torch.randn(2 * OC, IC, generator=gen) * 0.02).to(DEV)
+    nat, sc, ge = fp6.weight_quantize_native_cuda(E, M, w, True)
+    forms = [lambda: fp6.to_native(packed, E, M), lambda: fp6.to_native(packed.t().contiguous().t(), E, M), lambda: fp6.to_native(torch.cat([packed, packed])[OC:], E, M)]
+    for v in (w, w.half(), w.bfloat16()[16:], w.half().t().contiguous().t(), w[::2], torch.nn.Parameter(w[:48])):
+        forms += [lambda v=v, g=g: fp6.weight_quantize_native_cuda(E, M, v, g) for g in (False, True, 1, None)]
+    forms += [lambda s=s, g=g: fp6.weight_dequant_native_cuda(E, M, nat, s, 2 * OC, IC, g) for s in (sc, sc.repeat_interleave(2)[::2]) for g in (None, ge)]
+    forms += [lambda: fp6.weight_dequant_native_cuda(E, M, nat.view(torch.uint8), sc, 2 * OC, IC)]
+    refused = [lambda: fp6.to_native(packed.long(), E, M), lambda: fp6.to_native(packed[:, 1:], E, M), lambda: fp6.to_native(packed[:0], E, M), lambda: fp6.to_native(packed[:250], E, M),
+               lambda: fp6.to_native(packed, 4, 3), lambda: fp6.to_native(packed[0], E, M), lambda: fp6.to_native("w", E, M), lambda: fp6.weight_quantize_native_cuda(E, M, w[:, 1:]),
+               lambda: fp6.weight_quantize_native_cuda(E, M, w.double()), lambda: fp6.weight_quantize_native_cuda(E, M, w.cpu()), lambda: fp6.weight_quantize_native_cuda(E, M, w[:0]),
+               lambda: fp6.weight_quantize_native_cuda(4, 3, w), lambda: fp6.weight_quantize_native_cuda(E, M, w.flatten()[1:1 + 16 * IC].view(16, IC)),
+               lambda: fp6.weight_dequant_native_cuda(E, M, nat, sc, OC, IC), lambda: fp6.weight_dequant_native_cuda(E, M, nat, sc.cpu(), 2 * OC, IC),
+               lambda: fp6.weight_dequant_native_cuda(E, M, nat, sc, 2 * OC, IC, ge[:-1]), lambda: fp6.weight_dequant_native_cuda(E, M, nat, sc, 2 * OC, IC, ge.cpu()),
+               lambda: fp6.weight_dequant_native_cuda(E, M, None, sc, 2 * OC, IC), lambda: fp6.weight_dequant_native_cuda(E, M, nat, sc, 2 * OC, IC, 7)]
+    side, got, errors = torch.cuda.Stream(), [], []
+    for ext in (fp6._ext, None):
+        monkeypatch.setattr(fp6, "_ext", ext)
+        got.append([f() for f in forms])
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            got[-1] += [f() for f in forms]
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = [f() for f in forms[:4] + forms[-1:]]
+        graph.replay()
+        torch.cuda.synchronize()
+        got[-1] += [tuple(t.clone() for t in c) if isinstance(c, tuple) else c.clone() for c in captured]
+        kinds = []
+        for f in refused:
+            with pytest.raises(Exception) as e:
+                f()
+            kinds.append(e.type)
+        errors.append(kinds)
+        monkeypatch.undo()
+    assert errors[0] == errors[1]
+    for i, (a, b) in enumerate(zip(*got)):
+        a, b = (a if isinstance(a, tuple) else (a,)), (b if isinstance(b, tuple) else (b,))
+        assert len(a) == len(b) and all(u.dtype == v.dtype and u.shape == v.shape and torch.equal(u.view(torch.uint8), v.view(torch.uint8)) for u, v in zip(a, b)), i
+
+
+@pytest.mark.parametrize("E,M", FORMATS)
 def test_drop_in_call_through_extension_and_python_agree(E, M, monkeypatch):
     """Every accepted form of the drop-in call -- the three tensors in any order, strided activations and scales, odd batches, a split -- gives
     the same bits whether its checks run in the extension or in Python; a refused one is refused by both."""
