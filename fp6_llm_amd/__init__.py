@@ -36,7 +36,7 @@ if os.path.exists(_lib.LIB_PATH) and not os.environ.get("FP6MI_NO_TORCH_EXT"):
     try:
         _lib.lib()
         from . import _fp6mi_torch as _ext
-        if "bias" not in (_ext.linear_forward_native.__doc__ or "") or not hasattr(_ext, "weight_quantize_native"):   # the newest of the names and arguments used below
+        if "bias" not in (_ext.linear_forward_native.__doc__ or "") or not hasattr(_ext, "linear_forward_positional"):   # the newest of the names and arguments used below
             raise ImportError("the extension was built from an older tree")
     except (ImportError, OSError, AttributeError):   # extension not built or stale, or a stale library: the ctypes path reports what is wrong
         _ext = None
@@ -319,7 +319,7 @@ def linear_forward_native(EXPONENT, MANTISSA, in_feats, native_weight, scales, O
     group_exps: the tensor of pack_group_exps on the same GPU for weights with per-group exponents, else None.
     bias: contiguous float16 [OC] on the same GPU, added to the float32 sums before the one rounding, else None."""
     if _ext is not None:
-        return _ext.linear_forward_native(EXPONENT, MANTISSA, in_feats, native_weight, scales, OC, int(splitK), out, workspace, group_exps, bias)
+        return _ext.linear_forward_positional(EXPONENT, MANTISSA, in_feats, native_weight, scales, OC, int(splitK), out, workspace, group_exps, bias)
     _bits(EXPONENT, MANTISSA)
     if in_feats.dtype != torch.float16 or in_feats.dim() != 2:
         raise ValueError("in_feats must be a 2-D float16 tensor [B, IC]")
@@ -426,7 +426,7 @@ def linear_forward_eXmY_cuda(EXPONENT, MANTISSA, in_feats, weights, scales, spli
     """Drop-in for fp_eXmY_linear_forward_cuda (fp6_linear.cu:269-313): `weights` is the REFERENCE prepacked layout
     (int32 [OC, IC/32*x] on the GPU).  Its native-layout twin is built by one relayout kernel on first use."""
     if _ext is not None:
-        out = _ext.linear_forward_any_order(EXPONENT, MANTISSA, in_feats, weights, scales, int(splitK), _native_of)
+        out = _ext.linear_forward_any_order(EXPONENT, MANTISSA, in_feats, weights, scales, int(splitK), _native_of, _native_cache)
         if out is not None:
             return out
     in_feats, weights, scales = _sort_forward_args(in_feats, weights, scales)

@@ -3,6 +3,7 @@
 // A plain host translation unit: it touches torch only for tensors, the current stream and the device guard, and hands
 // raw pointers to libfp6mi.so.  The Python package uses it when it is built and falls back to its ctypes binding of the
 // same C ABI otherwise; both launch the same kernels.
+#include <torch/csrc/Exceptions.h>
 #include <torch/extension.h>
 
 #include <c10/hip/HIPGuard.h>
@@ -230,8 +231,27 @@ namespace {
 // linear_forward_eXmY_cuda of the Python package: the three tensors in either order (told apart by type and rank), its checks in their order,
 // and the GEMM.  The native twin comes from the package's own look-up, called with the very weight object the caller holds: `twin_of`
 // checks identity, address and version on every call.  None where an argument is no tensor: the package then says what is wrong.
-// A call on 4096 x 4096 at batch 1 is bound by the host (the kernel takes 4.0 us in a graph): 6.4-6.6 us a call with these checks in Python, 5.0-5.3 here.
-pybind11::object linear_forward_any_order(int64_t E, int64_t Mb, pybind11::handle a, pybind11::handle b, pybind11::handle c, int64_t splitK, pybind11::handle twin_of)
+// A call on 4096 x 4096 at batch 1 is bound by the host (the kernel takes 4.0 us in a graph): 6.4-6.6 us a call with these checks in Python, 4.7-4.9 here.
+// A twin that is there is found in the package's own dictionary without a call into Python: its entries are tuples that are replaced as a whole, under the
+// interpreter's lock, which is held here.
+const at::Tensor *known_twin(pybind11::handle cache, pybind11::handle weights, const at::Tensor &w, int64_t E, int64_t Mb)
+{
+    if (!PyDict_CheckExact(cache.ptr())) return nullptr;
+    const pybind11::object key = pybind11::reinterpret_steal<pybind11::object>(PyLong_FromVoidPtr(weights.ptr())); // id(weights)
+    PyObject              *entry = key ? PyDict_GetItemWithError(cache.ptr(), key.ptr()) : nullptr;               // (weakref, version, data_ptr, E, M, native tensor)
+    if (!entry || !PyTuple_CheckExact(entry) || PyTuple_GET_SIZE(entry) != 6) {
+        PyErr_Clear();
+        return nullptr;
+    }
+    auto number = [&](int i) { return PyLong_Check(PyTuple_GET_ITEM(entry, i)) ? PyLong_AsUnsignedLongLongMask(PyTuple_GET_ITEM(entry, i)) : ~0ull; };
+    PyObject *ref = PyTuple_GET_ITEM(entry, 0), *native = PyTuple_GET_ITEM(entry, 5);
+    if (!PyWeakref_Check(ref) || PyWeakref_GetObject(ref) != weights.ptr() || !THPVariable_Check(native)) return nullptr;
+    if (number(1) != w._version() || number(2) != reinterpret_cast<uintptr_t>(w.data_ptr()) || number(3) != (uint64_t)E || number(4) != (uint64_t)Mb) return nullptr;
+    return &THPVariable_Unpack(native);
+}
+
+pybind11::object linear_forward_any_order(int64_t E, int64_t Mb, pybind11::handle a, pybind11::handle b, pybind11::handle c, int64_t splitK, pybind11::handle twin_of,
+                                          pybind11::handle cache)
 {
     const pybind11::handle args[3] = { a, b, c };
     int                    weights = -1, scales = -1, feats = -1, ints = 0, halves = 0, vectors = 0, matrices = 0;
@@ -251,10 +271,48 @@ pybind11::object linear_forward_any_order(int64_t E, int64_t Mb, pybind11::handl
     if (!w.is_cuda()) bad("weights must be on the GPU");
     if (x.size(1) != IC) bad("in_feats has IC=" + std::to_string(x.size(1)) + " but the weights have IC=" + std::to_string(IC));
     if (!w.is_contiguous()) bad("weights must be contiguous");
-    const pybind11::object native = twin_of(args[weights], E, Mb);
-    return pybind11::cast(linear_forward_native(E, Mb, x, pybind11::cast<at::Tensor>(native), THPVariable_Unpack(args[scales].ptr()), OC, splitK, c10::nullopt, c10::nullopt,
-                                                c10::nullopt, c10::nullopt));
+    const at::Tensor *twin = known_twin(cache, args[weights], w, E, Mb);
+    const at::Tensor  native = twin ? *twin : pybind11::cast<at::Tensor>(twin_of(args[weights], E, Mb));
+    return pybind11::cast(linear_forward_native(E, Mb, x, native, THPVariable_Unpack(args[scales].ptr()), OC, splitK, c10::nullopt, c10::nullopt, c10::nullopt, c10::nullopt));
 }
+
+// linear_forward_native for the package itself, which hands over all eleven arguments in order: without pybind's dispatcher, which takes 0.3-0.4 us of a call for them.
+PyObject *linear_forward_positional(PyObject *, PyObject *const *args, Py_ssize_t count)
+{
+    HANDLE_TH_ERRORS
+    if (count != 11) {
+        PyErr_SetString(PyExc_TypeError, "linear_forward_positional takes 11 arguments");
+        return nullptr;
+    }
+    int64_t   numbers[4];
+    const int at[4] = { 0, 1, 5, 6 };
+    for (int i = 0; i < 4; i++) {
+        PyObject *n = PyNumber_Index(args[at[i]]);
+        if (!n) return nullptr; // (TypeError)
+        numbers[i] = PyLong_AsLongLong(n);
+        Py_DECREF(n);
+        if (numbers[i] == -1 && PyErr_Occurred()) return nullptr;
+    }
+    c10::optional<at::Tensor> more[4]; // out, workspace, group_exps, bias
+    for (int i = 2; i < 11; i++) {
+        if (i == 5 || i == 6 || (i > 6 && args[i] == Py_None)) continue;
+        if (!THPVariable_Check(args[i])) {
+            PyErr_Format(PyExc_TypeError, "argument %d of linear_forward_native must be a tensor, not %s", i, Py_TYPE(args[i])->tp_name);
+            return nullptr;
+        }
+        if (i > 6) more[i - 7] = THPVariable_Unpack(args[i]);
+    }
+    try {
+        return THPVariable_Wrap(linear_forward_native(numbers[0], numbers[1], THPVariable_Unpack(args[2]), THPVariable_Unpack(args[3]), THPVariable_Unpack(args[4]), numbers[2], numbers[3],
+                                                      more[0], more[1], more[2], more[3]));
+    } catch (const pybind11::builtin_exception &e) {
+        e.set_error();
+        return nullptr;
+    }
+    END_HANDLE_TH_ERRORS
+}
+PyMethodDef g_positional = { "linear_forward_positional", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&linear_forward_positional)), METH_FASTCALL,
+                             "linear_forward_native with all its arguments in order." };
 
 void clear_twins()
 {
@@ -360,6 +418,7 @@ PYBIND11_MODULE(_fp6mi_torch, m)
           pybind11::arg("native_weight"), pybind11::arg("scales"), pybind11::arg("OC"), pybind11::arg("splitK") = 1, pybind11::arg("out") = pybind11::none(),
           pybind11::arg("workspace") = pybind11::none(), pybind11::arg("group_exps") = pybind11::none(), pybind11::arg("bias") = pybind11::none());
     m.def("linear_forward_any_order", &linear_forward_any_order);
+    m.add_object("linear_forward_positional", pybind11::reinterpret_steal<pybind11::object>(PyCFunction_New(&g_positional, nullptr)));
     m.def("clear_workspaces", &clear_workspaces);
     m.def("clear_twins", &clear_twins);
     m.def("to_native", &to_native);
