@@ -195,12 +195,14 @@ inline double rounds_on_chip(const TuneCfg &c, size_t M, size_t N, int splitK)
 
 // What a launch takes however short K is, in 0.02 us: 2 us, and with a split 2 us for the reduction's launch and the partial sums at 8 TB/s, as
 // in tile_estimate_ns.  (Twice a time less the time at twice the K, over the table from 2048 columns on: 3-4 us unsplit, 5-8 us and the partial
-// sums with a split.)  Between 33 and 320 columns the splits are compared with this part carried over as it is and the rest in proportion; the shapes of one split
+// sums with a split.)  Up to 320 columns the splits are compared with this part carried over as it is and the rest in proportion; the shapes of one split
 // are not.  In proportion to K as a whole, a split's time shrank with the part that does not, and matrices of little K were cut that none of their
 // neighbours gains by: FP4 1280x2304 N 113 in eight (8.5 us, 5.5 unsplit), FP6 2048x3456 N 231 in four (11.0, 8.8), FP5 1536x1408 N 47 in three (5.9, 4.1).
 // Time of the choice / time of the best proposal on 324 matrices off the table, every proposal measured: N 33-80 1.07 before, 1.02 now, N 81-160 1.02 and
-// 1.01, N 161-320 1.03 and 1.02.  Left as they were: up to 32 columns (1.04 and 1.01, but 5 of 87 problems 3-13 % slower), and beyond 320, where the
-// few splits measured are for long K (11520x12800 N 456: 152 us in two pieces, 172 uncut).
+// 1.01, N 161-320 1.03 and 1.02.  Up to 16 columns, and 17 to 32 with K up to 3072 or M up to 2560, 81 of 600 drawn choices change by it, to 0.88 of the time in a graph
+// (0.52-1.11) and 0.80 in a stream, where a second launch costs the host 2.6 us (e3m2 2304x2176 N 13 in three 5.8 and 10.8 us, uncut 4.2 and 4.4; 2560x2688 N 5 in three 5.5 and 9.1,
+// uncut 3.8 and 4.7).  Left as they were: the other 17 to 32 columns (1.04-1.22 on ten problems whose tiles in six or eight gave way to the stream kernel uncut), and beyond 320,
+// where the few splits measured are for long K (11520x12800 N 456: 152 us in two pieces, 172 uncut).
 inline double fixed_part(size_t M, size_t N, int splitK)
 {
     return splitK == 1 ? 100.0 : 200.0 + (double)splitK * M * N * 8.0 / 8e6 / 0.02;
@@ -255,7 +257,7 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
                 of_shape[i] = a.t[i] = (float)t;
                 a.cfg[i] = LaunchCfg{ c.kind, c.nt, c.rt, c.wr, c.wk };
                 a.valid = true;
-                if (!a.measured && N > 32 && N <= 320) {
+                if (!a.measured && N <= 320 && (N <= 16 || N > 32 || K <= 3072 || M <= 2560)) {
                     const double there = std::fmin(fixed_part(Me, group->n, kSplits[i]), 0.8 * c.t), here = std::fmin(fixed_part(M, Nq, kSplits[i]), 0.8 * c.t);
                     a.t[i] = (float)((here + (c.t - there) * (double)K / (double)Ke * rounds) * (1.0 + 0.15 * dist[j]));
                 }
@@ -481,14 +483,15 @@ inline bool wide_replaces(const LaunchCfg &wide, float t, float narrow, size_t M
     return t < narrow * (N <= 400 || wide.nt <= 5 && wide.rt == 2 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
 }
 
-// The fastest split of the table's (3 % hysteresis towards fewer pieces) and its time in us; 0 where it holds none.  One that takes more than ws_bytes has to be
+// The fastest split of the table's (3 % hysteresis towards fewer pieces; 10 % towards a single launch that takes less than 8 us, which two take of the host alone) and its time
+// in us; 0 where it holds none.  One that takes more than ws_bytes has to be
 // the faster by the table's times as they stand too, which were what decided before narrow_estimate.
 inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N, size_t ws_bytes)
 {
     float best = 0.f;
     split = 0;
     for (int s : kSplits)
-        if (const float t = narrow_estimate(a, M, N, s); t > 0.f && (split == 0 || t * 1.03f < best)) {
+        if (const float t = narrow_estimate(a, M, N, s); t > 0.f && (split == 0 || t * (split == 1 && t < 8.f ? 1.1f : 1.03f) < best)) {
             if (split && fp6mi_workspace_bytes(M, N, s) > ws_bytes && a->t[split_index(s)] * 1.03f >= a->t[split_index(split)]) continue;
             split = s, best = t;
         }

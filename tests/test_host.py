@@ -974,3 +974,10 @@ def test_little_k_takes_the_stream_kernel_unsplit(OC, IC, N, shape):
     assert fp6.heuristic_splitk_mi355x(OC, N, IC) == 1
     assert _lib.lib().fp6mi_query_table(3, 2, OC, N, IC, 1, got) == 2
     assert tuple(got) == shape if shape else got[0] == 1
+
+
+@pytest.mark.parametrize("OC,IC,N,split", [(2048, 3264, 6, False), (1536, 3840, 2, False), (2304, 2176, 13, False), (2048, 2304, 26, False), (2560, 7744, 2, False), (9216, 1408, 24, False),
+                                           (1536, 28096, 13, True), (1280, 28288, 1, True), (4864, 9536, 25, True), (5120, 14784, 13, True), (1792, 22464, 3, True)])
+def test_small_batches_are_split_for_long_rows_only(OC, IC, N, split):
+    """Matrices off the table: measured, the first are 0.64 to 0.95 of the time uncut, the others 1.2 to 1.7."""
+    assert (fp6.heuristic_splitk_mi355x(OC, N, IC) > 1) == split
