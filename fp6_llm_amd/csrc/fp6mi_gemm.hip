@@ -1618,8 +1618,8 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 // 47.1 -> 43.1, 51.6 -> 45.2; fp32 8192x8192 95.2 -> 87.6, 98.7 -> 91.9.
 //
 // Two organisations of the same arithmetic.  quant_fused: one workgroup of eight wavefronts per 16-row tile reads
-// its rows, finds the scales, and converts; the last two blocks of every wavefront are still in its registers then, with 16-bit weights the one
-// before them in LDS, and the others are read again, latest first (8192x8192: a quarter of the weights twice).
+// its rows, finds the scales, and converts; the last two blocks of every wavefront (three of 32-bit weights) are still in its registers then, with 16-bit
+// weights the one before them in LDS, and the others are read again, latest first (8192x8192: a quarter of the weights twice).
 // quant_row_scales + quant_blocks: a workgroup takes a row, then a wavefront a block, and all weights are read twice.
 // Measured, us, e3m2, fused / two kernels (replayed from a graph, through more memory than the caches hold):
 //               bf16            bf16 groups     fp32            fp32 groups
@@ -1627,18 +1627,21 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 //   1024x4096     7.6 /   8.3     9.2 /   8.6    11.4 /  11.1    12.5 /  11.5
 //   1536x4096     8.0 /   9.9     9.6 /  10.4    12.9 /  13.9    14.1 /  14.2
 //   2048x4096     8.9 /  11.0    10.2 /  11.5    14.3 /  16.5    15.5 /  16.9
-//   2048x6144    12.3 /  13.5    13.9 /  14.1    20.2 /  22.3    22.1 /  23.0
+//   2048x6144    12.3 /  13.5    13.9 /  14.1    17.7 /  22.3    19.6 /  23.0
 //   2048x8192    15.6 /  16.2    18.9 /  16.6    26.9 /  26.9    29.6 /  27.7
-//   2560x8192    16.8 /  19.3    19.6 /  19.7    30.6 /  33.4    32.4 /  33.7
-//   2816x16384   36.0 /  37.3    40.0 /  37.9    65.4 /  68.7    69.2 /  68.6
-//   4096x8192    23.1 /  28.7    24.8 /  29.5    47.7 /  50.1    49.2 /  50.6
-//   8192x8192    42.9 /  52.7    45.0 /  52.7    93.3 /  95.2    98.6 /  94.6
-//   4096x28672   85.8 /  89.4    89.9 /  89.6   164 / 180       168 / 180
+//   2560x8192    16.8 /  19.3    19.6 /  19.7    28.3 /  33.4    30.9 /  33.7
+//   2816x16384   36.0 /  37.3    40.0 /  37.9    61.9 /  68.7    64.1 /  68.6
+//   4096x8192    23.1 /  28.7    24.8 /  29.5    41.2 /  50.1    43.0 /  50.6
+//   8192x8192    42.9 /  52.7    45.0 /  52.7    87.1 /  95.2    86.6 /  94.6
+//   4096x28672   85.8 /  89.4    89.9 /  89.6   158 / 180       158 / 180
 //  16384x4096    37.2 /  53.6    38.8 /  53.7    72.2 /  93.6    76.1 /  93.8
 // Few workgroups do not pull enough from memory to pay for a second pass over a long row: fused from 160 tiles on, and below that up to K = 3072 or three
-// times the rows.  On the wrong side of that line bf16 of 1024x4096 (9 %) and 2048x8192 (4 %), group exponents of 2816x16384 (6 %) and, in fp32 with them, 8192x8192 (4 %) and 1024x3072 (4 %).
-// (A block of every wavefront in LDS and two in registers leave room for two workgroups to a CU.  Three in registers and one in LDS, nothing read
-// twice at 8192 columns, were slower with one workgroup to a CU, and held to 128 registers they spill.)
+// times the rows.  On the wrong side of that line bf16 of 1024x4096 (9 %) and 2048x8192 (4 %), group exponents of 2816x16384 (6 %) and, in fp32 with them, 1024x3072 (4 %).
+// (16-bit weights: a block of every wavefront in LDS and two in registers leave room for two workgroups to a CU.  Three in registers and one in LDS, nothing
+// read twice at 8192 columns, were slower with one workgroup to a CU, and held to 128 registers they spill.
+// 32-bit weights, of which two blocks take 202 registers: a CU holds one workgroup either way, so a third block takes the other 54.  us, e3m2, two blocks -> three:
+// 4096x6144 29.5 -> 25.1, 14336x6144 99.6 -> 87.7, 8192x8192 91.1 -> 83.1, 8192x11008 113 -> 106, 8192x28672 323 -> 313; up to 4096 columns, where no
+// wavefront has a third, within 1 %.  A block of 16 KB in LDS beside two gives the same, beside three it costs 10 % but at 8192 columns.)
 // A conversion in double precision, code by code through a byte array in scratch memory, took 532 us at 8192x8192.
 // ---------------------------------------------------------------------------------------------------------------
 struct bf16_t { uint16_t bits; };
@@ -1841,8 +1844,8 @@ __device__ __forceinline__ void quantize_block(const WeightPiece<T> (&x)[8], flo
     store_native_strings<FM>(str[0], str[1], native + blk * Fmt<FM>::block_bytes, (lane >> 2) + 16 * (lane & 3));
 }
 
-// One block more of every wavefront waits in LDS, where a row has more than KEEP of them a wavefront and the weights 16 bits (64 KB; 32-bit ones would
-// take 128 KB and with it the CU's second workgroup).  It goes there straight from memory, lane l to byte 16 * l of its piece.
+// One block more of every wavefront waits in LDS, where a row has more than KEEP of them a wavefront and the weights 16 bits (64 KB; for the
+// 128 KB of 32-bit ones see above).  It goes there straight from memory, lane l to byte 16 * l of its piece.
 template <typename T, int WAVES> constexpr uint32_t quant_stash_bytes() { return sizeof(T) == 2 ? WAVES * 8 * 1024 : 0; }
 
 template <int FM, typename T, bool GROUPS, int WAVES, int KEEP>
@@ -2239,7 +2242,7 @@ template <int FM> int op_quantize(void *stream, void *native, void *scales, void
         typedef std::remove_cv_t<std::remove_pointer_t<decltype(typed)>> T;
         constexpr bool GROUPS = decltype(groups_c)::value;
         if (M / 16 >= 160 || K <= 3072 || K <= M * 3) { // (where the two organisations cross: see quant_fused)
-            constexpr int WAVES = 8, KEEP = 2;
+            constexpr int WAVES = 8, KEEP = sizeof(T) == 2 ? 2 : 3;
             const uint32_t stash = units > WAVES * KEEP ? quant_stash_bytes<T, WAVES>() : 0; // what some wavefront needs
             if (stash)
                 if (int rc = allow_dynamic_lds<quant_fused<FM, T, GROUPS, WAVES, KEEP>>(stash)) return rc;
