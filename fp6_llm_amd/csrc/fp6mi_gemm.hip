@@ -1238,218 +1238,11 @@ __global__ __launch_bounds__(4 * kWave, 2) void gemm_prefill(const uint8_t *W, c
 // bytes takes 36 us).
 // ---------------------------------------------------------------------------------------------------------------
 template <int FM, bool GS, int NT, int RT, int WK>
-__device__ __forceinline__ void wide_tile(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X, half_t *__restrict__ C,
-                                          float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K, uint32_t units, uint32_t splitK, uint32_t nblocks)
-{
-    constexpr int TM = 4 * RT * 16, TN = NT * 16, kStage = TN * 256, NTHREADS = 4 * WK * kWave;
-    constexpr int NA = (NT + 1) / 2, NB = NT / 2; // column tiles of the first and of the second half step
-    constexpr int kDma = TN / 16; // transfers of 1 KB (four rows) per wavefront and chunk
-    // loads a wavefront issues for certain after its last transfer of a chunk and before the chunk's barrier
-    constexpr int kRawLoads = (Fmt<FM>::bits == 4 ? 1 : 2) + (GS ? 1 : 0), kAfterDma = RT * kRawLoads;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int col = lane & 15, q = lane >> 4, wr = wave & 3, wk = WK == 1 ? 0 : wave >> 2;
-
-    const TileId   id = tile_of<TM, TN>(splitK, nblocks, N, K);
-    const uint32_t mb = id.mb, split = id.split, nb = id.nb;
-    const uint32_t nbase = nb * TN, R0 = (mb * 4 + wr) * RT;
-    uint32_t       u0 = 0, u1 = units;
-    if (splitK > 1) {
-        const uint32_t avg = units / splitK, extra = units % splitK;
-        u0 = split * avg + (split < extra ? split : extra);
-        u1 = u0 + avg + (split < extra ? 1u : 0u);
-    }
-
-    v4f acc[RT][NT];
-#pragma unroll
-    for (int r = 0; r < RT; r++)
-#pragma unroll
-        for (int t = 0; t < NT; t++) acc[r][t] = (v4f){ 0.f, 0.f, 0.f, 0.f };
-
-    // raw codes: scalar offsets into one buffer per wavefront (its RT row tiles), so that no address takes vector registers
-    const uint32_t tile_stride = units * Fmt<FM>::block_bytes; // 32 bits: the launcher bounds K
-    const auto     wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W + (size_t)R0 * tile_stride), 0, (int)(RT * tile_stride), 0x00027000);
-    const auto     gbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(GS ? gexp + (size_t)R0 * units * 32 : W), 0, (int)(RT * units * 32), 0x00027000);
-    constexpr int  kSets = RT * NT < 28 ? 2 : 1; // sets of raw codes: two where registers allow, which are then asked for a chunk and a half ahead
-    RawHalf        raw[kSets][RT];
-    auto           load_raw = [&](auto half_c, RawHalf (&raw)[RT], int r, uint32_t u) __attribute__((always_inline)) { // pieces as in load_raw_half
-        constexpr int  H = decltype(half_c)::value, kPiece = Fmt<FM>::bits == 6 ? 2048 : 1024;
-        const uint32_t at = r * tile_stride + u * Fmt<FM>::block_bytes;
-        raw[r].p = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16 + H * kPiece, at, 0));
-        if constexpr (Fmt<FM>::bits == 6) raw[r].s = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(wbuf, lane * 16 + 1024 + 8 * H, at, 0));
-        if constexpr (Fmt<FM>::bits == 5) raw[r].s[0] = __builtin_amdgcn_raw_buffer_load_b32(wbuf, lane * 8 + 2048 + 4 * H, at, 0);
-        if constexpr (GS) raw[r].g = __builtin_amdgcn_raw_buffer_load_b8(gbuf, 2 * col + H, (r * units + u) * 32, 0);
-    };
-
-    // transfers of activations: as in gemm_prefill
-    typedef __attribute__((address_space(3))) void lvoid;
-    uint8_t *const xstage = lds + wk * 2 * kStage;
-    const uint32_t xrow0 = 4 * wr + q, xpiece = (lane & 15) ^ xrow0; // xrow0 < 16
-    const uint32_t xoff0 = xrow0 * K * 2, xlast = (N - nbase < (uint32_t)TN ? N - 1 - nbase : TN - 1) * K * 2; // 32 bits: the launcher bounds K
-    auto           row_offset = [&](int j) __attribute__((always_inline)) {
-        uint32_t o = xoff0;
-        asm volatile("" : "+v"(o));
-        o += (uint32_t)j * 32u * K;
-        return o < xlast ? o : xlast;
-    };
-    const auto xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(X + (size_t)nbase * K), 0, (int)(xlast + K * 2), 0x00027000);
-    auto       transfer = [&](int j, uint32_t h, uint32_t stage) __attribute__((always_inline)) {
-        const uint32_t pos = h * 128 + xpiece * 8, off = row_offset(j) + (pos < K ? pos * 2 : 0xc0000000u); // (row offset + 2K < 2^29)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, (lvoid *)(xstage + stage * kStage + (wr + 4 * j) * 1024), 16, off, 0, 0, 0);
-    };
-
-    // B operands: half the column tiles of one MFMA step at a time, in two sets; half step i of a chunk is step i / 2, column tiles from NA * (i % 2) on
-    v8h            b[2][NA];
-    const uint8_t *xread = xstage + col * 256;
-    auto           read_b = [&](int i, uint32_t stage) __attribute__((always_inline)) {
-        const uint8_t *p = xread + stage * kStage + (((4 * (i >> 1) + q) ^ col) * 16) + (i & 1) * NA * 16 * 256;
-#pragma unroll
-        for (int t = 0; t < (i & 1 ? NB : NA); t++) b[i & 1][t] = *reinterpret_cast<const v8h *>(p + t * 16 * 256);
-    };
-
-    // Chunk h (half H of a block) from stage `st`; its B operands of half step 0 are in b, its raw codes in (or on the way to) set `st` of raw.  The
-    // next chunk of this wavefront is h + WK.  (LAST: a last odd one of two K halves, which fetches nothing.  No other copy of the code is special: after
-    // the last chunk another one is fetched and not used.)
-    v32h a[RT];
-    auto chunk = [&](auto half_c, auto next_c, uint32_t h, auto st_c, auto last_c) __attribute__((always_inline)) {
-        constexpr bool LAST = decltype(last_c)::value;
-        constexpr int  H = decltype(half_c)::value, st = decltype(st_c)::value, set = kSets == 2 ? st : 0;
-        const uint32_t hx = h + WK < 2 * u1 ? h + WK : h, hr = h + kSets * WK, u_raw = hr < 2 * u1 ? hr >> 1 : u1 - 1;
-        sections<8>([&](auto i_c) __attribute__((always_inline)) {
-            constexpr int i = decltype(i_c)::value;
-            if constexpr (i == 0) {
-#pragma unroll
-                for (int r = 0; r < RT; r++) a[r] = convert_raw_half<FM, GS, H>(raw[set][r]);
-            }
-            if constexpr (i == 4 && !LAST) { // (half of the converted fragments are used up: their registers hold these)
-#pragma unroll
-                for (int r = 0; r < RT; r++) load_raw(std::conditional_t<kSets == 2, decltype(half_c), decltype(next_c)>{}, raw[set], r, u_raw);
-            }
-            if constexpr (i < 4 && !LAST) {
-#pragma unroll
-                for (int j = i * kDma / 4; j < (i + 1) * kDma / 4; j++) transfer(j, hx, st ^ 1);
-            }
-            if constexpr (i == 7 && LAST) {
-                wait_transfers_and_barrier<0>();
-            } else if constexpr (i == 7) { // the next chunk's activations have landed, for every wavefront
-                wait_transfers_and_barrier<kAfterDma>();
-                __builtin_amdgcn_sched_barrier(0);
-                read_b(0, st ^ 1);
-            } else {
-                read_b(i + 1, st);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int t = 0; t < (i & 1 ? NB : NA); t++)
-#pragma unroll
-                for (int r = 0; r < RT; r++)
-                    acc[r][(i & 1) * NA + t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(slice8(a[r], i >> 1), b[i & 1][t], acc[r][(i & 1) * NA + t], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        });
-    };
-
-    typedef std::integral_constant<int, 0> Half0;
-    typedef std::integral_constant<int, 1> Half1;
-    if (u0 < u1) { // (more splits than K blocks leave some empty: their partial sums are zeros)
-        auto fill = [&](auto half_c, auto next_c) __attribute__((always_inline)) {
-#pragma unroll
-            for (int j = 0; j < kDma; j++) transfer(j, 2 * u0 + decltype(half_c)::value, 0);
-#pragma unroll
-            for (int r = 0; r < RT; r++) load_raw(half_c, raw[0], r, u0);
-            if constexpr (kSets == 2) {
-#pragma unroll
-                for (int r = 0; r < RT; r++) load_raw(next_c, raw[kSets - 1], r, WK == 1 ? u0 : u0 + 1 < u1 ? u0 + 1 : u0);
-            }
-            wait_transfers_and_barrier<0>();
-            read_b(0, 0);
-        };
-        if constexpr (WK == 1) {
-            fill(Half0{}, Half1{});
-            for (uint32_t u = u0; u < u1; u++) {
-                chunk(Half0{}, Half1{}, 2 * u, Half0{}, std::false_type{});
-                chunk(Half1{}, Half0{}, 2 * u + 1, Half1{}, std::false_type{});
-            }
-        } else {
-            // (every wavefront passes the same number of barriers)
-            auto run = [&](auto half_c) __attribute__((always_inline)) {
-                constexpr int H = decltype(half_c)::value;
-                fill(half_c, half_c);
-                uint32_t u = u0;
-                for (; u + 2 <= u1; u += 2) {
-                    chunk(half_c, half_c, 2 * u + H, Half0{}, std::false_type{});
-                    chunk(half_c, half_c, 2 * u + 2 + H, Half1{}, std::false_type{});
-                }
-                if (u < u1) chunk(half_c, half_c, 2 * u + H, Half0{}, std::true_type{});
-            };
-            if (wk == 0)
-                run(Half0{});
-            else
-                run(Half1{});
-        }
-    }
-    wait_transfers_and_barrier<0>(); // nothing is on its way to LDS any more, and nobody reads operands
-
-    // output: as in the other tile kernels, through LDS; the row scales are asked for here, one round trip at the end of a long K loop
-    v4h sc4[RT];
-#pragma unroll
-    for (int r = 0; r < RT; r++) {
-        const half_t *p = scales + (R0 + r) * 16 + 4 * q;
-        sc4[r] = (v4h){ p[0], p[1], p[2], p[3] };
-    }
-    if constexpr (WK == 2) { // each half of the wavefronts hands the other one's half of the columns over: [half][wr][r][t][lane]
-        float *red = reinterpret_cast<float *>(lds);
-        auto   at = [&](int half, int r, int t) { return reinterpret_cast<v4f *>(red + ((((half * 4 + wr) * RT + r) * NA + t) * 64 + lane) * 4); };
-#pragma unroll
-        for (int r = 0; r < RT; r++)
-#pragma unroll
-            for (int t = 0; t < NA; t++)
-                if (t < NB || wk == 1) *at(wk ^ 1, r, t) = wk == 0 ? acc[r][NA + (t < NB ? t : 0)] : acc[r][t];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < RT; r++)
-#pragma unroll
-            for (int t = 0; t < NA; t++)
-                if (t < NB || wk == 0) acc[r][t] = (wk == 0 ? acc[r][t] : acc[r][NA + (t < NB ? t : 0)]) + *at(wk, r, t);
-        __syncthreads();
-    }
-    if (splitK == 1) {
-        const half_t *bias = ws ? bias_of(ws) + mb * TM : nullptr;
-        if constexpr (WK == 1) {
-            tile_park<FM, NT, RT, 4, half_t>(acc, sc4, lds, wr, col, q, bias);
-        } else if constexpr (NA == NB) { // (the column tiles that a wavefront holds results of)
-            tile_park<FM, NT, RT, 4, half_t, 0, NA>(acc, sc4, lds + (size_t)wk * NA * 16 * (TM * 2 + 16), wr, col, q, bias);
-        } else {
-            if (wk == 0)
-                tile_park<FM, NT, RT, 4, half_t, 0, NA>(acc, sc4, lds, wr, col, q, bias);
-            else
-                tile_park<FM, NT, RT, 4, half_t, 0, NB>(acc, sc4, lds + (size_t)NA * 16 * (TM * 2 + 16), wr, col, q, bias);
-        }
-        __syncthreads();
-        tile_flush<NT, RT, 4, NTHREADS, half_t>(C, lds, M, N, mb, nbase, tid);
-    } else {
-        // fp32 partial sums in two turns, one half of the columns each: both at once take more LDS than the K loop
-        float *out = ws + (size_t)split * N * M;
-        if (WK == 1 || wk == 0) tile_park<FM, NT, RT, 4, float, 0, NA>(acc, sc4, lds, wr, col, q);
-        __syncthreads();
-        tile_flush<NA, RT, 4, NTHREADS, float>(out, lds, M, N, mb, nbase, tid);
-        __syncthreads();
-        if constexpr (WK == 1) {
-            tile_park<FM, NT, RT, 4, float, NA, NT>(acc, sc4, lds, wr, col, q);
-        } else {
-            if (wk == 1) tile_park<FM, NT, RT, 4, float, 0, NB>(acc, sc4, lds, wr, col, q);
-        }
-        __syncthreads();
-        tile_flush<NB, RT, 4, NTHREADS, float>(out, lds, M, N, mb, nbase + NA * 16, tid);
-    }
-}
-
-template <int FM, bool GS, int NT, int RT, int WK>
 __global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X,
                                                             half_t *__restrict__ C, float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
                                                             uint32_t units, uint32_t splitK, uint32_t nblocks)
 {
-    wide_tile<FM, GS, NT, RT, WK>(W, scales, gexp, X, C, ws, M, N, K, units, splitK, nblocks);
+#include "fp6mi_wide_tile.inc"
 }
 
 // gemm_span: the same organisation with the tile widths between gemm_wide's: 128 x 48, 128 x 80, 128 x 112, 256 x 80 and 256 x 112, and 256 x 96 with the halves of K
@@ -1464,7 +1257,7 @@ __global__ __launch_bounds__(4 * WK *kWave, RT == 2 && NT <= 4 ? 4 : 2) void gem
                                                             half_t *__restrict__ C, float *__restrict__ ws, uint32_t M, uint32_t N, uint32_t K,
                                                             uint32_t units, uint32_t splitK, uint32_t nblocks)
 {
-    wide_tile<FM, GS, NT, RT, WK>(W, scales, gexp, X, C, ws, M, N, K, units, splitK, nblocks);
+#include "fp6mi_wide_tile.inc"
 }
 
 // Native layout -> fp16 [M,K], with the GEMM's own conversion code.  One lane per (row tile, K block, lane) triple.
