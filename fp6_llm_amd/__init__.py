@@ -233,6 +233,10 @@ def weight_dequant_native_cuda(EXPONENT, MANTISSA, native_weight, fp16_scale, OC
         raise ValueError("native_weight and fp16_scale must be on the same GPU")
     if native_weight.numel() * native_weight.element_size() != (OC // 16) * ((IC + 255) // 256) * _BLOCK_BYTES[1 + EXPONENT + MANTISSA]:
         raise ValueError("native_weight has the wrong size for OC=%d IC=%d" % (OC, IC))
+    if not native_weight.is_contiguous():
+        raise ValueError("native_weight must be contiguous")
+    if fp16_scale.dtype != torch.float16 or fp16_scale.numel() < OC:   # (the kernel reads OC of them)
+        raise ValueError("fp16_scale must be float16, one for each of the OC rows")
     out = torch.empty((OC, IC), dtype=torch.float16, device=native_weight.device)
     with torch.cuda.device(native_weight.device):
         stream = torch.cuda.current_stream().cuda_stream

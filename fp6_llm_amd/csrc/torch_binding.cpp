@@ -371,6 +371,8 @@ pybind11::object weight_dequant_native(int64_t E, int64_t Mb, pybind11::handle n
     static const int kBlockBytes[] = { 2048, 2560, 3072 }; // 4, 5 and 6 bits
     if ((int64_t)w->numel() * (int64_t)w->element_size() != OC / 16 * ((IC + 255) / 256) * kBlockBytes[E + Mb - 3])
         bad("native_weight has the wrong size for OC=" + std::to_string(OC) + " IC=" + std::to_string(IC));
+    if (!w->is_contiguous()) bad("native_weight must be contiguous");
+    if (s->scalar_type() != at::kHalf || s->numel() < OC) bad("fp16_scale must be float16, one for each of the OC rows"); // (the kernel reads OC of them)
     c10::hip::HIPGuard guard(dev.index());
     const at::Tensor   out = at::empty({ OC, IC }, at::TensorOptions().dtype(at::kHalf).device(dev)), sc = s->contiguous();
     void              *stream = c10::hip::getCurrentHIPStream(dev.index()).stream();

@@ -717,6 +717,24 @@ def test_weight_preparation_through_extension_and_python_agree(E, M, monkeypatch
 
 
 @pytest.mark.parametrize("E,M", FORMATS)
+def test_dequantizer_takes_a_scale_for_every_row(E, M, monkeypatch):
+    """Fewer scales than rows, other types and strided codes are refused on the host, by the extension and in Python; strided, offset and longer scales are taken."""
+    print("case dequantizer scales", E, M, flush=True)
+    OC, IC = 256, 320
+    nat, sc = fp6.weight_quantize_native_cuda(E, M, (torch.randn(OC, IC, generator=torch.Generator().manual_seed(E + M)) * 0.02).to(DEV))
+    want = fp6.weight_dequant_native_cuda(E, M, nat, sc, OC, IC)
+    refused = [(nat, sc[:-1]), (nat, sc[:0]), (nat, sc[0]), (nat, sc.float()), (nat, sc.bfloat16()), (nat.repeat_interleave(2)[::2], sc)]
+    taken = [sc.repeat_interleave(2)[::2], torch.cat([sc[:3], sc])[3:], sc.reshape(16, OC // 16), torch.cat([sc, sc])]
+    for ext in (fp6._ext, None):
+        monkeypatch.setattr(fp6, "_ext", ext)
+        for w, s in refused:
+            with pytest.raises(ValueError):
+                fp6.weight_dequant_native_cuda(E, M, w, s, OC, IC)
+        for s in taken:
+            assert torch.equal(fp6.weight_dequant_native_cuda(E, M, nat, s, OC, IC).view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("E,M", FORMATS)
 def test_drop_in_call_through_extension_and_python_agree(E, M, monkeypatch):
     """Every accepted form of the drop-in call -- the three tensors in any order, strided activations and scales, odd batches, a split -- gives
     the same bits whether its checks run in the extension or in Python; a refused one is refused by both."""

@@ -981,3 +981,25 @@ def test_little_k_takes_the_stream_kernel_unsplit(OC, IC, N, shape):
 def test_small_batches_are_split_for_long_rows_only(OC, IC, N, split):
     """Matrices off the table: measured, the first are 0.64 to 0.95 of the time uncut, the others 1.2 to 1.7."""
     assert (fp6.heuristic_splitk_mi355x(OC, N, IC) > 1) == split
+
+
+class _OnGpu:
+    """A CPU tensor that says it is on the GPU, for checks that come before the first use of a device."""
+
+    def __init__(self, t):
+        self._t, self.device = t, torch.device("cuda", 0)
+
+    def __getattr__(self, name):
+        return getattr(self._t, name)
+
+
+@pytest.mark.parametrize("OC,IC", [(16, 64), (256, 320)])
+def test_dequantizer_refuses_scales_and_weights_it_would_read_wrongly(OC, IC, monkeypatch):
+    """Fewer scales than rows would be read out of range, other types and strided codes as other values: refused before anything is allocated or launched."""
+    monkeypatch.setattr(fp6, "_ext", None)
+    for E, M in fp6.FORMATS:
+        native, scales = torch.zeros(fp6.native_bytes(E, M, OC, IC) // 4, dtype=torch.int32), torch.ones(OC, dtype=torch.float16)
+        strided = torch.zeros(2 * native.numel(), dtype=torch.int32)[::2]
+        for w, s in ((native, scales[:-1]), (native, scales[:0]), (native, scales[0]), (native, scales.float()), (native, scales.bfloat16()), (strided, scales)):
+            with pytest.raises(ValueError):
+                fp6.weight_dequant_native_cuda(E, M, _OnGpu(w), _OnGpu(s), OC, IC)
