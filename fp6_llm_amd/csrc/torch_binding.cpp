@@ -287,11 +287,12 @@ PyObject *linear_forward_positional(PyObject *, PyObject *const *args, Py_ssize_
     int64_t   numbers[4];
     const int at[4] = { 0, 1, 5, 6 };
     for (int i = 0; i < 4; i++) {
-        PyObject *n = PyNumber_Index(args[at[i]]);
-        if (!n) return nullptr; // (TypeError)
-        numbers[i] = PyLong_AsLongLong(n);
-        Py_DECREF(n);
-        if (numbers[i] == -1 && PyErr_Occurred()) return nullptr;
+        pybind11::detail::make_caster<int64_t> number; // (takes and refuses what the dispatcher would)
+        if (!number.load(args[at[i]], true)) {
+            PyErr_Format(PyExc_TypeError, "argument %d of linear_forward_native must be an integer of 64 bits, not %s", at[i], Py_TYPE(args[at[i]])->tp_name);
+            return nullptr;
+        }
+        numbers[i] = number;
     }
     c10::optional<at::Tensor> more[4]; // out, workspace, group_exps, bias
     for (int i = 2; i < 11; i++) {

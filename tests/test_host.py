@@ -1,6 +1,8 @@
 """CPU-side product code (libfp6mi.so through the C ABI and the Python API) against the oracle and the golden fixtures.
 No GPU compute is called here; the library must load and export every symbol that include/fp6mi.h declares."""
 import ctypes
+import decimal
+import fractions
 import glob
 import hashlib
 import json
@@ -1003,3 +1005,30 @@ def test_dequantizer_refuses_scales_and_weights_it_would_read_wrongly(OC, IC, mo
         for w, s in ((native, scales[:-1]), (native, scales[:0]), (native, scales[0]), (native, scales.float()), (native, scales.bfloat16()), (strided, scales)):
             with pytest.raises(ValueError):
                 fp6.weight_dequant_native_cuda(E, M, _OnGpu(w), _OnGpu(s), OC, IC)
+
+
+class _Whole:
+    def __init__(self, index):
+        if index:
+            self.__class__ = type("Index", (), {"__index__": lambda _: 256})
+        else:
+            self.__class__ = type("Int", (), {"__int__": lambda _: 256, "__float__": lambda _: 256.0})
+
+
+@pytest.mark.parametrize("value", [256, True, 0, -1, 2 ** 63 - 1, 2 ** 63, -2 ** 70, 256.0, "256", None, 1j, np.int64(256), np.uint8(3), np.float32(256), np.float16(256), np.float64(256),
+                                   np.array(256), np.array(256.0), np.array([2, 3]), fractions.Fraction(256), decimal.Decimal(256), torch.tensor(256), torch.tensor(256.0), torch.tensor([2, 3]),
+                                   torch.tensor(256).half(), float("nan"), np.float32("nan"), _Whole(True), _Whole(False)], ids=lambda v: type(v).__name__ + " " + str(v)[:12])
+def test_positional_call_takes_the_numbers_that_the_dispatcher_takes(value):
+    """Formats, rows and splits given as whole numbers of any kind: one entry point gets as far as the other (here to the first check, of tensors that are not on a GPU), or raises the same."""
+    if fp6._ext is None:
+        pytest.skip("the extension is not built")
+    x, w, s = torch.zeros(1, 256, dtype=torch.float16), torch.zeros(fp6.native_bytes(3, 2, 256, 256) // 4, dtype=torch.int32), torch.ones(256, dtype=torch.float16)
+    for at in (0, 1, 5, 6):
+        args = [3, 2, x, w, s, 256, 1, None, None, None, None]
+        args[at] = value
+        ended = []
+        for call in (fp6._ext.linear_forward_native, fp6._ext.linear_forward_positional):
+            with pytest.raises(Exception) as e:
+                call(*args)
+            ended.append((e.type, str(e.value) if e.type is ValueError else ""))
+        assert ended[0] == ended[1], at
