@@ -424,9 +424,11 @@ PYBIND11_MODULE(_fp6mi_torch, m)
     m.add_object("linear_forward_positional", pybind11::reinterpret_steal<pybind11::object>(PyCFunction_New(&g_positional, nullptr)));
     m.def("clear_workspaces", &clear_workspaces);
     m.def("clear_twins", &clear_twins);
-    m.def("to_native", &to_native);
-    m.def("weight_dequant_native", &weight_dequant_native);
-    m.def("weight_quantize_native", &weight_quantize_native);
+    // (noconvert: whole numbers only, as in Python; the caster would round np.float32(3.7) to a format that exists)
+    m.def("to_native", &to_native, pybind11::arg("packed"), pybind11::arg("E").noconvert(), pybind11::arg("M").noconvert());
+    m.def("weight_dequant_native", &weight_dequant_native, pybind11::arg("E").noconvert(), pybind11::arg("M").noconvert(), pybind11::arg("native"), pybind11::arg("scales"),
+          pybind11::arg("OC").noconvert(), pybind11::arg("IC").noconvert(), pybind11::arg("group_exps"));
+    m.def("weight_quantize_native", &weight_quantize_native, pybind11::arg("E").noconvert(), pybind11::arg("M").noconvert(), pybind11::arg("weight"), pybind11::arg("group_scales"));
     // the reference's bindings, name for name (fp6_llm/csrc/pybind.cpp:8-15)
     m.def("linear_forward_cuda", &fp6_linear_forward_cuda, "Computes FP6-FP16 GEMM.", pybind11::arg("in_feats"), pybind11::arg("weights"),
           pybind11::arg("scales"), pybind11::arg("splitK") = 1);

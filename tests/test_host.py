@@ -1032,3 +1032,21 @@ def test_positional_call_takes_the_numbers_that_the_dispatcher_takes(value):
                 call(*args)
             ended.append((e.type, str(e.value) if e.type is ValueError else ""))
         assert ended[0] == ended[1], at
+
+
+@pytest.mark.parametrize("whole", [3, np.int64(3), np.uint8(3), torch.tensor(3), np.array(3)], ids=lambda v: type(v).__name__)
+@pytest.mark.parametrize("broken", [3.0, np.float32(3), np.float32(3.7), torch.tensor(3.7), fractions.Fraction(7, 2), "3", None], ids=lambda v: type(v).__name__ + str(v)[:12])
+def test_weight_preparation_takes_whole_numbers_only(whole, broken):
+    """The extension's entry points, like the Python path behind them, refuse a format or a size that is no integer instead of cutting its fraction off.  (A tensor that is
+    not on a GPU ends a call whose numbers are taken with None.)"""
+    if fp6._ext is None:
+        pytest.skip("the extension is not built")
+    t = torch.zeros(256, 12, dtype=torch.int32)
+    calls = [lambda v: fp6._ext.to_native(t, v, 2), lambda v: fp6._ext.to_native(t, 3, v), lambda v: fp6._ext.weight_quantize_native(v, 2, t, False),
+             lambda v: fp6._ext.weight_quantize_native(3, v, t, False), lambda v: fp6._ext.weight_dequant_native(v, 2, t, t, 256, 64, None),
+             lambda v: fp6._ext.weight_dequant_native(3, v, t, t, 256, 64, None), lambda v: fp6._ext.weight_dequant_native(3, 2, t, t, v, 64, None),
+             lambda v: fp6._ext.weight_dequant_native(3, 2, t, t, 256, v, None)]
+    for call in calls:
+        assert call(whole) is None
+        with pytest.raises(TypeError):
+            call(broken)
