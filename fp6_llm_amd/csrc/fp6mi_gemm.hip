@@ -1288,6 +1288,10 @@ __global__ __launch_bounds__(256) void dequant_native(half_t *__restrict__ out, 
         v = v * sc;                                    // one round-to-nearest-even, like fp16_rn(value * scale)
         *reinterpret_cast<v8h *>(mine + m * kRow + 64 * s + 16 * q) = v;
     }
+    // The reads below are of other lanes' writes.  The LDS unit serves a wavefront in order, so no instruction is needed, but the compiler has to leave them in this order.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const uint32_t k = U * 256 + 8 * (lane & 31);
 #pragma unroll
     for (int i = 0; i < 8; i++) {

@@ -189,3 +189,18 @@ def test_tile_kernel_without_a_bias_holds_no_code_for_one(tmp_path_factory):
     for shape, n in loads.items():
         RT = int(re.findall(r"Li(\d+)E", shape)[2])
         assert n[1] - n[0] == RT, (shape, n)
+
+
+def test_dequantizer_writes_a_block_to_lds_before_it_reads_other_lanes_rows(tmp_path_factory):
+    """dequant_native's lanes read back rows that other lanes of their wavefront wrote.  The source says so with a fence between the two (without one the order would rest on
+    the compiler not telling a lane's own addresses apart), and every write stands ahead of every read in the built code."""
+    with open(os.path.join(ROOT, "fp6_llm_amd", "csrc", "fp6mi_gemm.hip")) as f:
+        body = re.search(r"void dequant_native\(.*?\n}\n", f.read(), re.S).group(0)
+    write, read = body.index("reinterpret_cast<v8h *>(mine"), body.index("reinterpret_cast<const v4u *>(mine")
+    order = [body.find(text, write) for text in ('__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront")', "__builtin_amdgcn_wave_barrier()", '__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront")')]
+    assert [write] + order + [read] == sorted([write] + order + [read])
+    kernels = instructions(tmp_path_factory, "dequant_native")
+    assert len(kernels) == 8, sorted(kernels)   # four formats, with and without group exponents
+    for name, code in kernels.items():
+        writes, reads = ([i for i, c in enumerate(code) if c.startswith(op)] for op in ("ds_write", "ds_read"))
+        assert len(writes) >= 8 and len(reads) >= 8 and max(writes) < min(reads), name
