@@ -435,14 +435,15 @@ inline float wide_estimate(const WideShape &w, int xbits, size_t M, size_t N, si
     return t + (splitK > 1 ? w.split + w.split_out * (float)splitK * out : w.out * out);
 }
 
-// the fastest of the shapes for a given split, and its time in us; 0 where none fits
-inline float wide_best(LaunchCfg &c, int xbits, size_t M, size_t N, size_t K, int splitK, bool groups)
+// the fastest of the shapes for a given split, with gemm_span's among them or not, and its time in us; 0 where none fits
+inline float wide_best(LaunchCfg &c, int xbits, size_t M, size_t N, size_t K, int splitK, bool groups, bool spans)
 {
     float best = 0.f;
     if (N <= 96 || K > (size_t)1 << 20 || (size_t)splitK > (K + 255) / 256) return best;
     for (const WideShape &w : kWide) {
         const bool span = w.nt % 2 || (w.nt == 6 && w.rt == 4 && w.wk == 2); // gemm_span's: see kWide
-        float      t = wide_estimate(w, xbits, M, N, K, splitK, groups);
+        if (span && !spans) continue;
+        float t = wide_estimate(w, xbits, M, N, K, splitK, groups);
         if (span) {
             const size_t last = M / (64u * w.rt) * ((N + 16 * w.nt - 1) / (16 * w.nt)) * splitK % w.slots; // workgroups of the last round, 0 for a full one
             t *= (splitK > 1 || K < 1536 ? 1.04f : 1.025f) + ((splitK > 1 || (w.nt == 7 && w.rt == 2)) && (last == 0 || 4 * last >= 3 * (size_t)w.slots) ? 0.03f : 0.f);
@@ -504,14 +505,14 @@ inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N, si
 inline LaunchCfg final_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, bool groups, int cus)
 {
     LaunchCfg wide;
-    if (cus == 256 && N > 96)
-        if (const float t = wide_best(wide, xbits, M, N, K, splitK, groups); t > 0.f) {
+    for (bool spans : { true, false }) // (wide_replaces asks more of gemm_span's small tiles: where one of them is the fastest but not by enough, gemm_wide's fastest still may be)
+        if (const float t = cus == 256 && N > 96 ? wide_best(wide, xbits, M, N, K, splitK, groups, spans) : 0.f; t > 0.f) {
             const TuneAnswer *a = tune_lookup(xbits, M, N, K);
             const float       here = narrow_estimate(a, M, N, splitK);
             if (wide_replaces(wide, t, groups ? 1.06f * here : here, M, N, K)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
             LaunchCfg ungrouped = wide;
             int       split;
-            if (here <= 0.f && wide_replaces(ungrouped, groups ? wide_best(ungrouped, xbits, M, N, K, splitK, false) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N, K)) return wide;
+            if (here <= 0.f && wide_replaces(ungrouped, groups ? wide_best(ungrouped, xbits, M, N, K, splitK, false, spans) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N, K)) return wide;
         }
     return pick_cfg(xbits, M, N, K, splitK, cus);
 }
@@ -627,16 +628,19 @@ static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus
     if (M == 0 || N == 0 || K == 0 || num_cus <= 0) return 1;
     size_t units = (K + 255) / 256;
     if (num_cus == 256) { // the fastest split by the times of measured neighbours, or of gemm_wide where it takes their place (3 % hysteresis towards fewer splits)
-        int               best_s, wide_s = 0;
-        const float       best_t = best_narrow(best_s, tune_lookup(xbits, M, N, K), M, N, ws_bytes);
-        float             wide_t = 0.f;
-        LaunchCfg         wide = {};
-        for (int s : kSplits) {
-            LaunchCfg c;
-            if (fp6mi_workspace_bytes(M, N, s) > ws_bytes) break;
-            if (const float t = wide_best(c, xbits, M, N, K, s, false); t > 0.f && (wide_s == 0 || t * 1.03f < wide_t)) wide_s = s, wide_t = t, wide = c;
+        int         best_s;
+        const float best_t = best_narrow(best_s, tune_lookup(xbits, M, N, K), M, N, ws_bytes);
+        for (bool spans : { true, false }) { // (as in final_cfg)
+            int       wide_s = 0;
+            float     wide_t = 0.f;
+            LaunchCfg wide = {};
+            for (int s : kSplits) {
+                LaunchCfg c;
+                if (fp6mi_workspace_bytes(M, N, s) > ws_bytes) break;
+                if (const float t = wide_best(c, xbits, M, N, K, s, false, spans); t > 0.f && (wide_s == 0 || t * 1.03f < wide_t)) wide_s = s, wide_t = t, wide = c;
+            }
+            if (wide_replaces(wide, wide_t, best_t, M, N, K)) return wide_s; // (final_cfg launches gemm_wide or gemm_span then)
         }
-        if (wide_replaces(wide, wide_t, best_t, M, N, K)) return wide_s; // (final_cfg launches gemm_wide then)
         if (best_s) return best_s;
     }
     if (N > 16) {

@@ -1050,3 +1050,14 @@ def test_weight_preparation_takes_whole_numbers_only(whole, broken):
         assert call(whole) is None
         with pytest.raises(TypeError):
             call(broken)
+
+
+@pytest.mark.parametrize("E,M,OC,IC,N,split,shape", [
+    (2, 3, 2560, 1856, 789, 1, (2, 6, 2, 4, 2)), (3, 2, 2048, 2624, 1219, 1, (2, 6, 2, 4, 2)), (3, 2, 2048, 2432, 1218, 1, (2, 6, 2, 4, 2)), (2, 1, 6400, 11136, 202, 4, (2, 8, 4, 4, 2)),
+    (2, 3, 3584, 12480, 411, 4, (2, 8, 4, 4, 2))])
+def test_a_tile_of_gemm_span_that_is_not_ahead_by_enough_leaves_the_place_to_gemm_wide(E, M, OC, IC, N, split, shape):
+    """Where gemm_span's tile is expected to be the fastest, but not by the margin it is held to, gemm_wide's own fastest is asked as before.  Measured, us, the table's shape that was
+    taken instead and this one: 17.4 and 14.1, 22.5 and 18.9, 21.1 and 18.0, 47.7 (uncut) and 40.7, 51.0 (in two) and 48.7."""
+    got = (ctypes.c_int * 5)()
+    assert fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M) == split
+    assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, split, 0, got) == 0 and tuple(got) == shape
