@@ -1262,12 +1262,16 @@ __global__ __launch_bounds__(4 * WK *kWave, RT == 2 && NT <= 4 ? 4 : 2) void gem
 
 // Native layout -> fp16 [M,K], with the GEMM's own conversion code.  One lane per (row tile, K block, lane) triple.
 // Bound by its writes, two thirds to four fifths of the bytes.  A lane holds eight columns of a row: stored as they are, a wavefront writes 64 bytes into each of 16 rows, half
-// lines that meet their other half in L2.  So its block passes through LDS (its own part, no barrier) and leaves two whole rows of 512 bytes at a time, past the caches.  us,
-// e3m2, half lines / whole lines of 128 bytes (exchanged between lanes) / here: 8192x8192 38.6 / 35.0 / 32.5 (5.7 TB/s read and written), 28672x8192 124.6 / 111.8 / 104.2,
-// 3584x8128 19.9 / 17.7 / 14.3 (group exponents), 4096x4096 9.9 / 10.4 / 8.0, 2048x2048 4.6 / 4.7 / 3.7.
+// lines that meet their other half in L2.  So its block passes through LDS (its own part, no barrier) and leaves two whole rows of 512 bytes at a time.
+// How they leave: what was written is read next, by a GEMM as a rule.  Up to 224 MiB (kDequantKept) the stores are written through L2 and stay in the 256 MiB of the memory-side
+// cache; larger outputs go past the caches.  us, e3m2, alone and with the F.linear over N rows right behind: half lines / plain stores of rows / past the caches / written through:
+//   4096x4096  9.9 / 8.8 / 8.5 / 8.4, N 512 36.8 / 36.5 / 40.9 / 37.0        3584x8128 19.1 / 16.1 / 14.8 / 15.2, N 1024 84.4 / 81.5 / 95.1 / 80.9
+//   8192x8192  35.0 / 30.8 / 32.8 / 28.9, N 512 102.6 / 99.4 / 108.4 / 96.8  14336x8192 (224 MiB) 56.0 / 50.1 / 54.3 / 47.9, N 256 129 / 124 / 145 / 121, N 512 177 / 176 / 163 / 174
+//   16384x8192 62.6 / 56.2 / 61.2 / 53.8, N 512 203 / 204 / 181 / 201        28672x8192 124 / 111 / 105 / 104, N 512 308 / 299 / 285 / 299
+constexpr size_t kDequantKept = (size_t)224 << 20;
 template <int FM, bool GS>
 __global__ __launch_bounds__(256) void dequant_native(half_t *__restrict__ out, const uint8_t *__restrict__ W, const half_t *__restrict__ scales,
-                                                     const uint8_t *__restrict__ gexp, uint32_t M, uint32_t K, uint32_t units)
+                                                     const uint8_t *__restrict__ gexp, uint32_t M, uint32_t K, uint32_t units, uint32_t kept)
 {
     constexpr int  kRow = 528; // 16 bytes of padding: the reads of the 16 rows of a column start in different banks
     __shared__ __attribute__((aligned(16))) uint8_t stage[4][16 * kRow];
@@ -1293,11 +1297,23 @@ __global__ __launch_bounds__(256) void dequant_native(half_t *__restrict__ out, 
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const uint32_t k = U * 256 + 8 * (lane & 31);
+    auto           row = [&](int r) { return *reinterpret_cast<const v4u *>(mine + r * kRow + 16 * (lane & 31)); };
+    if (kept) {
+        constexpr int kWriteThrough = 16; // sc1: the scope is the device
+        const auto    obuf = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)(M * K * 2), 0x00027000);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int r = 2 * i + (lane >> 5);
-        const v4u v = *reinterpret_cast<const v4u *>(mine + r * kRow + 16 * (lane & 31));
-        if (k < K) __builtin_nontemporal_store(v, reinterpret_cast<v4u *>(out + (size_t)(R * 16 + r) * K + k));
+        for (int i = 0; i < 8; i++) {
+            const uint32_t r = 2 * i + (lane >> 5);
+            const v4u      v = row(r);
+            if (k < K) __builtin_amdgcn_raw_buffer_store_b128(v, obuf, ((R * 16 + r) * K + k) * 2, 0, kWriteThrough);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int r = 2 * i + (lane >> 5);
+            const v4u v = row(r);
+            if (k < K) __builtin_nontemporal_store(v, reinterpret_cast<v4u *>(out + (size_t)(R * 16 + r) * K + k));
+        }
     }
 }
 
@@ -2018,12 +2034,13 @@ template <int FM> int op_dequant(void *stream, void *out, const void *W, const v
     size_t      blocks = (M / 16) * units;
     dim3        grid((uint32_t)((blocks + 3) / 4));
     hipStream_t st = static_cast<hipStream_t>(stream);
+    const uint32_t kept = M * K <= kDequantKept / 2; // (and every offset below 2^28)
     if (gexp)
         hipLaunchKernelGGL((dequant_native<FM, true>), grid, dim3(256), 0, st, static_cast<half_t *>(out), static_cast<const uint8_t *>(W),
-                           static_cast<const half_t *>(sc), static_cast<const uint8_t *>(gexp), (uint32_t)M, (uint32_t)K, units);
+                           static_cast<const half_t *>(sc), static_cast<const uint8_t *>(gexp), (uint32_t)M, (uint32_t)K, units, kept);
     else
         hipLaunchKernelGGL((dequant_native<FM, false>), grid, dim3(256), 0, st, static_cast<half_t *>(out), static_cast<const uint8_t *>(W),
-                           static_cast<const half_t *>(sc), static_cast<const uint8_t *>(nullptr), (uint32_t)M, (uint32_t)K, units);
+                           static_cast<const half_t *>(sc), static_cast<const uint8_t *>(nullptr), (uint32_t)M, (uint32_t)K, units, kept);
     return (int)hipGetLastError();
 }
 

@@ -204,3 +204,10 @@ def test_dequantizer_writes_a_block_to_lds_before_it_reads_other_lanes_rows(tmp_
     for name, code in kernels.items():
         writes, reads = ([i for i, c in enumerate(code) if c.startswith(op)] for op in ("ds_write", "ds_read"))
         assert len(writes) >= 8 and len(reads) >= 8 and max(writes) < min(reads), name
+
+
+def test_dequantizer_keeps_what_the_last_level_cache_holds(tmp_path_factory):
+    """What dequant_native writes is read next.  Its outputs go past the caches only where they are larger than the memory-side cache; the others are written through to it."""
+    for name, code in instructions(tmp_path_factory, "dequant_native").items():
+        stores = [c for c in code if re.match(r"(buffer|global)_store_dwordx4", c)]
+        assert sum(c.startswith("buffer") and c.endswith(" sc1") for c in stores) == 8 and sum(c.startswith("global") and c.endswith(" nt") for c in stores) == 8 and len(stores) == 16, (name, stores)

@@ -734,6 +734,28 @@ def test_dequantizer_takes_a_scale_for_every_row(E, M, monkeypatch):
             assert torch.equal(fp6.weight_dequant_native_cuda(E, M, nat, s, OC, IC).view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("E,M,OC,groups", [(3, 2, 14448, False), (3, 2, 14464, False), (2, 2, 14464, True), (2, 3, 14448, True), (2, 1, 14464, False)])
+def test_dequantizer_on_both_sides_of_the_size_that_caches_hold(E, M, OC, groups):
+    """Outputs of up to 224 MiB and larger ones leave by other stores (8128 columns: the last block of a row is cut): the same bits as its slices of 2048 rows, which are
+    small and compared with the oracle, and not a byte beside the output."""
+    print("case dequantizer stores", E, M, OC, groups, flush=True)
+    IC, L, guard = 8128, _lib.lib(), 256
+    gen = torch.Generator(device=DEV).manual_seed(OC + M)
+    w = torch.randn(OC, IC, generator=gen, device=DEV, dtype=torch.float16) * 0.02
+    native, sc, *rest = fp6.weight_quantize_native_cuda(E, M, w, groups)
+    buf = torch.full((OC * IC + 2 * guard,), -1, dtype=torch.int16, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    args = [E, M, stream, buf[guard:].data_ptr(), native.data_ptr(), sc.data_ptr()] + ([rest[0].data_ptr()] if groups else []) + [OC, IC]
+    assert (L.fp6mi_dequant_native_grouped_gpu if groups else L.fp6mi_dequant_native_gpu)(*args) == 0
+    torch.cuda.synchronize()
+    assert (buf[:guard] == -1).all() and (buf[-guard:] == -1).all()
+    got = buf[guard:-guard].view(OC, IC)
+    for r in range(0, OC, 2048):
+        n = min(2048, OC - r)
+        part, ex = native.view(OC // 16, -1)[r // 16:(r + n) // 16].reshape(-1), rest[0].view(OC // 16, -1)[r // 16:(r + n) // 16].reshape(-1) if groups else None
+        assert torch.equal(got[r:r + n], fp6.weight_dequant_native_cuda(E, M, part, sc[r:r + n], n, IC, ex).view(torch.int16)), r
+
+
 @pytest.mark.parametrize("E,M", FORMATS)
 def test_drop_in_call_through_extension_and_python_agree(E, M, monkeypatch):
     """Every accepted form of the drop-in call -- the three tensors in any order, strided activations and scales, odd batches, a split -- gives
