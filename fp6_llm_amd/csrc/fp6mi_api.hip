@@ -393,12 +393,7 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
 // time, the smallest tiles most.  The shape and split that come out smallest are 0.8 % behind the best of these shapes on average, with a constant term, rates
 // and splits only 1.1 %.
 // gemm_span's tiles (odd widths, and 256 x 96 with the halves of K side by side) were fitted later, to 252 problems of N 97-1500 on which all twelve were measured (4-5 %
-// off; what group exponents cost was taken from their neighbours).  They are asked from K 1024 up to N 3072, what lies beyond not having been measured (128 x 48 up to N 600:
-// beyond, shapes of the table whose place it took were up to 11 % ahead of it), and have to be 2.5 % ahead of gemm_wide's, with a split or K below 1536 4 %, and
-// with a last round more than three quarters full 3 % more for a split and for 128 x 112, which take that much longer there than their rows say (e3m2 2048x2176 N 1635 18.2 us, with
-// 128 x 128 17.0; 1792x26048 N 1048 in three 107, with 256 x 128 in four 99): on those
-// problems 118 of 250 choices fell to them at a margin of 2 %, time / time of gemm_wide's best 0.93, 3 over 1.02; without a margin 150, 0.94, 7 over 1.02 and up to 1.11.
-// On 300 problems that no line was drawn on (N 97-3500, group exponents on 30 %) 76 calls changed: 0.94 (0.87-1.01) of the time before, with group exponents the same.
+// off; what group exponents cost was taken from their neighbours).  Where they are asked, and what they have to be ahead by: span_margin.
 struct WideShape {
     int   nt, rt, wk, slots;              // column tiles, row tiles per wavefront, K halves; workgroups that 256 CUs hold
     float full, full_k, full_kg;          // a full round: us, us per column of K, the same with group exponents on top
@@ -435,20 +430,48 @@ inline float wide_estimate(const WideShape &w, int xbits, size_t M, size_t N, si
     return t + (splitK > 1 ? w.split + w.split_out * (float)splitK * out : w.out * out);
 }
 
-// the fastest of the shapes for a given split, with gemm_span's among them or not, and its time in us; 0 where none fits
-inline float wide_best(LaunchCfg &c, int xbits, size_t M, size_t N, size_t K, int splitK, bool groups, bool spans)
+// What gemm_span's tile has to be ahead of gemm_wide's by; 0: it is not asked.  2.5 %, with a split or K below 1536 4 %, and with a last round more than three quarters full 3 % more
+// for a split and for 128 x 112, which take that much longer there than their rows say (e3m2 2048x2176 N 1635 18.2 us, with 128 x 128 17.0).  From K 1024 up to N 3072, what lies
+// beyond not having been measured; 128 x 48 up to N 600 (beyond, shapes of the table whose place it took were up to 11 % ahead of it).
+// The rows of the 128-row tiles, fitted to K of some thousand, expect too little of a long K: measured / expected on 1900 problems 1.02 up to K 4096 and 1.12 beyond for 128 x 80, 1.02 and
+// 1.11 for 128 x 112, 1.05 and 1.13-1.19 (K of a piece from 8192 on) for 128 x 48; gemm_wide's tiles and the 256-row ones 0.99-1.05.  Against gemm_wide at the same split they hold all the same
+// (128 x 80: 0.95 of its time on 213 problems, none above 1.00; 128 x 48 0.98), but not everywhere, and not across splits.  Time / time of what is launched instead:
+//   * 128 x 112 uncut beyond N 1400: 1.02 of 128 x 128 (138 problems; 0.965 up to there); with a last round below seven eighths and K from 8192: 1.09 (1.05-1.13) of 128 x 96;
+//   * 256 x 80 uncut, more columns than rows, K from 4096: 1.09 (1.03-1.15) of 128 x 128 on 33 of 60 problems, which a margin of 8 % finds;
+//   * uncut tiles of 128 rows in the place of a cut one: 1.06 (0.94-1.22) of gemm_wide's, 1.08-1.12 of a 256-row one; uncut 256 x 80 beyond K 20480: 1.025.  They leave the choice of a split to the others;
+//   * 128 x 48 in the place of the table's shape, K of a piece from 4096 and a single round of up to 256 workgroups: 1.09 (0.86-1.32).  wide_replaces allows for it.
+// All of it together, against the choice without gemm_span: 600 problems of N 97-4096 that it changes 0.93, 8 above 1.03 (the largest 1.05); 450 unsplit 0.92, 8 (1.08); 450 of a given split 0.93, 7 (1.11).
+// Without these lines, on as many, 0.94 with 53 above 1.03 (1.23), 0.92 with 23 (1.30: e2m3 1536x16448 N 2161 122 -> 159 us) and 0.93 with 11 (1.08).
+inline float span_margin(const WideShape &w, size_t M, size_t N, size_t K, int splitK)
+{
+    const bool   span112 = w.rt == 2 && w.nt == 7;
+    const size_t last = M / (64u * w.rt) * ((N + 16 * w.nt - 1) / (16 * w.nt)) * splitK % w.slots; // workgroups of the last round, 0 for a full one
+    if (K < 1024 || N > (w.nt == 3 ? 600 : span112 && splitK == 1 ? 1400 : 3072)) return 0.f;
+    if (span112 && splitK == 1 && K >= 8192 && last && 8 * last < 7 * (size_t)w.slots) return 0.f;
+    if (w.nt == 5 && w.rt == 4 && splitK == 1 && N > M && K >= 4096) return 1.08f;
+    return (splitK > 1 || K < 1536 ? 1.04f : 1.025f) + ((splitK > 1 || span112) && (last == 0 || 4 * last >= 3 * (size_t)w.slots) ? 0.03f : 0.f);
+}
+
+// Which of gemm_span's tiles are asked: none; those that take part in the choice of a split; all.
+enum class Spans { kNone, kForSplit, kAll };
+inline bool span_asked(const WideShape &w, Spans spans, size_t K, int splitK)
+{
+    if (spans != Spans::kForSplit) return spans == Spans::kAll;
+    return w.rt == 2 ? splitK > 1 && w.nt != 7 : w.nt != 5 || splitK > 1 || K <= 20480;
+}
+
+// the fastest of the shapes for a given split, and its time in us; 0 where none fits
+inline float wide_best(LaunchCfg &c, int xbits, size_t M, size_t N, size_t K, int splitK, bool groups, Spans spans)
 {
     float best = 0.f;
     if (N <= 96 || K > (size_t)1 << 20 || (size_t)splitK > (K + 255) / 256) return best;
     for (const WideShape &w : kWide) {
-        const bool span = w.nt % 2 || (w.nt == 6 && w.rt == 4 && w.wk == 2); // gemm_span's: see kWide
-        if (span && !spans) continue;
         float t = wide_estimate(w, xbits, M, N, K, splitK, groups);
-        if (span) {
-            const size_t last = M / (64u * w.rt) * ((N + 16 * w.nt - 1) / (16 * w.nt)) * splitK % w.slots; // workgroups of the last round, 0 for a full one
-            t *= (splitK > 1 || K < 1536 ? 1.04f : 1.025f) + ((splitK > 1 || (w.nt == 7 && w.rt == 2)) && (last == 0 || 4 * last >= 3 * (size_t)w.slots) ? 0.03f : 0.f);
+        if (w.nt % 2 || (w.nt == 6 && w.rt == 4 && w.wk == 2)) { // gemm_span's
+            const float margin = span_asked(w, spans, K, splitK) ? span_margin(w, M, N, K, splitK) : 0.f;
+            if (margin == 0.f) continue;
+            t *= margin;
         }
-        if (span && (K < 1024 || N > (w.nt == 3 ? 600 : 3072))) continue;
         if (best == 0.f || t < best) best = t, c = LaunchCfg{ 2, w.nt, w.rt, 4, w.wk };
     }
     return best;
@@ -477,9 +500,11 @@ inline float narrow_estimate(const TuneAnswer *a, size_t M, size_t N, int splitK
 // (0.56-1.28), 71 of them over 1.02; with 0.9 it takes 44 of them at 0.91 and 4 are over 1.02 (9472x17024 N 1984 in FP4 1.28, the others up to 1.03); on 34 problems of N 401-640 as good as with 0.95, 1 over 1.02 for 5.
 // Out of the table's reach K up to 512 takes 2^22 outputs: 23 problems below that took 1.02 of the time of the rules' tiles (0.90-1.22: 5632x256 N 325 4.9 us -> 5.9);
 // of the 177 others, 0.87 (0.63-1.09), 8 are over 1.02.
-inline bool wide_replaces(const LaunchCfg &wide, float t, float narrow, size_t M, size_t N, size_t K)
+// (128 x 48 with a long K in a single round takes longer than its row says: see span_margin.)
+inline bool wide_replaces(const LaunchCfg &wide, float t, float narrow, size_t M, size_t N, size_t K, int splitK)
 {
     if (t <= 0.f) return false;
+    if (wide.nt == 3 && K / splitK >= 4096 && M / 128 * ((N + 47) / 48) * splitK <= 256) t *= 1.2f;
     if (narrow <= 0.f) return M * N >= (size_t)1 << (K <= 512 ? 22 : 20);
     return t < narrow * (N <= 400 || wide.nt <= 5 && wide.rt == 2 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
 }
@@ -504,16 +529,22 @@ inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N, si
 // (0.37-1.26) by the rules.
 inline LaunchCfg final_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, bool groups, int cus)
 {
-    LaunchCfg wide;
-    for (bool spans : { true, false }) // (wide_replaces asks more of gemm_span's small tiles: where one of them is the fastest but not by enough, gemm_wide's fastest still may be)
-        if (const float t = cus == 256 && N > 96 ? wide_best(wide, xbits, M, N, K, splitK, groups, spans) : 0.f; t > 0.f) {
-            const TuneAnswer *a = tune_lookup(xbits, M, N, K);
-            const float       here = narrow_estimate(a, M, N, splitK);
-            if (wide_replaces(wide, t, groups ? 1.06f * here : here, M, N, K)) return wide; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
+    if (cus == 256 && N > 96) {
+        const TuneAnswer *a = tune_lookup(xbits, M, N, K);
+        const float       here = narrow_estimate(a, M, N, splitK);
+        LaunchCfg         wide = {};
+        auto              replaces = [&](Spans spans) { // (sets `wide`)
+            const float t = wide_best(wide, xbits, M, N, K, splitK, groups, spans);
+            if (wide_replaces(wide, t, groups ? 1.06f * here : here, M, N, K, splitK)) return true; // (the table's rows are row scales only; group exponents cost those kernels 3-10 %)
             LaunchCfg ungrouped = wide;
             int       split;
-            if (here <= 0.f && wide_replaces(ungrouped, groups ? wide_best(ungrouped, xbits, M, N, K, splitK, false, spans) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N, K)) return wide;
-        }
+            return here <= 0.f && t > 0.f &&
+                   wide_replaces(ungrouped, groups ? wide_best(ungrouped, xbits, M, N, K, splitK, false, spans) : t, best_narrow(split, a, M, N, SIZE_MAX), M, N, K, splitK);
+        };
+        // (wide_replaces asks more of gemm_span's small tiles than of most others.  Where gemm_wide's fastest passes, a span tile that is faster still is launched, too.)
+        if (replaces(Spans::kAll)) return wide;
+        if (replaces(Spans::kNone)) return wide_best(wide, xbits, M, N, K, splitK, groups, Spans::kAll), wide;
+    }
     return pick_cfg(xbits, M, N, K, splitK, cus);
 }
 
@@ -630,16 +661,19 @@ static int heuristic_splitk(int xbits, size_t M, size_t N, size_t K, int num_cus
     if (num_cus == 256) { // the fastest split by the times of measured neighbours, or of gemm_wide where it takes their place (3 % hysteresis towards fewer splits)
         int         best_s;
         const float best_t = best_narrow(best_s, tune_lookup(xbits, M, N, K), M, N, ws_bytes);
-        for (bool spans : { true, false }) { // (as in final_cfg)
-            int       wide_s = 0;
-            float     wide_t = 0.f;
-            LaunchCfg wide = {};
+        auto wide_split = [&](Spans spans, float &t, LaunchCfg &wide) {
+            int split = 0;
             for (int s : kSplits) {
                 LaunchCfg c;
                 if (fp6mi_workspace_bytes(M, N, s) > ws_bytes) break;
-                if (const float t = wide_best(c, xbits, M, N, K, s, false, spans); t > 0.f && (wide_s == 0 || t * 1.03f < wide_t)) wide_s = s, wide_t = t, wide = c;
+                if (const float ts = wide_best(c, xbits, M, N, K, s, false, spans); ts > 0.f && (split == 0 || ts * 1.03f < t)) split = s, t = ts, wide = c;
             }
-            if (wide_replaces(wide, wide_t, best_t, M, N, K)) return wide_s; // (final_cfg launches gemm_wide or gemm_span then)
+            return split;
+        };
+        for (Spans spans : { Spans::kForSplit, Spans::kNone }) { // (as in final_cfg, which launches gemm_wide or gemm_span then)
+            float     t = 0.f;
+            LaunchCfg wide = {};
+            if (const int split = wide_split(spans, t, wide); wide_replaces(wide, t, best_t, M, N, K, split)) return split;
         }
         if (best_s) return best_s;
     }

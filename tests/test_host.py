@@ -1053,11 +1053,49 @@ def test_weight_preparation_takes_whole_numbers_only(whole, broken):
 
 
 @pytest.mark.parametrize("E,M,OC,IC,N,split,shape", [
-    (2, 3, 2560, 1856, 789, 1, (2, 6, 2, 4, 2)), (3, 2, 2048, 2624, 1219, 1, (2, 6, 2, 4, 2)), (3, 2, 2048, 2432, 1218, 1, (2, 6, 2, 4, 2)), (2, 1, 6400, 11136, 202, 4, (2, 8, 4, 4, 2)),
+    (2, 3, 2560, 1856, 789, 1, (2, 5, 2, 4, 2)), (3, 2, 2048, 2624, 1219, 1, (2, 5, 2, 4, 2)), (3, 2, 2048, 2432, 1218, 1, (2, 5, 2, 4, 2)), (2, 1, 6400, 11136, 202, 4, (2, 8, 4, 4, 2)),
     (2, 3, 3584, 12480, 411, 4, (2, 8, 4, 4, 2))])
 def test_a_tile_of_gemm_span_that_is_not_ahead_by_enough_leaves_the_place_to_gemm_wide(E, M, OC, IC, N, split, shape):
-    """Where gemm_span's tile is expected to be the fastest, but not by the margin it is held to, gemm_wide's own fastest is asked as before.  Measured, us, the table's shape that was
-    taken instead and this one: 17.4 and 14.1, 22.5 and 18.9, 21.1 and 18.0, 47.7 (uncut) and 40.7, 51.0 (in two) and 48.7."""
+    """Where gemm_span's tile is expected to be the fastest, but not by the margin that it is held to against the table, gemm_wide's own fastest is asked, which is held to less; if that
+    passes, the span tile, which is ahead of it, is launched at that split.  Measured, us, the table's shape that was taken instead, gemm_wide's and this one: 17.4, 14.7 and 13.8; 22.5,
+    20.0 and 19.0; 21.0, 18.0 and 17.2; 47.7 (uncut) and 40.7; 51.0 (in two) and 48.7."""
+    got = (ctypes.c_int * 5)()
+    assert fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M) == split
+    assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, split, 0, got) == 0 and tuple(got) == shape
+
+
+W64, W96, W128, T96, T128 = (2, 4, 2, 4, 2), (2, 6, 2, 4, 2), (2, 8, 2, 4, 2), (2, 6, 4, 4, 1), (2, 8, 4, 4, 2)   # gemm_wide: 64-128 columns; 256 rows
+S48, S80, S112, S80T, S96T, S112T = (2, 3, 2, 4, 2), (2, 5, 2, 4, 2), (2, 7, 2, 4, 2), (2, 5, 4, 4, 2), (2, 6, 4, 4, 2), (2, 7, 4, 4, 2)   # gemm_span
+
+
+@pytest.mark.parametrize("E,M,OC,IC,N,grouped,split,shape", [
+    # from K 1024
+    (2, 2, 2560, 960, 1926, 0, 1, T96), (2, 2, 2560, 1024, 1926, 0, 1, S80T), (2, 1, 8192, 960, 440, 0, 1, W64), (2, 1, 8192, 1024, 440, 0, 1, S112),
+    # 128 x 48 up to N 600, 128 x 112 uncut up to 1400, the others up to 3072
+    (3, 2, 1536, 11328, 601, 0, 1, W64), (3, 2, 2304, 3584, 600, 0, 1, S48), (3, 2, 2304, 3584, 601, 0, 1, W64), (3, 2, 2304, 2624, 1400, 1, 1, S112), (3, 2, 2304, 2624, 1401, 1, 1, W128),
+    (2, 2, 2048, 2176, 3072, 0, 1, S96T), (2, 2, 2048, 2176, 3073, 0, 1, T128),
+    # 128 x 112 uncut with K from 8192: not where the last round is less than seven eighths full; a last round from three quarters on counts 3 % more
+    (2, 2, 2560, 8128, 1225, 0, 1, S112), (2, 2, 2560, 8192, 1225, 0, 1, W128), (3, 2, 5632, 20800, 408, 1, 1, W96), (2, 1, 3328, 6144, 784, 0, 1, S112), (2, 1, 3328, 6144, 785, 0, 1, W96),
+    (3, 2, 2048, 2176, 1635, 0, 1, W128),
+    # 256 x 80 uncut, more columns than rows, K from 4096
+    (3, 2, 2048, 4032, 2552, 0, 1, S80T), (3, 2, 2048, 4096, 2552, 0, 1, S96T), (2, 3, 1536, 16448, 2161, 0, 1, W128),
+    # 128 x 48 in a single round against the table's shapes, K of a piece from 4096
+    (3, 2, 1280, 8064, 195, 0, 2, S48), (3, 2, 1280, 8192, 195, 0, 2, (1, 2, 1, 4, 4)), (2, 3, 2048, 4032, 579, 0, 1, S48), (2, 3, 2048, 4096, 579, 0, 1, (2, 4, 2, 4, 4)),
+    (2, 2, 2816, 18304, 326, 1, 1, (2, 4, 2, 4, 4)), (2, 2, 2048, 26816, 582, 0, 1, (2, 4, 2, 4, 4))])
+def test_where_gemm_span_is_launched(E, M, OC, IC, N, grouped, split, shape):
+    """The shapes on both sides of each line of span_margin and wide_replaces."""
+    got = (ctypes.c_int * 5)()
+    assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, split, grouped, got) == 0 and tuple(got) == shape
+
+
+@pytest.mark.parametrize("E,M,OC,IC,N,split,shape", [
+    # uncut tiles of 128 rows, and 128 x 112 in pieces, decide no split: measured, us, uncut and this one 52.8 and 45.7, 66.8 and 59.2, 55.5 and 49.3, 92.4 and 83.5 (with 256 x 128), 46.8 and 42.8
+    (2, 3, 3328, 8640, 585, 3, T128), (3, 2, 4352, 11200, 543, 3, T128), (2, 2, 5120, 9152, 451, 3, T128), (3, 2, 3584, 12800, 945, 2, S112T), (2, 2, 9984, 7488, 216, 3, T128),
+    # where the others answer with the same split they are launched
+    (2, 2, 4608, 4544, 777, 1, S112), (3, 2, 8192, 4992, 445, 1, S112), (2, 1, 20736, 4992, 142, 1, S48),
+    # those of 256 rows decide splits, uncut 256 x 80 up to K 20480
+    (3, 2, 17408, 7168, 196, 1, S80T), (2, 2, 4864, 5632, 1067, 1, S96T), (2, 3, 2816, 20480, 1552, 1, S80T), (2, 3, 2816, 20544, 1552, 3, (2, 8, 4, 4, 1))])
+def test_which_tiles_of_gemm_span_choose_a_split(E, M, OC, IC, N, split, shape):
     got = (ctypes.c_int * 5)()
     assert fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M) == split
     assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, split, 0, got) == 0 and tuple(got) == shape
