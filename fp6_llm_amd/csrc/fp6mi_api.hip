@@ -311,8 +311,9 @@ inline bool prefill_replaces(const TuneAnswer &a, int i, size_t M, size_t N, siz
     return !a.exact && prefill_tile_wins(a.cfg[i], M, N, K, kSplits[i], 256);
 }
 
-// K up to which a split never pays, by the rules: its launch and partial sums (3 us and more) against at most five and a half K blocks.  On 440 problems off the table with
-// K 64-1472 and N 17-500 the best split was 1 every time.
+// K up to which the rules, which answer where the table does not, never split: its launch and partial sums (3 us and more) against at most five and a half K blocks.  On 440
+// problems out of the table's reach with K 64-1472 and N 17-500 the best split was 1 every time.  (The table, whose least K is 2048, reaches K 1408 for some M and N and answers
+// there for itself, in up to three pieces; K up to 1344 is the rules' everywhere.)
 constexpr size_t kLittleK = 1408;
 
 // Launch shape for a given splitK.
@@ -370,13 +371,16 @@ inline LaunchCfg pick_cfg(int xbits, size_t M, size_t N, size_t K, int splitK, i
     // Little K, few outputs: the stream kernel over several column blocks, whose workgroups are many and done when their few K blocks are.  Per CU w workgroups of 16 x 16
     // outputs; time here / the rules' tile unsplit / the best of all shapes, on 190 problems (M 256-28672, N 17-500): two and three K blocks up to w = 8 0.64 and 1.01 (up to
     // 1.17 of the tile's beyond); from five on w up to 3 0.53-0.70 and 1.00-1.03, up to 4 0.75-0.79 and 1.02, up to 6 0.90-0.97 and 1.00-1.06, and beyond it the tiles are level
-    // or ahead.  On 200 other problems (K 256-1472, M from 512, group exponents on 30 %) 95 calls changed: 0.65 (0.39-1.00) of the time before, of 200 with K from 1024 83: 0.66 (0.41-1.03).  us, before -> here: e2m1 1280x1216 N 21
-    // 6.7 -> 3.2, e2m2 3584x1088 N 20 7.2 -> 3.8, 2304x1088 N 31 7.8 -> 3.9, e3m2 3328x1344 N 41 6.5 -> 4.9.  (A single K block leaves all wavefronts but one idle;
-    // four of them stay with the tiles of four K wavefronts, which take them in one chunk: 0.74 here.)
+    // or ahead.  On 1500 other problems that it changes (K 64-1472, N 17-500, group exponents on 30 %) 0.62 of the time before in a graph, 0.86 in a stream, 6 above 1.03 (up to
+    // 1.09); N 33-96 at w 5 to 6 1.00 (0.92-1.11).  us, before -> here: e2m1 1280x1216 N 21 6.7 -> 3.2, e2m2 3584x1088 N 20 7.2 -> 3.8, 2304x1088 N 31 7.8 -> 3.9, e3m2 3328x1344
+    // N 41 6.5 -> 4.9.  5 bits: two row tiles on eight wavefronts take 135-142 registers there, 122-128 with 6 and 4 bits, and a CU holds one such workgroup instead of two: beyond
+    // 128 columns 1.04 (0.99-1.09) of the tile's time where it would need a second round (w 2 to 4; 512x1280 N 385 6.1 -> 6.6), level up to 128 columns.  (A single K block leaves
+    // all wavefronts but one idle; four of them stay with the tiles of four K wavefronts, which take them in one chunk: 0.74 here.)
     const size_t columns = (N + 15) / 16, wgs = tiles * columns, some = (size_t)cus;
     if (splitK == 1 && K <= kLittleK && units > 1 && units != 4 && wgs <= (units < 4 ? 8 : 6) * some) {
         if (units < 4) return LaunchCfg{ 0, 1, wgs < 3 * some ? 1 : 2, 1, 4 };
-        return LaunchCfg{ 0, 1, wgs <= some ? 1 : wgs > 2 * some && (tiles + 2) / 3 * columns <= some ? 3 : 2, 1, wgs <= 4 * some ? 8 : 4 };
+        const bool three = wgs > 2 * some && (tiles + 2) / 3 * columns <= some, one_to_a_cu = xbits == 5 && wgs <= 4 * some;
+        if (wgs <= 2 * some || three || !one_to_a_cu || N <= 128) return LaunchCfg{ 0, 1, wgs <= some ? 1 : three ? 3 : 2, 1, wgs <= 4 * some ? 8 : 4 };
     }
     c.kind = 1;
     const TileShape *t = nullptr;

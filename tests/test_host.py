@@ -1099,3 +1099,18 @@ def test_which_tiles_of_gemm_span_choose_a_split(E, M, OC, IC, N, split, shape):
     got = (ctypes.c_int * 5)()
     assert fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M) == split
     assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, split, 0, got) == 0 and tuple(got) == shape
+
+
+@pytest.mark.parametrize("E,M,OC,IC,N,shape", [
+    # 5 bits: beyond 128 columns no second round of two row tiles on eight wavefronts; three tiles where they fill one, four wavefronts beyond four outputs' tiles a CU, other formats as before
+    (2, 2, 512, 1280, 256, (0, 1, 2, 1, 8)), (2, 2, 512, 1280, 257, (0, 1, 3, 1, 8)), (2, 2, 512, 1280, 385, (1, 2, 1, 4, 4)), (3, 2, 512, 1280, 385, (0, 1, 2, 1, 8)), (2, 1, 512, 1280, 385, (0, 1, 2, 1, 8)),
+    (2, 2, 1280, 1152, 144, (0, 1, 3, 1, 8)), (2, 2, 1280, 1152, 145, (1, 2, 1, 4, 4)), (2, 2, 2048, 1280, 128, (0, 1, 2, 1, 8)), (2, 2, 2048, 1280, 129, (0, 1, 2, 1, 4)), (2, 2, 2560, 1216, 78, (0, 1, 2, 1, 8)),
+    # K 1344 is the rules' whatever M and N are, K 1408 is in the table's reach
+    (3, 2, 1280, 1344, 200, (0, 1, 2, 1, 4)), (3, 2, 28672, 1344, 17, (1, 2, 2, 4, 2)), (3, 2, 1280, 1408, 200, None), (3, 2, 4096, 1408, 24, None)])
+def test_little_k_by_format_and_where_the_table_begins(E, M, OC, IC, N, shape):
+    got = (ctypes.c_int * 5)()
+    source = _lib.lib().fp6mi_query_table(E, M, OC, N, IC, 1, got)
+    if shape:
+        assert source == 2 and tuple(got) == shape and fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M) == 1
+    else:
+        assert source == 1
