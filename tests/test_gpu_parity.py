@@ -393,6 +393,27 @@ def test_stream_kernel_over_many_column_blocks_of_little_k(E, M, OC, IC, N, grou
     check_close(y.cpu().numpy(), ref, "little K")
 
 
+@pytest.mark.parametrize("E,M", FORMATS)
+@pytest.mark.parametrize("groups", [False, True])
+def test_stream_kernel_over_column_blocks_with_a_short_last_workgroup(E, M, groups):
+    """80 row tiles in workgroups of three, of which the last holds two, over nine column blocks with 1 to 16 columns in the last, five and a half K blocks."""
+    OC, IC, L = 1280, 1344, _lib.lib()
+    codes, sc, ex = quant.quantize_groupwise(_grouped_weights(E + 8 * M, OC, IC), E, M)
+    raw = quant.pack_raw(codes, E, M)
+    dense = oracle.dequant_grouped_from_definition(codes, sc, ex, E, M) if groups else oracle.dequant(raw, sc, E, M)
+    gexp = fp6.pack_group_exps(torch.from_numpy(ex), OC, IC).to(DEV) if groups else None
+    for N in (129, 144):
+        shape = (ctypes.c_int * 5)()
+        assert L.fp6mi_query_kernel(E, M, OC, N, IC, 1, groups, shape) == 0 and tuple(shape) == (0, 1, 3, 1, 8) and OC // 16 % 3 == 2
+        print("case short last workgroup", E, M, groups, N, flush=True)
+        x = synth.activations(N, N, IC)
+        native, scd, xd = upload(raw, sc, x, E, M)
+        out = torch.full((N + 1, OC), float("nan"), dtype=torch.float16, device=DEV)
+        y = fp6.linear_forward_native(E, M, xd, native, scd, OC, 1, out=out[:N], group_exps=gexp)
+        assert torch.isnan(out[N]).all()
+        check_close(y.cpu().numpy(), oracle.gemm_f64(dense, x), "N=%d" % N)
+
+
 def test_unsupported_launch_shape_is_rejected():
     raw, sc, x = synth.uniform_problem(1, 256, 256, 4)
     native, scd, xd = upload(raw, sc, x, 3, 2)
@@ -1198,6 +1219,17 @@ def test_bias_in_the_epilogues(E, M, OC, IC, BS, splitK, shape, groups):
         run(bias[:-1])
     with pytest.raises(ValueError):
         run(bias.float())
+
+
+@pytest.mark.parametrize("E,M,OC,IC,BS,splitK,shape", [
+    (2, 1, 768, 1728, 549, 1, (2, 3, 2, 4, 2)), (3, 2, 1792, 1088, 1157, 1, (2, 5, 2, 4, 2)), (2, 3, 8192, 1088, 397, 1, (2, 7, 2, 4, 2)), (2, 2, 22016, 1152, 130, 1, (2, 5, 4, 4, 2)),
+    (2, 2, 17408, 1600, 243, 1, (2, 6, 4, 4, 2)), (2, 1, 5120, 1088, 1157, 1, (2, 7, 4, 4, 2)),
+    (2, 2, 1280, 1920, 146, 3, (2, 3, 2, 4, 2)), (2, 3, 4096, 2432, 313, 2, (2, 5, 2, 4, 2)), (2, 2, 8448, 4992, 97, 2, (2, 7, 2, 4, 2)), (2, 2, 11264, 2624, 142, 2, (2, 5, 4, 4, 2)),
+    (3, 2, 768, 5952, 1429, 4, (2, 6, 4, 4, 2)), (2, 1, 12032, 7616, 100, 3, (2, 7, 4, 4, 2))])
+@pytest.mark.parametrize("groups", [False, True])
+def test_bias_in_the_epilogues_of_gemm_span(E, M, OC, IC, BS, splitK, shape, groups):
+    """As for the other kernels, for each of gemm_span's tiles, unsplit and in pieces: the two halves of K hold different numbers of columns of an odd width."""
+    test_bias_in_the_epilogues(E, M, OC, IC, BS, splitK, shape, groups)
 
 
 def test_module_prefill_route_dequantizes_and_matches():

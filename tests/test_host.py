@@ -1114,3 +1114,56 @@ def test_little_k_by_format_and_where_the_table_begins(E, M, OC, IC, N, shape):
         assert source == 2 and tuple(got) == shape and fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M) == 1
     else:
         assert source == 1
+
+
+def test_a_module_finds_buffers_parameters_and_submodules():
+    """FPxLinear looks for a buffer before nn.Module does, and finds and refuses what nn.Module does: with and without a bias, before __init__, copied, pickled, with its buffers
+    replaced or taken out, and as a subclass with parameters and modules of its own."""
+    import copy
+    import pickle
+
+    from fp6_llm_amd import module
+
+    class Wrapped(module.FPxLinear):
+        def __init__(self):
+            super().__init__(64, 256, bias=torch.ones(256, dtype=torch.float16))
+            self.gain = torch.nn.Parameter(torch.ones(3))
+            self.inner = torch.nn.Linear(2, 2)
+
+        @property
+        def broken(self):
+            raise AttributeError("broken has no value")
+
+    plain, wrapped = module.FPxLinear(64, 256), Wrapped()
+    assert plain.bias is None and plain.group_exps is None and wrapped.bias is wrapped._buffers["bias"] and wrapped.gain is wrapped._parameters["gain"] and wrapped.inner is wrapped._modules["inner"]
+    for m in (plain, wrapped):
+        assert m.scales is m._buffers["scales"] and m.weight_native is m._buffers["weight_native"]
+        for name in ("nothing", "_buffer", "weight"):
+            with pytest.raises(AttributeError, match=name):
+                getattr(m, name)
+            assert not hasattr(m, name)
+    with pytest.raises(AttributeError):
+        wrapped.broken
+    bare = module.FPxLinear.__new__(module.FPxLinear)   # before nn.Module has made its dictionaries
+    for name in ("_buffers", "scales", "training_steps"):
+        with pytest.raises(AttributeError):
+            getattr(bare, name)
+    for other in (copy.deepcopy(plain), copy.copy(plain), pickle.loads(pickle.dumps(plain))):
+        assert torch.equal(other.scales, plain.scales) and other.bias is None and list(other.state_dict()) == list(plain.state_dict())
+    plain.scales = torch.full_like(plain.scales, 2.0)
+    assert plain.scales is plain._buffers["scales"] and (plain.scales == 2).all()
+    swapped = torch.zeros_like(plain.scales)
+    got = torch.func.functional_call(_Reads(plain), {"layer.scales": swapped}, ())
+    assert got is swapped and plain.scales is not swapped
+    del plain.scales
+    with pytest.raises(AttributeError, match="scales"):
+        plain.scales
+
+
+class _Reads(torch.nn.Module):
+    def __init__(self, layer):
+        super().__init__()
+        self.layer = layer
+
+    def forward(self):
+        return self.layer.scales
