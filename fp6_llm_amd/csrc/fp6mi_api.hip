@@ -167,7 +167,7 @@ inline bool cfg_fits(const TuneCfg &c, size_t M) { return c.kind != 255 && (c.ki
 // 16384 and 17920 rows differ by 9 % in size but by a whole round of 64-row workgroups; sweeps off the grid showed that
 // this, not the distance, decides which neighbour's shape is right.  Farther neighbours pay 15 % per octave of distance.
 struct TuneGroup { int xb; size_t n, begin, end; }; // entries [begin, end) of kTune share format and batch (the table is sorted by them)
-struct TuneAnswer { bool valid, measured, exact; size_t n; LaunchCfg cfg[kNumSplits]; float t[kNumSplits]; }; // index i: splitK = kSplits[i]; t in 0.02 us, 0 = no proposal; measured: this very (M, K) at this or the next larger measured batch; exact: at this batch; n: the measured batch that answers
+struct TuneAnswer { bool valid, measured, exact; size_t n; LaunchCfg cfg[kNumSplits]; float t[kNumSplits], by_k[kNumSplits]; }; // index i: splitK = kSplits[i]; t in 0.02 us, 0 = no proposal; by_k: t in proportion to K as a whole; measured: this very (M, K) at this or the next larger measured batch; exact: at this batch; n: the measured batch that answers
 
 const std::vector<TuneGroup> &tune_groups()
 {
@@ -199,10 +199,13 @@ inline double rounds_on_chip(const TuneCfg &c, size_t M, size_t N, int splitK)
 // are not.  In proportion to K as a whole, a split's time shrank with the part that does not, and matrices of little K were cut that none of their
 // neighbours gains by: FP4 1280x2304 N 113 in eight (8.5 us, 5.5 unsplit), FP6 2048x3456 N 231 in four (11.0, 8.8), FP5 1536x1408 N 47 in three (5.9, 4.1).
 // Time of the choice / time of the best proposal on 324 matrices off the table, every proposal measured: N 33-80 1.07 before, 1.02 now, N 81-160 1.02 and
-// 1.01, N 161-320 1.03 and 1.02.  Up to 16 columns, and 17 to 32 with K up to 3072 or M up to 2560, 81 of 600 drawn choices change by it, to 0.88 of the time in a graph
-// (0.52-1.11) and 0.80 in a stream, where a second launch costs the host 2.6 us (e3m2 2304x2176 N 13 in three 5.8 and 10.8 us, uncut 4.2 and 4.4; 2560x2688 N 5 in three 5.5 and 9.1,
-// uncut 3.8 and 4.7).  Left as they were: the other 17 to 32 columns (1.04-1.22 on ten problems whose tiles in six or eight gave way to the stream kernel uncut), and beyond 320,
-// where the few splits measured are for long K (11520x12800 N 456: 152 us in two pieces, 172 uncut).
+// 1.01, N 161-320 1.03 and 1.02.  So it is up to 16 columns, and 17 to 32 with K up to 3072 or M up to 2560.  Time / time by proportion of what changes by it: an uncut launch in the place
+// of a cut one, which in a stream saves the host 2.6 us besides, 0.87 in a graph (0.56-1.16) and 0.78 in a stream (0.64-1.05) on 891 problems up to 16 columns, 0.85 (0.61-1.17) and
+// 0.82 (0.65-1.14) on 343 beyond (e3m2 2304x2176 N 13 in three 5.8 and 10.8 us, uncut 4.2 and 4.4; 2560x2688 N 5 in three 5.5 and 9.1, uncut 3.8 and 4.7); a graph alone is the slower by it
+// where few rows meet a long K (M up to 1536 and K from 9216 1.05 and 0.85 in a stream: e2m1 1536x12480 N 3 in four 6.3 and 7.9, uncut 7.4 and 7.4).  Another cut is 0.99 and 1.00 on 216
+// up to 16 columns, one of them 1.12.  From 17 on the stream kernel in three or four pieces, which the times above prefer to the tile kernel in six or eight, is behind it: 1.09 (0.94-1.27) on 62
+// problems (e2m2 2048x14144 N 21 12.1 us, in eight 10.0), so that best_narrow leaves those as proportion has them.  Left as they were: the other 17 to 32 columns (1.04-1.22 on ten problems
+// whose tiles in six or eight gave way to the stream kernel uncut), and beyond 320, where the few splits measured are for long K (11520x12800 N 456: 152 us in two pieces, 172 uncut).
 inline double fixed_part(size_t M, size_t N, int splitK)
 {
     return splitK == 1 ? 100.0 : 200.0 + (double)splitK * M * N * 8.0 / 8e6 / 0.02;
@@ -243,7 +246,6 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
     a.n = group ? group->n : 0;
     if (count > 0 && dist[0] == 0.f) count = 1, a.measured = true, a.exact = group->n == N; // measured: nothing to carry over
     const size_t units = (K + 255) / 256;
-    float        of_shape[kNumSplits] = {}; // what the shapes of a split are compared by
     for (int j = 0; j < count; j++) {
         const TuneEntry &e = *near[j];
         const size_t     Me = (size_t)e.m256 * 256, Ke = (size_t)e.k64 * 64, Nq = N > group->n ? N : group->n;
@@ -253,8 +255,8 @@ const TuneAnswer *tune_lookup(int xbits, size_t M, size_t N, size_t K)
             const double rounds = rounds_on_chip(c, M, Nq, kSplits[i]) / rounds_on_chip(c, Me, group->n, kSplits[i]);
             double       t = (double)c.t * (double)K / (double)Ke * (1.0 + 0.15 * dist[j]);
             t *= rounds;
-            if (a.t[i] == 0.f || (float)t < of_shape[i]) {
-                of_shape[i] = a.t[i] = (float)t;
+            if (a.t[i] == 0.f || (float)t < a.by_k[i]) { // (the shapes of one split are compared in proportion)
+                a.by_k[i] = a.t[i] = (float)t;
                 a.cfg[i] = LaunchCfg{ c.kind, c.nt, c.rt, c.wr, c.wk };
                 a.valid = true;
                 if (!a.measured && N <= 320 && (N <= 16 || N > 32 || K <= 3072 || M <= 2560)) {
@@ -513,7 +515,8 @@ inline bool wide_replaces(const LaunchCfg &wide, float t, float narrow, size_t M
     return t < narrow * (N <= 400 || wide.nt <= 5 && wide.rt == 2 ? 0.9f : N <= 640 ? 0.95f : 1.15f);
 }
 
-// The fastest split of the table's (3 % hysteresis towards fewer pieces; 10 % towards a single launch that takes less than 8 us, which two take of the host alone) and its time
+// The fastest split of the table's (3 % hysteresis towards fewer pieces; 10 % towards a single launch against pieces expected to take less than 8 us, since two launches take
+// that of the host alone) and its time
 // in us; 0 where it holds none.  One that takes more than ws_bytes has to be
 // the faster by the table's times as they stand too, which were what decided before narrow_estimate.
 inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N, size_t ws_bytes)
@@ -525,6 +528,13 @@ inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N, si
             if (split && fp6mi_workspace_bytes(M, N, s) > ws_bytes && a->t[split_index(s)] * 1.03f >= a->t[split_index(split)]) continue;
             split = s, best = t;
         }
+    if (N > 16 && N <= 32 && split > 1 && a->cfg[split_index(split)].kind == 0) { // a tile kernel in more pieces where proportion says so: see fixed_part
+        int   cut = 0;
+        float least = 0.f;
+        for (int i = 0; i < kNumSplits; i++)
+            if (const float t = a->by_k[i]; t > 0.f && (cut == 0 || t * 1.03f < least)) cut = i, least = t;
+        if (cut && a->cfg[cut].kind != 0) split = kSplits[cut], best = a->t[cut] * 0.02f;
+    }
     return best;
 }
 // The launch shape of a call: gemm_wide's, or that of the table and the rules.  A split that the table does not hold for a problem it does hold (in other

@@ -1167,3 +1167,13 @@ class _Reads(torch.nn.Module):
 
     def forward(self):
         return self.layer.scales
+
+
+@pytest.mark.parametrize("E,M,OC,IC,N,split,shape", [
+    (2, 2, 2048, 14144, 21, 8, (1, 2, 1, 4, 4)), (3, 2, 2304, 7360, 18, 6, (1, 2, 1, 4, 4)), (3, 2, 2304, 6784, 24, 6, (1, 2, 1, 4, 4)), (2, 1, 2048, 19264, 25, 8, (1, 2, 1, 4, 4)),
+    (2, 2, 2048, 14144, 16, 4, (0, 1, 2, 1, 8)), (2, 2, 2048, 2176, 21, 1, (0, 1, 1, 1, 4))])   # up to 16 columns, and uncut, it is the stream kernel's
+def test_a_cut_stream_kernel_does_not_replace_a_cut_tile_kernel(E, M, OC, IC, N, split, shape):
+    """17 to 32 columns, matrices off the table: measured, us, in three or four pieces of the stream kernel and here, 12.1 and 10.0, 10.3 and 9.0, 10.7 and 9.2."""
+    got = (ctypes.c_int * 5)()
+    assert fp6.heuristic_splitk_mi355x(OC, N, IC, EXPONENT=E, MANTISSA=M) == split
+    assert _lib.lib().fp6mi_query_kernel(E, M, OC, N, IC, split, 0, got) == 0 and tuple(got) == shape
