@@ -532,7 +532,7 @@ inline float best_narrow(int &split, const TuneAnswer *a, size_t M, size_t N, si
         int   cut = 0;
         float least = 0.f;
         for (int i = 0; i < kNumSplits; i++)
-            if (const float t = a->by_k[i]; t > 0.f && (cut == 0 || t * 1.03f < least)) cut = i, least = t;
+            if (const float t = a->by_k[i]; t > 0.f && (least == 0.f || t * 1.03f < least)) cut = i, least = t;
         if (cut && a->cfg[cut].kind != 0) split = kSplits[cut], best = a->t[cut] * 0.02f;
     }
     return best;
