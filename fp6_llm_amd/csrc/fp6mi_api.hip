@@ -622,7 +622,7 @@ const char *fp6mi_tuning_info(void)
         ;
 }
 
-int fp6mi_version(void) { return 141; } // 141: gemm_span (odd column tiles of the wide kernel), little K on the stream kernel, splits of small batches off the table, dequantizer and quantizer kernels; 140: where gemm_wide is taken and with which splits, instances of gemm_tile for a bias, the quantizer chooses its arithmetic before a block; 139: a bias in the epilogues of the GEMM kernels, the quantizer's arithmetic; 138: gemm_wide (launch kind 2 with four rows of one or two wavefronts) in the place of larger tiles from 97 columns on, the other kernels unchanged; 137: group exponents of 128 rows through LDS in the wave-specialized kernel, panels of 256-row tiles only for activations beyond L2; 136: tiles of 48, 80 and 96 columns, deeper rings in the wave-specialized kernel of 128 rows, panels; 135: prefill kernel (launch kind 2 with 2 x 2 wavefronts), relayout and quantizer kernels rewritten, the other GEMM kernels unchanged; 134: three row tiles per workgroup in the small-batch kernel (any M: the last workgroup takes what is left), no other kernel changed; 133: wave-specialized tile kernel (launch kind 2) for large batches; 132: split-K reduction runs on the XCD that wrote the partial sums, every grid size gets XCD-contiguous tiles; 131: tile kernel stores through LDS; 130: small-batch kernel loads activations as whole rows and turns them into operand order through LDS
+int fp6mi_version(void) { return 142; } // 142: where gemm_span, little K and the stream kernel in pieces are taken, the dequantizer's stores; 141: gemm_span (odd column tiles of the wide kernel), little K on the stream kernel, splits of small batches off the table, dequantizer and quantizer kernels; 140: where gemm_wide is taken and with which splits, instances of gemm_tile for a bias, the quantizer chooses its arithmetic before a block; 139: a bias in the epilogues of the GEMM kernels, the quantizer's arithmetic; 138: gemm_wide (launch kind 2 with four rows of one or two wavefronts) in the place of larger tiles from 97 columns on, the other kernels unchanged; 137: group exponents of 128 rows through LDS in the wave-specialized kernel, panels of 256-row tiles only for activations beyond L2; 136: tiles of 48, 80 and 96 columns, deeper rings in the wave-specialized kernel of 128 rows, panels; 135: prefill kernel (launch kind 2 with 2 x 2 wavefronts), relayout and quantizer kernels rewritten, the other GEMM kernels unchanged; 134: three row tiles per workgroup in the small-batch kernel (any M: the last workgroup takes what is left), no other kernel changed; 133: wave-specialized tile kernel (launch kind 2) for large batches; 132: split-K reduction runs on the XCD that wrote the partial sums, every grid size gets XCD-contiguous tiles; 131: tile kernel stores through LDS; 130: small-batch kernel loads activations as whole rows and turns them into operand order through LDS
 
 int fp6mi_prepack_ref(int E, int Mb, void *packed, const void *raw, size_t M, size_t K) { return fp6mi::prepack_ref(E, Mb, packed, raw, M, K); }
 int fp6mi_unpack_ref(int E, int Mb, void *raw, const void *packed, size_t M, size_t K) { return fp6mi::unpack_ref(E, Mb, raw, packed, M, K); }
