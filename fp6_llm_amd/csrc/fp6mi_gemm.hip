@@ -1248,9 +1248,10 @@ __global__ __launch_bounds__(4 * WK *kWave, RT *NT <= 8 ? 4 : 2) void gemm_wide(
 // gemm_span: the same organisation with the tile widths between gemm_wide's: 128 x 48, 128 x 80, 128 x 112, 256 x 80 and 256 x 112, and 256 x 96 with the halves of K
 // side by side, all of eight wavefronts.  What bounds a GEMM of some hundred columns is the same as there, and on top of it what the tile grid adds: columns that no tile
 // is full of (777 columns are 7 tiles of 128 or of 112), a last round of few workgroups, and CUs with a single workgroup of four wavefronts.  A half step holds (NT + 1) / 2
-// column tiles, the other one NT / 2.  Measured, us, the best there was -> here: e2m2 with group exponents 4608x4544 N 777 35.2 -> 32.3 (128 x 112), e2m1 20736x4992 N 142
-// 41.5 -> 35.6 (128 x 48), e2m2 3584x3200 N 1293 36.5 -> 31.7 and e3m2 17408x7168 N 196 72.0 -> 64.0 (256 x 80), 8192x4992 N 445 39.3 -> 35.5 (128 x 112), e2m2 4864x5632
-// N 1067 60.6 -> 54.8 (256 x 96).  Left out: 256 x 48, 256 x 64, 256 x 80 and 256 x 112 of four wavefronts and 256 x 48, 256 x 64 of eight (0.4 % over all problems
+// column tiles, the other one NT / 2.  Measured, us, what is launched without it -> here: e2m2 with group exponents 4608x4544 N 777 34.0 -> 31.3 (128 x 112), e2m1 20736x4992 N 142
+// 39.9 -> 33.6 (128 x 48), e2m2 3584x3200 N 1293 37.2 -> 31.2 and e3m2 17408x7168 N 196 70.7 -> 62.8 (256 x 80), 8192x4992 N 445 40.8 -> 39.4 (128 x 112), e2m2 4864x5632
+// N 1067 60.3 -> 53.8 (256 x 96).  256 x 112 takes all 256 registers with 6-bit weights and spills one, with group exponents eleven: written once a launch, of which one, four or seven
+// are read back every two K blocks, between a barrier and the chunk's transfers (no counted wait sees them).  Left out: 256 x 48, 256 x 64, 256 x 80 and 256 x 112 of four wavefronts and 256 x 48, 256 x 64 of eight (0.4 % over all problems
 // measured), and the same tiles for 33 to 96 columns (88 problems, the best of them with what there is: 0.990).
 template <int FM, bool GS, int NT, int RT, int WK>
 __global__ __launch_bounds__(4 * WK *kWave, RT == 2 && NT <= 4 ? 4 : 2) void gemm_span(const uint8_t *W, const half_t *__restrict__ scales, const uint8_t *gexp, const half_t *X,
@@ -1428,32 +1429,33 @@ __global__ __launch_bounds__(256) void relayout_ref_to_native(uint8_t *__restric
 // sign handling made that 10 operations a weight (17 us of 46 at 8192x8192); they are left to the wavefronts that have met an Inf, a NaN or a
 // scale that is no normal number, the others take 5 (quantize_string's PLAIN).  us, e3m2, before -> now, row scales and group exponents: bf16 8192x8192
 // 45.9 -> 41.9, 49.6 -> 44.0; 3072x8192 23.5 -> 18.9, 26.1 -> 20.7; 28672x8192 141 -> 136, 142 -> 137; 8192x28672 176 -> 165, 183 -> 176; fp16 8192x8192
-// 47.1 -> 43.1, 51.6 -> 45.2; fp32 8192x8192 95.2 -> 87.6, 98.7 -> 91.9.
+// 47.1 -> 43.1, 51.6 -> 45.2; fp32 8192x8192, then with two blocks kept, 95.2 -> 87.6, 98.7 -> 91.9 (another card than below).
 //
 // Two organisations of the same arithmetic.  quant_fused: one workgroup of eight wavefronts per 16-row tile reads
 // its rows, finds the scales, and converts; the last two blocks of every wavefront (three of 32-bit weights) are still in its registers then, with 16-bit
 // weights the one before them in LDS, and the others are read again, latest first (8192x8192: a quarter of the weights twice).
 // quant_row_scales + quant_blocks: a workgroup takes a row, then a wavefront a block, and all weights are read twice.
-// Measured, us, e3m2, fused / two kernels (replayed from a graph, through more memory than the caches hold):
+// Measured, us, e3m2, fused / two kernels (replayed from a graph, through more memory than the caches hold; the fp32 columns, both sides of them, on another card than the bf16 ones):
 //               bf16            bf16 groups     fp32            fp32 groups
-//   1024x3072     6.4 /   7.9     7.4 /   8.2     9.9 /  10.1    10.8 /  10.4
-//   1024x4096     7.6 /   8.3     9.2 /   8.6    11.4 /  11.1    12.5 /  11.5
-//   1536x4096     8.0 /   9.9     9.6 /  10.4    12.9 /  13.9    14.1 /  14.2
-//   2048x4096     8.9 /  11.0    10.2 /  11.5    14.3 /  16.5    15.5 /  16.9
-//   2048x6144    12.3 /  13.5    13.9 /  14.1    17.7 /  22.3    19.6 /  23.0
-//   2048x8192    15.6 /  16.2    18.9 /  16.6    26.9 /  26.9    29.6 /  27.7
-//   2560x8192    16.8 /  19.3    19.6 /  19.7    28.3 /  33.4    30.9 /  33.7
-//   2816x16384   36.0 /  37.3    40.0 /  37.9    61.9 /  68.7    64.1 /  68.6
-//   4096x8192    23.1 /  28.7    24.8 /  29.5    41.2 /  50.1    43.0 /  50.6
-//   8192x8192    42.9 /  52.7    45.0 /  52.7    87.1 /  95.2    86.6 /  94.6
-//   4096x28672   85.8 /  89.4    89.9 /  89.6   158 / 180       158 / 180
-//  16384x4096    37.2 /  53.6    38.8 /  53.7    72.2 /  93.6    76.1 /  93.8
+//   1024x3072     6.4 /   7.9     7.4 /   8.2     8.5 /  10.2     9.7 /  10.4
+//   1024x4096     7.6 /   8.3     9.2 /   8.6    10.6 /  11.2    11.7 /  11.4
+//   1536x4096     8.0 /   9.9     9.6 /  10.4    12.8 /  14.1    14.0 /  14.3
+//   2048x4096     8.9 /  11.0    10.2 /  11.5    14.7 /  17.0    15.7 /  17.1
+//   2048x6144    12.3 /  13.5    13.9 /  14.1    19.2 /  22.5    19.8 /  22.6
+//   2048x8192    15.6 /  16.2    18.9 /  16.6    25.7 /  26.9    27.5 /  27.3
+//   2560x8192    16.8 /  19.3    19.6 /  19.7    28.8 /  33.1    31.2 /  33.1
+//   2816x16384   36.0 /  37.3    40.0 /  37.9    61.7 /  68.1    64.0 /  66.1
+//   4096x8192    23.1 /  28.7    24.8 /  29.5    43.8 /  49.9    45.3 /  48.3
+//   8192x8192    42.9 /  52.7    45.0 /  52.7    85.3 /  93.7    87.5 /  90.1
+//   4096x28672   85.8 /  89.4    89.9 /  89.6   158 / 174       157 / 173
+//  16384x4096    37.2 /  53.6    38.8 /  53.7    71.4 /  93.5    75.8 /  91.6
 // Few workgroups do not pull enough from memory to pay for a second pass over a long row: fused from 160 tiles on, and below that up to K = 3072 or three
-// times the rows.  On the wrong side of that line bf16 of 1024x4096 (9 %) and 2048x8192 (4 %), group exponents of 2816x16384 (6 %) and, in fp32 with them, 1024x3072 (4 %).
+// times the rows.  On the wrong side of that line bf16 of 1024x4096 (9 %) and 2048x8192 (4 %), 16-bit weights with group exponents of 2816x16384 (6 %) and fp32 of 1024x4096 (6 %) and 2048x8192 (5 %).
 // (16-bit weights: a block of every wavefront in LDS and two in registers leave room for two workgroups to a CU.  Three in registers and one in LDS, nothing
 // read twice at 8192 columns, were slower with one workgroup to a CU, and held to 128 registers they spill.
-// 32-bit weights, of which two blocks take 202 registers: a CU holds one workgroup either way, so a third block takes the other 54.  us, e3m2, two blocks -> three:
-// 4096x6144 29.5 -> 25.1, 14336x6144 99.6 -> 87.7, 8192x8192 91.1 -> 83.1, 8192x11008 113 -> 106, 8192x28672 323 -> 313; up to 4096 columns, where no
+// 32-bit weights, of which two blocks take 202 registers: a CU holds one workgroup either way, so a third block, 64 registers, takes the other 54 and spills eight, which are
+// written once and read back once a row tile, around the search for its maxima (36 bytes of scratch a lane; the loops over blocks touch none).  us, e3m2, two blocks -> three:
+// 4096x6144 29.8 -> 25.2, 14336x6144 99.8 -> 88.6, 8192x8192 95.6 -> 85.3, 8192x11008 114 -> 108, 8192x28672 316 -> 306; up to 4096 columns, where no
 // wavefront has a third, within 1 %.  A block of 16 KB in LDS beside two gives the same, beside three it costs 10 % but at 8192 columns.)
 // A conversion in double precision, code by code through a byte array in scratch memory, took 532 us at 8192x8192.
 // ---------------------------------------------------------------------------------------------------------------
