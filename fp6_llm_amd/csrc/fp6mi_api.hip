@@ -442,18 +442,22 @@ inline float wide_estimate(const WideShape &w, int xbits, size_t M, size_t N, si
 // The rows of the 128-row tiles, fitted to K of some thousand, expect too little of a long K: measured / expected on 1900 problems 1.02 up to K 4096 and 1.12 beyond for 128 x 80, 1.02 and
 // 1.11 for 128 x 112, 1.05 and 1.13-1.19 (K of a piece from 8192 on) for 128 x 48; gemm_wide's tiles and the 256-row ones 0.99-1.05.  Against gemm_wide at the same split they hold all the same
 // (128 x 80: 0.95 of its time on 213 problems, none above 1.00; 128 x 48 0.98), but not everywhere, and not across splits.  Time / time of what is launched instead:
-//   * 128 x 112 uncut beyond N 1400: 1.02 of 128 x 128 (138 problems; 0.965 up to there); with a last round below seven eighths and K from 8192: 1.09 (1.05-1.13) of 128 x 96;
-//   * 256 x 80 uncut, more columns than rows, K from 4096: 1.09 (1.03-1.15) of 128 x 128 on 33 of 60 problems, which a margin of 8 % finds;
-//   * uncut tiles of 128 rows in the place of a cut one: 1.06 (0.94-1.22) of gemm_wide's, 1.08-1.12 of a 256-row one; uncut 256 x 80 beyond K 20480: 1.025.  They leave the choice of a split to the others;
+//   * 128 x 112 uncut without group exponents, beyond N 1400: 1.03 of 128 x 128 (109 problems; 0.965 up to there); with a last round below seven eighths and K from 8192: 1.09 (1.07-1.14) of
+//     128 x 96, and 1.06 of the table's shapes.  With group exponents it holds against all (0.87-0.99 on 372 problems) but 128 x 96, K from 8192: 1.08-1.11 where their rows are within 15 %;
+//   * 256 x 80 uncut, more columns than rows, K from 4096: 1.09 (1.03-1.15) of 128 x 128 on 33 of 60 problems, which a margin of 8 % finds; it is ahead of the other span tiles all
+//     the same (0.94 of 256 x 96, 0.91-0.96, on 103 problems);
+//   * uncut tiles of 128 rows in the place of a cut one: 1.06 (0.94-1.22) of gemm_wide's, 1.08-1.12 of a 256-row one; 128 x 112 in pieces 1.02, uncut 256 x 80 beyond K 20480
+//     1.025.  They leave the choice of a split to the others;
 //   * 128 x 48 in the place of the table's shape, K of a piece from 4096 and a single round of up to 256 workgroups: 1.09 (0.86-1.32).  wide_replaces allows for it.
-// All of it together, against the choice without gemm_span: 600 problems of N 97-4096 that it changes 0.93, 8 above 1.03 (the largest 1.05); 450 unsplit 0.92, 8 (1.08); 450 of a given split 0.93, 7 (1.11).
-// Without these lines, on as many, 0.94 with 53 above 1.03 (1.23), 0.92 with 23 (1.30: e2m3 1536x16448 N 2161 122 -> 159 us) and 0.93 with 11 (1.08).
-inline float span_margin(const WideShape &w, size_t M, size_t N, size_t K, int splitK)
+// All of it together, against the choice without gemm_span: 1200 problems of N 97-4096 that it changes 0.93, 24 above 1.03 (up to 1.10, one 1.25: e3m2 15616x6656 N 132 with group
+// exponents); 900 unsplit 0.91, 14 (1.10); 900 of a given split 0.93, 17 (1.11).
+// Without these lines, on half as many, 0.94 with 53 above 1.03 (1.23), 0.92 with 23 (1.30: e2m3 1536x16448 N 2161 122 -> 159 us) and 0.93 with 11 (1.08).
+inline float span_margin(const WideShape &w, size_t M, size_t N, size_t K, int splitK, bool groups)
 {
     const bool   span112 = w.rt == 2 && w.nt == 7;
     const size_t last = M / (64u * w.rt) * ((N + 16 * w.nt - 1) / (16 * w.nt)) * splitK % w.slots; // workgroups of the last round, 0 for a full one
-    if (K < 1024 || N > (w.nt == 3 ? 600 : span112 && splitK == 1 ? 1400 : 3072)) return 0.f;
-    if (span112 && splitK == 1 && K >= 8192 && last && 8 * last < 7 * (size_t)w.slots) return 0.f;
+    if (K < 1024 || N > (w.nt == 3 ? 600 : span112 && splitK == 1 && !groups ? 1400 : 3072)) return 0.f;
+    if (span112 && splitK == 1 && !groups && K >= 8192 && last && 8 * last < 7 * (size_t)w.slots) return 0.f;
     if (w.nt == 5 && w.rt == 4 && splitK == 1 && N > M && K >= 4096) return 1.08f;
     return (splitK > 1 || K < 1536 ? 1.04f : 1.025f) + ((splitK > 1 || span112) && (last == 0 || 4 * last >= 3 * (size_t)w.slots) ? 0.03f : 0.f);
 }
@@ -469,17 +473,20 @@ inline bool span_asked(const WideShape &w, Spans spans, size_t K, int splitK)
 // the fastest of the shapes for a given split, and its time in us; 0 where none fits
 inline float wide_best(LaunchCfg &c, int xbits, size_t M, size_t N, size_t K, int splitK, bool groups, Spans spans)
 {
-    float best = 0.f;
+    float best = 0.f, t96 = 0.f, t80 = 0.f; // t96: of gemm_wide's 128 x 96; t80: of 256 x 80, where it is held to more against gemm_wide
     if (N <= 96 || K > (size_t)1 << 20 || (size_t)splitK > (K + 255) / 256) return best;
     for (const WideShape &w : kWide) {
         float t = wide_estimate(w, xbits, M, N, K, splitK, groups);
+        if (w.nt == 6 && w.rt == 2) t96 = t;
         if (w.nt % 2 || (w.nt == 6 && w.rt == 4 && w.wk == 2)) { // gemm_span's
-            const float margin = span_asked(w, spans, K, splitK) ? span_margin(w, M, N, K, splitK) : 0.f;
-            if (margin == 0.f) continue;
+            const float margin = span_asked(w, spans, K, splitK) ? span_margin(w, M, N, K, splitK, groups) : 0.f;
+            if (margin == 0.f || (groups && w.nt == 7 && w.rt == 2 && splitK == 1 && K >= 8192 && t * 1.15f > t96)) continue;
+            if (margin == 1.08f) t80 = t * 1.025f;
             t *= margin;
         }
         if (best == 0.f || t < best) best = t, c = LaunchCfg{ 2, w.nt, w.rt, 4, w.wk };
     }
+    if (t80 > 0.f && t80 < best && c.rt == 4 && c.wk == 2 && c.nt < 8) c.nt = 5; // (another of gemm_span's is ahead of gemm_wide's, and this one of it)
     return best;
 }
 
